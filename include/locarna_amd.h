@@ -205,9 +205,11 @@ int lcg_batch_create(lcg_pair *const *pairs, int32_t npairs, int32_t device, lcg
  * override the defaults, and nonzero fields override both.  Results do not
  * depend on the shape (integer results bit for bit). */
 typedef struct {
-    int32_t waves;          /* fill of D: waves per workgroup, 1..16 (default 16) */
+    int32_t waves;          /* fill of D: waves per workgroup, 1..16 (default 16; 8 with fewer pairs than CUs
+                               where the band fill applies) */
     int32_t wgs_per_cu;     /* fill: workgroups per CU, 1..4, with at least as many pairs as CUs (1) */
-    int32_t wg_per_pair;    /* fill: workgroups per pair, 1..64, with fewer pairs than CUs (CUs / pairs) */
+    int32_t wg_per_pair;    /* fill: workgroups per pair, 1..64, with fewer pairs than CUs; 0: chosen per pair
+                               by its estimated work (general fill: CUs / pairs) */
     int32_t top_waves;      /* top level + traceback: waves per workgroup, 1..16 (4) */
     int32_t top_wgs_per_cu; /* top level + traceback: workgroups per CU, 1..4 (4) */
     int32_t pf_waves;       /* LocARNA-P: waves per workgroup, 1..8 (8) */

@@ -35,6 +35,7 @@
 
 #include <climits>
 #include <mutex>
+#include <type_traits>
 
 #include "device_layout.h"
 
@@ -106,7 +107,8 @@ struct Pair {
     const int *__restrict__ cptr;   // global
     int4 *cand;                     // global: (al|bl<<16, j, D, min_col(al-1))
     const int *fbp, *fbk;           // LDS: fill blocks of row i, (p, first entry)
-    int *fcand;                     // global: fill entries, 3 ints each
+    const int2 *__restrict__ fcand; // global: fill entries (p | q<<16, j | min_col(p-1)<<16)
+    int2 *fband;                    // global: fill entries by band cells (LCG_FBAND, D)
     const int *__restrict__ amscore;
     int *D;
     int *edges;
@@ -138,7 +140,7 @@ __device__ __forceinline__ int sig_col(const Pair &P, int j) {
 __device__ __forceinline__ int row_lo(const Pair &P, int i, int bl) { return max(bl, P.mn[i]); }
 __device__ __forceinline__ int row_hi(const Pair &P, int i, int br) { return min(br - 1, P.mx[i]); }
 
-// fill-list entry: (p | q<<16, j | min_col(p-1)<<16, D)
+// fill-list entry (fcand and the D of fband)
 struct FillEntry {
     int pq, jm, D;
 };
@@ -347,12 +349,13 @@ __device__ void group_fill_fixed(const Pair &P, int al, int bl, int ar, int br, 
             }
     };
     const FillEntry none{0, 0, 0};
-    // one unpredicated 12-byte load per lane: lanes past the row's range
-    // read its last entry (or entry 0 of the pair; a group implies arc
-    // matches), and arc_slot ignores them through its lane flag
+    // unpredicated loads: lanes past the row's range read its last entry
+    // (or entry 0 of the pair; a group implies arc matches), and arc_slot
+    // ignores them through its lane flag
     auto fetch = [&](int t, int t1) {
         const int tt = t < t1 ? t : max(t1 - 1, 0);
-        return *reinterpret_cast<const FillEntry *>(P.fcand + 3 * tt);
+        const int2 e = P.fcand[tt];
+        return FillEntry{e.x, e.y, P.fband[tt].y};
     };
     for (int c = lane; c < br - bl; c += 64) Srow[c] = LCG_NEG;
     // row al (init row): M(al, bl) = 0, M(al, j) = alpha + sum gapB
@@ -529,6 +532,416 @@ __device__ void fill_group(const Pair &P, int al, int bl, int ar, int br, int W,
         group_fill_fixed<TAB, GLOBAL, 4, 4, COUNT>(P, al, bl, ar, br, W, base, counts);
     else
         group_fill<TAB, GLOBAL, false>(P, al, bl, ar, br, W, base, true, true, nullptr, counts);
+}
+
+// ---- band fill: arc-match groups with the lanes over the columns of the
+// band row (column mn[i] + l in lane l), so that a row of w band columns takes
+// w lanes wherever the group's columns lie.  Rows of a region are stored
+// whole (cell x of the pair at M - coff[al] + x), cells left of bl near minus
+// infinity, so that a fill entry names its source cell and its column by two
+// numbers that hold for every group of the pair (LCG_FBAND) and needs no test
+// against the group: an entry costs one 8-byte load, one LDS gather, an add
+// and an LDS atomic.
+//   LPG 32: two groups of one left end in one wave (rows of at most 31
+//     columns), their regions interleaved, so that an entry is loaded and
+//     decoded once for both and one 8-byte gather serves both;
+//   LPG 64: one group, NC chunks of 64 columns.
+// An arc spans at least three positions (i - p >= 3), so the arc terms of
+// rows i .. i+3 read rows up to i-1 only: four rows are gathered together and
+// the four rows of the recursion then run on registers (M, E and the row's
+// operands, read together beforehand).  Rows al+1 .. al+3 have no arc terms;
+// they run while the entries of the next four rows are loaded, and every
+// block's entries are loaded while the block before runs.
+// Bound: a wave's instruction stream (about 450 instructions per block of
+// four rows at 4-5 cycles each, most of a row of left ends' waves idle while
+// its longest group runs) and, with many arc terms, the LDS (an atomic of 64
+// lanes on 25 columns takes 8-19 cycles by how the lanes meet, a random
+// gather 10).  The LDS holds the regions of only 7-12 waves per CU.  Against
+// the fixed-column kernel: 2016 pairs of 60-200 nt 53.5 -> 36.6 ms, 120
+// local pairs of 35-149 nt 65.9 -> 18.8 ms (with the pairs dealt by work),
+// four 500-nt pairs 61.9 -> 17.4 ms, one pair of 75 nt 2.10 -> 0.78 ms.
+// Tried and slower or equal: the rows' scalars through the scalar cache
+// (34.9 / 17.8 / 18.2 / 0.84 ms), regions of one size per row (37.3 ms for
+// the first), 128 instead of 256 entries of a row loaded ahead (37.7 ms).
+struct BandView {
+    const int2 *pc;   // LDS: (F slope prefix, symbol code) of every column
+    const int *end;   // LDS: per row i the end of the fill-list prefix p > al
+};
+
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// lane l receives lane l+1's value; lane 63 receives `last`
+__device__ __forceinline__ int wave_shift_down(int v, int last) {
+    return __builtin_amdgcn_update_dpp(last, v, 0x130, 0xf, 0xf, false);  // wave_shl:1
+}
+
+// inclusive prefix max over each LPG lanes
+template <int LPG>
+__device__ __forceinline__ int group_scan_max(int v) {
+    const int id = INT_MIN;
+    v = max(v, dpp<0x111, 0xf>(id, v));
+    v = max(v, dpp<0x112, 0xf>(id, v));
+    v = max(v, dpp<0x114, 0xf>(id, v));
+    v = max(v, dpp<0x118, 0xf>(id, v));
+    v = max(v, dpp<0x142, 0xa>(id, v));
+    if (LPG == 64) v = max(v, dpp<0x143, 0xc>(id, v));
+    return v;
+}
+
+// lambdas that must not become calls (captures in memory)
+#define LCG_INLINE __attribute__((always_inline))
+
+// Fill of the groups (al, bl0) and, with LPG 32, (al, bl1), rows up to
+// ar - 1.  Every row al .. ar - 1 has at most 31 (LPG 32), 64 or 128 columns.
+// Minus infinity: E is bounded below by LCG_NEG, which bounds s and M; cells
+// that have no finite value (left of bl, above the band) gain at most the
+// positive scores of one path, far less than 2^28, and stay below
+// LCG_NEG_LIMIT.
+// `later` is called once, after the first twelve rows (all where there are fewer).
+template <bool TAB, int LPG, int NC, class Later>
+__device__ __forceinline__ void band_fill(const Pair &P, const BandView &V, int al, int bl0, int bl1, int ar, int *base,
+                                          Later later) {
+    constexpr int G = 64 / LPG, CW = LPG * NC, SR = CW * G;
+    constexpr int PQ = NC == 1 ? 4 : 2;  // chunks of 64 entries of a row loaded a block ahead
+    const int lane = lane_id(), l = lane % LPG, g = lane / LPG;
+    const int bl = (G == 2 && g) ? bl1 : bl0;
+    const int lg = l * G + g;  // the lane's place in a row of S or M
+    const int nrows = ar - al - 1;
+    const int alpha = P.alpha, calpha = P.alpha - P.alpha_pos;
+    int *S = base;
+#pragma unroll
+    for (int k = 0; k < 4 * SR / 64; ++k) S[64 * k + lane] = LCG_NEG;
+    const int c0 = uniform(P.coff[al]);
+    int *Mo = base + 4 * SR - c0 * G;  // cell x of the pair at Mo + x * G
+    // lane r: row al+r of the current 64 rows: band (first column, width), cell
+    // offset, gap score, row of sigma, fill-list prefix (read by lane number
+    // below, so that no row waits for a load)
+    int tmw, tco, tga, tsg, tt0, tt1;
+    auto table = [&](int r) LCG_INLINE {
+        const int i = min(al + r + lane, P.n);
+        const int mn = P.mn[i];
+        tmw = mn | (min(max(P.mx[i] - mn + 1, 0), 0x7fff) << 16);
+        tco = P.coff[i] * G;
+        tga = P.gapA[i];
+        tsg = TAB ? i : P.codeA[i] * LCG_NCODES;
+        tt0 = P.fbk[2 * P.fbp[i] + 1];
+        tt1 = V.end[i];
+    };
+    table(0);
+    // rows al+r .. al+r+3 (r a multiple of 4): prefix starts, counts, the first
+    // 64 PQ entries of each (the loads run past a row's entries, over the
+    // arena's pad for the last row), first column and width, and by column the
+    // F slope prefix and the symbol code (TAB: the column)
+    int st[4], cnt[4] = {0, 0, 0, 0}, most = 0, rmw[4];
+    int2 pe[PQ][4], pc[4][NC];
+    auto columns = [&](int r) LCG_INLINE {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            rmw[k] = readlane(tmw, (r + k) & 63);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) pc[k][c] = V.pc[min(rmw[k] & 0xffff, P.m) + 64 * c + l];
+        }
+    };
+    auto entries = [&](int r) LCG_INLINE {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            st[k] = readlane(tt0, (r + k) & 63);
+            cnt[k] = r + k <= nrows ? readlane(tt1, (r + k) & 63) - st[k] : 0;
+        }
+        most = max(max(cnt[0], cnt[1]), max(cnt[2], cnt[3]));
+        auto load = [&](int q) LCG_INLINE {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) pe[q][k] = (P.fband + st[k] + 64 * q)[(unsigned)lane];
+        };
+        load(0);
+        if (most > 64) load(1);
+        if (PQ > 2 && most > 128) {
+            load(PQ - 2);
+            load(PQ - 1);
+        }
+    };
+    columns(0);
+    // init row al: M(al, bl) = 0, M(al, j) = alpha + sum of gapB(bl+1 .. j)
+    int Mp[NC], Ep[NC];
+    int mnp = rmw[0] & 0xffff;
+    {
+        const int pb = V.pc[bl].x;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int lc = 64 * c + l, j = mnp + lc;
+            const int v = alpha + pc[0][c].x - pb - P.alpha_pos * (j - bl);
+            Mp[c] = (lc >= (rmw[0] >> 16) || j < bl) ? LCG_NEG : j == bl ? 0 : v;
+            Ep[c] = LCG_NEG;
+            (Mo + c0 * G)[64 * c * G + lg] = Mp[c];
+        }
+    }
+    int colv = alpha;  // M(i, bl)
+    region_sync<false>();
+    for (int r0 = 0; r0 <= nrows; r0 += 4) {  // rows al+r0 .. al+r0+3
+        // ---- arc terms of four rows
+        auto gather = [&](const int2 &e, bool in, int &v0, int &v1) LCG_INLINE {
+            const int x = in ? e.x & 0xffffff : c0;
+            if (G == 2) {
+                const int2 m2 = *reinterpret_cast<const int2 *>(Mo + 2 * x);
+                v0 = m2.x + e.y;
+                v1 = m2.y + e.y;
+            } else {
+                v0 = Mo[x] + e.y;
+            }
+        };
+        auto scatter = [&](const int2 &e, int k, int v0, int v1) LCG_INLINE {
+            int *s = S + k * SR + G * (int)((unsigned)e.x >> 24);
+            atomicMax(s, v0);
+            if (G == 2) atomicMax(s + 1, v1);
+        };
+        auto arcs4 = [&](int q) LCG_INLINE {
+            int v0[4], v1[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) gather(pe[q][k], 64 * q + lane < cnt[k], v0[k], v1[k]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (64 * q + lane < cnt[k]) scatter(pe[q][k], k, v0[k], v1[k]);
+        };
+        if (most > 0) {
+            arcs4(0);
+            if (most > 64) arcs4(1);
+            if (PQ > 2 && most > 128) {
+                arcs4(PQ - 2);
+                arcs4(PQ - 1);
+            }
+            if (most > 64 * PQ)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    for (int t = 64 * PQ; t < cnt[k]; t += 256) {
+                        int2 e[4];
+                        int v0[4], v1[4];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) e[q] = (P.fband + st[k] + t + 64 * q)[(unsigned)lane];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) gather(e[q], t + 64 * q + lane < cnt[k], v0[q], v1[q]);
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            if (t + 64 * q + lane < cnt[k]) scatter(e[q], k, v0[q], v1[q]);
+                    }
+        }
+        region_sync<false>();
+        // ---- the rows' operands, then the next block's entries and columns
+        int sv[4][NC], pr[4][NC], sg[4][NC], cmw[4], cco[4], cga[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            cmw[k] = rmw[k];
+            cco[k] = readlane(tco, (r0 + k) & 63);
+            cga[k] = readlane(tga, (r0 + k) & 63);
+            const int sr = readlane(tsg, (r0 + k) & 63);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                pr[k][c] = pc[k][c].x;
+                sg[k][c] = TAB ? P.gsig[sr * (P.m + 1) + pc[k][c].y] : P.sig[sr + pc[k][c].y];
+                int *sp = S + k * SR + 64 * c * G + lg;
+                sv[k][c] = *sp;
+                *sp = LCG_NEG;
+            }
+        }
+        if (r0 + 4 <= nrows) {
+            if (((r0 + 4) & 63) == 0) table(r0 + 4);
+            entries(r0 + 4);
+            columns(r0 + 4);
+        }
+        // ---- the rows
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (r0 + k > nrows) break;
+            if (r0 + k == 0) continue;
+            const int mni = cmw[k] & 0xffff, w = cmw[k] >> 16, gA = cga[k];
+            const int d = mni - mnp;
+            mnp = mni;
+            colv += gA;
+            if (d >= 2) {
+                // all but the last column of the shift
+                int m2[NC], e2[NC];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const int x = 64 * c + l + d - 1;  // source column
+                    m2[c] = e2[c] = LCG_NEG;
+#pragma unroll
+                    for (int s = 0; s < NC; ++s) {
+                        const int a = (g * LPG + (x & (LPG - 1))) << 2;
+                        const int mv = __builtin_amdgcn_ds_bpermute(a, Mp[s]);
+                        const int ev = __builtin_amdgcn_ds_bpermute(a, Ep[s]);
+                        const bool here = x < CW && (NC == 1 || (x >> 6) == s);
+                        m2[c] = here ? mv : m2[c];
+                        e2[c] = here ? ev : e2[c];
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < NC; ++c) Mp[c] = m2[c], Ep[c] = e2[c];
+            }
+            int up[NC], dg[NC];
+            if (d >= 1) {
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const bool last = c + 1 == NC;
+                    dg[c] = Mp[c];
+                    up[c] = wave_shift_down(Mp[c], last ? LCG_NEG : readlane(Mp[last ? c : c + 1], 0));
+                    Ep[c] = wave_shift_down(Ep[c], last ? LCG_NEG : readlane(Ep[last ? c : c + 1], 0));
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    up[c] = Mp[c];
+                    dg[c] = wave_shift_up(Mp[c], c == 0 ? LCG_NEG : readlane(Mp[c == 0 ? 0 : c - 1], 63));
+                }
+            }
+            int ylast = LCG_NEG, pxlast = INT_MIN;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int lc = 64 * c + l;
+                const int e = max(max(Ep[c] + gA, up[c] + (gA + alpha)), LCG_NEG);
+                // (with two groups the last lane of the first holds the other's)
+                Ep[c] = LPG == 64 || lc < w ? e : LCG_NEG;
+                int s = max(max(dg[c] + sg[k][c], e), sv[k][c]);
+                s = (mni == bl - lc) ? colv : s;  // column bl (its own E is never read)
+                // F(j) = Pre(j) + alpha - alpha_pos + max_{k<j} (s(k) - Pre(k))
+                const int y = s - pr[k][c];
+                int yl = wave_shift_up(y, ylast);
+                if (LPG == 32) yl = l == 0 ? LCG_NEG : yl;  // not from the other group
+                int px = group_scan_max<LPG>(yl);
+                if (NC > 1) {
+                    px = max(px, pxlast);
+                    ylast = readlane(y, 63);
+                    pxlast = readlane(px, 63);
+                }
+                Mp[c] = lc < w ? max(s, px + pr[k][c] + calpha) : LCG_NEG;
+                // lanes past the row write into the next rows, which are
+                // written later, or the overhang
+                (Mo + cco[k] + 64 * c * G)[lg] = Mp[c];
+            }
+        }
+        if (r0 == 8 || (r0 < 8 && r0 + 4 > nrows)) later();
+        region_sync<false>();
+    }
+}
+
+// D of the arc match of group entry `ga`, of score sc, from M(ar-1, br-1) = mv
+__device__ __forceinline__ int arcmatch_D(const Pair &P, const int4 &ga, int mv, int sc) {
+    if (P.nolp) {
+        // aligner.cc:612-657: the inner arc match (its right ends are ar, br)
+        // ends the stack or continues it; its D comes from a later row,
+        // written before.  With stacking only a stackable arc match has a D,
+        // with its stacked score
+        const int y = P.inner[ga.z];  // always one (the host lists no other)
+        const int sx = P.stacking ? P.amst[ga.z] : sc;
+        return (unsigned)y < (unsigned)P.nam && sx != LCG_NEG ? max(mv + P.amscore[y], P.D[y]) + sx : LCG_NEG;
+    }
+    int v = mv + sc;
+    if (P.stacking) {
+        // aligner.cc:574-610: a stackable arc match with an inner one may
+        // take the inner one's D (a later row, written before) plus its
+        // stacked score
+        const int y = P.inner[ga.z];
+        const int st = P.amst[ga.z];
+        if ((unsigned)y < (unsigned)P.nam && st != LCG_NEG) v = max(v, P.D[y] + st);
+    }
+    return v;
+}
+
+// D of an arc match, not normalized (the reference's InftyInt sum)
+__device__ __forceinline__ void store_D(const Pair &P, const int4 &ga, int v) {
+    P.cand[ga.y].z = v;
+    P.fband[ga.w].y = v;
+    P.D[ga.z] = v;
+}
+
+// A group of a row's task list, of the list that the lanes hold (places below
+// 64) or of the list in memory.
+struct BandGroup {
+    int bl, ar, b, e;  // left end, largest right end, range in gams
+};
+__device__ __forceinline__ BandGroup band_group(const int4 &held, const int4 *__restrict__ tasks, int u) {
+    int x, b, e;
+    if (u < 64) {
+        x = readlane(held.x, u), b = readlane(held.y, u), e = readlane(held.z, u);
+    } else {
+        const int4 t = tasks[u];
+        x = uniform(t.x), b = uniform(t.y), e = uniform(t.z);
+    }
+    return BandGroup{x & 0xffff, (int)((unsigned)x >> 16), b, e};
+}
+
+// The groups of a row of left ends at places u and, with LPG 32, u + 1 of
+// their list filled, and the D of their arc matches written.  The first 64
+// arc matches and their scores are loaded before they are needed.
+template <bool TAB, int LPG, int NC>
+__device__ __forceinline__ void band_task(const Pair &P, const BandView &V, const int4 &held,
+                                          const int4 *__restrict__ tasks, const int4 *__restrict__ gams, int al, int u,
+                                          bool two, int *base) {
+    constexpr int G = 64 / LPG;
+    const int lane = lane_id();
+    const BandGroup a = band_group(held, tasks, u), b = two ? band_group(held, tasks, u + 1) : a;
+    const int na = a.e - a.b, nt = na + (two ? b.e - b.b : 0);
+    auto place = [&](int t) LCG_INLINE { return t >= na ? b.b + t - na : a.b + t; };
+    int4 ga = gams[place(min(lane, nt - 1))];
+    int sc = 0;
+    band_fill<TAB, LPG, NC>(P, V, al, a.bl, b.bl, a.ar, base, [&]() LCG_INLINE { sc = P.amscore[ga.z]; });
+    const int *Mo = base + 4 * LPG * NC * G - G * P.coff[al];
+    for (int t = lane; t < nt; t += 64) {
+        if (t >= 64) {
+            ga = gams[place(t)];
+            sc = P.amscore[ga.z];
+        }
+        const int i = (ga.x & 0xffff) - 1, j = (ga.x >> 16) - 1;
+        store_D(P, ga, arcmatch_D(P, ga, Mo[(P.coff[i] + j - P.mn[i]) * G + (t >= na)], sc));
+    }
+}
+
+// The groups g0 .. g1-1 of row al (tasks: their list, longest first; held:
+// its first 64 by lane): dealt in this order to the K members and the waves of
+// each, which take them in turns up and down; a wave's region is as large as
+// its first task's, the number of waves is what the pool holds, and a wave
+// passes from one task to the next without a barrier.  Two groups per wave
+// where the band rows are narrow, unless there are fewer pairs than CUs and
+// every group gets a wave of its own (the row's time is then that of its
+// longest task).
+template <bool TAB>
+__device__ __forceinline__ void band_row(const Pair &P, const BandView &V, const BatchParams &bp, const int4 &held,
+                                         const int4 *__restrict__ tasks, const int4 *__restrict__ gams, int al, int ng,
+                                         int member, int K, int *pool) {
+    const int lane = lane_id(), wave = uniform(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    const int c0 = P.coff[al];
+    const int ar = (int)((unsigned)readlane(held.x, 0) >> 16);
+    int w = 0;
+    for (int i = al + lane; i < ar; i += 64) w = max(w, P.mx[i] - P.mn[i] + 1);
+    w = readlane(group_scan_max<64>(w), 63);
+    // member mem's waves for tasks of `per` groups with rows of CW columns:
+    // region ends of its first 16 tasks by lane; returns the waves that fit.
+    // Member 0 has the longest tasks: the choice that all members must make
+    // alike is made with its list.
+    int size = 0, end = 0;
+    auto fit = [&](int per, int CW, int mem) LCG_INLINE {
+        const int u = per * (mem + K * lane);
+        const bool valid = u < ng && lane < nw;
+        // places from 64 on are no longer than the last one held
+        const int a = (int)((unsigned)__shfl(held.x, min(u, 63)) >> 16);
+        size = valid ? LCG_BAND_REGION(per, CW, P.coff[a] - c0) : 0;
+        end = wave_scan_add(size);
+        return (int)__popcll(__ballot(valid && end <= bp.pool_ints));
+    };
+    auto run = [&](auto lpg, auto nc, int ns) LCG_INLINE {
+        constexpr int LPG = decltype(lpg)::value, NC = decltype(nc)::value, per = 64 / LPG;
+        if (wave >= ns) return;
+        int *base = pool + (readlane(end, wave) - readlane(size, wave));
+        for (int r = 0; per * (member + K * r * ns) < ng; ++r) {
+            const int u = per * (member + K * (r * ns + ((r & 1) ? ns - 1 - wave : wave)));
+            if (u < ng) band_task<TAB, LPG, NC>(P, V, held, tasks, gams, al, u, per == 2 && u + 1 < ng, base);
+        }
+    };
+    using std::integral_constant;
+    if (w <= 31 && ng > 1 && fit(2, 32, 0) > 0 && !(bp.band_latency && ng <= K * fit(1, 64, 0)))
+        run(integral_constant<int, 32>(), integral_constant<int, 1>(), fit(2, 32, member));
+    else if (w <= 64)
+        run(integral_constant<int, 64>(), integral_constant<int, 1>(), fit(1, 64, member));
+    else
+        run(integral_constant<int, 64>(), integral_constant<int, 2>(), fit(1, 128, member));
 }
 
 // stored value of cell (i, j) of the group (origin al, bl; bound br)
@@ -1149,7 +1562,8 @@ __device__ __forceinline__ Pair load_pair(const PairDesc &d, int *arena, int *ld
     P.cand = reinterpret_cast<int4 *>(arena + d.cand);
     P.fbp = fbp;
     P.fbk = fbk;
-    P.fcand = arena + d.fcand;
+    P.fcand = reinterpret_cast<const int2 *>(arena + d.fcand);
+    P.fband = reinterpret_cast<int2 *>(arena + d.fband);
     P.amscore = arena + d.amscore;
     P.D = arena + d.D;
     P.edges = arena + d.edges;
@@ -1178,6 +1592,19 @@ __device__ __forceinline__ Pair load_pair(const PairDesc &d, int *arena, int *ld
 // Group schedule word G[5] = round | wave << 12 | member << 16.
 #define LCG_SPIN_LIMIT (1 << 22)
 
+// Arrival at a pair's barrier and bounded wait for `target` arrivals (one
+// thread of each member); an expired wait marks the pair's status.
+__device__ __forceinline__ void meet(int *counter, int target, int spin_lim, int *status) {
+    atomicAdd(counter, 1);
+    for (int spin = 0; spin_lim < 0 || atomicAdd(counter, 0) < target; ++spin) {
+        if (spin > spin_lim) {
+            atomicExch(status, 2);
+            break;
+        }
+        __builtin_amdgcn_s_sleep(2);
+    }
+}
+
 template <bool TAB, bool SL>
 __device__ __forceinline__ void fill_pairs(const PairDesc *__restrict__ descs, const int *__restrict__ order,
                                            int *queue, int *arena, int *barriers, int *scratch, BatchParams bp) {
@@ -1200,6 +1627,10 @@ __device__ __forceinline__ void fill_pairs(const PairDesc *__restrict__ descs, c
         const int k = s_pair;
         if (k >= bp.npairs) break;
         const PairDesc d = descs[order[k]];
+        if (d.band_need && d.band_need <= bp.band) {  // the band fill's
+            __syncthreads();
+            continue;
+        }
         if (member == 0) {
             if (bp.count && threadIdx.x < 4) arena[d.out + 4 + threadIdx.x] = 0;
             if (threadIdx.x == 0) arena[d.out + 3] = 0;  // status
@@ -1210,14 +1641,7 @@ __device__ __forceinline__ void fill_pairs(const PairDesc *__restrict__ descs, c
             // members count into the pair's words after member 0 cleared them
             if (threadIdx.x == 0) {
                 __threadfence();
-                atomicAdd(&barriers[k], 1);
-                for (int spin = 0; spin_lim < 0 || atomicAdd(&barriers[k], 0) < K; ++spin) {
-                    if (spin > spin_lim) {
-                        atomicExch(&arena[d.out + 3], 2);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(2);
-                }
+                meet(&barriers[k], K, spin_lim, &arena[d.out + 3]);
             }
         }
         int passed = (K > 1 && counts) ? 1 : 0;  // barrier generations passed
@@ -1254,9 +1678,7 @@ __device__ __forceinline__ void fill_pairs(const PairDesc *__restrict__ descs, c
                         const int4 ga = gams[t];
                         const int ar = ga.x & 0xffff, br = ga.x >> 16;
                         const int v = sl_best(P, base, gal, gbl, gar, gbr, W, ar - 1, br - 1, nullptr) + P.amscore[ga.z];
-                        P.cand[ga.y].z = v;
-                        P.fcand[3 * ga.w + 2] = v;
-                        P.D[ga.z] = v;
+                        store_D(P, ga, v);
                     }
                     region_sync<true>();
                 } else if (!SL && mg >= 0) {
@@ -1274,29 +1696,7 @@ __device__ __forceinline__ void fill_pairs(const PairDesc *__restrict__ descs, c
                         const int4 ga = gams[t];
                         const int ar = ga.x & 0xffff, br = ga.x >> 16;
                         const int mv = Mst[(ar - 1 - gal) * W + (br - 1 - row_lo(P, ar - 1, gbl))];
-                        int v = mv + P.amscore[ga.z];
-                        if (P.nolp) {
-                            // aligner.cc:612-657: the inner arc match (its right
-                            // ends are ar, br) ends the stack or continues it;
-                            // its D comes from a later row, written before.  With
-                            // stacking only a stackable arc match has a D, with
-                            // its stacked score
-                            const int y = P.inner[ga.z];  // always one (the host lists no other)
-                            const int sx = P.stacking ? P.amst[ga.z] : P.amscore[ga.z];
-                            v = (unsigned)y < (unsigned)P.nam && sx != LCG_NEG
-                                    ? max(mv + P.amscore[y], P.D[y]) + sx
-                                    : LCG_NEG;
-                        } else if (P.stacking) {
-                            // aligner.cc:574-610: a stackable arc match with an
-                            // inner one may take the inner one's D (a later row,
-                            // written before) plus its stacked score
-                            const int y = P.inner[ga.z];
-                            const int st = P.amst[ga.z];
-                            if ((unsigned)y < (unsigned)P.nam && st != LCG_NEG) v = max(v, P.D[y] + st);
-                        }
-                        P.cand[ga.y].z = v;  // D, not normalized (the reference's InftyInt sum)
-                        P.fcand[3 * ga.w + 2] = v;
-                        P.D[ga.z] = v;
+                        store_D(P, ga, arcmatch_D(P, ga, mv, P.amscore[ga.z]));
                     }
                 }
                 __threadfence_block();
@@ -1309,16 +1709,7 @@ __device__ __forceinline__ void fill_pairs(const PairDesc *__restrict__ descs, c
                 __threadfence();
                 __syncthreads();
                 ++passed;
-                if (threadIdx.x == 0) {
-                    atomicAdd(&barriers[k], 1);
-                    for (int spin = 0; spin_lim < 0 || atomicAdd(&barriers[k], 0) < K * passed; ++spin) {
-                        if (spin > spin_lim) {
-                            atomicExch(&arena[d.out + 3], 2);
-                            break;
-                        }
-                        __builtin_amdgcn_s_sleep(2);
-                    }
-                }
+                if (threadIdx.x == 0) meet(&barriers[k], K * passed, spin_lim, &arena[d.out + 3]);
                 __syncthreads();
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             }
@@ -1347,6 +1738,122 @@ extern "C" __global__ void __launch_bounds__(1024) lcg_fill_pairs_sl(const PairD
                                                                      int *arena, int *barriers, int *scratch,
                                                                      BatchParams bp) {
     fill_pairs<false, true>(descs, order, queue, arena, barriers, scratch, bp);
+}
+
+// Fill of D by the band kernels, for the pairs they apply to
+// (PairDesc.band_need): K members share a pair as in fill_pairs, one barrier
+// per row of left ends; the host deals the largest pairs to several members
+// each and queues the others.
+template <bool TAB>
+__device__ __forceinline__ void fill_band(const PairDesc *__restrict__ descs, const int *__restrict__ order, int *queue,
+                                          int *arena, int *barriers, const int *__restrict__ deal, BatchParams bp) {
+    extern __shared__ int lds[];
+    __shared__ int s_pair;
+    const int wave = threadIdx.x >> 6;
+    const int lane = lane_id();
+    int *pool = lds + bp.hdr_ints;
+    const int spin_lim = bp.spin_limit ? bp.spin_limit : LCG_SPIN_LIMIT;
+    // this fill's part of the LDS header: F slope prefix and code of every
+    // column, groups of every left end, and per row of A the cursor in its
+    // fill blocks and the end of its fill-list prefix p > al, kept a row of
+    // left ends ahead in two buffers (a thread keeps its own rows)
+    int2 *pc = reinterpret_cast<int2 *>(lds + bp.band_lds);
+    const int step = bp.max_len + 2;
+    int *lrows = lds + bp.band_lds + 2 * (bp.max_len + 1 + LCG_BAND_COLS);
+    int *cursor = lrows + step, *ends = cursor + step;
+    for (int iter = 0;; ++iter) {
+        // the pairs dealt to workgroups by the host first, then the queue
+        const bool mine = iter == 0 && (int)blockIdx.x < bp.dealt;
+        int K = 1, member = 0;
+        if (mine) {
+            member = deal[3 * blockIdx.x + 1];
+            K = deal[3 * blockIdx.x + 2];
+        }
+        if (threadIdx.x == 0)
+            s_pair = mine ? deal[3 * blockIdx.x] : bp.dealt_pairs + atomicAdd(queue, 1);
+        __syncthreads();
+        const int k = uniform(s_pair);
+        if (k >= bp.npairs) break;
+        const PairDesc d = descs[order[k]];
+        if (d.band_need && d.band_need <= bp.pool_ints) {
+            if (member == 0 && threadIdx.x == 0) arena[d.out + 3] = 0;  // status
+            const Pair P = load_pair(d, arena, lds, bp);
+            for (int t = threadIdx.x; t <= d.n + 1; t += blockDim.x) lrows[t] = arena[d.rows + t];
+            __syncthreads();
+            if (wave == 0) {
+                int carry = 0;
+                for (int j0 = 0; j0 <= d.m + LCG_BAND_COLS; j0 += 64) {
+                    const int j = j0 + lane;
+                    const bool in = j >= 1 && j <= d.m;
+                    const int ps = wave_scan_add(in ? P.gapB[j] + P.alpha_pos : 0);
+                    if (j <= d.m + LCG_BAND_COLS) pc[j] = make_int2(carry + ps, TAB ? min(j, d.m) : in ? P.codeB[j] : 0);
+                    carry += readlane(ps, 63);
+                }
+            }
+            auto next_row = [&](int al) {  // the next row of left ends with groups, 0: none
+                while (al >= 1 && lrows[al + 1] == lrows[al]) --al;
+                return uniform(al);
+            };
+            auto advance = [&](int *end, int al) {  // prefix p > al
+                for (int i = threadIdx.x; i <= d.n; i += blockDim.x) {
+                    int b = cursor[i];
+                    const int be = P.fbp[i + 1];
+                    while (b < be && P.fbk[2 * b] > al) ++b;
+                    cursor[i] = b;
+                    end[i] = P.fbk[2 * b + 1];
+                }
+            };
+            for (int i = threadIdx.x; i <= d.n; i += blockDim.x) cursor[i] = P.fbp[i];
+            int al = next_row(d.n), buf = 0, passed = 0;
+            advance(ends, al);
+            const int4 *gtask = reinterpret_cast<const int4 *>(arena + d.gtask);
+            const int4 *gams = reinterpret_cast<const int4 *>(arena + d.gams);
+            // the next row's first 64 groups, by lane
+            auto hold = [&](int al) {
+                const int g0 = uniform(lrows[al + 1]), ng = uniform(lrows[al]) - g0;
+                return gtask[g0 + min(lane, ng - 1)];
+            };
+            int4 held = al >= 1 ? hold(al) : make_int4(0, 0, 0, 0);
+            __syncthreads();
+            while (al >= 1) {
+                const int nal = next_row(al - 1);
+                const int4 now = held;
+                if (nal >= 1) held = hold(nal);
+                advance(ends + (buf ^ 1) * step, nal);
+                const BandView V{pc, ends + buf * step};
+                const int g0 = uniform(lrows[al + 1]), ng = uniform(lrows[al]) - g0;
+                band_row<TAB>(P, V, bp, now, gtask + g0, gams, al, ng, member, K, pool);
+                if (K > 1) {
+                    // every member's D of the row is written before any
+                    // member reads it in a later row
+                    __threadfence();
+                    __syncthreads();
+                    ++passed;
+                    if (threadIdx.x == 0) meet(&barriers[k], K * passed, spin_lim, &arena[d.out + 3]);
+                    __syncthreads();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                } else {
+                    __threadfence_block();
+                    __syncthreads();
+                }
+                al = nal;
+                buf ^= 1;
+            }
+        }
+        __syncthreads();
+    }
+}
+extern "C" __global__ void __launch_bounds__(1024) lcg_fill_band(const PairDesc *__restrict__ descs,
+                                                                 const int *__restrict__ order, int *queue,
+                                                                 int *arena, int *barriers,
+                                                                 const int *__restrict__ deal, BatchParams bp) {
+    fill_band<false>(descs, order, queue, arena, barriers, deal, bp);
+}
+extern "C" __global__ void __launch_bounds__(1024) lcg_fill_band_tab(const PairDesc *__restrict__ descs,
+                                                                     const int *__restrict__ order, int *queue,
+                                                                     int *arena, int *barriers,
+                                                                     const int *__restrict__ deal, BatchParams bp) {
+    fill_band<true>(descs, order, queue, arena, barriers, deal, bp);
 }
 
 extern "C" __global__ void lcg_reset_barriers(int *barriers, int n) {
@@ -1584,7 +2091,7 @@ extern "C" int lcg_launch_gather(const PairDesc *descs, const int *res_off, cons
 }
 
 extern "C" __global__ void lcg_reset_queue(int *queue) {
-    if (threadIdx.x == 0) *queue = 0;
+    if (threadIdx.x < 48) queue[threadIdx.x] = 0;  // the three counters
 }
 
 // Scratch of the allocation-free run (lcg_batch_run_noalloc in batch.cpp):
@@ -1623,46 +2130,42 @@ extern "C" int lcg_noalloc_scratch(int device, int **ptr, long long *ints) {
 }
 
 extern "C" int lcg_launch_align(const PairDesc *descs, const int *order, int *queue, int *arena, int *scratch,
-                                int *barriers, BatchParams bp, int grid, int waves, size_t lds_bytes, BatchParams bp_top,
-                                int top_grid, int top_waves, size_t top_lds_bytes, const int *lambda, int top_only,
+                                int *barriers, const LaunchParts *parts, const int *lambda, int top_only,
                                 hipEvent_t mid, hipStream_t stream, const int4 *restr) {
     static bool attr_set = false;
     if (!attr_set) {
         const void *kernels[] = {(const void *)lcg_fill_pairs,    (const void *)lcg_top_pairs,
                                  (const void *)lcg_fill_pairs_tab, (const void *)lcg_top_pairs_tab,
-                                 (const void *)lcg_fill_pairs_sl,  (const void *)lcg_top_pairs_sl};
+                                 (const void *)lcg_fill_pairs_sl,  (const void *)lcg_top_pairs_sl,
+                                 (const void *)lcg_fill_band,      (const void *)lcg_fill_band_tab};
         for (const void *k : kernels) {
             hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256);
             if (e != hipSuccess) return (int)e;
         }
         attr_set = true;
     }
-    // two work counters, 64 bytes apart; the per-pair barrier counters of
-    // the multi-workgroup fill
-    hipLaunchKernelGGL(lcg_reset_queue, dim3(1), dim3(64), 0, stream, queue + 16);
+    const LaunchPart &F = parts->fill, &B = parts->band, &T = parts->top;
+    // three work counters, 64 bytes apart; the per-pair barrier counters of
+    // the multi-workgroup fills (a pair is in one of them)
+    hipLaunchKernelGGL(lcg_reset_queue, dim3(1), dim3(64), 0, stream, queue);
     if (!top_only) {  // the fill of D (skipped when only the top level is redone)
-        hipLaunchKernelGGL(lcg_reset_queue, dim3(1), dim3(64), 0, stream, queue);
-        if (bp.wg_per_pair > 1)
-            hipLaunchKernelGGL(lcg_reset_barriers, dim3(1), dim3(256), 0, stream, barriers, bp.npairs);
-        if (bp.struct_local)
-            hipLaunchKernelGGL(lcg_fill_pairs_sl, dim3(grid), dim3(waves * 64), lds_bytes, stream, descs, order,
-                               queue, arena, barriers, scratch, bp);
-        else if (bp.sigma_table)
-            hipLaunchKernelGGL(lcg_fill_pairs_tab, dim3(grid), dim3(waves * 64), lds_bytes, stream, descs, order,
-                               queue, arena, barriers, scratch, bp);
-        else
-            hipLaunchKernelGGL(lcg_fill_pairs, dim3(grid), dim3(waves * 64), lds_bytes, stream, descs, order, queue,
-                               arena, barriers, scratch, bp);
+        if ((F.waves && F.bp.wg_per_pair > 1) || (B.waves && B.bp.dealt))
+            hipLaunchKernelGGL(lcg_reset_barriers, dim3(1), dim3(256), 0, stream, barriers, T.bp.npairs);
+        if (B.waves)
+            hipLaunchKernelGGL(B.bp.sigma_table ? lcg_fill_band_tab : lcg_fill_band, dim3(B.grid), dim3(B.waves * 64),
+                               B.lds_bytes, stream, descs, order, queue + 32, arena, barriers, parts->deal, B.bp);
+        if (F.waves)
+            hipLaunchKernelGGL(F.bp.struct_local  ? lcg_fill_pairs_sl
+                               : F.bp.sigma_table ? lcg_fill_pairs_tab
+                                                  : lcg_fill_pairs,
+                               dim3(F.grid), dim3(F.waves * 64), F.lds_bytes, stream, descs, order, queue, arena,
+                               barriers, scratch, F.bp);
     }
-    if (mid) hipEventRecord(mid, stream);
-    if (bp_top.struct_local)
-        hipLaunchKernelGGL(lcg_top_pairs_sl, dim3(top_grid), dim3(top_waves * 64), top_lds_bytes, stream, descs,
-                           order, queue + 16, arena, scratch, bp_top, lambda, restr);
-    else if (bp_top.sigma_table)
-        hipLaunchKernelGGL(lcg_top_pairs_tab, dim3(top_grid), dim3(top_waves * 64), top_lds_bytes, stream, descs,
-                           order, queue + 16, arena, scratch, bp_top, lambda, restr);
-    else
-        hipLaunchKernelGGL(lcg_top_pairs, dim3(top_grid), dim3(top_waves * 64), top_lds_bytes, stream, descs, order,
-                           queue + 16, arena, scratch, bp_top, lambda, restr);
+    if (mid) (void)hipEventRecord(mid, stream);
+    hipLaunchKernelGGL(T.bp.struct_local  ? lcg_top_pairs_sl
+                       : T.bp.sigma_table ? lcg_top_pairs_tab
+                                          : lcg_top_pairs,
+                       dim3(T.grid), dim3(T.waves * 64), T.lds_bytes, stream, descs, order, queue + 16, arena, scratch,
+                       T.bp, lambda, restr);
     return (int)hipGetLastError();
 }

@@ -40,10 +40,8 @@ extern "C" int lcg_launch_compact_build(const CompactDesc *cds, const PairDesc *
                                         hipStream_t stream);
 
 extern "C" int lcg_launch_align(const PairDesc *descs, const int *order, int *queue, int *arena, int *scratch,
-                                int *barriers, BatchParams bp, int grid, int waves, size_t lds_bytes, BatchParams bp_top,
-                                int top_grid,
-                                int top_waves, size_t top_lds_bytes, const int *lambda, int top_only, hipEvent_t mid,
-                                hipStream_t stream, const int32_t *restr = nullptr);  // int4 per pair
+                                int *barriers, const LaunchParts *parts, const int *lambda, int top_only,
+                                hipEvent_t mid, hipStream_t stream, const int32_t *restr = nullptr);  // int4 per pair
 
 struct lcg_pair {
     lcg_params params;
@@ -100,7 +98,9 @@ size_t layout_pair(PairDesc &d, int n, int m, int ncells, int ngroups, int nam, 
     d.sigma = take(table ? (size_t)(n + 1) * (m + 1) : LCG_NCODES * LCG_NCODES);
     d.rows = take((size_t)n + 2);
     d.rounds = take((size_t)n + 2);
+    align(4);
     d.groups = take((size_t)LCG_GROUP_INTS * ngroups);
+    d.gtask = take(4 * (size_t)ngroups);
     align(4);
     d.gams = take(4 * (size_t)nam);
     d.amscore = take(nam);
@@ -108,7 +108,9 @@ size_t layout_pair(PairDesc &d, int n, int m, int ncells, int ngroups, int nam, 
     align(4);
     d.cand = take(4 * (size_t)nam);
     d.fptr = take((size_t)n + 2);
-    d.fcand = take(3 * (size_t)nam);
+    align(2);
+    d.fcand = take(2 * (size_t)nam);
+    d.fband = take(2 * (size_t)nam);
     d.fblk = take(2 * (size_t)nfblk);
     d.f2c = take(nam);
     d.D = take(nam);
@@ -129,7 +131,7 @@ size_t layout_pair(PairDesc &d, int n, int m, int ncells, int ngroups, int nam, 
 void rebase(PairDesc &d, int32_t base) {
     int32_t *offs[] = {&d.band, &d.codes, &d.gaps, &d.sigma, &d.rows, &d.groups, &d.gams, &d.amscore,
                        &d.cptr, &d.cand, &d.D, &d.edges, &d.structs, &d.tstack, &d.out, &d.rounds,
-                       &d.fptr, &d.fblk, &d.fcand, &d.f2c, &d.inner, &d.c2a, &d.amst};
+                       &d.fptr, &d.fblk, &d.fcand, &d.f2c, &d.inner, &d.c2a, &d.amst, &d.fband, &d.gtask};
     for (int32_t *o : offs) *o += base;
 }
 
@@ -140,7 +142,7 @@ bool image_in_place(const PairDesc &d, int32_t base, int32_t size, const std::ve
                     bool stacking = false) {
     const int32_t offs[] = {d.band, d.codes, d.gaps, d.sigma, d.rows, d.groups, d.gams, d.amscore, d.cptr, d.cand,
                             d.D, d.edges, d.structs, d.tstack, d.out, d.rounds, d.fptr, d.fblk, d.fcand, d.f2c,
-                            d.inner, d.c2a, d.amst};
+                            d.inner, d.c2a, d.amst, d.fband, d.gtask};
     for (int32_t o : offs)
         if (o < base || o > base + size) return false;
     if (stacking && d.amst + d.nam > base + size) return false;  // --stacking scores present
@@ -166,6 +168,26 @@ void top_region(const std::vector<int> &mn, const std::vector<int> &mx, int n, i
         if (i > 0) cells += std::max(0, std::min(m, mx[i]) - std::max(1, mn[i]) + 1);
     }
     top_ints = ((m + 1) + wtop + (n + 1) * wtop + 3) & ~3;
+}
+
+// Order of the arcs of B within a fill block (the arc matches of one arc of
+// A): first the first arc of every right end (ascending), then the second
+// ones, and so on (right ends by right adjacency order), so that neighbouring
+// fill entries end in different columns: the fill combines the entries of a
+// row by LDS atomics, which are serialized where lanes meet in a column.
+// Returns the place of every arc in that order.
+std::vector<int> fill_order(const BasePairs &bB, int m) {
+    std::vector<int> place(bB.num_bps(), 0);
+    int t = 0;
+    for (size_t r = 0, left = 1; left; ++r) {
+        left = 0;
+        for (int j = 0; j <= m; ++j) {
+            const auto &lst = bB.right_adj(j);
+            if (r < lst.size()) place[lst[r]] = t++;
+            left += r + 1 < lst.size();
+        }
+    }
+    return place;
 }
 
 void pack(lcg_pair &P) {
@@ -317,6 +339,7 @@ void pack(lcg_pair &P) {
     d.rows = reserve(blob, rows.size());
     std::copy(rows.begin(), rows.end(), blob.begin() + d.rows);
     d.rounds = reserve(blob, rows.size());  // filled by the batch's LDS schedule
+    while (blob.size() & 3) blob.push_back(0);
     d.groups = reserve(blob, (size_t)LCG_GROUP_INTS * groups.size());
     for (size_t g = 0; g < groups.size(); ++g) {
         int32_t *G8 = &blob[d.groups + LCG_GROUP_INTS * g];
@@ -326,6 +349,22 @@ void pack(lcg_pair &P) {
         G8[3] = groups[g].b;
         G8[4] = groups[g].e;
         G8[7] = groups[g].lds;
+    }
+    d.gtask = reserve(blob, 4 * groups.size());
+    {
+        std::vector<int> idx(groups.size());
+        std::iota(idx.begin(), idx.end(), 0);
+        std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) {
+            return groups[x].al != groups[y].al ? groups[x].al > groups[y].al : groups[x].ar > groups[y].ar;
+        });
+        for (size_t t = 0; t < idx.size(); ++t) {
+            const G &g = groups[idx[t]];
+            int32_t *T = &blob[d.gtask + 4 * t];
+            T[0] = g.bl | (g.ar << 16);
+            T[1] = g.b;
+            T[2] = g.e;
+            T[3] = idx[t];
+        }
     }
     while (blob.size() & 3) blob.push_back(0);
     d.gams = reserve(blob, 4 * (size_t)nam);  // (--noLP: only the arc matches with an inner one have an entry)
@@ -366,11 +405,14 @@ void pack(lcg_pair &P) {
     blob[d.cptr + ncells] = t;
     if (t != nam) throw failure("internal: arc match right-end lists incomplete");
     // fill-D candidate list: the arc matches of row i (right end in A),
-    // blocks of one arc of A by left end p descending, j ascending in a block
+    // blocks of one arc of A by left end p descending, in fill order in a block
+    const std::vector<int> place = fill_order(bB, m);
     std::vector<std::vector<int>> by_rightA(n + 1);
     for (int k = 0; k < nam; ++k) by_rightA[bA.arc(ams.arcmatch(k).arcA).right].push_back(k);
     d.fptr = reserve(blob, (size_t)n + 2);
-    d.fcand = reserve(blob, 3 * (size_t)nam);
+    while (blob.size() & 1) blob.push_back(0);
+    d.fcand = reserve(blob, 2 * (size_t)nam);
+    d.fband = reserve(blob, 2 * (size_t)nam);
     std::vector<int32_t> blk;
     std::vector<int> fentry_of(nam, -1);
     int tf = 0;
@@ -381,9 +423,7 @@ void pack(lcg_pair &P) {
             const ArcMatch &ax = ams.arcmatch(x), &ay = ams.arcmatch(y);
             const int px = bA.arc(ax.arcA).left, py = bA.arc(ay.arcA).left;
             if (px != py) return px > py;
-            const int jx = bB.arc(ax.arcB).right, jy = bB.arc(ay.arcB).right;
-            if (jx != jy) return jx < jy;
-            return bB.arc(ax.arcB).left > bB.arc(ay.arcB).left;
+            return place[ax.arcB] < place[ay.arcB];
         });
         int last_p = -1;
         for (int k : lst) {
@@ -394,9 +434,11 @@ void pack(lcg_pair &P) {
                 blk.push_back(tf);
                 last_p = p;
             }
-            blob[d.fcand + 3 * tf] = p | (q << 16);
-            blob[d.fcand + 3 * tf + 1] = j | (tc.min_col(p - 1) << 16);
-            blob[d.fcand + 3 * tf + 2] = LCG_NEG;
+            blob[d.fcand + 2 * tf] = p | (q << 16);
+            blob[d.fcand + 2 * tf + 1] = j | (tc.min_col(p - 1) << 16);
+            const int src = blob[d.band + 2 * (n + 1) + p - 1] + (q - 1 - tc.min_col(p - 1));
+            blob[d.fband + 2 * tf] = (int32_t)LCG_FBAND(src, j - tc.min_col(i));
+            blob[d.fband + 2 * tf + 1] = LCG_NEG;
             fentry_of[k] = tf++;
         }
     }
@@ -530,6 +572,11 @@ void prepare_compaction_inputs(lcg_pair &P) {
     };
     side(bA, *P.A, n, true);
     side(bB, *P.B, m, false);
+    c.fordB = reserve(img, NB);
+    {
+        const std::vector<int> place = fill_order(bB, m);
+        for (int b = 0; b < NB; ++b) img[c.fordB + place[b]] = b;
+    }
     c.band = reserve(img, 2 * (size_t)(n + 1));
     for (int i = 0; i <= n; ++i) {
         img[c.band + i] = tc.min_col(i);
@@ -892,7 +939,6 @@ struct lcg_batch {
     int32_t *d_order = nullptr;
     int32_t *d_queue = nullptr;
     int32_t *d_barriers = nullptr;  // per-pair arrival counters (multi-workgroup fill)
-    int wg_per_pair = 1;
     int32_t *d_scratch = nullptr;
     hipStream_t stream = nullptr;      // the stream every launch and copy of the batch goes to
     hipStream_t own_stream = nullptr;  // the batch's own stream (destroyed with it)
@@ -905,14 +951,15 @@ struct lcg_batch {
     // what choosing one needs (CU count, LDS header ints, largest region)
     lcg_shape req{};
     lcg_shape eff{};
-    int cus = 1, hdr = 0, gmax = 4, top_max = 4, max_len = 1;
+    int cus = 1, hdr = 0, band_ints = 0, gmax = 4, top_max = 4, max_len = 1;
     int sl_max = 0;  // --struct-local: ints of the largest group region (global scratch per wave)
-    BatchParams bp;      // fill-D kernel
-    int waves = 1, grid = 1;
-    size_t lds_bytes = 0;
-    BatchParams bp_top;  // top-level / traceback kernel
-    int top_waves = 1, top_grid = 1;
-    size_t top_lds_bytes = 0;
+    BatchParams bp;       // general fill of D
+    BatchParams bp_band;  // band fill of D
+    BatchParams bp_top;   // top level / traceback
+    LaunchParts parts{};  // grids, waves and LDS of the three launches (their bp is filled in per run)
+    std::vector<int32_t> deal;    // workgroups of the band fill with a pair of their own (deal_pairs)
+    int32_t *d_deal = nullptr;    // 3 per CU
+    int fill_waves = 1;   // waves of the general fill, also where no pair of the batch takes it
     bool have_results = false;
     bool fetched = false;
     bool run_invalid = false;  // the fetched run's status words reported an expired wait
@@ -1153,7 +1200,7 @@ int device_count_and_layout(lcg_batch &B, lcg_pair *const *pairs, int npairs, st
         cin.insert(cin.end(), P->cimg.begin(), P->cimg.end());
         CompactDesc c = P->cdesc;
         int32_t *offs[] = {&c.arcsA, &c.arcsB, &c.wA, &c.wB, &c.ptA, &c.ptB, &c.lA, &c.lB,
-                           &c.rpA, &c.rpB, &c.radjA, &c.radjB, &c.band, &c.tab, &c.hdr};
+                           &c.rpA, &c.rpB, &c.radjA, &c.radjB, &c.fordB, &c.band, &c.tab, &c.hdr};
         for (int32_t *o : offs) *o += base;
         const size_t words = (size_t)c.NA * c.W64;
         ws_ints = (ws_ints + 1) & ~(size_t)1;
@@ -1310,6 +1357,7 @@ constexpr int kLdsIntsCu = (160 * 1024 - 512) / 4;  // static LDS of the kernels
 
 struct FillShape {
     int waves, wgs_per_cu, K, pool;
+    int band_waves, band_wgs_per_cu, band_K, band_pool;  // band fill, pool 0: not used; K 0: by work
 };
 struct TopShape {
     int waves, wgs_per_cu, pool;
@@ -1336,6 +1384,22 @@ int choose_fill(const lcg_batch &B, FillShape &s, char *err, int errlen) {
     const int np = B.npairs;
     s.K = pick(B.req.wg_per_pair, "LCG_WG_PER_PAIR", np < B.cus ? std::min(64, B.cus / np) : 1, 1, 64);
     s.K = std::min(s.K, std::max(1, B.cus / np));  // all workgroups of the fill stay co-resident
+    // band fill: one workgroup of 16 waves per CU (2016 pairs of 60-200 nt: 36.6
+    // ms; 12 waves 37.2, 8 waves 41.4, two of 8 waves 76.0: the regions of a
+    // row are then half as many at a time); with fewer pairs than CUs 8 waves
+    // (120 local pairs 18.8 ms against 19.3, four 500-nt pairs 17.4 against 18.1)
+    s.band_waves = pick(B.req.waves, "LCG_WAVES", np < B.cus ? 8 : 16, 1, 16);
+    s.band_wgs_per_cu = pick(B.req.wgs_per_cu, "LCG_WGS_PER_CU", 1, 1, 4);
+    s.band_K = pick(B.req.wg_per_pair, "LCG_WG_PER_PAIR", 0, 1, 64);
+    s.band_K = std::min(s.band_K, std::max(1, B.cus / np));
+    int need = 0;
+    for (const PairDesc &d : B.descs) need = std::max(need, d.band_need);
+    s.band_pool = 0;
+    if (need > 0)
+        for (; s.band_wgs_per_cu >= 1; --s.band_wgs_per_cu) {
+            s.band_pool = std::max(0, kLdsIntsCu / s.band_wgs_per_cu - B.hdr - B.band_ints) & ~3;
+            if (s.band_pool >= need || s.band_wgs_per_cu == 1) break;
+        }
     return LCG_OK;
 }
 
@@ -1363,26 +1427,98 @@ bool schedule_all(lcg_batch &B, const FillShape &s) {
     return true;
 }
 
+// Deals the first pairs of the work order to workgroups of the band fill:
+// K each where that is asked for, else as many to each as keep the estimated
+// makespan smallest (a pair of work w on k workgroups takes w (1 + 0.14 (k -
+// 1)) / k: 80, 43, 27 and 20 ms for k = 1, 2, 4 and 8 on four 500-nt pairs),
+// with a group of an average row of left ends for every one.
+// All of them are resident at once (at most one per CU); the pairs that are
+// not dealt are queued.  Three ints per workgroup: place in the order, member,
+// members.
+void deal_pairs(lcg_batch &B, const FillShape &s) {
+    const int np = B.npairs, slots = B.cus;
+    auto time = [&](int q, int k) { return (double)B.work[B.order[q]] * (1 + 0.14 * (k - 1)) / k; };
+    auto most = [&](int q) {
+        const PairDesc &d = B.descs[B.order[q]];
+        if (!d.band_need || d.band_need > s.band_pool) return 1;
+        return std::max(2, std::min(16, d.ngroups / std::max(1, d.n)));
+    };
+    std::vector<int> K(np, 1);
+    int dealt = np < slots ? np : 0;
+    if (s.band_K > 0) {
+        if (s.band_K > 1) {
+            dealt = np;  // band_K * np workgroups at most one per CU
+            std::fill(K.begin(), K.end(), s.band_K);
+        }
+    } else {
+        double total = 0;
+        for (int q = 0; q < np; ++q) total += time(q, 1);
+        // smallest makespan that the slots allow, by bisection
+        double lo = total / slots, hi = std::max(time(0, 1), 2 * lo);
+        std::vector<int> kk(np);
+        for (int it = 0; it < 20; ++it) {
+            const double T = it == 0 ? hi : 0.5 * (lo + hi);
+            long used = 0;
+            double rest = 0;
+            for (int q = 0; q < np; ++q) {
+                const int cap = most(q);
+                int k = 1;
+                while (k < cap && time(q, k) > T) ++k;
+                kk[q] = k;
+                if (k > 1 || np < slots) used += k;
+                else rest += time(q, 1);
+            }
+            // queued pairs fill their workgroups to about 0.9
+            if (used + rest / (0.9 * T) <= slots) {
+                hi = T;
+                K = kk;
+            } else {
+                lo = T;
+            }
+        }
+        for (int q = 0; q < np; ++q)
+            if (K[q] > 1) dealt = std::max(dealt, q + 1);
+    }
+    B.deal.clear();
+    for (int q = 0; q < dealt; ++q)
+        for (int m = 0; m < K[q]; ++m) B.deal.insert(B.deal.end(), {q, m, K[q]});
+    const int wgs = (int)B.deal.size() / 3;
+    B.bp_band.dealt = wgs;
+    B.bp_band.dealt_pairs = dealt;
+    B.parts.band.grid = std::max(wgs, dealt == np ? 0 : std::min(np, B.cus * s.band_wgs_per_cu));
+}
+
 // Launch parameters of both kernels for the chosen shapes.
 void apply_shape(lcg_batch &B, const FillShape &s, const TopShape &t) {
     const int np = B.npairs;
-    B.wg_per_pair = s.K;
-    B.waves = s.waves;
-    B.lds_bytes = (size_t)(B.hdr + s.pool) * 4;
+    B.bp.hdr_ints = B.hdr;
+    B.bp.band = s.band_pool;
     B.bp.pool_ints = s.pool;
     B.bp.wg_per_pair = s.K;
-    B.grid = s.K > 1 ? np * s.K : std::min(np, B.cus * s.wgs_per_cu);
+    int nband = 0;
+    for (const PairDesc &d : B.descs) nband += d.band_need && d.band_need <= s.band_pool;
+    B.parts.fill.waves = nband < np ? s.waves : 0;
+    B.parts.fill.grid = s.K > 1 ? np * s.K : std::min(np, B.cus * s.wgs_per_cu);
+    B.parts.fill.lds_bytes = (size_t)(B.hdr + s.pool) * 4;
+    B.fill_waves = s.waves;
+    B.parts.band.waves = nband > 0 ? s.band_waves : 0;
+    B.parts.band.lds_bytes = (size_t)(B.hdr + B.band_ints + s.band_pool) * 4;
+    B.bp_band = B.bp;
+    B.bp_band.hdr_ints = B.hdr + B.band_ints;
+    B.bp_band.pool_ints = s.band_pool;
+    B.bp_band.wg_per_pair = s.band_K;
+    deal_pairs(B, s);
     B.bp.sl_stride = B.sl_max;
     B.bp_top = B.bp;
     B.bp_top.pool_ints = t.pool;
     // the traceback's structure-local regions use the per-wave scratch too
     B.bp_top.scratch_stride = std::max(B.top_max, B.sl_max);
-    B.top_waves = t.waves;
-    B.top_lds_bytes = (size_t)(B.hdr + t.pool) * 4;
-    B.top_grid = std::min(np, B.cus * t.wgs_per_cu);
-    B.eff.waves = s.waves;
-    B.eff.wgs_per_cu = s.wgs_per_cu;
-    B.eff.wg_per_pair = s.K;
+    B.parts.top.waves = t.waves;
+    B.parts.top.lds_bytes = (size_t)(B.hdr + t.pool) * 4;
+    B.parts.top.grid = std::min(np, B.cus * t.wgs_per_cu);
+    B.eff.waves = nband ? s.band_waves : s.waves;
+    B.eff.wgs_per_cu = nband ? s.band_wgs_per_cu : s.wgs_per_cu;
+    B.eff.wg_per_pair = nband ? s.band_K : s.K;
     B.eff.top_waves = t.waves;
     B.eff.top_wgs_per_cu = t.wgs_per_cu;
 }
@@ -1390,9 +1526,34 @@ void apply_shape(lcg_batch &B, const FillShape &s, const TopShape &t) {
 // global scratch of a batch: the top level's per-wave regions and, with
 // --struct-local, the fill's and traceback's eight-state regions
 size_t scratch_ints(const lcg_batch &B) {
-    const size_t top = (size_t)B.top_grid * B.top_waves * std::max(B.top_max, B.sl_max);
-    const size_t fill = (size_t)B.grid * B.waves * B.sl_max;
+    const size_t top = (size_t)B.parts.top.grid * B.parts.top.waves * std::max(B.top_max, B.sl_max);
+    const size_t fill = (size_t)B.parts.fill.grid * B.fill_waves * B.sl_max;
     return std::max(top, fill);
+}
+
+hipError_t upload_deal(lcg_batch &B) {
+    if (B.deal.empty()) return hipSuccess;
+    return hipMemcpy(B.d_deal, B.deal.data(), B.deal.size() * 4, hipMemcpyHostToDevice);
+}
+
+// The launches of a run.  A counting run takes the general fill for every
+// pair: its kernels count cells and candidates.
+LaunchParts run_parts(const lcg_batch &B, int trace, int count) {
+    LaunchParts L = B.parts;
+    L.deal = B.d_deal;
+    L.fill.bp = B.bp;
+    L.band.bp = B.bp_band;
+    L.top.bp = B.bp_top;
+    for (LaunchPart *x : {&L.fill, &L.band, &L.top}) {
+        x->bp.trace = trace;
+        x->bp.count = count;
+    }
+    if (count) {
+        L.fill.waves = B.fill_waves;
+        L.fill.bp.band = 0;
+        L.band.waves = 0;
+    }
+    return L;
 }
 }  // namespace
 
@@ -1471,6 +1632,33 @@ extern "C" int lcg_batch_create_shaped(lcg_pair *const *pairs, int32_t npairs, i
             work[k] = P->cells;
         }
     }
+    // pairs the band fill takes: band bounds that do not decrease, rows of at
+    // most LCG_BAND_COLS columns; the pool must hold a region of one group
+    // (rows al .. below the largest right end of A's arcs with left end al)
+    const char *fc = std::getenv("LCG_FIXED_COLS");
+    const bool fixed_cols = !fc || std::atoi(fc) != 0;
+    bool band = false;
+    for (int k = 0; k < npairs && fixed_cols && !p0.struct_local; ++k) {
+        const lcg_pair &X = *pairs[k];
+        const std::vector<int> &mn = X.tc->min_cols(), &mx = X.tc->max_cols();
+        const int n = X.A->length();
+        if (!std::is_sorted(mn.begin(), mn.end()) || !std::is_sorted(mx.begin(), mx.end())) continue;
+        std::vector<int> coff(n + 2, 0);
+        int w = 0;
+        for (int i = 0; i <= n; ++i) {
+            const int x = std::max(0, mx[i] - mn[i] + 1);
+            w = std::max(w, x);
+            coff[i + 1] = coff[i] + x;
+        }
+        if (w > LCG_BAND_COLS) continue;
+        int cells = 0;
+        for (int a = 0; a < X.bA->num_bps(); ++a) {
+            const Arc &x = X.bA->arc(a);
+            cells = std::max(cells, coff[x.right] - coff[x.left]);
+        }
+        B->descs[k].band_need = LCG_BAND_REGION(1, w <= 64 ? 64 : 128, cells);
+        band = true;
+    }
     int max_len = 1, gmax = 4, top_max = 4, nfblk_max = 1;
     for (const PairDesc &d : B->descs) B->sl_max = std::max(B->sl_max, d.slmax);
     for (const PairDesc &d : B->descs) {
@@ -1479,7 +1667,16 @@ extern "C" int lcg_batch_create_shaped(lcg_pair *const *pairs, int32_t npairs, i
         nfblk_max = std::max(nfblk_max, d.nfblk);
         top_max = std::max(top_max, d.top_ints);
     }
-    // longest pairs first (greedy LPT over the persistent workgroups)
+    // longest pairs first (greedy LPT over the persistent workgroups).  Work of
+    // a pair: its DP cells and the arc terms they read, about 0.7 arc matches
+    // per band cell and DP cell; the fill of pairs of 60-200 nt takes 1.6 ns a
+    // cell and 0.39 ns an arc term (2.1, 3.7, 10.3 and 12.8 ms for pairs of
+    // 1.1, 1.4, 3.7 and 3.1 million cells and 0.9, 3.8, 11.9 and 21 million
+    // terms, alone on a CU)
+    for (int k = 0; k < npairs; ++k) {
+        const PairDesc &d = B->descs[k];
+        work[k] = (int64_t)((double)work[k] * (1.0 + 0.17 * d.nam / std::max(1, d.ncells)));
+    }
     B->work = work;
     B->order.resize(npairs);
     std::iota(B->order.begin(), B->order.end(), 0);
@@ -1495,6 +1692,10 @@ extern "C" int lcg_batch_create_shaped(lcg_pair *const *pairs, int32_t npairs, i
     const int fptr_lds = 7 * max_len + 72;
     const int fblk_lds = fptr_lds + max_len + 2;
     B->hdr = (fblk_lds + 2 * nfblk_max + 3) & ~3;
+    // the band fill's part of the header: F slope and symbol code of every
+    // column; groups of every left end, block cursor and fill-list prefix end
+    // (two buffers) of every row
+    if (band) B->band_ints = (2 * (max_len + 1 + LCG_BAND_COLS) + 4 * (max_len + 2) + 3) & ~3;
     B->cus = cus;
     B->gmax = gmax;
     B->top_max = top_max;
@@ -1520,21 +1721,23 @@ extern "C" int lcg_batch_create_shaped(lcg_pair *const *pairs, int32_t npairs, i
     }
     B->bp.trace = 1;
     B->bp.npairs = npairs;
-    B->bp.hdr_ints = B->hdr;
     B->bp.fptr_lds = fptr_lds;
     B->bp.fblk_lds = fblk_lds;
     B->bp.max_len = max_len;
     B->bp.count = 0;
     B->bp.scratch_stride = top_max;
-    B->bp.fixed_cols = 1;
-    if (const char *f = std::getenv("LCG_FIXED_COLS")) B->bp.fixed_cols = std::atoi(f) != 0;
+    B->bp.fixed_cols = fixed_cols;
+    B->bp.band_lds = B->hdr;
+    B->bp.band_latency = npairs < cus;
     apply_shape(*B, fs, ts);
-    if ((e = hipMalloc(&B->d_arena, B->arena_ints * 4)) != hipSuccess) return hip_fail(e, err, errlen);
+    if ((e = hipMalloc(&B->d_arena, (B->arena_ints + LCG_ARENA_PAD) * 4)) != hipSuccess) return hip_fail(e, err, errlen);
     if ((e = hipMalloc(&B->d_descs, sizeof(PairDesc) * npairs)) != hipSuccess) return hip_fail(e, err, errlen);
     if ((e = hipMalloc(&B->d_order, 4 * (size_t)npairs)) != hipSuccess) return hip_fail(e, err, errlen);
     if ((e = hipMalloc(&B->d_queue, 256)) != hipSuccess) return hip_fail(e, err, errlen);
     if ((e = hipMalloc(&B->d_barriers, 4 * (size_t)npairs)) != hipSuccess) return hip_fail(e, err, errlen);
     if ((e = hipMalloc(&B->d_scratch, scratch_ints(*B) * 4)) != hipSuccess) return hip_fail(e, err, errlen);
+    if ((e = hipMalloc(&B->d_deal, 12 * (size_t)cus)) != hipSuccess) return hip_fail(e, err, errlen);
+    if ((e = upload_deal(*B)) != hipSuccess) return hip_fail(e, err, errlen);
     if (deferred)  // the compaction writes the image over a cleared arena
         e = hipMemsetAsync(B->d_arena, 0, B->arena_ints * 4, B->stream);
     else
@@ -1592,6 +1795,7 @@ lcg_batch::~lcg_batch() {
     if (B->d_order) hipFree(B->d_order);
     if (B->d_queue) hipFree(B->d_queue);
     if (B->d_barriers) hipFree(B->d_barriers);
+    if (B->d_deal) hipFree(B->d_deal);
     if (B->d_scratch) hipFree(B->d_scratch);
     if (B->d_restr) hipFree(B->d_restr);
     if (B->d_kscratch) hipFree(B->d_kscratch);
@@ -1677,44 +1881,50 @@ extern "C" int lcg_batch_set_stream(lcg_batch *B, void *stream) {
 extern "C" int lcg_batch_set_spin_limit(lcg_batch *B, int32_t polls) {
     if (!B || polls < -1) return LCG_E_ARG;
     B->bp.spin_limit = polls;
+    B->bp_band.spin_limit = polls;
     B->bp_top.spin_limit = polls;
     return LCG_OK;
 }
 
 extern "C" int lcg_batch_config(const lcg_batch *B, int32_t *waves, int32_t *workgroups, int32_t *lds_bytes) {
     if (!B) return LCG_E_ARG;
-    if (waves) *waves = B->waves;
-    if (workgroups) *workgroups = B->grid;
-    if (lds_bytes) *lds_bytes = (int32_t)B->lds_bytes;
+    const LaunchPart &f = B->parts.band.waves ? B->parts.band : B->parts.fill;
+    if (waves) *waves = f.waves;
+    if (workgroups) *workgroups = f.grid;
+    if (lds_bytes) *lds_bytes = (int32_t)f.lds_bytes;
     return LCG_OK;
 }
 
 extern "C" int lcg_batch_run(lcg_batch *B, int32_t mode, int32_t trace, float *device_ms) {
     if (!B || mode < 0 || mode > 2) return LCG_E_ARG;
     HIPCHECK(hipSetDevice(B->device));
-    BatchParams bp = B->bp;
-    bp.trace = (trace & 1) ? 1 : 0;
-    bp.count = (trace & 2) ? 1 : 0;
-    if (mode == 2 && bp.count) return LCG_E_ARG;
-    BatchParams top = B->bp_top;
-    top.trace = bp.trace;
-    top.count = bp.count;
+    const int with_trace = (trace & 1) ? 1 : 0, count = (trace & 2) ? 1 : 0;
+    if (mode == 2 && count) return LCG_E_ARG;
+    LaunchParts parts = run_parts(*B, with_trace, count);
+    auto launch = [&](const int32_t *order, hipEvent_t mid, hipStream_t stream) {
+        return lcg_launch_align(B->d_descs, order, B->d_queue, B->d_arena, B->d_scratch, B->d_barriers, &parts, nullptr,
+                                0, mid, stream);
+    };
     HIPCHECK(hipEventRecord(B->ev0, B->stream));
     if (mode == 0) {
-        int rc = lcg_launch_align(B->d_descs, B->d_order, B->d_queue, B->d_arena, B->d_scratch, B->d_barriers, bp, B->grid, B->waves,
-                                  B->lds_bytes, top, B->top_grid, B->top_waves, B->top_lds_bytes, nullptr, 0, B->ev_mid, B->stream);
-        if (rc) return hip_fail((hipError_t)rc);
+        if (int rc = launch(B->d_order, B->ev_mid, B->stream)) return hip_fail((hipError_t)rc);
     } else if (mode == 1) {
-        BatchParams one = bp, one_top = top;
-        one.npairs = 1;
-        one_top.npairs = 1;
+        // one pair per launch, by the fill that takes it
+        const LaunchParts all = parts;
         for (int k = 0; k < B->npairs; ++k) {
-            int rc = lcg_launch_align(B->d_descs, B->d_order + k, B->d_queue, B->d_arena, B->d_scratch, B->d_barriers, one, B->wg_per_pair, B->waves,
-                                      B->lds_bytes, one_top, 1, B->top_waves, B->top_lds_bytes, nullptr, 0, nullptr, B->stream);
-            if (rc) return hip_fail((hipError_t)rc);
+            const PairDesc &d = B->descs[B->order[k]];
+            const bool band = d.band_need && d.band_need <= all.fill.bp.band;
+            parts.fill.waves = band ? 0 : all.fill.waves;
+            parts.band.waves = band ? all.band.waves : 0;
+            for (LaunchPart *x : {&parts.fill, &parts.band, &parts.top}) {
+                x->bp.npairs = 1;
+                x->grid = x == &parts.fill ? x->bp.wg_per_pair : 1;
+            }
+            parts.band.bp.dealt = parts.band.bp.dealt_pairs = 0;  // one workgroup from the queue
+            if (int rc = launch(B->d_order + k, nullptr, B->stream)) return hip_fail((hipError_t)rc);
         }
     } else {
-        if (!B->graph_exec || B->graph_trace != bp.trace) {
+        if (!B->graph_exec || B->graph_trace != with_trace) {
             if (B->graph_exec) hipGraphExecDestroy(B->graph_exec);
             if (B->graph) hipGraphDestroy(B->graph);
             B->graph_exec = nullptr;
@@ -1722,8 +1932,7 @@ extern "C" int lcg_batch_run(lcg_batch *B, int32_t mode, int32_t trace, float *d
             hipStream_t cs;
             HIPCHECK(hipStreamCreate(&cs));
             HIPCHECK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-            int rc = lcg_launch_align(B->d_descs, B->d_order, B->d_queue, B->d_arena, B->d_scratch, B->d_barriers, bp, B->grid, B->waves,
-                                      B->lds_bytes, top, B->top_grid, B->top_waves, B->top_lds_bytes, nullptr, 0, nullptr, cs);
+            int rc = launch(B->d_order, nullptr, cs);
             hipGraph_t g = nullptr;
             hipError_t ec = hipStreamEndCapture(cs, &g);
             hipStreamDestroy(cs);
@@ -1731,7 +1940,7 @@ extern "C" int lcg_batch_run(lcg_batch *B, int32_t mode, int32_t trace, float *d
             if (ec != hipSuccess) return hip_fail(ec);
             B->graph = g;
             HIPCHECK(hipGraphInstantiate(&B->graph_exec, g, nullptr, nullptr, 0));
-            B->graph_trace = bp.trace;
+            B->graph_trace = with_trace;
         }
         HIPCHECK(hipGraphLaunch(B->graph_exec, B->stream));
     }
@@ -1746,7 +1955,7 @@ extern "C" int lcg_batch_run(lcg_batch *B, int32_t mode, int32_t trace, float *d
     }
     B->have_results = true;
     B->fetched = false;
-    B->traced = bp.trace != 0;
+    B->traced = with_trace != 0;
     B->norm_valid = false;
     return LCG_OK;
 }
@@ -1770,14 +1979,11 @@ extern "C" int lcg_batch_run_noalloc(lcg_batch *B, int32_t trace) {
     if (int rc = lcg_noalloc_scratch(B->device, &S, &cap)) return hip_fail((hipError_t)rc);
     const long long bar_off = 64;                                 // queues at 0 and 16
     const long long top_off = (bar_off + B->npairs + 63) & ~63LL;  // 256-byte aligned
-    const long long per_wg = (long long)B->top_waves * B->top_max;
+    const long long per_wg = (long long)B->parts.top.waves * B->top_max;
     if (top_off + per_wg > cap) return LCG_E_CAPACITY;
-    const int top_grid = (int)std::min<long long>(B->top_grid, (cap - top_off) / per_wg);
-    BatchParams bp = B->bp, top = B->bp_top;
-    bp.trace = top.trace = trace & 1;
-    bp.count = top.count = 0;
-    if (int rc = lcg_launch_align(B->d_descs, B->d_order, S, B->d_arena, S + top_off, S + bar_off, bp, B->grid,
-                                  B->waves, B->lds_bytes, top, top_grid, B->top_waves, B->top_lds_bytes, nullptr, 0,
+    LaunchParts parts = run_parts(*B, trace & 1, 0);
+    parts.top.grid = (int)std::min<long long>(parts.top.grid, (cap - top_off) / per_wg);
+    if (int rc = lcg_launch_align(B->d_descs, B->d_order, S, B->d_arena, S + top_off, S + bar_off, &parts, nullptr, 0,
                                   nullptr, B->stream))
         return hip_fail((hipError_t)rc);
     B->fill_ms = B->top_ms = -1;
@@ -1796,12 +2002,9 @@ inline int32_t res(const lcg_batch *B, int k, int32_t off);
 // top level and traceback again over the D of the last run).
 int run_with_penalty(lcg_batch *B, bool top_only, float *device_ms) {
     HIPCHECK(hipSetDevice(B->device));
-    BatchParams bp = B->bp, top = B->bp_top;
-    bp.trace = top.trace = 1;
-    bp.count = top.count = 0;
+    const LaunchParts parts = run_parts(*B, 1, 0);
     HIPCHECK(hipEventRecord(B->ev0, B->stream));
-    int rc = lcg_launch_align(B->d_descs, B->d_order, B->d_queue, B->d_arena, B->d_scratch, B->d_barriers, bp,
-                              B->grid, B->waves, B->lds_bytes, top, B->top_grid, B->top_waves, B->top_lds_bytes,
+    int rc = lcg_launch_align(B->d_descs, B->d_order, B->d_queue, B->d_arena, B->d_scratch, B->d_barriers, &parts,
                               B->d_lambda, top_only ? 1 : 0, nullptr, B->stream);
     if (rc) return hip_fail((hipError_t)rc);
     HIPCHECK(hipEventRecord(B->ev1, B->stream));
@@ -1947,7 +2150,7 @@ int restricted_top(lcg_batch *B, int k, const int32_t r[4], bool trace, int64_t 
     if (need > B->kscratch_ints) {
         if (B->d_kscratch) HIPCHECK(hipFree(B->d_kscratch));
         B->d_kscratch = nullptr;
-        HIPCHECK(hipMalloc(&B->d_kscratch, need * B->top_waves * 4));
+        HIPCHECK(hipMalloc(&B->d_kscratch, need * B->parts.top.waves * 4));
         B->kscratch_ints = need;
     }
     if (!B->d_restr) HIPCHECK(hipMalloc(&B->d_restr, 16 * (size_t)B->npairs));
@@ -1959,14 +2162,12 @@ int restricted_top(lcg_batch *B, int k, const int32_t r[4], bool trace, int64_t 
     for (int t = 0; t < B->npairs && pos < 0; ++t)
         if (B->order[t] == k) pos = t;
     if (pos < 0) return LCG_E_STATE;
-    BatchParams bp = B->bp, top = B->bp_top;
-    bp.npairs = top.npairs = 1;
-    bp.trace = top.trace = trace ? 1 : 0;
-    bp.count = top.count = 0;
-    top.scratch_stride = (int32_t)B->kscratch_ints;
-    int rc = lcg_launch_align(B->d_descs, B->d_order + pos, B->d_queue, B->d_arena, B->d_kscratch, B->d_barriers, bp,
-                              1, B->waves, B->lds_bytes, top, 1, B->top_waves, B->top_lds_bytes, nullptr, 1, nullptr,
-                              B->stream, B->d_restr);
+    LaunchParts parts = run_parts(*B, trace ? 1 : 0, 0);
+    parts.top.bp.npairs = 1;
+    parts.top.grid = 1;
+    parts.top.bp.scratch_stride = (int32_t)B->kscratch_ints;
+    int rc = lcg_launch_align(B->d_descs, B->d_order + pos, B->d_queue, B->d_arena, B->d_kscratch, B->d_barriers, &parts,
+                              nullptr, 1, nullptr, B->stream, B->d_restr);
     if (rc) return hip_fail((hipError_t)rc);
     HIPCHECK(hipStreamSynchronize(B->stream));
     B->fill_ms = B->top_ms = -1;
@@ -3155,6 +3356,7 @@ extern "C" int lcg_batch_reshape(lcg_batch *B, const lcg_shape *shape, char *err
     }
     const size_t old_scratch = scratch_ints(*B);
     apply_shape(*B, fs, ts);
+    HIPCHECK(upload_deal(*B));
     const size_t new_scratch = scratch_ints(*B);
     if (new_scratch > old_scratch) {
         HIPCHECK(hipFree(B->d_scratch));
@@ -3230,10 +3432,10 @@ extern "C" int lcg_batch_autotune(lcg_batch *B, int32_t path, int32_t reps, lcg_
         };
         if (np >= cus) {
             const int wg[][2] = {{16, 1}, {12, 1}, {8, 1}, {8, 2}, {4, 2}, {4, 4}};
-            for (auto &x : wg) add_fill(x[0], x[1], 1);
+            for (auto &x : wg) add_fill(x[0], x[1], 0);
         } else {
             const int kmax = std::min(64, cus / np);
-            std::vector<int> ks = {kmax, kmax / 2, kmax / 4, 1};
+            std::vector<int> ks = {kmax, kmax / 2, kmax / 4, 1};  // besides the starting shape's
             ks.erase(std::remove_if(ks.begin(), ks.end(), [](int k) { return k < 1; }), ks.end());
             std::sort(ks.begin(), ks.end(), std::greater<int>());
             ks.erase(std::unique(ks.begin(), ks.end()), ks.end());

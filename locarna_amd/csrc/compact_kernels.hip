@@ -83,7 +83,7 @@ __device__ __forceinline__ void block_scan2(int a, int b, int &ea, int &eb, int 
 
 struct CPair {
     int n, m, NA, NB, W64;
-    const int *arcsA, *arcsB, *wA, *wB, *ptA, *ptB, *lA, *lB, *rpA, *rpB, *radjA, *radjB, *tab;
+    const int *arcsA, *arcsB, *wA, *wB, *ptA, *ptB, *lA, *lB, *rpA, *rpB, *radjA, *radjB, *fordB, *tab;
     int tau, ribosum, dlen, dend;
     const int *mn, *mx, *coff;  // LDS: band of A's rows, band cell offsets
     uint64_t *bits;
@@ -109,6 +109,7 @@ __device__ CPair make_cpair(const CompactDesc &c, const int *cin, int *ws, int *
     P.rpB = cin + c.rpB;
     P.radjA = cin + c.radjA;
     P.radjB = cin + c.radjB;
+    P.fordB = cin + c.fordB;
     P.tab = cin + c.tab;
     P.tau = c.tau;
     P.ribosum = c.ribosum;
@@ -500,15 +501,16 @@ __global__ __launch_bounds__(CT) void lcg_compact_build(const CompactDesc *__res
     }
     // fill-list row pointers: first block of right end i
     for (int i = threadIdx.x; i <= P.n + 1; i += CT) arena[d.fptr + i] = P.sblk[P.rpA[i]];
-    // fill entries of a block: arcs of B in right adjacency order
+    // fill entries of a block: arcs of B in fill order
     for (int bi = threadIdx.x >> 6; bi < nblk; bi += CW) {
         const int a = P.blka[bi];
         const int p = left_of(P.arcsA[a]);
-        const int mnp = P.mn[p - 1];
+        const int i = right_of(P.arcsA[a]);
+        const int mnp = P.mn[p - 1], mni = P.mn[i];
         int tf = P.blks[bi];
         for (int base = 0; base < P.NB; base += 64) {
             const int v = base + lane;
-            const int b = v < P.NB ? P.radjB[v] : 0;
+            const int b = v < P.NB ? P.fordB[v] : 0;
             const bool ok = v < P.NB && has_bit(P, a, b);
             const uint64_t mask = __ballot(ok);
             if (ok) {
@@ -516,10 +518,11 @@ __global__ __launch_bounds__(CT) void lcg_compact_build(const CompactDesc *__res
                 const int x = am_index(P, a, b);
                 const int arcB = P.arcsB[b];
                 if (t < nam && x < nam) {
-                    int *F = arena + d.fcand + 3 * (size_t)t;
-                    F[0] = p | (left_of(arcB) << 16);
-                    F[1] = right_of(arcB) | (mnp << 16);
-                    F[2] = LCG_NEG;
+                    const int q = left_of(arcB), j = right_of(arcB);
+                    *reinterpret_cast<int2 *>(arena + d.fcand + 2 * (size_t)t) =
+                        make_int2(p | (q << 16), j | (mnp << 16));
+                    *reinterpret_cast<int2 *>(arena + d.fband + 2 * (size_t)t) =
+                        make_int2((int)LCG_FBAND(P.coff[p - 1] + (q - 1 - mnp), j - mni), LCG_NEG);
                     P.fof[x] = t;
                 } else {
                     s_status = 2;
@@ -599,6 +602,11 @@ __global__ __launch_bounds__(CT) void lcg_compact_build(const CompactDesc *__res
                 --s;
             }
             idx[s] = x;
+        }
+        for (int t = 0; t < cnt; ++t) {  // the band fill's order: ar descending
+            const int *G = Gt + (size_t)idx[t] * LCG_GROUP_INTS;
+            reinterpret_cast<int4 *>(arena + d.gtask)[g0 + t] =
+                make_int4((G[0] >> 16) | ((G[1] & 0xffff) << 16), G[3], G[4], idx[t]);
         }
         for (int mm = 0; mm < K; ++mm) load[mm] = 0;
         for (int t = 0; t < cnt; ++t) {

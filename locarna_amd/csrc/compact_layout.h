@@ -43,7 +43,8 @@ typedef struct {
     int32_t ws_sched;      // 3 * ngroups + K * (n + 2): schedule scratch
     int32_t hdr, hdr_len;  // head of the pair's image (band, codes, gap
                            // scores, sigma), copied to the arena by pass 2
-    int32_t pad[2];
+    int32_t fordB;         // NB: arcs of B in the order of a fill block (fill_order)
+    int32_t pad;
 } CompactDesc;  // 36 ints
 
 // Per-pair results of the counting pass (and status of the build pass).

@@ -34,11 +34,19 @@
 //                                       right end i), rows i ascending, p
 //                                       descending within a row: (p, first
 //                                       fill entry); sentinel (0, nam)
-//   fcand:    3 per entry               the arc matches again, by block,
-//                                       j ascending: (p | q<<16,
-//                                       j | min_col(p-1)<<16, D(am)); a group
+//   fcand:    2 per entry               the arc matches again, by block, a
+//                                       block's in fill order: (p | q<<16,
+//                                       j | min_col(p-1)<<16); a group
 //                                       with left end al reads the prefix
 //                                       p > al of each row
+//   fband:    2 per entry               the same entries by band cells:
+//                                       (LCG_FBAND of the cell (p-1, q-1)
+//                                       and of the column of j in row i,
+//                                       D(am))
+//   gtask:    4 per group               the groups of each left end by ar
+//                                       descending (their order within
+//                                       equal ar): (bl | ar<<16, am_begin,
+//                                       am_end, group)
 //   f2c:      per fill entry            its index in cand (cell order)
 //   D:        per arc match (output of the fill, reference index order)
 //   edges:    n + m + 1 slots (output): slot i+j holds the edge that reaches
@@ -60,12 +68,18 @@
 // the current row, M the matrix rows al..ar-1 (row i stored from column
 // max(bl, min_col(i))).
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 
 #define LCG_NEG (-(1 << 29))        /* normalized minus infinity */
 #define LCG_NEG_LIMIT (-(1 << 28))  /* values below are minus infinity */
 #define LCG_GROUP_INTS 8
 #define LCG_NCODES 8
+/* Words of the band fill, whose rows hold at most LCG_BAND_COLS columns, so
+ * that a pair has less than 2^24 band cells and a column of a row fits 8
+ * bits (pairs with wider rows do not use them). */
+#define LCG_FBAND(src, c) (((uint32_t)(src) & 0xffffffu) | ((uint32_t)(c) << 24))
+#define LCG_BAND_COLS 128 /* widest band row of the band kernels */
 
 typedef struct {
     int32_t n, m;
@@ -85,7 +99,11 @@ typedef struct {
     int32_t c2a;       // --noLP / --stacking only: candidate entry -> arc match
     int32_t amst;      // --stacking only: per arc match its stacked score, LCG_NEG if not stackable
     int32_t slmax;     // --struct-local: ints of the largest group region (eight states)
-} PairDesc;  // 33 ints
+    int32_t fband, gtask;
+    int32_t band_need; // pool ints the band kernels need for this pair, 0: they do not
+                       // apply (a band row wider than LCG_BAND_COLS, or bounds that decrease)
+    int32_t pad;
+} PairDesc;  // 37 ints
 
 typedef struct {
     int32_t alpha;           // indel opening
@@ -97,7 +115,7 @@ typedef struct {
     int32_t max_len;         // max sequence length over the batch
     int32_t count;           // count DP cells and arc candidates (out[4..11])
     int32_t scratch_stride;  // ints of global scratch per (workgroup, wave)
-    int32_t fixed_cols;      // fill narrow groups with the fixed-column kernel
+    int32_t fixed_cols;      // fill narrow groups with the fixed-column kernels
     int32_t fptr_lds;        // LDS offsets (ints) of the pair's fptr and fblk
     int32_t fblk_lds;
     int32_t wg_per_pair;     // workgroups sharing one pair in the fill of D
@@ -114,4 +132,32 @@ typedef struct {
     int32_t exclusion;       // --exclusion: score of one excluded block
     int32_t sl_stride;       // ints of global scratch per (workgroup, wave) of the
                              // fill with --struct-local
+    int32_t band;            // general fill: pool ints of the band fill, which takes the
+                             // pairs that need no more (0: no band fill)
+    int32_t band_lds;        // band fill: LDS offset (ints, even) of its part of the header
+    int32_t dealt;           // band fill: workgroups with a pair of their own to start
+    int32_t dealt_pairs;     // with, and the pairs they have; the others are queued
+    int32_t band_latency;    // fewer pairs than CUs: a group per wave where the
+                             // waves and the pool allow it, not two
 } BatchParams;
+
+// One kernel launch of a run (waves 0: not launched).
+typedef struct {
+    BatchParams bp;
+    int32_t grid, waves;
+    size_t lds_bytes;
+} LaunchPart;
+// The launches of a run: general fill, band fill, top level / traceback.
+// deal (device): 3 per workgroup of the band fill below bp.dealt: place in
+// the work order, member, members.
+typedef struct {
+    LaunchPart fill, band, top;
+    const int32_t *deal;
+} LaunchParts;
+
+// LDS ints of a region of the band fill: rows of CW columns per group, G
+// groups per wave, `cells` band cells per group: the arc maxima of four rows,
+// the matrix and the overhang of an unpredicated row store.
+#define LCG_BAND_REGION(G, CW, cells) ((4 * (G) * (CW) + (G) * ((cells) + (CW)) + 3) & ~3)
+// ints past the arena's last image: the band fill loads fill entries 64 at a time
+#define LCG_ARENA_PAD 512

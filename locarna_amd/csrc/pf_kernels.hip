@@ -436,8 +436,8 @@ __device__ __forceinline__ PfEnt pf_fetch(const PfPair &P, int t, int t1) {
     PfEnt e;
     struct PJ {
         int x, y;
-    };  // 4-byte aligned pair (one 8-byte load)
-    const PJ pj = *reinterpret_cast<const PJ *>(P.fcand + 3 * tt);
+    };
+    const PJ pj = *reinterpret_cast<const PJ *>(P.fcand + 2 * tt);
     e.pq = pj.x;
     e.jm = pj.y;
     e.D = P.fD[tt];
