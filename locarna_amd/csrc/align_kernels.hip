@@ -1824,14 +1824,19 @@ __device__ __forceinline__ void fill_band(const PairDesc *__restrict__ descs, co
                 const int g0 = uniform(lrows[al + 1]), ng = uniform(lrows[al]) - g0;
                 band_row<TAB>(P, V, bp, now, gtask + g0, gams, al, ng, member, K, pool);
                 if (K > 1) {
-                    // every member's D of the row is written before any
-                    // member reads it in a later row
-                    __threadfence();
+                    // every member's D of the row is written before any member
+                    // reads it in a later row: the waves' stores are in the L2
+                    // before one wave writes it back, and after the barrier
+                    // drops what the CU's L1 holds
+                    __threadfence_block();
                     __syncthreads();
                     ++passed;
-                    if (threadIdx.x == 0) meet(&barriers[k], K * passed, spin_lim, &arena[d.out + 3]);
+                    if (threadIdx.x == 0) {
+                        __threadfence();
+                        meet(&barriers[k], K * passed, spin_lim, &arena[d.out + 3]);
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                    }
                     __syncthreads();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
                 } else {
                     __threadfence_block();
                     __syncthreads();
