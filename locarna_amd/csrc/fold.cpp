@@ -6,8 +6,8 @@
 // with p > --min-prob (RnaData, rna_data.cc:509-547) and writes them as a
 // `#PP 2.0` text (RnaData::write_pp, rna_data.cc:1242-1350).  Here the
 // partition function is the McCaskill recursion over the energy model of
-// fold_model.h, run by lcg_fold_seqs (fold_kernels.hip), one workgroup per
-// sequence; the text is the same writer's layout.
+// fold_model.h, run by lcg_fold_seqs (fold_kernels.hip), one workgroup or
+// several per sequence; the text is the same writer's layout.
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
@@ -23,15 +23,17 @@
 #include "host.hpp"
 #include "locarna_amd.h"
 
+extern "C" size_t lcg_fold_lds_bytes(int nmax, int nch);
 extern "C" int lcg_launch_fold(const FoldDesc *descs, const signed char *codes, const double *tabs, double *mats,
-                               double *outs, double *zout, int nseq, int nmax, hipStream_t stream);
+                               double *outs, double *zout, int *counters, int *status, const int *seq_of, int grid,
+                               int nmax, int nch, hipStream_t stream);
 
 struct lcg_fold {
     lcg_fold_params p{};
     std::vector<std::string> seq;  // normalized: upper case, T -> U
     std::vector<int> W;
     std::vector<size_t> out;       // offset of sequence k's P band in `bands`
-    std::vector<double> bands;     // P and P2 bands of every sequence
+    std::unique_ptr<double[]> bands;  // P and P2 bands of every sequence
     std::vector<double> Z;     // scaled partition functions
     std::vector<double> logz;  // natural logarithms of the partition functions
     float device_ms = 0, wall_ms = 0;
@@ -51,8 +53,9 @@ void set_err(char *err, int errlen, const std::string &msg) {
 }
 
 // Boltzmann factors of the loop terms, laid out as fold_layout.h describes;
-// the terms depend on the pair types only through weak / strong except the
-// stacks and the one-base bulges (which include a stack)
+// the terms depend on the pair types only through weak / strong, each pair
+// adding its own term to the energy, except the stacks and the one-base
+// bulges (which include a stack)
 std::vector<double> factor_table(int nmax) {
     using namespace locarna_amd::fold_model;
     std::vector<double> T(LCG_FOLD_TAB_HP + 2 * (size_t)(nmax + 2), 0.0);
@@ -60,14 +63,14 @@ std::vector<double> factor_table(int nmax) {
     for (int l1 = 0; l1 <= MAX_LOOP; ++l1)
         for (int l2 = 0; l1 + l2 <= MAX_LOOP; ++l2) {
             if (l1 + l2 < 2) continue;
-            for (int wo = 0; wo < 2; ++wo)
-                for (int wi = 0; wi < 2; ++wi) {
-                    const int to = rep[wo], ti = rep[wi];
-                    const double e = (l1 == 0 || l2 == 0) ? bulge_energy(l1 + l2, to, ti, 0.0)
-                                                          : interior_energy(l1, l2, to, ti);
-                    T[LCG_FOLD_TAB_LOOP + (l1 * 31 + l2) * 4 + wo * 2 + wi] = bf(e);
-                }
+            const double e = (l1 == 0 || l2 == 0) ? bulge_energy(l1 + l2, rep[0], rep[0], 0.0)
+                                                  : interior_energy(l1, l2, rep[0], rep[0]);
+            T[LCG_FOLD_TAB_LOOP + l1 * 31 + l2] = bf(e);
         }
+    for (int w = 0; w < 2; ++w) {
+        T[LCG_FOLD_TAB_GI + w] = bf(interior_energy(1, 1, rep[0], rep[w]) - interior_energy(1, 1, rep[0], rep[0]));
+        T[LCG_FOLD_TAB_GU + w] = bf(bulge_energy(2, rep[0], rep[w], 0.0) - bulge_energy(2, rep[0], rep[0], 0.0));
+    }
     for (int to = 1; to <= 6; ++to)
         for (int ti = 1; ti <= 6; ++ti) {
             char X, Xp, Y, Yp;
@@ -97,6 +100,38 @@ signed char code_of(char c) {
     case 'U': return 3;
     default: return 4;
     }
+}
+
+// Workgroups of each sequence (FoldDesc.K), chunks of 64 cells per batch, and
+// the sequence and member of every workgroup, longest sequences first.  Up to
+// 256 nt a sequence has one workgroup: 64 of 60-200 nt take 2.45 ms so and
+// 2.79 ms on several, one of 75 nt 1.10 and 1.17 ms (a barrier per diagonal
+// takes longer than the cells it divides).  Longer ones get one per 64 cells
+// as far as the CUs go: two of 700-800 nt 26.8 ms against 121 ms.
+std::vector<int> deal_workgroups(std::vector<FoldDesc> &descs, int cus, int nmax, int &nch) {
+    const int count = (int)descs.size();
+    auto chunks = [&](const FoldDesc &d) { return std::max(1, (d.n + 63) / 64); };
+    int cap = 1;
+    if (nmax > 256)
+        for (int c = 2; c <= 64; ++c) {
+            long sum = 0;
+            for (const FoldDesc &d : descs) sum += std::min(c, chunks(d));
+            if (sum > cus) break;
+            cap = c;
+        }
+    nch = cap > 1 || nmax <= 64 ? 1 : nmax <= 128 ? 2 : 4;
+    while (nch > 1 && lcg_fold_lds_bytes(nmax, nch) > 160 * 1024 - 1024) nch /= 2;
+    std::vector<int> by_len(count), out;
+    for (int k = 0; k < count; ++k) by_len[k] = k;
+    std::stable_sort(by_len.begin(), by_len.end(), [&](int a, int b) { return descs[a].n > descs[b].n; });
+    for (int k : by_len) {
+        descs[k].K = std::min(cap, chunks(descs[k]));
+        for (int m = 0; m < descs[k].K; ++m) {
+            out.push_back(k);
+            out.push_back(m);
+        }
+    }
+    return out;
 }
 
 struct DevBuf {
@@ -152,12 +187,12 @@ extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fo
         codes.push_back(4);
         for (char c : s) codes.push_back(code_of(c));
         codes.push_back(4);
-        const size_t sz = (size_t)(n + 2) * W;
+        D.S = (n + 2 + 15) & ~15;
         D.mat = (long long)mat;
         D.out = (long long)outd;
         F->out[k] = outd;
-        mat += 6 * sz;
-        outd += 2 * sz;
+        mat += ((size_t)6 * W + LCG_FOLD_RINGS + 2) * D.S + LCG_FOLD_PAD;
+        outd += 2 * (size_t)(n + 2) * W;
         F->W[k] = W;
         F->seq[k] = std::move(s);
         nmax = std::max(nmax, n);
@@ -170,14 +205,23 @@ extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fo
         return LCG_E_HIP;
     };
     if ((e = hipSetDevice(device)) != hipSuccess) return hip_fail(e);
-    DevBuf dd, dc, dt, dm, dout, dz;
+    int cus = 1;
+    if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device)) != hipSuccess)
+        return hip_fail(e);
+    int nch = 4;
+    const std::vector<int> seq_of = deal_workgroups(descs, cus, nmax, nch);
+    const int grid = (int)seq_of.size() / 2;
+    DevBuf dd, dc, dt, dm, dout, dz, db, ds;
     if ((e = hipMalloc(&dd.p, sizeof(FoldDesc) * count)) || (e = hipMalloc(&dc.p, codes.size())) ||
         (e = hipMalloc(&dt.p, tabs.size() * sizeof(double))) || (e = hipMalloc(&dm.p, mat * sizeof(double))) ||
-        (e = hipMalloc(&dout.p, outd * sizeof(double))) || (e = hipMalloc(&dz.p, count * sizeof(double))))
+        (e = hipMalloc(&dout.p, outd * sizeof(double))) || (e = hipMalloc(&dz.p, count * sizeof(double))) ||
+        (e = hipMalloc(&db.p, (count + 1) * sizeof(int))) || (e = hipMalloc(&ds.p, seq_of.size() * sizeof(int))))
         return hip_fail(e);
     if ((e = hipMemcpy(dc.p, codes.data(), codes.size(), hipMemcpyHostToDevice)) ||
-        (e = hipMemcpy(dt.p, tabs.data(), tabs.size() * sizeof(double), hipMemcpyHostToDevice)))
+        (e = hipMemcpy(dt.p, tabs.data(), tabs.size() * sizeof(double), hipMemcpyHostToDevice)) ||
+        (e = hipMemcpy(ds.p, seq_of.data(), seq_of.size() * sizeof(int), hipMemcpyHostToDevice)))
         return hip_fail(e);
+    if ((e = hipMemsetAsync(dm.p, 0, mat * sizeof(double), 0))) return hip_fail(e);
     hipEvent_t ev0, ev1;
     if ((e = hipEventCreate(&ev0))) return hip_fail(e);
     if ((e = hipEventCreate(&ev1))) {
@@ -204,9 +248,15 @@ extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fo
             rc = hip_fail(e);
             break;
         }
+        // arrival counters of the sequences on several workgroups, and the status
+        if ((e = hipMemsetAsync(db.p, 0, (count + 1) * sizeof(int), 0))) {
+            rc = hip_fail(e);
+            break;
+        }
         (void)hipEventRecord(ev0, 0);
         int lr = lcg_launch_fold((const FoldDesc *)dd.p, (const signed char *)dc.p, (const double *)dt.p,
-                                 (double *)dm.p, (double *)dout.p, (double *)dz.p, count, nmax, 0);
+                                 (double *)dm.p, (double *)dout.p, (double *)dz.p, (int *)db.p, (int *)db.p + count,
+                                 (const int *)ds.p, grid, nmax, nch, 0);
         (void)hipEventRecord(ev1, 0);
         if (lr) {
             rc = hip_fail((hipError_t)lr);
@@ -223,6 +273,18 @@ extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fo
         if ((e = hipMemcpy(F->Z.data(), dz.p, count * sizeof(double), hipMemcpyDeviceToHost))) {
             rc = hip_fail(e);
             break;
+        }
+        if (grid > count) {  // some sequences on several workgroups
+            int expired = 0;
+            if ((e = hipMemcpy(&expired, (int *)db.p + count, sizeof(int), hipMemcpyDeviceToHost))) {
+                rc = hip_fail(e);
+                break;
+            }
+            if (expired) {
+                set_err(err, errlen, "a wait between the workgroups of a sequence expired");
+                rc = LCG_E_STATE;
+                break;
+            }
         }
         bool all = true;
         for (int k = 0; k < count; ++k) {
@@ -253,8 +315,8 @@ extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fo
                 break;
             }
     if (rc == LCG_OK) {
-        F->bands.resize(outd);
-        if ((e = hipMemcpy(F->bands.data(), dout.p, outd * sizeof(double), hipMemcpyDeviceToHost))) rc = hip_fail(e);
+        F->bands.reset(new double[outd]);
+        if ((e = hipMemcpy(F->bands.get(), dout.p, outd * sizeof(double), hipMemcpyDeviceToHost))) rc = hip_fail(e);
         for (int k = 0; k < count; ++k) F->logz[k] = std::log(F->Z[k]) + (double)F->seq[k].size() * (-g[k] / kT);
     }
     (void)hipEventDestroy(ev0);
@@ -271,7 +333,7 @@ extern "C" int lcg_fold_probs(const lcg_fold *f, int32_t k, double *P, double *P
     const int64_t need = (int64_t)(n + 1) * (n + 1);
     if ((!P && !P2) || cap < need) return LCG_E_ARG;
     const size_t sz = (size_t)(n + 2) * W;
-    const double *bp = f->bands.data() + f->out[k];
+    const double *bp = f->bands.get() + f->out[k];
     for (int pass = 0; pass < 2; ++pass) {
         double *M = pass ? P2 : P;
         if (!M) continue;
@@ -302,7 +364,7 @@ extern "C" int64_t lcg_fold_write_pp(const lcg_fold *f, int32_t k, const char *n
     const std::string &s = f->seq[k];
     const int n = (int)s.size(), W = f->W[k];
     const size_t sz = (size_t)(n + 2) * W;
-    const double *bp = f->bands.data() + f->out[k];
+    const double *bp = f->bands.get() + f->out[k];
     const double cut = f->p.min_prob;
     const bool stack = f->p.stacking != 0;
     // RnaData::write_pp (rna_data.cc:1242-1350): the sequence block with a

@@ -3,98 +3,137 @@
 // that mlocarna runs once per sequence (locarna_rnafold_pp ->
 // RnaEnsemble, rna_ensemble.cc:141-193; mlocarna:3148-3188).
 //
-// One workgroup of 16 waves folds one sequence.  The inside pass walks the
-// diagonals d = j - i upward; the cells of a diagonal are independent, a
-// quarter wave (16 lanes) per cell, and the lanes of a cell split its terms
-// (interior loops, multiloop splits) and sum them with a butterfly; 16
-// lanes per cell measured faster than 8, 32 or 64 on 64 sequences of 60-200 nt
-// (the work is latency-bound: more cells in flight per wave).  The exterior
-// prefix sums Z5 (forward) and Z5b (their adjoints) run on one wave.  The
-// outside pass walks the diagonals downward and gathers, for every cell, the
-// terms of the enclosing cells that use it (the pull form of the adjoint of
-// the inside recursions), so that no cell is written by more than one wave
-// and the result does not depend on the schedule.  The probabilities
-// P = Qb Qbb / Z and the stacked joint probabilities are written as the
-// outside value of a cell is known.
-//
 // Recursions (1-based, t = pair type of (i, j), 0 when (i, j) cannot pair):
-//   Qb(i,j)  = H(i,j) + sum_{k,l} L(i,j,k,l) Qb(k,l)
-//              + MLC TP(t) sum_u Qm(i+1,u-1) Qm1(u,j-1)
-//   Qm1(i,j) = sum_{l <= j} Qb(i,l) BR(i,l)
-//   Qm(i,j)  = sum_{u >= i} (1 + Qm(i,u-1)) Qm1(u,j)
-//   Z5(j)    = Z5(j-1) + sum_k Z5(k-1) Qb(k,j) EXT(k,j),  Z = Z5(n)
+//   Qb(i,j)  = H(i,j) + sum_{k,l} L(i,j,k,l) Qb(k,l) + MLC TP(t) M2(i+1,j-1)
+//   Qm1(i,j) = s Qm1(i,j-1) + Qb(i,j) BR(t)
+//   M2(i,j)  = sum_u Qm(i,u-1) Qm1(u,j)
+//   Y(i,j)   = Qm1(i,j) + s Y(i+1,j),  Qm(i,j) = Y(i,j) + M2(i,j)
+//   Z5(j)    = s Z5(j-1) + sum_k Z5(k-1) Qb(k,j) EXT(k,j),  Z = Z5(n)
+// and outside, the pull form of the adjoints (b marks them; every cell is
+// written once and the result does not depend on the schedule):
+//   X(a,e)    = Qmb(a,e) + MLC TP Qbb(a-1,e+1)
+//   Qmb(a,e)  = sum_j X(a,j) Qm1(e+1,j)
+//   U(a,e)    = Qmb(a,e) + s U(a-1,e)
+//   Qm1b(a,e) = sum_i X(i,e) Qm(i,a-1) + U(a,e)
+//   R(a,e)    = Qm1b(a,e) + s R(a,e+1)
+//   Qbb(a,e)  = Z5b(e) Z5(a-1) EXT + sum_{i,j} L(i,j,a,e) Qbb(i,j)
+//               + BR (s R(a,e+1) + Qm1b(a,e))
+// so that besides the interior loops one sum over the splits is left inside
+// and two outside.  P = Qb Qbb / Z, P2(i,j) = Qbb(i,j) stack Qb(i+1,j-1) / Z.
 // Every value of a segment of L bases is stored times sigma^-L (sigma per
 // sequence, FoldDesc.log_sigma; ViennaRNA's per-nucleotide pf_scale), so
-// each term carries sigma^-(bases it adds): SC[l1 + l2 + 2] on an interior
-// loop, SC[2] on a multiloop's closing pair, SC[d + 1] on a hairpin, SC[j - l]
-// on the unpaired tail of a branch, SC[1] per exterior base.  The
-// probabilities do not depend on sigma; log Z = log Z5(n) + n log sigma.
+// each term carries sigma^-(bases it adds): s = sigma^-1 per unpaired base,
+// sigma^-(l1 + l2 + 2) on an interior loop.  The probabilities do not depend
+// on sigma; log Z = log Z5(n) + n log sigma.
+//
+// A loop's factor is the product of one for (l1, l2) and one for each of its
+// pairs (weak or not), except for stacks and one-base bulges.  Qb is also
+// stored times the inner pair's factor, so that a term of an interior loop is
+// one load and one multiply-add with a factor that is the same for all cells.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "fold_layout.h"
 
 namespace {
 
-constexpr int FT = LCG_FOLD_THREADS;
-#ifndef LCG_FOLD_CELL_LANES
-#define LCG_FOLD_CELL_LANES 16
-#endif
-// lanes per cell: a wave works on 64 / CL cells of a diagonal at once
-constexpr int CL = LCG_FOLD_CELL_LANES;
-
-// sum over the CL lanes of a cell
-__device__ __forceinline__ double cell_sum(double v) {
-#pragma unroll
-    for (int o = CL / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
+constexpr int FT = LCG_FOLD_THREADS, NWV = FT / 64;
+constexpr int MAXLOOP = LCG_FOLD_MAXLOOP;
 
 __device__ __forceinline__ int weak(int t) { return (0x72 >> t) & 1; }
+__device__ __forceinline__ double readlane_d(double v, int l) {
+    const long long x = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((int)x, l), hi = __builtin_amdgcn_readlane((int)(x >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | lo);
+}
 
 struct Seq {
     const signed char *cs;  // codes in LDS, position i at cs[i]
     const int *ptab;        // pair type of (code a, code b) at a * 5 + b
-    int n, W;
-    // pair type of (i, j) with the hairpin and span limits, 0 if none
-    __device__ __forceinline__ int pt(int i, int j) const {
-        const int d = j - i;
-        return (d >= 4 && d < W) ? ptab[cs[i] * 5 + cs[j]] : 0;
-    }
+    // pair type of (i, i + d), 0 if none
+    __device__ __forceinline__ int pt(int i, int j) const { return ptab[cs[i] * 5 + cs[j]]; }
 };
 
-__device__ __forceinline__ double loopf(const double *T, int l1, int l2, int to, int ti) {
-    const int s = l1 + l2;
-    if (s == 0) return T[LCG_FOLD_TAB_STACK + to * 8 + ti];
-    if (s == 1) return T[LCG_FOLD_TAB_BULGE1 + to * 8 + ti];
-    return T[LCG_FOLD_TAB_LOOP + (l1 * 31 + l2) * 4 + weak(to) * 2 + weak(ti)];
+// The loop terms of a wave, one per lane: lanes 0..3 bulges of two bases and
+// more, lanes 4..31 interior loops, by loop size within each kind.  Wave w
+// has every 16th of the 58 bulges and 435 interior loops.
+struct Terms {
+    int s, l1;     // unpaired bases (99: none), those of the 5' side
+    double f;      // factor with two strong pairs, times sigma^-(s + 2)
+};
+
+__device__ __forceinline__ Terms wave_terms(int w, int lane, const double *tabs, double log_sigma) {
+    Terms t{99, 0, 0.0};
+    int l2 = 0;
+    if (lane < 4) {
+        const int e = w + NWV * lane;
+        if (e < 2 * (MAXLOOP - 1)) {
+            t.s = 2 + e / 2;
+            t.l1 = (e & 1) ? t.s : 0;
+        }
+    } else if (lane < 32) {
+        int x = w + NWV * (lane - 4), s = 2;
+        while (s <= MAXLOOP && x >= s - 1) x -= s - 1, ++s;
+        if (s <= MAXLOOP) {
+            t.s = s;
+            t.l1 = 1 + x;
+        }
+    }
+    if (t.s < 99) {
+        l2 = t.s - t.l1;
+        t.f = tabs[LCG_FOLD_TAB_LOOP + t.l1 * (MAXLOOP + 1) + l2] * exp(-(double)(t.s + 2) * log_sigma);
+    }
+    return t;
 }
 
-// number of (l1, l2) entries with l1 + l2 <= s
-__device__ __forceinline__ int loop_count(int s) { return s < 0 ? 0 : (s + 1) * (s + 2) / 2; }
+// Arrival at a sequence's barrier and bounded wait for `target` arrivals.
+__device__ __forceinline__ void meet(int *counter, int target, int *status) {
+    atomicAdd(counter, 1);
+    for (int spin = 0; atomicAdd(counter, 0) < target; ++spin) {
+        if (spin > (1 << 22)) {
+            atomicExch(status, 2);
+            break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
 
 }  // namespace
 
-extern "C" __global__ __launch_bounds__(FT) void lcg_fold_seqs(const FoldDesc *descs, const signed char *codes,
-                                                               const double *tabs, double *mats, double *outs,
-                                                               double *zout, int nseq) {
-    extern __shared__ double lds[];
-    const int sq = blockIdx.x;
-    if (sq >= nseq) return;
-    const FoldDesc D = descs[sq];
-    const int n = D.n, W = D.W;
-    double *T = lds;                       // fixed factor table
-    double *Z5 = T + LCG_FOLD_TAB_FIXED;   // n + 1
-    double *Z5b = Z5 + (n + 1);            // n + 1
-    double *SC = Z5b + (n + 1);            // n + 2: SC[L] = sigma^-L
-    int *ptab = (int *)(SC + (n + 2));     // 25
-    unsigned short *LL = (unsigned short *)(ptab + 28);  // LCG_FOLD_NLOOP: l1 | l2 << 8
-    signed char *cs = (signed char *)(LL + LCG_FOLD_NLOOP + 8);  // n + 2
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = FT / 64;
-    const int cl = lane % CL, cg = wave * (64 / CL) + lane / CL, ncg = nw * (64 / CL);
+// K workgroups fold a sequence, each the batches of 64 NCH cells of a
+// diagonal that are its own.  The lanes of a wave are the cells of a chunk of
+// 64; the waves of the workgroup split the terms of their sums (every 16th
+// each), so that a load is 64 neighbours, many are in flight, and no lane
+// waits for another; the partial sums meet in LDS, one wave per chunk adds
+// them up and finishes its cells.  The interior loops are summed for the
+// cells that can pair only (3 of 8 on random sequences), listed by a wave
+// that has no chunk to finish.
+// Bound: per diagonal the instructions of 16 waves (about 200 each for the
+// interior loops), three trips to the L2 and two barriers: 6-10 us, and with
+// several workgroups 7 us more for the barrier between them.  Against a
+// quarter wave per cell with gathered terms and five more sums over the
+// splits: 64 sequences of 60-200 nt, span 100, 5.53 -> 2.45 ms; two of
+// 700-800 nt without a limit 300 -> 26.8 ms; one of 75 nt 1.21 -> 1.10 ms.
+template <int NCH>
+__device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const signed char *codes, const double *tabs,
+                                         double *mats, double *outs, double *zout, int *counter, int *status,
+                                         double *lds) {
+    constexpr int NB = 64 * NCH;  // cells per batch
+    const int n = D.n, W = D.W, S = D.S, K = D.K;
+    double *part = lds;                    // [sum][wave][cell]: M2 or Qmb, interior loops, Qm1b
+    double *T = part + 3 * NWV * NB;       // factor table from the stacks on
+    double *Z5 = T + (LCG_FOLD_TAB_HP - LCG_FOLD_TAB_STACK), *Z5b = Z5 + (n + 1);  // n + 1 each
+    int *ptab = (int *)(Z5b + (n + 1));    // 25
+    unsigned short *list = (unsigned short *)(ptab + 28);  // two buffers of NB: cells that can pair
+    unsigned short *place = list + 2 * NB;                 // two buffers of NB: their places in the list
+    int *count = (int *)(place + 2 * NB);                  // two buffers
+    signed char *cs = (signed char *)(count + 2);          // n + 2
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto tab = [&](int x) { return T[x - LCG_FOLD_TAB_STACK]; };
 
-    for (int x = tid; x < LCG_FOLD_TAB_FIXED; x += FT) T[x] = tabs[x];
+    for (int x = tid; x < LCG_FOLD_TAB_HP - LCG_FOLD_TAB_STACK; x += FT) T[x] = tabs[LCG_FOLD_TAB_STACK + x];
     for (int x = tid; x < n + 2; x += FT) cs[x] = (x >= 1 && x <= n) ? codes[D.codes + x] : (signed char)4;
-    for (int x = tid; x < n + 2; x += FT) SC[x] = exp(-(double)x * D.log_sigma);
     if (tid < 25) {
         // canonical pairs AU, CG, GC, UA, GU, UG as types 1..6
         const int a = tid / 5, b = tid % 5;
@@ -107,218 +146,361 @@ extern "C" __global__ __launch_bounds__(FT) void lcg_fold_seqs(const FoldDesc *d
         else if (a == 3 && b == 2) t = 6;
         ptab[tid] = t;
     }
-    for (int e = tid; e < LCG_FOLD_NLOOP; e += FT) {
-        int s = 0;
-        while (loop_count(s) <= e) ++s;
-        const int l1 = e - loop_count(s - 1);
-        LL[e] = (unsigned short)(l1 | ((s - l1) << 8));
-    }
-    __syncthreads();
-
-    const Seq S{cs, ptab, n, W};
-    const size_t sz = (size_t)(n + 2) * W;
-    double *Qb = mats + D.mat, *Qm = Qb + sz, *Qm1 = Qm + sz;
-    double *Qbb = Qm1 + sz, *Qmb = Qbb + sz, *Qm1b = Qmb + sz;
-    double *P = outs + D.out, *P2 = P + sz;
+    const Seq Q{cs, ptab};
+    const Terms tm = wave_terms(wave, lane, tabs, D.log_sigma);
+    // place of a term's cell from the cell (i, d) inside and outside
+    const int off_in = tm.s < 99 ? -(2 + tm.s) * S + 1 + tm.l1 : 0, off_out = -off_in;
+    const double s1 = exp(-D.log_sigma), s2 = s1 * s1, s3 = s2 * s1;
+    const size_t sz = (size_t)W * S;
+    double *Qb = mats + D.mat, *QI = Qb + sz, *QU = QI + sz, *Qm = QU + sz, *Qm1 = Qm + sz, *X = Qm1 + sz;
+    double *ring = X + sz;
+    double *M2 = ring, *Y = ring + 3 * (size_t)S;  // inside: 3 and 2 diagonals
+    double *U = ring + 5 * (size_t)S, *R = ring + 7 * (size_t)S, *Qbb = ring + 9 * (size_t)S;  // outside: 2, 2, 4
+    const size_t osz = (size_t)(n + 2) * W;
+    double *P = outs + D.out, *P2 = P + osz;
     const double *hp = tabs + LCG_FOLD_TAB_HP;
-    const double mlc = T[LCG_FOLD_TAB_MLC];
-
-    // ---------------- inside
-    for (int d = 0; d < W; ++d) {
-        for (int c = cg; c < n - d; c += ncg) {
-            const int i = 1 + c, j = i + d;
-            double qb = 0, qm1 = 0, qm = 0;
-            if (d >= 4) {
-                const int t = S.pt(i, j);
-                if (t) {
-                    double s = 0;
-                    const int cnt = loop_count(min(LCG_FOLD_MAXLOOP, d - 6));
-#pragma unroll 4
-                    for (int e = cl; e < cnt; e += CL) {
-                        const int l1 = LL[e] & 255, l2 = LL[e] >> 8;
-                        const int k = i + 1 + l1, l = j - 1 - l2;
-                        const int ti = S.pt(k, l);
-                        // the load does not wait for the pair test: (k, l)
-                        // lies in the band and holds 0 where it cannot pair
-                        const double q = Qb[(size_t)k * W + (l - k)];
-                        s += (ti ? loopf(T, l1, l2, t, ti) * SC[l1 + l2 + 2] : 0.0) * q;
-                    }
-                    double mq = 0;
-                    for (int u = i + 6 + cl; u <= j - 5; u += CL)
-                        mq += Qm[(size_t)(i + 1) * W + (u - 2 - i)] * Qm1[(size_t)u * W + (j - 1 - u)];
-                    s = cell_sum(s);
-                    mq = cell_sum(mq);
-                    qb = hp[(d - 1) * 2 + weak(t)] * SC[d + 1] + s + mq * mlc * T[LCG_FOLD_TAB_TP + weak(t)] * SC[2];
-                }
-                double a1 = 0;
-                for (int l = i + 4 + cl; l < j; l += CL) {
-                    const int tl = S.pt(i, l);
-                    const double q = Qb[(size_t)i * W + (l - i)];  // 0 where (i, l) cannot pair
-                    a1 += (tl ? T[LCG_FOLD_TAB_BRANCH + weak(tl)] * SC[j - l] : 0.0) * q;
-                }
-                a1 = cell_sum(a1);
-                if (t) a1 += qb * T[LCG_FOLD_TAB_BRANCH + weak(t)];
-                qm1 = a1;
-                double a2 = 0;
-                for (int u = i + 1 + cl; u <= j - 4; u += CL)
-                    a2 += (SC[u - i] + Qm[(size_t)i * W + (u - 1 - i)]) * Qm1[(size_t)u * W + (j - u)];
-                qm = cell_sum(a2) + qm1;
-            }
-            if (cl == 0) {
-                const size_t x = (size_t)i * W + d;
-                Qb[x] = qb;
-                Qm1[x] = qm1;
-                Qm[x] = qm;
-            }
-        }
-        __syncthreads();
-    }
-
-    // ---------------- exterior loop: Z5 forward, then its adjoints.  The
-    // sum of column j reads Z5 up to j - 5 only, so four consecutive columns
-    // are summed at once (a quarter wave each) and chained in order.
-    if (wave == 0) {
-        const int g = lane >> 4, gl = lane & 15;
-        double zlast = 1.0;
-        if (lane == 0) Z5[0] = 1.0;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        for (int j0 = 1; j0 <= n; j0 += 4) {
-            const int j = j0 + g;
-            double f = 0;
-            if (j <= n)
-                for (int k = max(1, j - W + 1) + gl; k <= j - 4; k += 16) {
-                    const int t = S.pt(k, j);
-                    const double q = Qb[(size_t)k * W + (j - k)];
-                    f += (t ? Z5[k - 1] * T[LCG_FOLD_TAB_EXT + weak(t)] : 0.0) * q;
-                }
-#pragma unroll
-            for (int o = 8; o > 0; o >>= 1) f += __shfl_xor(f, o);
-            const double z0 = zlast * SC[1] + __shfl(f, 0), z1 = z0 * SC[1] + __shfl(f, 16),
-                         z2 = z1 * SC[1] + __shfl(f, 32), z3 = z2 * SC[1] + __shfl(f, 48);
-            if (lane == 0) {
-                Z5[j0] = z0;
-                if (j0 + 1 <= n) Z5[j0 + 1] = z1;
-                if (j0 + 2 <= n) Z5[j0 + 2] = z2;
-                if (j0 + 3 <= n) Z5[j0 + 3] = z3;
-            }
-            zlast = j0 + 3 <= n ? z3 : j0 + 2 <= n ? z2 : j0 + 1 <= n ? z1 : z0;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        }
-        // Z5b(m) = Z5b(m+1) + sum_j Z5b(j) Qb(m+1,j) EXT reads Z5b from m + 5 up
-        double glast = 1.0;
-        if (lane == 0) Z5b[n] = 1.0;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        for (int m0 = n - 1; m0 >= 0; m0 -= 4) {
-            const int m = m0 - g;
-            double f = 0;
-            if (m >= 0)
-                for (int j = m + 5 + gl; j <= min(n, m + W); j += 16) {
-                    const int t = S.pt(m + 1, j);
-                    const double q = Qb[(size_t)(m + 1) * W + (j - m - 1)];
-                    f += (t ? Z5b[j] * T[LCG_FOLD_TAB_EXT + weak(t)] : 0.0) * q;
-                }
-#pragma unroll
-            for (int o = 8; o > 0; o >>= 1) f += __shfl_xor(f, o);
-            const double z0 = glast * SC[1] + __shfl(f, 0), z1 = z0 * SC[1] + __shfl(f, 16),
-                         z2 = z1 * SC[1] + __shfl(f, 32), z3 = z2 * SC[1] + __shfl(f, 48);
-            if (lane == 0) {
-                Z5b[m0] = z0;
-                if (m0 - 1 >= 0) Z5b[m0 - 1] = z1;
-                if (m0 - 2 >= 0) Z5b[m0 - 2] = z2;
-                if (m0 - 3 >= 0) Z5b[m0 - 3] = z3;
-            }
-            glast = m0 - 3 >= 0 ? z3 : m0 - 2 >= 0 ? z2 : m0 - 1 >= 0 ? z1 : z0;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        }
-        if (lane == 0) zout[sq] = Z5[n];
-    }
+    int passed = 0, buf = 0;
     __syncthreads();
+
+    // the cells of batch b of diagonal d that can pair, into a list buffer
+    auto make_list = [&](int d, int b, int to) {
+        int c = 0;
+#pragma unroll
+        for (int h = 0; h < NCH; ++h) {
+            const int i = b * NB + 64 * h + lane + 1;
+            const bool ok = d >= 4 && d < W && i + d <= n && Q.pt(i, i + d) != 0;
+            const unsigned long long m = __ballot(ok);
+            const int at = c + __popcll(m & ((1ull << lane) - 1));
+            if (ok) {
+                list[to * NB + at] = (unsigned short)(64 * h + lane);
+                place[to * NB + 64 * h + lane] = (unsigned short)at;
+            }
+            c += __popcll(m);
+        }
+        if (lane == 0) count[to] = c;
+    };
+    // end of a diagonal: every workgroup's cells are written before any
+    // workgroup reads them
+    auto diagonal_done = [&]() {
+        if (K > 1) {
+            // the waves' stores are in the L2 before one wave writes it back
+            // and, after the barrier, drops what the CU's L1 holds
+            __threadfence_block();
+            __syncthreads();
+            ++passed;
+            if (tid == 0) {
+                __threadfence();
+                meet(counter, K * passed, status);
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            }
+            __syncthreads();
+        } else {
+            __threadfence_block();
+            __syncthreads();
+        }
+    };
+    // sums over the loop terms for the listed cells of batch b: term q of
+    // cell i at band[off(q) + i], off by lane
+    auto loops = [&](int b, int lim, const double *band_u, const double *band_i, int off) {
+        const int c = count[buf];
+        const unsigned long long in = __ballot(tm.s <= lim);
+        const int nu = __popcll(in & 15), ni = __popcll(in >> 4);
+        for (int h = 0; 64 * h < c; ++h) {
+            const int x = 64 * h + lane;
+            const unsigned i = b * NB + list[buf * NB + (x < c ? x : 0)] + 1;
+            // terms [q0, q0 + N) of the wave with their loads in flight
+            // together; those past q1 (the terms go by loop size, the limit
+            // cuts a tail) load the last one's cell and count nothing
+            auto terms = [&](auto nt, const double *band, int q0, int q1, double acc) {
+                constexpr int N = decltype(nt)::value;
+                double v[N];
+#pragma unroll
+                for (int u = 0; u < N; ++u)
+                    v[u] = (band + __builtin_amdgcn_readlane(off, min(q0 + u, q1 - 1)))[i];
+#pragma unroll
+                for (int u = 0; u < N; ++u) acc = fma(v[u], q0 + u < q1 ? readlane_d(tm.f, q0 + u) : 0.0, acc);
+                return acc;
+            };
+            double au = 0, ai = 0;
+            if (nu > 0) au = terms(std::integral_constant<int, 4>(), band_u, 0, nu, au);
+            for (int q = 4; q < 4 + ni; q += 14) ai = terms(std::integral_constant<int, 14>(), band_i, q, 4 + ni, ai);
+            part[(NWV + wave) * NB + x] = au;
+            part[(2 * NWV + wave) * NB + x] = ai;
+        }
+    };
+    auto total = [&](int sum, int x) {
+        double v = 0;
+#pragma unroll
+        for (int w = 0; w < NWV; ++w) v += part[(sum * NWV + w) * NB + x];
+        return v;
+    };
+
+    const int nbatch = (n + NB - 1) / NB;
+    // ---------------- inside
+    if (wave == 0) make_list(4, member, 0);
+    __syncthreads();
+    for (int d = 4; d < W; ++d) {
+        const double hs = exp(-(double)(d + 1) * D.log_sigma);
+        for (int b = member; b < nbatch && b * NB < n - d; b += K) {
+            // partial sums
+            double m2[NCH];
+#pragma unroll
+            for (int h = 0; h < NCH; ++h) m2[h] = 0;
+#pragma unroll 4
+            for (int a = 4 + wave; a <= d - 5; a += NWV) {
+                const double *x = Qm + (size_t)a * S + b * NB + 1 + lane;
+                const double *y = Qm1 + (size_t)(d - 1 - a) * S + b * NB + 1 + lane + a + 1;
+#pragma unroll
+                for (int h = 0; h < NCH; ++h) m2[h] += x[64 * h] * y[64 * h];
+            }
+#pragma unroll
+            for (int h = 0; h < NCH; ++h) part[wave * NB + 64 * h + lane] = m2[h];
+            loops(b, min(MAXLOOP, d - 6), QU + (size_t)d * S, QI + (size_t)d * S, off_in);
+            __syncthreads();
+            // finish the cells; the next batch's list
+            const int nb = b + K < nbatch && (b + K) * NB < n - d ? b + K : member;
+            if (wave == NWV - 1) make_list(nb == member ? d + 1 : d, nb, buf ^ 1);
+            for (int h = wave; h < NCH; h += NWV - 1) {
+                const int c = 64 * h + lane, i = b * NB + c + 1, j = i + d;
+                if (wave == NWV - 1 || j > n) break;
+                const size_t x = (size_t)d * S + i;
+                const int t = Q.pt(i, j);
+                const double q1p = Qm1[x - S], yp = d > 4 ? Y[(size_t)((d - 1) & 1) * S + i + 1] : 0.0;
+                double qb = 0;
+                if (t) {
+                    const int wk = weak(t), at = place[buf * NB + c];
+                    // the bulges and interior loops, stacks and one-base bulges
+                    double l = total(1, at) * tab(LCG_FOLD_TAB_GU + wk) + total(2, at) * tab(LCG_FOLD_TAB_GI + wk);
+                    if (d >= 6) l += tab(LCG_FOLD_TAB_STACK + t * 8 + Q.pt(i + 1, j - 1)) * s2 * Qb[x - 2 * S + 1];
+                    if (d >= 7)
+                        l += s3 * (tab(LCG_FOLD_TAB_BULGE1 + t * 8 + Q.pt(i + 1, j - 2)) * Qb[x - 3 * S + 1] +
+                                   tab(LCG_FOLD_TAB_BULGE1 + t * 8 + Q.pt(i + 2, j - 1)) * Qb[x - 3 * S + 2]);
+                    const double mq = d > 5 ? M2[(size_t)((d - 2) % 3) * S + i + 1] : 0.0;
+                    qb = hp[(d - 1) * 2 + wk] * hs + l + mq * tab(LCG_FOLD_TAB_MLC) * tab(LCG_FOLD_TAB_TP + wk) * s2;
+                    Qb[x] = qb;
+                    QI[x] = qb * tab(LCG_FOLD_TAB_GI + wk);
+                    QU[x] = qb * tab(LCG_FOLD_TAB_GU + wk);
+                } else {
+                    Qb[x] = QI[x] = QU[x] = 0.0;
+                }
+                const double qm1 = (d > 4 ? q1p * s1 : 0.0) + (t ? qb * tab(LCG_FOLD_TAB_BRANCH + weak(t)) : 0.0);
+                const double y = qm1 + s1 * yp, m = total(0, c);
+                Qm1[x] = qm1;
+                Qm[x] = y + m;
+                M2[(size_t)(d % 3) * S + i] = m;
+                Y[(size_t)(d & 1) * S + i] = y;
+                P[(size_t)i * W + d] = t ? qb * tab(LCG_FOLD_TAB_EXT + weak(t)) : 0.0;
+            }
+            buf ^= 1;
+            if (nb != member) __syncthreads();
+        }
+        diagonal_done();
+        // a workgroup without cells on this diagonal has made no list
+        if (member * NB >= n - d) {
+            if (wave == 0) make_list(d + 1, member, buf);
+            __syncthreads();
+        }
+    }
+
+    // ---------------- exterior loop, by wave 0 of every workgroup: Z5
+    // forward, pushing each Z5(k-1) over the row of pairs (k, j), then the
+    // adjoints Z5b, gathered over rows.  A pair spans at least 4, so four rows
+    // are taken at once.
+    for (int x = tid; x <= n; x += FT) Z5[x] = Z5b[x] = 0.0;
+    __syncthreads();
+    if (wave == 0) {
+        double z = 1.0;  // Z5(k0 - 1)
+        if (lane == 0) Z5[0] = 1.0;
+        for (int k0 = 1; k0 <= n; k0 += 4) {
+            // Z5[j] holds the pairs ending in j until j is reached
+            double zk[4];
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                zk[k] = z;  // Z5(k0 + k - 1)
+                if (k0 + k <= n) z = z * s1 + Z5[k0 + k];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            if (lane < 4 && k0 + lane <= n) Z5[k0 + lane] = lane == 0 ? zk[1] : lane == 1 ? zk[2] : lane == 2 ? zk[3] : z;
+            for (int j0 = k0 + 4; j0 <= min(n, k0 + 3 + W - 1); j0 += 64) {
+                const int j = j0 + lane;
+                double f = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int e = j - k0 - k;
+                    if (j <= n && e >= 4 && e < W && k0 + k <= n) f += zk[k] * P[(size_t)(k0 + k) * W + e];
+                }
+                if (j <= n) Z5[j] += f;
+            }
+        }
+        if (lane == 0) Z5b[n] = 1.0;
+        double g = 1.0;  // Z5b(m0 + 1)
+        for (int m0 = n - 1; m0 >= 0; m0 -= 4) {
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            double f[4] = {0, 0, 0, 0};
+            for (int j0 = m0 + 2; j0 <= min(n, m0 + W); j0 += 64) {
+                const int j = j0 + lane;
+                const double zb = j <= n ? Z5b[j] : 0.0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int m = m0 - k, e = j - m - 1;  // row m + 1
+                    if (m >= 0 && j <= n && e >= 4 && e < W) f[k] += zb * P[(size_t)(m + 1) * W + e];
+                }
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) f[k] += __shfl_xor(f[k], o);
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (m0 - k < 0) break;
+                g = g * s1 + f[k];
+                if (lane == 0) Z5b[m0 - k] = g;
+            }
+        }
+        if (member == 0 && lane == 0) *zout = Z5[n];
+    }
+    // the rows of P are read before any workgroup overwrites them
+    diagonal_done();
     const double Z = Z5[n];
 
-    // ---------------- outside (gathered adjoints), probabilities
-    for (int d = W - 1; d >= 0; --d) {
-        for (int c = cg; c < n - d; c += ncg) {
-            const int a = 1 + c, e = a + d;
-            double qmb = 0, qm1b = 0, qbb = 0, p = 0, p2 = 0;
-            if (d >= 4) {
-                // Qm(a, e): inside Qb(a-1, j) as Qm(i+1, u-1), inside Qm(a, j) as Qm(i, u-1)
-                double s = 0;
-                if (a >= 2)
-                    for (int j = e + 6 + cl; j <= min(n, a + W - 2); j += CL) {
-                        const int t = S.pt(a - 1, j);
-                        const double o = Qbb[(size_t)(a - 1) * W + (j - a + 1)], q = Qm1[(size_t)(e + 1) * W + (j - e - 2)];
-                        s += (t ? mlc * T[LCG_FOLD_TAB_TP + weak(t)] * SC[2] : 0.0) * o * q;
-                    }
-                for (int j = e + 5 + cl; j <= min(n, a + W - 1); j += CL)
-                    s += Qmb[(size_t)a * W + (j - a)] * Qm1[(size_t)(e + 1) * W + (j - e - 1)];
-                qmb = cell_sum(s);
-                // Qm1(a, e): inside Qb(i, e+1) as Qm1(u, j-1), inside Qm(i, e) as Qm1(u, j)
-                s = 0;
-                if (e + 1 <= n)
-                    for (int i = max(1, e + 2 - W) + cl; i <= a - 6; i += CL) {
-                        const int t = S.pt(i, e + 1);
-                        const double o = Qbb[(size_t)i * W + (e + 1 - i)], q = Qm[(size_t)(i + 1) * W + (a - 2 - i)];
-                        s += (t ? mlc * T[LCG_FOLD_TAB_TP + weak(t)] * SC[2] : 0.0) * o * q;
-                    }
-                for (int i = max(1, e - W + 1) + cl; i <= a - 1; i += CL)
-                    s += Qmb[(size_t)i * W + (e - i)] * (SC[a - i] + Qm[(size_t)i * W + (a - 1 - i)]);
-                qm1b = cell_sum(s) + qmb;
-                // Qb(a, e): exterior loop, enclosing pairs, multiloop branches
-                const int t = S.pt(a, e);
-                if (t) {
-                    double si = 0, sb = 0;
-                    const int cnt = loop_count(min(LCG_FOLD_MAXLOOP, W - 3 - d));
+    // ---------------- outside, probabilities
+    auto has_cells = [&](int d) { return member * NB < n - d; };
+    if (wave == 0) make_list(W - 1, member, buf);
+    __syncthreads();
+    for (int d = W - 1; d >= 4; --d) {
+        for (int b = member; b < nbatch && b * NB < n - d; b += K) {
+            // terms outside the sequence read cells that are never written (0): past
+            // the last cell of a diagonal, which is also where an index below 1 leads
+            double q1[NCH], q2[NCH];
+#pragma unroll
+            for (int h = 0; h < NCH; ++h) q1[h] = q2[h] = 0;
+            const int a0 = b * NB + 1 + lane;
+            const int top = min(W - 1, n - 1 - b * NB);  // diagonals with a cell of the batch
 #pragma unroll 4
-                    for (int q = cl; q < cnt; q += CL) {
-                        const int l1 = LL[q] & 255, l2 = LL[q] >> 8;
-                        const int i = a - 1 - l1, j = e + 1 + l2;
-                        const bool in = i >= 1 && j <= n;
-                        // (i, j) in range lies in the band (cnt bounds l1 + l2); the load
-                        // does not wait for the pair test, cells that cannot pair hold 0
-                        const double o = in ? Qbb[(size_t)i * W + (j - i)] : 0.0;
-                        const int to = in ? S.pt(i, j) : 0;
-                        si += (to ? loopf(T, l1, l2, to, t) * SC[l1 + l2 + 2] : 0.0) * o;
-                    }
-                    for (int j = e + 1 + cl; j <= min(n, a + W - 1); j += CL)
-                        sb += Qm1b[(size_t)a * W + (j - a)] * SC[j - e];
-                    si = cell_sum(si);
-                    sb = cell_sum(sb);
-                    qbb = Z5b[e] * Z5[a - 1] * T[LCG_FOLD_TAB_EXT + weak(t)] + si +
-                          T[LCG_FOLD_TAB_BRANCH + weak(t)] * (sb + qm1b);
-                    const double qb = Qb[(size_t)a * W + d];
-                    p = qb * qbb / Z;
-                    if (d >= 6) {
-                        const int ti = S.pt(a + 1, e - 1);
-                        if (ti)
-                            p2 = qbb * T[LCG_FOLD_TAB_STACK + t * 8 + ti] * SC[2] * Qb[(size_t)(a + 1) * W + (d - 2)] / Z;
-                    }
+            for (int e = d + 5 + wave; e <= top; e += NWV) {
+                const double *x = X + (size_t)e * S + a0, *y = Qm1 + (size_t)(e - d - 1) * S + a0 + d + 1;
+#pragma unroll
+                for (int h = 0; h < NCH; ++h) q1[h] += x[64 * h] * y[64 * h];
+            }
+            const int btop = min(W - 1 - d, b * NB + NB - 1);
+#pragma unroll 4
+            for (int e = 5 + wave; e <= btop; e += NWV) {
+                const double *x = X + (size_t)(d + e) * S + a0 - e, *y = Qm + (size_t)(e - 1) * S + a0 - e;
+#pragma unroll
+                for (int h = 0; h < NCH; ++h) q2[h] += x[64 * h] * y[64 * h];
+            }
+            loops(b, min(MAXLOOP, W - 3 - d), QU + (size_t)d * S, QI + (size_t)d * S, off_out);
+            // the sums of the splits share the first third in turn
+#pragma unroll
+            for (int h = 0; h < NCH; ++h) part[wave * NB + 64 * h + lane] = q1[h];
+            __syncthreads();
+            double qmb = 0, lu = 0, li = 0;
+            const int c = 64 * wave + lane, a = b * NB + c + 1, e = a + d;
+            const bool mine = wave < NCH && e <= n;
+            const int t = mine ? Q.pt(a, e) : 0;
+            if (mine) qmb = total(0, c);
+            if (t) {
+                const int at = place[buf * NB + c];
+                lu = total(1, at);
+                li = total(2, at);
+            }
+            const int nb = b + K < nbatch && (b + K) * NB < n - d ? b + K : member;
+            if (wave == NWV - 1) make_list(nb == member ? d - 1 : d, nb, buf ^ 1);
+            __syncthreads();
+#pragma unroll
+            for (int h = 0; h < NCH; ++h) part[wave * NB + 64 * h + lane] = q2[h];
+            __syncthreads();
+            if (mine) {
+                const size_t x = (size_t)d * S + a;
+                const bool up = a >= 2, right = e < n;
+                const double u = qmb + (up && d + 1 < W ? s1 * U[(size_t)((d + 1) & 1) * S + a - 1] : 0.0);
+                const double qm1b = total(0, c) + u;
+                const double sb = right && d + 1 < W ? s1 * R[(size_t)((d + 1) & 1) * S + a] : 0.0;
+                double xv = qmb;
+                if (up && right && d + 2 < W) {
+                    const int to = Q.pt(a - 1, e + 1);
+                    if (to)
+                        xv += tab(LCG_FOLD_TAB_MLC) * tab(LCG_FOLD_TAB_TP + weak(to)) * s2 *
+                              Qbb[(size_t)((d + 2) & 3) * S + a - 1];
                 }
+                double qbb = 0, p = 0, p2 = 0;
+                if (t) {
+                    const int wk = weak(t);
+                    double l = lu * tab(LCG_FOLD_TAB_GU + wk) + li * tab(LCG_FOLD_TAB_GI + wk);
+                    if (up && right && d + 2 < W)
+                        l += tab(LCG_FOLD_TAB_STACK + Q.pt(a - 1, e + 1) * 8 + t) * s2 *
+                             Qbb[(size_t)((d + 2) & 3) * S + a - 1];
+                    if (d + 3 < W) {
+                        const double *q = Qbb + (size_t)((d + 3) & 3) * S;
+                        if (up && e + 2 <= n) l += tab(LCG_FOLD_TAB_BULGE1 + Q.pt(a - 1, e + 2) * 8 + t) * s3 * q[a - 1];
+                        if (a >= 3 && right) l += tab(LCG_FOLD_TAB_BULGE1 + Q.pt(a - 2, e + 1) * 8 + t) * s3 * q[a - 2];
+                    }
+                    qbb = Z5b[e] * Z5[a - 1] * tab(LCG_FOLD_TAB_EXT + wk) + l +
+                          tab(LCG_FOLD_TAB_BRANCH + wk) * (sb + qm1b);
+                    p = Qb[x] * qbb / Z;
+                    if (d >= 6) {
+                        const int ti = Q.pt(a + 1, e - 1);
+                        if (ti) p2 = qbb * tab(LCG_FOLD_TAB_STACK + t * 8 + ti) * s2 * Qb[x - 2 * S + 1] / Z;
+                    }
+                    QI[x] = qbb * tab(LCG_FOLD_TAB_GI + wk);
+                    QU[x] = qbb * tab(LCG_FOLD_TAB_GU + wk);
+                } else {
+                    QI[x] = QU[x] = 0.0;
+                }
+                X[x] = xv;
+                U[(size_t)(d & 1) * S + a] = u;
+                R[(size_t)(d & 1) * S + a] = qm1b + sb;
+                Qbb[(size_t)(d & 3) * S + a] = qbb;
+                P[(size_t)a * W + d] = p;
+                P2[(size_t)a * W + d] = p2;
             }
-            if (cl == 0) {
-                const size_t x = (size_t)a * W + d;
-                Qmb[x] = qmb;
-                Qm1b[x] = qm1b;
-                Qbb[x] = qbb;
-                P[x] = p;
-                P2[x] = p2;
-            }
+            buf ^= 1;
+            if (nb != member) __syncthreads();
         }
-        __syncthreads();
+        diagonal_done();
+        if (!has_cells(d)) {
+            if (wave == 0) make_list(d - 1, member, buf);
+            __syncthreads();
+        }
     }
 }
 
-extern "C" size_t lcg_fold_lds_bytes(int nmax) {
-    return (size_t)(LCG_FOLD_TAB_FIXED + 2 * (nmax + 1) + (nmax + 2)) * sizeof(double) + 28 * sizeof(int) +
-           (LCG_FOLD_NLOOP + 8) * sizeof(unsigned short) + (size_t)(nmax + 2);
+// Chunks per batch: one with several workgroups on the sequence, else as many
+// as its diagonals have, up to nch (what the LDS allows).
+extern "C" __global__ __launch_bounds__(FT) void lcg_fold_seqs(const FoldDesc *descs, const signed char *codes,
+                                                               const double *tabs, double *mats, double *outs,
+                                                               double *zout, int *counters, int *status,
+                                                               const int *seq_of, int nch) {
+    extern __shared__ double lds[];
+    const int sq = seq_of[2 * blockIdx.x], member = seq_of[2 * blockIdx.x + 1];
+    const FoldDesc D = descs[sq];
+    if (D.K > 1 || D.n <= 64 || nch == 1)
+        fold_seq<1>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, lds);
+    else if (D.n <= 128)
+        fold_seq<2>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, lds);
+    else
+        fold_seq<4>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, lds);
 }
 
+extern "C" size_t lcg_fold_lds_bytes(int nmax, int nch) {
+    const int nb = 64 * nch;
+    const size_t doubles = 3 * NWV * nb + (LCG_FOLD_TAB_HP - LCG_FOLD_TAB_STACK) + 2 * (nmax + 1);
+    return doubles * sizeof(double) + 28 * sizeof(int) + 4 * nb * sizeof(unsigned short) + 2 * sizeof(int) +
+           (size_t)(nmax + 2);
+}
+
+// grid workgroups: sequence and member of each in seq_of; nch 1, 2 or 4.
 extern "C" int lcg_launch_fold(const FoldDesc *descs, const signed char *codes, const double *tabs, double *mats,
-                               double *outs, double *zout, int nseq, int nmax, hipStream_t stream) {
-    const size_t lds = lcg_fold_lds_bytes(nmax);
+                               double *outs, double *zout, int *counters, int *status, const int *seq_of, int grid,
+                               int nmax, int nch, hipStream_t stream) {
+    const size_t lds = lcg_fold_lds_bytes(nmax, nch);
     if (hipError_t e = hipFuncSetAttribute((const void *)lcg_fold_seqs, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)lds))
         return (int)e;
-    if (nseq <= 0) return 0;
-    hipLaunchKernelGGL(lcg_fold_seqs, dim3(nseq), dim3(FT), lds, stream, descs, codes, tabs, mats, outs, zout, nseq);
+    if (grid <= 0) return 0;
+    hipLaunchKernelGGL(lcg_fold_seqs, dim3(grid), dim3(FT), lds, stream, descs, codes, tabs, mats, outs, zout, counters,
+                       status, seq_of, nch);
     return (int)hipGetLastError();
 }

@@ -1,0 +1,55 @@
+"""The folding kernel at the edges of its batches and workgroups: lengths
+around 64, 128 and 256 nt (1, 2, 4 chunks of cells a batch) and above (several
+workgroups per sequence), spans below and above the interior-loop limit, alone
+and together, against the folding oracle (1e-10 absolute on probabilities, as
+sums of up to 500 positive terms per cell in another order allow, 1e-12
+relative on log Z); and the probability texts against printf's rounding."""
+import numpy as np
+import pytest
+
+from locarna_amd import api, synth
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _seqs(lens, seed):
+    return [synth.sequences(seed + k, 1, n, n, 0.5, 0.6)[0] for k, n in enumerate(lens)]
+
+
+def _check(seqs, span):
+    F = api.Fold(seqs, max_bp_span=span, min_prob=0.0005)
+    for k, s in enumerate(seqs):
+        P, P2 = F.probs(k)
+        Po, P2o, lz = oracle.fold(s, span)
+        assert np.abs(P - Po).max() <= 1e-10, (len(s), span)
+        assert np.abs(P2 - P2o).max() <= 1e-10, (len(s), span)
+        assert abs(F.log_z(k) - lz) <= 1e-12 * max(1.0, abs(lz)), (len(s), span)
+    F.destroy()
+
+
+@pytest.mark.parametrize("n", [5, 9, 10, 11, 40, 63, 64, 65, 127, 128, 129, 192, 255, 256, 257, 321])
+@pytest.mark.parametrize("span", [-1, 7, 36, 70])
+def test_one_sequence(n, span):
+    _check(_seqs([n], 40 + n), span)
+
+
+@pytest.mark.parametrize("lens", [[1, 4, 64, 65, 128, 129, 250], [300, 12, 90, 64, 257]])
+def test_together(lens):
+    _check(_seqs(lens, 90), 100)
+
+
+def test_probability_digits():
+    F = api.Fold(_seqs([150, 140], 7), max_bp_span=100, min_prob=1e-6)
+    for k in range(2):
+        P, _ = F.probs(k)
+        for line in F.pp(k, "x").split("#BPCUT")[1].split("\n")[1:]:
+            f = line.split()
+            if len(f) != 3:
+                continue
+            p = P[int(f[0]), int(f[1])]
+            want = "%.4g" % p
+            if len(want) > 8:
+                want = "%.3e" % p
+            assert f[2] == want.replace("e-0", "e-"), (p, f[2])
+    F.destroy()
