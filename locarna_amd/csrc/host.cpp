@@ -728,7 +728,46 @@ std::string clustal_blocks(const std::vector<std::pair<std::string, const std::s
     return text;
 }
 
+namespace {
+// format_prob of p in [1e-4, 1) without printf: the four significant digits
+// are the nearest integer to p 10^k; false where that is too close to a tie
+// for the product's rounding, or p lies outside.
+bool format_prob_digits(double p, std::string &txt) {
+    if (!(p >= 1e-4 && p < 1)) return false;
+    int lead = 1;  // p = 0.ddd.. x 10^(1 - lead): zeros after the point + 1
+    double x = p * 1e4;
+    while (x < 1000) x *= 10, ++lead;
+    const double r = std::floor(x);
+    const double half = x - r - 0.5;
+    if (std::fabs(half) < 1e-6 || lead > 4) return false;
+    int d = (int)r + (half > 0);
+    if (d == 10000) {  // rounded up to the next power of ten
+        d = 1000;
+        if (--lead == 0) return false;
+    }
+    char buf[16];
+    if (lead == 4 && d % 10) {  // 0.000dddd has more than 8 characters: d.ddde-4
+        buf[0] = (char)('0' + d / 1000), buf[1] = '.', buf[2] = (char)('0' + d / 100 % 10);
+        buf[3] = (char)('0' + d / 10 % 10), buf[4] = (char)('0' + d % 10);
+        buf[5] = 'e', buf[6] = '-', buf[7] = '4';
+        txt.assign(buf, 8);
+        return true;
+    }
+    int n = 0;
+    buf[n++] = '0', buf[n++] = '.';
+    for (int k = 1; k < lead; ++k) buf[n++] = '0';
+    for (int k = 1000; k > 0 && d > 0; k /= 10) {  // %g drops trailing zeros
+        buf[n++] = (char)('0' + d / k);
+        d %= k;
+    }
+    txt.assign(buf, n);
+    return true;
+}
+}  // namespace
+
 std::string format_prob(double p) {
+    std::string fast;
+    if (format_prob_digits(p, fast)) return fast;
     // a stream with precision 4 and the default float field writes what
     // printf's %.4g writes, the scientific field with precision 3 what %.3e
     // writes (the streams' num_put is specified by those conversions)
