@@ -2485,6 +2485,7 @@ int pf_setup(lcg_batch &B) {
         f.scal = take(4);
         f.out = take(4);
         f.fD = take(h.nam);
+        f.fDb = take(h.nam);
         const int cap = B.frags.empty() ? 0 : (int)B.frags[k].size();
         f.frag = take(8 * (size_t)cap);
         f.nfrag = 0;

@@ -117,6 +117,7 @@ struct PfPair {
     const int *fcand;      // int arena: fill entries (p | q<<16, j | min_col(p-1)<<16, -)
     const int *f2c;        // fill entry -> candidate entry
     double *fD;            // inside D per fill entry
+    double *fDb;           // outside dZ/dD per fill entry: the fixed-column kernels' part
     double *fq;            // fragment match queries (8 doubles each)
     int nfq;
 };
@@ -707,7 +708,7 @@ __device__ __forceinline__ double pf_rev_fixed(const PfPair &P, int al, int bl, 
             const int rl = max(bl, e.jm >> 16);
             if (in && q > bl && j >= jlo && j <= hi && q - 1 >= rl && e.D != 0.0) {
                 atomicAdd(&Mb[(p - 1 - al) * W + (q - 1 - rl)], rowB[j - lo] * e.D * ps);
-                if (FULL) atomicAdd(&P.Dbar[P.f2c[tt]], rowB[j - lo] * Mst[(p - 1 - al) * W + (q - 1 - rl)] * ps);
+                if (FULL) atomicAdd(&P.fDb[tt], rowB[j - lo] * Mst[(p - 1 - al) * W + (q - 1 - rl)] * ps);
             }
         };
         if (t1 > t0) arc(ce, t0 + lane, t0 + lane < t1);
@@ -847,6 +848,7 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                 pfa[f.Dc + t] = 0.0;
                 pfa[f.Dbar + t] = 0.0;
                 pfa[f.fD + t] = 0.0;
+                pfa[f.fDb + t] = 0.0;
             }
             for (int t = threadIdx.x; t < d.ncells; t += blockDim.x) {
                 pfa[f.edge_full + t] = 0.0;
@@ -859,12 +861,15 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
         }
         if (threadIdx.x == 0) s_open = 0.0;
         int passed = 0;  // barrier generations passed
-        // all members' global writes before any member goes on
+        // all members' global writes before any member goes on; one wave's
+        // device-scope fences after the workgroup's own barrier (each writes the
+        // L2 back or drops the L1)
         auto pair_barrier = [&]() {
-            __threadfence();
+            __threadfence_block();
             __syncthreads();
             ++passed;
             if (threadIdx.x == 0) {
+                __threadfence();
                 atomicAdd(&barriers[k], 1);
                 for (int spin = 0; spin_lim < 0 || atomicAdd(&barriers[k], 0) < K * passed; ++spin) {
                     if (spin > spin_lim) {
@@ -873,9 +878,9 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                     }
                     __builtin_amdgcn_s_sleep(2);
                 }
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             }
             __syncthreads();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         };
         PfPair P;
         P.mn = mn;
@@ -902,6 +907,7 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
         P.fcand = arena + d.fcand;
         P.f2c = arena + d.f2c;
         P.fD = pfa + f.fD;
+        P.fDb = pfa + f.fDb;
         P.fq = pfa + f.frag;
         P.nfq = f.nfrag;
         if (K > 1) {
@@ -1033,6 +1039,8 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
         }
         const double Z = pfa[f.out + 0];
         const double thr = pfa[f.scal + 2];
+        // dZ/dD of the arc match of a gams entry, complete before its row
+        auto dbar = [&](const int4 &ga) { return P.Dbar[ga.y] + P.fDb[ga.w]; };
         // ---- outside over the groups, rows al = 1 .. n
         for (int al = 1; al <= n; ++al) {
             const int g0 = rows[al + 1], g1 = rows[al];
@@ -1048,7 +1056,7 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                     bool any = false;
                     for (int t = G[3] + lane; t < G[4]; t += 64) {
                         const int4 ga = gams[t];
-                        if (P.Dc[ga.y] * P.Dbar[ga.y] / Z > thr) any = true;
+                        if (P.Dc[ga.y] * dbar(ga) / Z > thr) any = true;
                     }
                     const bool sig = __ballot(any) != 0;
                     if (off >= 0) {
@@ -1076,10 +1084,10 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                             lds_fence();
                             for (int t = G[3] + lane; t < G[4]; t += 64) {
                                 const int4 ga = gams[t];
-                                if (pass == 1 && !(P.Dc[ga.y] * P.Dbar[ga.y] / Z > thr)) continue;
+                                if (pass == 1 && !(P.Dc[ga.y] * dbar(ga) / Z > thr)) continue;
                                 const int ar = ga.x & 0xffff, br = ga.x >> 16;
                                 const int x = fixed_at(gal, gbl, gbr, W, ar - 1, br - 1);
-                                if (x >= 0) atomicAdd(&Mb[x], P.Dbar[ga.y] * P.eam[ga.y]);
+                                if (x >= 0) atomicAdd(&Mb[x], dbar(ga) * P.eam[ga.y]);
                             }
                             scratch_sync();  // Es/Ss (global) and the seeds (LDS) before the sweep
                             if (pass == 0) {
@@ -1103,7 +1111,7 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                             const int4 ga = gams[t];
                             const int ar = ga.x & 0xffff, br = ga.x >> 16;
                             if (R.stored(P, ar - 1, br - 1))
-                                atomicAdd(R.at(R.Mb, P, ar - 1, br - 1), P.Dbar[ga.y] * P.eam[ga.y]);
+                                atomicAdd(R.at(R.Mb, P, ar - 1, br - 1), dbar(ga) * P.eam[ga.y]);
                         }
                         scratch_sync();
                         pf_reverse(P, R, true, P.edge_full, &s_open);
@@ -1112,8 +1120,8 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                             for (int t = G[3] + lane; t < G[4]; t += 64) {
                                 const int4 ga = gams[t];
                                 const int ar = ga.x & 0xffff, br = ga.x >> 16;
-                                if (P.Dc[ga.y] * P.Dbar[ga.y] / Z > thr && R.stored(P, ar - 1, br - 1))
-                                    atomicAdd(R.at(R.Mb, P, ar - 1, br - 1), P.Dbar[ga.y] * P.eam[ga.y]);
+                                if (P.Dc[ga.y] * dbar(ga) / Z > thr && R.stored(P, ar - 1, br - 1))
+                                    atomicAdd(R.at(R.Mb, P, ar - 1, br - 1), dbar(ga) * P.eam[ga.y]);
                             }
                             scratch_sync();
                             pf_reverse(P, R, false, P.edge_ref, nullptr);
@@ -1125,6 +1133,8 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
             }
             if (K > 1) pair_barrier();
         }
+        for (int t = member * blockDim.x + threadIdx.x; t < d.nam; t += K * blockDim.x)
+            P.Dbar[P.f2c[t]] += P.fDb[t];
         // fragment queries: the inside of each block (the virtual arc match
         // (i-1, j+1; k-1, l+1), AlignerP::compute_fragment_match_prob,
         // aligner_p.icc:1440-1479), one wave per query in its global scratch

@@ -13,6 +13,10 @@
 //                       P(am) > sqrt(min_am_prob))
 //   scal[4]             exp(indel_opening / T), pf_scale, sqrt(min_am_prob)
 //   out[4]              Z, expected-openings weight
+//   fDb[nam]            the part of Dbar that the fixed-column kernels sum, per
+//                       fill entry (neighbouring lanes add to neighbouring
+//                       words, and no index is loaded in front of the add);
+//                       added to Dbar at the end
 //   fD[nam]             inside D per fill entry (the fill list of the int
 //                       arena, for the candidate gathers of the group kernels)
 //   frag[8 cap]         fragment match queries, 8 doubles each: i, j, k, l,
@@ -41,7 +45,8 @@ typedef struct {
     int32_t sched, rin, rout;  // int schedule buffer
     int32_t frag, nfrag;       // fragment match queries of the run
     int32_t fso;               // int schedule buffer: forward-store offset per group
-} PfDesc;  // 17 ints
+    int32_t fDb;               // double arena: the fixed-column kernels' part of Dbar
+} PfDesc;  // 18 ints
 
 typedef struct {
     int32_t npairs;
