@@ -2560,7 +2560,6 @@ int pf_setup(lcg_batch &B) {
     // the pool together, the others run in per-wave global scratch (offset
     // -1).  Word: round | wave<<12 | member<<16.
     std::vector<int32_t> sched;
-    size_t max_fixed = 0;
     std::vector<int> Kp(np, 1);  // workgroups of each pair
     for (int q = 0; q < nst; ++q) Kp[B.order[q]] = K;
     for (int k = 0; k < np; ++k) {
@@ -2583,7 +2582,7 @@ int pf_setup(lcg_batch &B) {
                     const int gal = G[0] & 0xffff, gbl = G[0] >> 16, gar = G[1] & 0xffff, gbr = G[1] >> 16;
                     if (gbr - gbl - 1 > 128 || gar - gal - 1 > 128) return -1;
                     const long cells = (long)(gar - gal) * G[2];
-                    const long sz = (gbr - gbl) + (pass == 0 ? 1 : 2) * cells;
+                    const long sz = 4 * (gbr - gbl) + (pass == 0 ? 1 : 2) * cells;
                     return sz <= pool ? ((sz + 1) & ~1L) : -1;
                 };
                 auto rows_of = [&](int g) {
@@ -2621,8 +2620,6 @@ int pf_setup(lcg_batch &B) {
                         S[1] = sz > 0 ? (int32_t)used[r] : -1;
                         if (sz > 0) {
                             used[r] += sz;
-                            const int32_t *G = A + gbase + g * LCG_GROUP_INTS;
-                            max_fixed = std::max(max_fixed, (size_t)2 * ((G[1] & 0xffff) - (G[0] & 0xffff)) * G[2]);
                         }
                         cnt[r] += 1;
                     }
@@ -2635,8 +2632,8 @@ int pf_setup(lcg_batch &B) {
         (void)gbase;
     }
     // forward-value store: every group that runs the fixed-column kernels in
-    // both passes gets 3 (ar - al) W doubles (E, s, M) while the store stays
-    // within its budget; the others are recomputed by the outside pass
+    // both passes gets (ar - al) W doubles (M) while the store stays within
+    // its budget; the others are recomputed by the outside pass
     const size_t store_budget = (size_t)1 << 31;  // doubles (16 GiB)
     size_t store = 0;
     for (int k = 0; k < np; ++k) {
@@ -2649,13 +2646,12 @@ int pf_setup(lcg_batch &B) {
             const int32_t *S = &sched[f.sched + 4 * (size_t)g];
             if (S[1] < 0 || S[3] < 0) continue;
             const int32_t *G = A + d.groups + g * LCG_GROUP_INTS;
-            const size_t need = (3 * (size_t)((G[1] & 0xffff) - (G[0] & 0xffff)) * G[2] + 3) & ~(size_t)3;
+            const size_t need = ((size_t)((G[1] & 0xffff) - (G[0] & 0xffff)) * G[2] + 3) & ~(size_t)3;
             if (store + need > store_budget) continue;
             sched[f.fso + (size_t)g] = (int32_t)(store / 4);
             store += need;
         }
     }
-    stride = std::max(stride, max_fixed);
     B.pbp.scratch_stride = (int32_t)((stride + 31) & ~(size_t)31);
     hipError_t e;
     // all workgroups resident at once (one per CU): static members + the rest

@@ -382,85 +382,162 @@ __device__ void pf_reverse(const PfPair &P, const Region &R, bool want_dbar, dou
 }
 
 // ---- fixed-column group kernels (columns bl+1 .. br-1 in NC chunks of 64
-// lanes, lane l of chunk c owns column bl+1+64c+l in every row; rows
-// al+1 .. ar-1 at most 128).  Region in LDS (doubles): [S: br-bl] [M:
-// (ar-al) W] [Mbar: (ar-al) W], rows stored from max(bl, min_col(i)) as in
-// the general layout.  The arc candidates of row i are the fill-list prefix
-// p > al (left ends descending), located from the LDS block table.
-
-struct PfEnt {
-    int pq, jm;
-    double D;
-};
-
+// lanes, the same column on the same lane in every row; rows al+1 .. ar-1).
+// Region in LDS (doubles): [S: 4 (br-bl)] [M: (ar-al) W] [Mbar: (ar-al) W],
+// rows stored from max(bl, min_col(i)) as in the general layout.
+//
+// Four rows are one block, rows al+r0 .. al+r0+3 (r0 a multiple of 4).  An
+// arc (p, i) spans at least three positions, so an arc term of row i reads
+// (the adjoint: adds to) row p - 1 <= i - 4, outside the block: the arc
+// entries of the four rows are handled together, packed on the lanes, before
+// the block's rows (the adjoint: after them), and the next block's are loaded
+// meanwhile.  The arc candidates of row i are the fill-list prefix p > al
+// (left ends descending), located from the LDS block table.
+// Bound: LDS holds 5 to 10 regions of a workgroup, so every SIMD has one to
+// three waves and the latency of a row's chain (LDS, scan, store) shows; a
+// row at a time cost a trip to memory and five to LDS each.  120 pairs of 150
+// nt, whole kernel, 105.3 -> 61.7 ms; 48 ragged pairs of 80-250 nt 170.7 ->
+// 98.5 ms; one pair of 88 nt, a wave at a time, 11.4 -> 7.0 ms.
 // lane l receives lane l-1's value, lane 0 `first` (DPP wave_shr:1)
 __device__ __forceinline__ double shift_up_d(double v, double first) { return dpp_d<0x138, 0xf>(first, v); }
-// lane l receives lane l+1's value, lane 63 `last` (DPP wave_shl:1)
-__device__ __forceinline__ double shift_down_d(double v, double last) { return dpp_d<0x130, 0xf>(last, v); }
 
-// candidate range [t0, t1) of rows al+1+r, r = lane + 64 h (RT tables: at
-// most 64 RT rows)
-template <int RT>
-__device__ __forceinline__ void pf_row_table(const PfPair &P, int al, int bl, int br, int nrows, int rt0[RT],
-                                             int rt1[RT]) {
-#pragma unroll
-    for (int h = 0; h < RT; ++h) {
-        const int r = lane_id() + 64 * h;
-        rt0[h] = rt1[h] = 0;
-        if (r < nrows) {
-            const int i = al + 1 + r;
-            if (max(bl + 1, P.mn[i]) <= min(br - 1, P.mx[i])) {
-                int b = P.fbp[i];
-                const int be = P.fbp[i + 1];
-                rt0[h] = P.fbk[2 * b + 1];
-                while (b < be && P.fbk[2 * b] > al) ++b;
-                rt1[h] = P.fbk[2 * b + 1];
-            }
-        }
-    }
-}
-template <int RT>
-__device__ __forceinline__ void pf_row_cands(const int rt0[RT], const int rt1[RT], int r, int &t0, int &t1) {
-    t0 = t1 = 0;
-#pragma unroll
-    for (int h = 0; h < RT; ++h)
-        if ((r >> 6) == h) {
-            t0 = __builtin_amdgcn_readlane(rt0[h], r & 63);
-            t1 = __builtin_amdgcn_readlane(rt1[h], r & 63);
-        }
-}
-// Unpredicated loads: lanes past the range read its last entry (or entry 0
-// of the pair; a group implies arc matches) and are ignored by the caller's
-// lane flag.
-__device__ __forceinline__ PfEnt pf_fetch(const PfPair &P, int t, int t1) {
-    const int tt = t < t1 ? t : max(t1 - 1, 0);
-    PfEnt e;
-    struct PJ {
-        int x, y;
-    };
-    const PJ pj = *reinterpret_cast<const PJ *>(P.fcand + 2 * tt);
-    e.pq = pj.x;
-    e.jm = pj.y;
-    e.D = P.fD[tt];
-    return e;
-}
 __device__ __forceinline__ void lds_fence() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); }
 
-// Inside fill of a group (aligner_p.icc:150-312), values as pf_fill.  When
-// Es/Ss are given (global scratch, layout of M), E and s = M - F of every
-// computed cell are stored for the adjoint.
-template <int NC, int RT = 2>
-__device__ __forceinline__ void pf_fwd_fixed(const PfPair &P, int al, int bl, int ar, int br, int W, double *base, double *Es,
-                             double *Ss) {
+// Prefix scan x_l = b_l + a_l x_{l-1} whose multipliers are the same for all
+// rows of a group: the products that each step needs are computed once, so
+// that a step is one move and one multiply-add.  Returns the product a_0 .. a_l.
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ void coef_step(double &a, double &m) {
+    m = a * dpp_d<CTRL, ROWMASK>(0.0, 1.0);  // 0 where the step has no source lane
+    a *= dpp_d<CTRL, ROWMASK>(1.0, a);
+}
+__device__ __forceinline__ double scan_coef(double a, double (&m)[6]) {
+    coef_step<0x111, 0xf>(a, m[0]);
+    coef_step<0x112, 0xf>(a, m[1]);
+    coef_step<0x114, 0xf>(a, m[2]);
+    coef_step<0x118, 0xf>(a, m[3]);
+    coef_step<0x142, 0xa>(a, m[4]);
+    coef_step<0x143, 0xc>(a, m[5]);
+    return a;
+}
+__device__ __forceinline__ double scan_lin(double b, const double (&m)[6]) {
+    b = fma(m[0], dpp_d<0x111, 0xf>(0.0, b), b);
+    b = fma(m[1], dpp_d<0x112, 0xf>(0.0, b), b);
+    b = fma(m[2], dpp_d<0x114, 0xf>(0.0, b), b);
+    b = fma(m[3], dpp_d<0x118, 0xf>(0.0, b), b);
+    b = fma(m[4], dpp_d<0x142, 0xa>(0.0, b), b);
+    return fma(m[5], dpp_d<0x143, 0xc>(0.0, b), b);
+}
+
+// Operands of rows al+rb .. al+rb+63, one per lane: band, gap weight, symbol,
+// fill entries [t0, t1); mnu, mxu: the band of the row above.
+struct PfRows {
+    int mn, mx, mnu, mxu, code, co, t0, t1;
+    double gA;
+    __device__ __forceinline__ void load(const PfPair &P, int al, int bl, int ar, int br, int rb) {
+        const int r = rb + lane_id(), i = min(al + r, ar - 1), u = max(i - 1, 0);
+        mn = P.mn[i];
+        mx = P.mx[i];
+        mnu = P.mn[u];
+        mxu = P.mx[u];
+        code = P.codeA[i] * LCG_NCODES;
+        co = P.coff[i];
+        gA = P.egA[i];
+        t0 = t1 = 0;
+        if (r >= 1 && al + r < ar && max(bl + 1, mn) <= min(br - 1, mx)) {
+            int b = P.fbp[i];
+            const int be = P.fbp[i + 1];
+            t0 = P.fbk[2 * b + 1];
+            while (b < be && P.fbk[2 * b] > al) ++b;
+            t1 = P.fbk[2 * b + 1];
+        }
+    }
+};
+__device__ __forceinline__ int rl(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+
+// The fill entries of a block's rows packed on the lanes, 64 PF_Q at a time:
+// entry, position in the fill list (-1: none) and the base that turns the
+// right-end column j into an LDS index of its row.
+#define PF_Q 4
+__device__ __forceinline__ int pick4(int x, int p1, int p2, int p3, int a0, int a1, int a2, int a3) {
+    const int lo = x < p1 ? a0 : a1, hi = x < p3 ? a2 : a3;
+    return x < p2 ? lo : hi;
+}
+struct PfBlock {
+    int o0, o1, o2, o3, p1, p2, p3, tot;  // fill entry minus packed index, packed starts, count
+    int b0, b1, b2, b3;                   // column bases of the rows
+    int pq[PF_Q], jm[PF_Q], tt[PF_Q], at[PF_Q];
+    double D[PF_Q];
+    __device__ __forceinline__ void rows(const PfRows &T, int r0) {
+        const int x = r0 & 63;
+        o0 = rl(T.t0, x);
+        p1 = rl(T.t1, x) - o0;
+        const int s1 = rl(T.t0, x + 1), s2 = rl(T.t0, x + 2), s3 = rl(T.t0, x + 3);
+        p2 = p1 + rl(T.t1, x + 1) - s1;
+        p3 = p2 + rl(T.t1, x + 2) - s2;
+        tot = p3 + rl(T.t1, x + 3) - s3;
+        o1 = s1 - p1;
+        o2 = s2 - p2;
+        o3 = s3 - p3;
+    }
+    __device__ __forceinline__ void load(const PfPair &P, int q, int x0) {
+        const int x = x0 + lane_id();
+        const int t = x < tot ? x + pick4(x, p1, p2, p3, o0, o1, o2, o3) : 0;
+        at[q] = pick4(x, p1, p2, p3, b0, b1, b2, b3);
+        struct PJ {
+            int x, y;
+        };
+        const PJ pj = *reinterpret_cast<const PJ *>(P.fcand + 2 * t);
+        pq[q] = pj.x;
+        jm[q] = pj.y;
+        D[q] = P.fD[t];
+        tt[q] = x < tot ? t : -1;
+    }
+    // the first 64 PF_Q entries
+    __device__ __forceinline__ void first(const PfPair &P) {
+        if (tot > 0) {
+            load(P, 0, 0);
+            load(P, 1, 64);
+        }
+        if (tot > 128) {
+            load(P, 2, 128);
+            load(P, 3, 192);
+        }
+    }
+    // fn(q0) handles entries q0 and q0 + 1, of all chunks
+    template <class Fn>
+    __device__ __forceinline__ void each(const PfPair &P, Fn fn) {
+        if (tot > 0) fn(0);
+        if (tot > 128) fn(2);
+        for (int x = 64 * PF_Q; x < tot; x += 64 * PF_Q) {
+#pragma unroll
+            for (int q = 0; q < PF_Q; ++q) load(P, q, x + 64 * q);
+            fn(0);
+            fn(2);
+        }
+    }
+};
+
+// Inside fill of a group (aligner_p.icc:150-312), values as pf_fill: M.
+template <int NC>
+__device__ __forceinline__ void pf_fwd_fixed(const PfPair &P, int al, int bl, int ar, int br, int W, double *base) {
     const int lane = lane_id();
     const double eo = P.eo, ps = P.ps;
-    double *Srow = base;
-    double *Mst = base + (br - bl);
-    const int nrows = ar - al - 1;
-    int rt0[RT], rt1[RT];
-    pf_row_table<RT>(P, al, bl, br, nrows, rt0, rt1);
-    for (int c = lane; c < br - bl; c += 64) Srow[c] = 0.0;
-    double Mp[NC], Ep[NC], gBc[NC];
+    const int SR = br - bl, nrows = ar - al - 1;
+    double *S = base, *Mst = base + 4 * SR;
+    for (int c = lane; c < 4 * SR; c += 64) S[c] = 0.0;
+    PfRows T;
+    T.load(P, al, bl, ar, br, 0);
+    PfBlock B;
+    auto block = [&](int r0) __attribute__((always_inline)) {
+        B.rows(T, r0);
+        B.first(P);
+    };
+    B.b0 = -bl - 1;
+    B.b1 = B.b0 + SR;
+    B.b2 = B.b1 + SR;
+    B.b3 = B.b2 + SR;
+    double Mp[NC], Ep[NC], cf[NC][6], ac[NC], gBo[NC];
     int cBc[NC];
     const int hi0 = min(br - 1, P.mx[al]);
     {
@@ -469,270 +546,310 @@ __device__ __forceinline__ void pf_fwd_fixed(const PfPair &P, int al, int bl, in
         for (int c = 0; c < NC; ++c) {
             const int j = bl + 1 + 64 * c + lane;
             const bool in = j <= hi0, col = j <= br - 1;
-            double a = in ? P.egB[j] : 1.0, b = 0.0;
-            wave_scan_affine(a, b);  // prefix products
-            Mp[c] = in ? carry * a : 0.0;
-            if (in) Mst[j - bl] = carry * a;
-            carry *= readlane_d(a, 63);
-            Ep[c] = 0.0;
-            gBc[c] = col ? P.egB[j] : 1.0;
+            const double g = col ? P.egB[j] : 1.0;
+            gBo[c] = g * eo;
             cBc[c] = col ? P.codeB[j] : 0;
+            ac[c] = scan_coef(g, cf[c]);
+            Mp[c] = in ? carry * ac[c] : 0.0;
+            if (in) Mst[j - bl] = Mp[c];
+            carry *= readlane_d(ac[c], 63);
+            Ep[c] = 0.0;
         }
         if (lane == 0) Mst[0] = 1.0 / ps;
     }
+    block(0);
     lds_fence();
     double colv = eo / ps;
     bool colopen = true;
     double Mcol_prev = 1.0 / ps;  // M(i-1, bl)
-    PfEnt cur[4];
-    {
-        int u0 = 0, u1 = 0;
-        if (nrows > 0) pf_row_cands<RT>(rt0, rt1, 0, u0, u1);
+    for (int r0 = 0; r0 <= nrows; r0 += 4) {
+        // arc terms ps * M(p-1, q-1) * D of the four rows, LDS atomic adds
+        B.each(P, [&](int q0) __attribute__((always_inline)) {
+            double v[2];
+            bool ok[2];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) cur[k] = pf_fetch(P, u0 + 64 * k + lane, u1);
-    }
-    for (int i = al + 1; i < ar; ++i) {
-        const int r = i - al - 1;
-        const int mni = P.mn[i];
-        double Mcol = 0.0;  // M(i, bl)
-        if (colopen && mni <= bl) {
-            colv *= P.egA[i];
-            Mcol = colv;
-        } else {
-            colopen = false;
-        }
-        const int lo = max(bl, mni), hi = min(br - 1, P.mx[i]);
-        double *row = Mst + (size_t)(r + 1) * W;
-        if (colopen && lane == 0) row[0] = colv;
-        const int jlo = max(bl + 1, mni);
-        int t0, t1;
-        pf_row_cands<RT>(rt0, rt1, r, t0, t1);
-        // arc terms ps * M(p-1, q-1) * D, candidate-parallel, LDS atomic adds
-        auto arc = [&](const PfEnt &e, bool in) {
-            const int p = e.pq & 0xffff, q = e.pq >> 16, j = e.jm & 0xffff;
-            const int rl = max(bl, e.jm >> 16);
-            const bool ok = in && q > bl && j >= jlo && j <= hi && q - 1 >= rl;
-            const double v = Mst[ok ? (p - 1 - al) * W + (q - 1 - rl) : 0] * e.D * ps;
-            if (ok) atomicAdd(&Srow[j - bl - 1], v);
-        };
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (t0 + 64 * k < t1) arc(cur[k], t0 + 64 * k + lane < t1);
-        for (int t = t0 + 256 + lane; t < t1; t += 64) arc(pf_fetch(P, t, t1), true);
-        if (r + 1 < nrows) {  // the next row's chunks
-            int u0, u1;
-            pf_row_cands<RT>(rt0, rt1, r + 1, u0, u1);
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (u0 + 64 * k < u1) cur[k] = pf_fetch(P, u0 + 64 * k + lane, u1);
-        }
-        lds_fence();
-        double Fcarry = 0.0, sprev = Mcol, dgin = Mcol_prev;
-        const double gA = P.egA[i];
-        const double *esrow = P.es + P.codeA[i] * LCG_NCODES;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const int j = bl + 1 + 64 * c + lane;
-            const bool act = j >= jlo && j <= hi;
-            const double up = Mp[c];
-            const double dg = shift_up_d(Mp[c], dgin);
-            dgin = readlane_d(Mp[c], 63);
-            double s = 0.0, e = 0.0;
-            if (act) {
-                const double ep = Ep[c];
-                e = ep * gA + (up - ep) * gA * eo;
-                Ep[c] = e;
-                const double sv = Srow[j - bl - 1];
-                Srow[j - bl - 1] = 0.0;
-                s = dg * esrow[cBc[c]] + e + sv;
+            for (int h = 0; h < 2; ++h) {
+                const int pq = B.pq[q0 + h], jm = B.jm[q0 + h];
+                const int p = pq & 0xffff, q = pq >> 16, j = jm & 0xffff, mc = max(bl, jm >> 16);
+                ok[h] = B.tt[q0 + h] >= 0 && q > bl && j < br && q - 1 >= mc;
+                v[h] = Mst[ok[h] ? (p - 1 - al) * W + (q - 1 - mc) : 0] * B.D[q0 + h] * ps;
             }
-            const double sl = shift_up_d(s, sprev);
-            double a = act ? gBc[c] : 1.0, b = act ? sl * gBc[c] * eo : 0.0;
-            wave_scan_affine(a, b);
-            const double F = a * Fcarry + b;
-            const double Mv = s + F;
-            if (act) {
-                const size_t idx = (size_t)(r + 1) * W + (j - lo);
-                row[j - lo] = Mv;
-                if (Es) {
-                    Es[idx] = e;
-                    Ss[idx] = s;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (ok[h]) atomicAdd(&S[B.at[q0 + h] + (B.jm[q0 + h] & 0xffff)], v[h]);
+        });
+        lds_fence();
+        // the rows' operands, then the next block's entries
+        double sv[4][NC], es[4][NC], gAk[4];
+        int mnk[4], mxk[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int x = (r0 + k) & 63;
+            mnk[k] = rl(T.mn, x);
+            mxk[k] = rl(T.mx, x);
+            gAk[k] = readlane_d(T.gA, x);
+            const int code = rl(T.code, x);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                double *sp = S + k * SR + min(64 * c + lane, SR - 1);
+                sv[k][c] = *sp;
+                *sp = 0.0;
+                es[k][c] = P.es[code + cBc[c]];
+            }
+        }
+        if (r0 + 4 <= nrows) {
+            if (((r0 + 4) & 63) == 0) T.load(P, al, bl, ar, br, r0 + 4);
+            block(r0 + 4);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int r = r0 + k;
+            if (r > nrows) break;
+            if (r == 0) continue;
+            const int mni = mnk[k];
+            const double gA = gAk[k];
+            double Mcol = 0.0;  // M(i, bl)
+            if (colopen && mni <= bl) {
+                colv *= gA;
+                Mcol = colv;
+            } else {
+                colopen = false;
+            }
+            const int lo = max(bl, mni), hi = min(br - 1, mxk[k]), jlo = max(bl + 1, mni);
+            double *row = Mst + r * W;
+            if (mni <= bl && lane == 0) row[0] = Mcol;
+            double Fcarry = 0.0, sprev = Mcol, dgin = Mcol_prev;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int j0 = bl + 1 + 64 * c, j = j0 + lane;
+                const double up = Mp[c];
+                const double last = c + 1 < NC ? readlane_d(up, 63) : 0.0;
+                // a chunk without a cell of the row
+                if (NC > 1 && (j0 > hi || j0 + 63 < jlo)) {
+                    Mp[c] = 0.0;
+                    dgin = last;
+                    Fcarry = 0.0;
+                    sprev = 0.0;
+                    continue;
+                }
+                const bool act = j >= jlo && j <= hi;
+                const double dg = shift_up_d(up, dgin);
+                dgin = last;
+                const double ep = Ep[c];
+                const double e = ep * gA + (up - ep) * gA * eo;
+                Ep[c] = act ? e : ep;
+                const double s = act ? dg * es[k][c] + e + sv[k][c] : 0.0;
+                double F = scan_lin(shift_up_d(s, sprev) * gBo[c], cf[c]);
+                if (c > 0) F = fma(ac[c], Fcarry, F);
+                const double Mv = s + F;
+                if (act) row[j - lo] = Mv;
+                Mp[c] = act ? Mv : 0.0;
+                if (c + 1 < NC) {
+                    Fcarry = readlane_d(F, 63);
+                    sprev = readlane_d(s, 63);
                 }
             }
-            Mp[c] = act ? Mv : 0.0;
-            Fcarry = readlane_d(F, 63);
-            sprev = readlane_d(s, 63);
+            Mcol_prev = Mcol;
         }
-        Mcol_prev = Mcol;
         lds_fence();
     }
 }
 
 // Adjoint of pf_fwd_fixed for a group whose Mbar rows (LDS, after M) hold the
-// seeds; Es/Ss from the forward recompute.  FULL: also Dbar (dZ/dD per
-// candidate entry) and the gap-opening weight (returned); edge receives the
-// match-edge weights.  Same terms as pf_reverse.
+// seeds.  FULL: also Dbar (dZ/dD per fill entry) and the gap-opening weight
+// (returned); edge receives the match-edge weights.  Same terms as pf_reverse.
 //
-// The sweep visits rows ar-1 .. al+1.  Once a row is done no later row reads
-// its Mbar, so each computed cell's Mbar is replaced by its sbar there; the
-// arc terms of the row read sbar from LDS.  The global accumulations (Dbar +=
-// sbar M(p-1,q-1) ps per arc candidate, edge += sbar M(i-1,j-1) es per cell)
-// are issued inside the sweep, next to the values they use (a separate pass
-// after the sweep that re-reads sbar and M measured slower).  The sweep's
-// Ss/Es loads (FULL) are issued a row ahead.
-template <int NC, bool FULL, int RT = 2>
-__device__ __forceinline__ double pf_rev_fixed(const PfPair &P, int al, int bl, int ar, int br, int W, double *base, const double *Es,
-                               const double *Ss, double *edge, double *edge2 = nullptr) {
+// The lanes hold the columns from the right (lane l of chunk c: br-1-64c-l),
+// so that the F adjoint is a prefix scan.  Blocks run from row ar-1 down.
+// Once a row is done no later row reads its Mbar, so each computed cell's
+// Mbar is replaced by its sbar there for the arc terms.
+//
+// Openings: with s = M - F, the weight sum_j Fbar_j gB_j o s_{j-1} equals
+// sum_j gB_j o M(i, j-1) U_j, U_j = Mbar_j + gB_{j+1} (1-o) U_{j+1} (F_j as a
+// recurrence driven by M(i, j-1), summed by parts); alike for E with U over the
+// rows and the adjoint of s without its vertical part.  Only positive terms,
+// and of the forward values only M is needed.
+template <int NC, bool FULL>
+__device__ __forceinline__ double pf_rev_fixed(const PfPair &P, int al, int bl, int ar, int br, int W, double *base,
+                               double *edge, double *edge2 = nullptr) {
     const int lane = lane_id();
-    const double eo = P.eo, ps = P.ps;
-    const double *Mst = base + (br - bl);
-    double *Mb = base + (br - bl) + (size_t)(ar - al) * W;
+    const double eo = P.eo, ec = 1.0 - P.eo, ps = P.ps;
+    const double *Mst = base + 4 * (br - bl);
+    double *Mb = base + 4 * (br - bl) + (ar - al) * W;
     const int nrows = ar - al - 1;
-    int rt0[RT], rt1[RT];
-    pf_row_table<RT>(P, al, bl, br, nrows, rt0, rt1);
-    double carry[NC], Eb[NC], gBc[NC];
+    double cf[NC][6], ac[NC], uf[NC][6], au[NC], gBo[NC], gBn[NC];
+    double cv[NC], cd[NC], Eb[NC], Ue[NC], left[NC];
     int cBc[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        const int j = bl + 1 + 64 * c + lane;
-        carry[c] = 0.0;
-        Eb[c] = 0.0;
-        gBc[c] = (j <= br - 1) ? P.egB[j] : 1.0;
-        cBc[c] = (j <= br - 1) ? P.codeB[j] : 0;
-    }
     // first stored column of row i of the region (row al from bl)
     auto lo_of = [&](int i) { return (i == al) ? bl : max(bl, P.mn[i]); };
-    // Ss of row i at column j - 1 and Es of row i - 1 at column j (clamped
-    // into the stored rows; the caller's flags decide whether they are used)
-    double ssc[NC], esc[NC];
-    auto load_se = [&](int i, double *ss, double *es) {
-        const int r = i - al - 1;
-        const int lo = lo_of(i), lo_u = lo_of(i - 1);
+    const int rs = nrows & ~3;
+    PfRows T;
+    T.load(P, al, bl, ar, br, rs & ~63);
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const int j = bl + 1 + 64 * c + lane;
-            ss[c] = Ss[(size_t)(r + 1) * W + min(max(j - 1 - lo, 0), W - 1)];
-            es[c] = Es[(size_t)r * W + min(max(j - lo_u, 0), W - 1)];
-        }
-    };
-    if (FULL && nrows > 0) load_se(ar - 1, ssc, esc);
+    for (int c = 0; c < NC; ++c) {
+        const int j = br - 1 - 64 * c - lane;
+        const bool col = j > bl;
+        const double gn = col && j < br - 1 ? P.egB[j + 1] : 0.0;
+        gBo[c] = (col ? P.egB[j] : 0.0) * eo;
+        gBn[c] = gn * eo;
+        cBc[c] = col ? P.codeB[j] : 0;
+        // the first lane's multiplier belongs to the chunk on the right: it
+        // enters with ac / au
+        ac[c] = scan_coef(gn, cf[c]);
+        if (FULL) au[c] = scan_coef(gn * ec, uf[c]);
+        cv[c] = cd[c] = Eb[c] = Ue[c] = 0.0;
+        // M(ar-1, j-1)
+        const int lo = lo_of(ar - 1), x = j - 1 - lo;
+        left[c] = (nrows > 0 && x >= 0 && j - 1 <= min(br - 1, P.mx[ar - 1])) ? Mst[nrows * W + min(x, W - 1)] : 0.0;
+    }
+    const int lc = (br - 2 - bl) >> 6, ll = (br - 2 - bl) & 63;  // chunk and lane of column bl+1
     double colcarry = 0.0;  // contribution of row i+1 to Mbar(i, bl)
     double open_acc = 0.0;
-    // first 64 fill entries of the row, fetched one row ahead; rows are
-    // visited downwards
-    PfEnt ce;
-    {
-        int u0 = 0, u1 = 0;
-        if (nrows > 0) pf_row_cands<RT>(rt0, rt1, nrows - 1, u0, u1);
-        ce = pf_fetch(P, u0 + lane, u1);
-    }
+    PfBlock B;
+    auto block = [&](int r0) __attribute__((always_inline)) {
+        B.rows(T, r0);
+        // Mbar index of column 0 of the block's rows
+        B.b0 = r0 * W - (r0 == 0 ? bl : max(bl, rl(T.mn, r0 & 63)));
+        B.b1 = (r0 + 1) * W - max(bl, rl(T.mn, (r0 + 1) & 63));
+        B.b2 = (r0 + 2) * W - max(bl, rl(T.mn, (r0 + 2) & 63));
+        B.b3 = (r0 + 3) * W - max(bl, rl(T.mn, (r0 + 3) & 63));
+        B.first(P);
+    };
+    block(rs);
     lds_fence();
-    for (int i = ar - 1; i > al; --i) {
-        const int r = i - al - 1;
-        PfEnt ne = ce;
-        double ssn[NC], esn[NC];
-        if (r > 0) {
-            int u0, u1;
-            pf_row_cands<RT>(rt0, rt1, r - 1, u0, u1);
-            if (u1 > u0) ne = pf_fetch(P, u0 + lane, u1);
-            if (FULL) load_se(i - 1, ssn, esn);
-        }
-        const int mni = P.mn[i];
-        const int lo = max(bl, mni), hi = min(br - 1, P.mx[i]), jlo = max(bl + 1, mni);
-        const bool colopen_i = mni <= bl;
-        const int lo_u = lo_of(i - 1), hi_u = min(br - 1, P.mx[i - 1]);
-        const int jlo_u = max(bl + 1, P.mn[i - 1]);
-        const bool upc_row = i - 1 > al;  // row i-1 computed (has E)
-        const double *rowM = Mst + (size_t)(r + 1) * W;
-        const double *rowU = Mst + (size_t)r * W;
-        double *rowB = Mb + (size_t)(r + 1) * W;
-        const double gA = P.egA[i];
-        const double *esrow = P.es + P.codeA[i] * LCG_NCODES;
-        double Fb_in = 0.0, gB_in = 0.0, d_in = 0.0;
-        double newcarry[NC];
-        double colcarry_next = 0.0, colb = 0.0;
-#pragma unroll
-        for (int cc = NC - 1; cc >= 0; --cc) {
-            const int j = bl + 1 + 64 * cc + lane;
-            const bool act = j >= jlo && j <= hi;
-            const double g = act ? rowB[j - lo] + carry[cc] : 0.0;
-            const double gB = act ? gBc[cc] : 0.0;
-            const double gB_next = shift_down_d(gB, gB_in);
-            double cm = act ? gB_next : 0.0, gg = g;
-            wave_suffix_affine(cm, gg);
-            const double Fb = cm * Fb_in + gg;  // Fbar_j
-            const double Fb_next = shift_down_d(Fb, Fb_in);
-            const double sb = act ? g + Fb_next * gB_next * eo : 0.0;
-            if (act) rowB[j - lo] = sb;  // this row's Mbar is not read again
-            const bool bcol = act && j == jlo && jlo == bl + 1 && colopen_i;  // s_{j-1} = M(i, bl)
-            if (FULL && act) {
-                const double sl = (j == jlo) ? (bcol ? rowM[0] : 0.0) : ssc[cc];
-                open_acc += Fb * sl * gB * eo;
-            }
-            if (cc == 0) colb = readlane_d(bcol ? Fb * gB * eo : 0.0, 0);
-            // E chain: E(i,j) = E(i-1,j) gA (1-o) + M(i-1,j) gA o
-            const double eb = act ? sb + Eb[cc] : 0.0;
-            const bool upst = j >= lo_u && j <= hi_u;
-            if (FULL && act) {
-                const double up = upst ? rowU[j - lo_u] : 0.0;
-                const bool upc = upc_row && j >= jlo_u && j <= hi_u;
-                const double Ep = upc ? esc[cc] : 0.0;
-                open_acc += eb * (up - Ep) * gA * eo;
-            }
-            Eb[cc] = act ? eb * gA * (1.0 - eo) : 0.0;
-            // match: s_j uses M(i-1, j-1) es
-            const bool dgst = act && j - 1 >= lo_u && j - 1 <= hi_u;
-            const double d = dgst ? sb * esrow[cBc[cc]] : 0.0;  // to Mbar(i-1, j-1)
-            if (dgst) {  // match-edge weight sbar M(i-1, j-1) es
-                const double w = d * rowU[j - 1 - lo_u];
-                atomicAdd(&edge[P.coff[i] - mni + j], w);
-                if (edge2) atomicAdd(&edge2[P.coff[i] - mni + j], w);
-            }
-            const double d_right = shift_down_d(d, d_in);
-            newcarry[cc] = upst ? (act ? eb * gA * eo : 0.0) + d_right : 0.0;
-            if (cc == 0) colcarry_next = readlane_d(d, 0);
-            d_in = readlane_d(d, 0);
-            Fb_in = readlane_d(Fb, 0);
-            gB_in = readlane_d(gB, 0);
-        }
-        // the init column cell (i, bl): one opening per value
-        if (FULL && colopen_i && lane == 0) open_acc += (rowB[0] + colcarry + colb) * rowM[0];
-        lds_fence();
-        // arc terms: Mbar(p-1, q-1) += sbar D ps
-        int t0, t1;
-        pf_row_cands<RT>(rt0, rt1, r, t0, t1);
-        // arc terms: Mbar(p-1, q-1) += sbar D ps and (FULL) Dbar += sbar
-        // M(p-1, q-1) ps of the candidate entry tt
-        auto arc = [&](const PfEnt &e, int tt, bool in) {
-            const int p = e.pq & 0xffff, q = e.pq >> 16, j = e.jm & 0xffff;
-            const int rl = max(bl, e.jm >> 16);
-            if (in && q > bl && j >= jlo && j <= hi && q - 1 >= rl && e.D != 0.0) {
-                atomicAdd(&Mb[(p - 1 - al) * W + (q - 1 - rl)], rowB[j - lo] * e.D * ps);
-                if (FULL) atomicAdd(&P.fDb[tt], rowB[j - lo] * Mst[(p - 1 - al) * W + (q - 1 - rl)] * ps);
-            }
-        };
-        if (t1 > t0) arc(ce, t0 + lane, t0 + lane < t1);
-        for (int t = t0 + 64 + lane; t < t1; t += 64) arc(pf_fetch(P, t, t1), t, true);
-        ce = ne;
-        if (FULL && r > 0) {
+    for (int r0 = rs; r0 >= 0; r0 -= 4) {
+        // operands of the four rows (NC 3: of each row in its turn, for the registers)
+        double mb[4][NC], up[4][NC], dg[4][NC], es[4][NC], gAk[4];
+        int mnk[4], mxk[4], mnu[4], mxu[4], cok[4];
+        auto operands = [&](int k) __attribute__((always_inline)) {
+            const int x = (r0 + k) & 63, r = min(r0 + k, nrows);
+            mnk[k] = rl(T.mn, x);
+            mxk[k] = rl(T.mx, x);
+            mnu[k] = rl(T.mnu, x);
+            mxu[k] = rl(T.mxu, x);
+            cok[k] = rl(T.co, x);
+            gAk[k] = readlane_d(T.gA, x);
+            const int code = rl(T.code, x);
+            const int lo = max(bl, mnk[k]), lou = r <= 1 ? bl : max(bl, mnu[k]);
+            const int hiu = min(br - 1, mxu[k]), ru = max(r - 1, 0) * W;
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
-                ssc[c] = ssn[c];
-                esc[c] = esn[c];
+                const int j = br - 1 - 64 * c - lane;
+                mb[k][c] = Mb[r * W + min(max(j - lo, 0), W - 1)];
+                const double u = Mst[ru + min(max(j - lou, 0), W - 1)];
+                const double d = Mst[ru + min(max(j - 1 - lou, 0), W - 1)];
+                up[k][c] = j >= lou && j <= hiu ? u : 0.0;
+                dg[k][c] = j - 1 >= lou && j - 1 <= hiu ? d : 0.0;
+                es[k][c] = P.es[code + cBc[c]];
             }
+        };
+        if (NC < 3)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) operands(k);
+#pragma unroll
+        for (int k = 3; k >= 0; --k) {
+            const int r = r0 + k;
+            if (r > nrows || r == 0) continue;
+            if (NC >= 3) operands(k);
+            const int mni = mnk[k];
+            const int lo = max(bl, mni), hi = min(br - 1, mxk[k]), jlo = max(bl + 1, mni);
+            const bool colopen = mni <= bl;
+            const int lou = r == 1 ? bl : max(bl, mnu[k]), hiu = min(br - 1, mxu[k]);
+            double *rowB = Mb + r * W;
+            const double gA = gAk[k], gAo = gA * eo, gAc = gA * ec;
+            double Fb_in = 0.0, U_in = 0.0, d_in = 0.0, colb = 0.0, cnext = 0.0;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int j0 = br - 1 - 64 * c, j = j0 - lane;
+                const bool here = !(NC > 1 && (j0 < jlo || j0 - 63 > hi));
+                const bool upst = j >= lou && j <= hiu;
+                double d = 0.0;
+                if (here) {
+                    const bool act = j >= jlo && j <= hi;
+                    const double g0 = act ? mb[k][c] + cd[c] : 0.0;
+                    const double gv = act ? cv[c] : 0.0;
+                    const double g = g0 + gv;
+                    double Fb = scan_lin(g, cf[c]);
+                    if (c > 0) Fb = fma(ac[c], Fb_in, Fb);
+                    const double Fb_next = shift_up_d(Fb, Fb_in);
+                    const double sp = act ? fma(Fb_next, gBn[c], g0) : 0.0;  // sbar without the vertical part
+                    const double sb = sp + gv;
+                    if (act) rowB[j - lo] = sb;
+                    const double eb = act ? sb + Eb[c] : 0.0;
+                    if (FULL) {
+                        double U = scan_lin(g, uf[c]);
+                        if (c > 0) U = fma(au[c], U_in, U);
+                        const double ue = act ? sp + Ue[c] : 0.0;
+                        // left is 0 outside the stored row, U left of its cells is not used
+                        open_acc += (act ? U * left[c] : 0.0) * gBo[c] + ue * up[k][c] * gAo;
+                        Ue[c] = ue * gAc;
+                        if (c + 1 < NC) U_in = readlane_d(U, 63);
+                    }
+                    Eb[c] = eb * gAc;
+                    // match: s_j uses M(i-1, j-1) es
+                    const bool dgst = act && j - 1 >= lou && j - 1 <= hiu;
+                    d = dgst ? sb * es[k][c] : 0.0;  // to Mbar(i-1, j-1)
+                    if (dgst) {  // match-edge weight sbar M(i-1, j-1) es
+                        const double w = d * dg[k][c];
+                        atomicAdd(&edge[cok[k] - mni + j], w);
+                        if (edge2) atomicAdd(&edge2[cok[k] - mni + j], w);
+                    }
+                    cv[c] = upst ? eb * gAo : 0.0;
+                    if (c == lc) {
+                        // s_{j-1} = M(i, bl) of column bl + 1
+                        if (jlo == bl + 1 && colopen && bl + 1 <= hi) colb = readlane_d(Fb * gBo[c], ll);
+                        cnext = readlane_d(d, ll);
+                    }
+                    if (c + 1 < NC) Fb_in = readlane_d(Fb, 63);
+                } else {
+                    Eb[c] = Ue[c] = cv[c] = 0.0;
+                    Fb_in = U_in = 0.0;
+                }
+                const double dr = shift_up_d(d, d_in);
+                cd[c] = upst ? dr : 0.0;
+                if (c + 1 < NC) d_in = readlane_d(d, 63);
+                if (FULL) left[c] = dg[k][c];
+            }
+            // the init column cell (i, bl): one opening per value
+            if (FULL && colopen && lane == 0) open_acc += (rowB[0] + colcarry + colb) * Mst[r * W];
+            colcarry = (lou == bl) ? cnext : 0.0;
         }
         lds_fence();
+        // arc terms: Mbar(p-1, q-1) += sbar D ps and (FULL) Dbar += sbar
+        // M(p-1, q-1) ps of the fill entry
+        B.each(P, [&](int q0) __attribute__((always_inline)) {
+            double sb[2], mv[2];
+            int x[2];
+            bool ok[2];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) carry[c] = newcarry[c];
-        colcarry = (lo_u == bl) ? colcarry_next : 0.0;
+            for (int h = 0; h < 2; ++h) {
+                const int pq = B.pq[q0 + h], jm = B.jm[q0 + h];
+                const int p = pq & 0xffff, q = pq >> 16, j = jm & 0xffff, mc = max(bl, jm >> 16);
+                ok[h] = B.tt[q0 + h] >= 0 && q > bl && j < br && q - 1 >= mc && B.D[q0 + h] != 0.0;
+                x[h] = ok[h] ? (p - 1 - al) * W + (q - 1 - mc) : 0;
+                sb[h] = Mb[ok[h] ? B.at[q0 + h] + j : 0] * ps;
+                if (FULL) mv[h] = Mst[x[h]];
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (ok[h]) {
+                    atomicAdd(&Mb[x[h]], sb[h] * B.D[q0 + h]);
+                    if (FULL) atomicAdd(&P.fDb[B.tt[q0 + h]], sb[h] * mv[h]);
+                }
+        });
+        if (r0 >= 4) {
+            if ((r0 & 63) == 0) T.load(P, al, bl, ar, br, r0 - 64);
+            block(r0 - 4);
+        }
+        lds_fence();
     }
     // init row al: one opening per value M(al, j), j > bl
     if (FULL) {
         const int hi0 = min(br - 1, P.mx[al]);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-            const int j = bl + 1 + 64 * c + lane;
-            if (j <= hi0) open_acc += (Mb[j - bl] + carry[c]) * Mst[j - bl];
+            const int j = br - 1 - 64 * c - lane;
+            if (j > bl && j <= hi0) open_acc += (Mb[j - bl] + cv[c] + cd[c]) * Mst[j - bl];
         }
     }
     // fragment queries: the computed cells hold sbar now (lanes over queries)
@@ -957,19 +1074,16 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                     const int off = S[4 * g + 1];
                     if (off >= 0) {
                         double *base = pool + off;
-                        // the forward values the outside pass reads (E, s, M), if stored
                         const int so = sched[f.fso + g];
-                        const size_t cells = (size_t)(gar - gal) * W;
-                        double *Es = so >= 0 ? fstore + 4 * (size_t)so : nullptr;
-                        double *Ss = so >= 0 ? Es + cells : nullptr;
+                        const int cells = (gar - gal) * W;
                         if (gbr - gbl - 1 <= 64)
-                            pf_fwd_fixed<1>(P, gal, gbl, gar, gbr, W, base, Es, Ss);
+                            pf_fwd_fixed<1>(P, gal, gbl, gar, gbr, W, base);
                         else
-                            pf_fwd_fixed<2>(P, gal, gbl, gar, gbr, W, base, Es, Ss);
-                        const double *Mst = base + (gbr - gbl);
-                        if (so >= 0) {
-                            double *Ms = Ss + cells;
-                            for (size_t c = lane; c < cells; c += 64) Ms[c] = Mst[c];
+                            pf_fwd_fixed<2>(P, gal, gbl, gar, gbr, W, base);
+                        const double *Mst = base + 4 * (gbr - gbl);
+                        if (so >= 0) {  // M, which the outside pass reads
+                            double *Ms = fstore + 4 * (size_t)so;
+                            for (int c = lane; c < cells; c += 64) Ms[c] = Mst[c];
                         }
                         for (int t = G[3] + lane; t < G[4]; t += 64) {
                             const int4 ga = gams[t];
@@ -1003,22 +1117,20 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
         if (wave == 0 && member == 0) {
             const int W = d.wtop;
             const size_t cells = (size_t)(n + 1) * W;
-            if (n <= 192 && m <= 192 && (size_t)(m + 1) + 2 * cells <= (size_t)bp.pool) {
-                // the whole LDS pool is free while the other waves wait: the
-                // fixed-column kernels (E, s of every cell in the wave's scratch)
+            if (n <= 192 && m <= 192 && 4 * (size_t)(m + 1) + 2 * cells <= (size_t)bp.pool) {
+                // the whole LDS pool is free while the other waves wait
                 double *base = pool;
-                double *Es = wscr, *Ss = wscr + cells;
-                pf_fwd_fixed<3, 3>(P, 0, 0, n + 1, m + 1, W, base, Es, Ss);
+                pf_fwd_fixed<3>(P, 0, 0, n + 1, m + 1, W, base);
                 const int xz = fixed_at(0, 0, m + 1, W, n, m);
-                const double Z = xz >= 0 ? base[(m + 1) + xz] : 0.0;
+                double *Mst = base + 4 * (m + 1);
+                const double Z = xz >= 0 ? Mst[xz] : 0.0;
                 if (lane == 0) pfa[f.out + 0] = Z;
-                double *Mb = base + (m + 1) + cells;
+                double *Mb = Mst + cells;
                 for (size_t c = lane; c < cells; c += 64) Mb[c] = 0.0;
                 lds_fence();
                 if (lane == 0 && xz >= 0) Mb[xz] = 1.0;
-                scratch_sync();  // Es/Ss (global) and the seed (LDS) before the sweep
-                const double o = pf_rev_fixed<3, true, 3>(P, 0, 0, n + 1, m + 1, W, base, Es, Ss, P.edge_full,
-                                                          P.edge_ref);
+                lds_fence();  // the seed before the sweep
+                const double o = pf_rev_fixed<3, true>(P, 0, 0, n + 1, m + 1, W, base, P.edge_full, P.edge_ref);
                 if (lane == 0) atomicAdd(&s_open, o);
             } else {
                 const Region R = region(0, 0, n + 1, m + 1, W);
@@ -1061,26 +1173,30 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                     const bool sig = __ballot(any) != 0;
                     if (off >= 0) {
                         double *base = pool + off;
-                        const size_t cells = (size_t)(gar - gal) * W;
-                        double *Mb = base + (gbr - gbl) + cells;
+                        const int cells = (gar - gal) * W;
+                        double *Mst = base + 4 * (gbr - gbl), *Mb = Mst + cells;
                         const bool nc1 = gbr - gbl - 1 <= 64;
                         const int so = sched[f.fso + g];
-                        double *Es = wscr, *Ss = wscr + cells;
                         if (so >= 0) {
-                            // the inside pass's forward values: M into the region
-                            Es = fstore + 4 * (size_t)so;
-                            Ss = Es + cells;
-                            const double *Ms = Ss + cells;
-                            double *Mst = base + (gbr - gbl);
-                            for (size_t c = lane; c < cells; c += 64) Mst[c] = Ms[c];
+                            // the inside pass's M into the region
+                            const double *Ms = fstore + 4 * (size_t)so;
+                            int c = lane;
+                            for (; c + 7 * 64 < cells; c += 8 * 64) {
+                                double v[8];
+#pragma unroll
+                                for (int q = 0; q < 8; ++q) v[q] = Ms[c + 64 * q];
+#pragma unroll
+                                for (int q = 0; q < 8; ++q) Mst[c + 64 * q] = v[q];
+                            }
+                            for (; c < cells; c += 64) Mst[c] = Ms[c];
                             lds_fence();
                         } else if (nc1) {
-                            pf_fwd_fixed<1>(P, gal, gbl, gar, gbr, W, base, Es, Ss);
+                            pf_fwd_fixed<1>(P, gal, gbl, gar, gbr, W, base);
                         } else {
-                            pf_fwd_fixed<2>(P, gal, gbl, gar, gbr, W, base, Es, Ss);
+                            pf_fwd_fixed<2>(P, gal, gbl, gar, gbr, W, base);
                         }
                         for (int pass = 0; pass < (sig ? 2 : 1); ++pass) {
-                            for (size_t c = lane; c < cells; c += 64) Mb[c] = 0.0;
+                            for (int c = lane; c < cells; c += 64) Mb[c] = 0.0;
                             lds_fence();
                             for (int t = G[3] + lane; t < G[4]; t += 64) {
                                 const int4 ga = gams[t];
@@ -1089,18 +1205,16 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                                 const int x = fixed_at(gal, gbl, gbr, W, ar - 1, br - 1);
                                 if (x >= 0) atomicAdd(&Mb[x], dbar(ga) * P.eam[ga.y]);
                             }
-                            scratch_sync();  // Es/Ss (global) and the seeds (LDS) before the sweep
+                            lds_fence();  // the seeds before the sweep
                             if (pass == 0) {
-                                const double o = nc1 ? pf_rev_fixed<1, true>(P, gal, gbl, gar, gbr, W, base, Es, Ss,
-                                                                                P.edge_full)
-                                                     : pf_rev_fixed<2, true>(P, gal, gbl, gar, gbr, W, base, Es, Ss,
-                                                                                P.edge_full);
+                                const double o = nc1 ? pf_rev_fixed<1, true>(P, gal, gbl, gar, gbr, W, base, P.edge_full)
+                                                     : pf_rev_fixed<2, true>(P, gal, gbl, gar, gbr, W, base, P.edge_full);
                                 if (lane == 0) atomicAdd(&s_open, o);
                             } else {
                                 if (nc1)
-                                    pf_rev_fixed<1, false>(P, gal, gbl, gar, gbr, W, base, Es, Ss, P.edge_ref);
+                                    pf_rev_fixed<1, false>(P, gal, gbl, gar, gbr, W, base, P.edge_ref);
                                 else
-                                    pf_rev_fixed<2, false>(P, gal, gbl, gar, gbr, W, base, Es, Ss, P.edge_ref);
+                                    pf_rev_fixed<2, false>(P, gal, gbl, gar, gbr, W, base, P.edge_ref);
                             }
                         }
                     } else {

@@ -30,10 +30,9 @@
 // wave<<12, outside LDS offset; offset -1: the group runs in global
 // scratch), the number of rounds of every row for both passes, and per
 // group the offset of its forward values in the store (units of 4 doubles;
-// -1: none, the outside pass recomputes them): E and s = M - F of every
-// computed cell and the region's M rows, (ar - al) W doubles each, written
-// by the inside pass and read by the outside pass instead of a second
-// forward fill.
+// -1: none, the outside pass recomputes them): the region's M rows,
+// (ar - al) W doubles, written by the inside pass and read by the outside
+// pass instead of a second forward fill.
 #pragma once
 #include <stdint.h>
 
