@@ -425,9 +425,9 @@ int64_t lcg_batch_write_bm_probs(const lcg_batch *batch, int32_t k, int32_t incl
 int lcg_batch_pf_sample(const lcg_batch *batch, int32_t k, uint64_t seed, int32_t nsamples, double *mean,
                         double *var, int32_t cap);
 /* LocARNA-P launch configuration of the batch (no counterpart in the
- * reference): the first `nstatic` pairs of the work order (largest first) run
- * on `wg_per_pair` workgroups each, the others one workgroup each from a
- * queue; `workgroups` in all. */
+ * reference): `nstatic` pairs, the first of the work order (largest first), run
+ * on `wg_per_pair` workgroups each or more, the others on one workgroup each;
+ * `workgroups` in all. */
 int lcg_batch_pf_config(lcg_batch *batch, int32_t *wg_per_pair, int32_t *nstatic, int32_t *workgroups);
 /* Z (AlignerP::align_inside) and the expected number of gap openings */
 int lcg_batch_pf_result(const lcg_batch *batch, int32_t k, double *Z, double *openings);

@@ -1003,6 +1003,7 @@ struct lcg_batch {
     double *d_pfscratch = nullptr;
     double *d_pfstore = nullptr;  // LocARNA-P forward values of the fixed-column groups (inside -> outside)
     int pf_grid = 0, pf_waves = 8;
+    int pf_split = 0, pf_nsplit = 0;  // fewest workgroups of a pair with several, pairs with several
     size_t pf_lds = 0;
     PfBatchParams pbp;
     bool pf_have = false;
@@ -2513,46 +2514,64 @@ int pf_setup(lcg_batch &B) {
     if (pool < 64) return LCG_E_CAPACITY;
     B.pbp.pool = pool;
     B.pf_lds = (size_t)4 * hdr_ints + (size_t)8 * (hdr_doubles + pool);
-    // workgroups per pair: with fewer pairs than CUs, K workgroups share a
-    // pair (all resident, one per CU)
+    // Workgroups per pair (members; all workgroups resident, one per CU): the
+    // numbers that make the slowest pair's estimated time smallest, the pairs
+    // that are not dealt being queued for the remaining workgroups.  A pair on
+    // k workgroups takes about (1 + 0.08 (k - 1)) / k of its time on one (120
+    // pairs of 150 nt 109 -> 62 ms on two each; 48 ragged pairs 202, 116 and 99
+    // ms on two, four and five each).  No more than a pair has groups per row:
+    // one pair of 88 nt (14 groups a row) takes 7.12 ms on 4, 6.90 on 16 and
+    // 7.03 on 64.
     int cus = 0;
     HIPCHECK(hipSetDevice(B.device));
     HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, B.device));
     const bool forced = B.req.pf_wg_per_pair > 0 || std::getenv("LCG_PF_WG_PER_PAIR");
-    int K = pick(B.req.pf_wg_per_pair, "LCG_PF_WG_PER_PAIR", np < cus ? std::min(64, cus / np) : 1, 1, 64);
-    K = std::min(K, std::max(1, cus / np));
-    // the first nst pairs of the work order get K workgroups each, statically;
-    // the others are pulled from the queue by the remaining workgroups.  With
-    // at most half as many pairs as CUs all pairs are static.  Otherwise the largest pairs
-    // get two workgroups where that shortens the estimated makespan (a pair
-    // on two workgroups measured about 1.75x faster; the rest by longest
-    // processing time first over the other workgroups).
-    int nst = K > 1 ? np : 0;
-    if (K == 1 && cus >= 4 && !forced) {
-        auto makespan = [&](int ns) {
-            double t = 0;
-            for (int q = 0; q < ns; ++q) t = std::max(t, (double)B.work[B.order[q]] / 1.75);
-            const int rest = cus - 2 * ns;
-            if (ns < np && rest < 1) return 1e300;
-            std::vector<double> load(std::max(rest, 1), 0.0);
-            for (int q = ns; q < np; ++q) {
-                auto it = std::min_element(load.begin(), load.end());
-                *it += (double)B.work[B.order[q]];
-            }
-            for (double x : load) t = std::max(t, x);
-            return t;
+    std::vector<int> Kq(np, 1);  // by place in the work order
+    int nst = 0;                 // pairs with workgroups of their own
+    if (forced) {
+        const int K = std::min(pick(B.req.pf_wg_per_pair, "LCG_PF_WG_PER_PAIR", 1, 1, 64), std::max(1, cus / np));
+        std::fill(Kq.begin(), Kq.end(), K);
+        nst = K > 1 ? np : 0;
+    } else {
+        auto time = [&](int q, int k) { return (double)B.work[B.order[q]] * (1 + 0.08 * (k - 1)) / k; };
+        auto most = [&](int q) {
+            const PairDesc &d = B.descs[B.order[q]];
+            return std::max(2, std::min(64, d.ngroups / std::max(1, d.n)));
         };
-        double best = makespan(0);
-        for (int ns = 1; 2 * ns <= cus && ns <= np; ++ns) {
-            const double t = makespan(ns);
-            if (t < best) {
-                best = t;
-                nst = ns;
-                K = 2;
+        double total = 0;
+        for (int q = 0; q < np; ++q) total += time(q, 1);
+        // smallest makespan that the workgroups allow, by bisection; queued
+        // pairs fill theirs to about 0.9
+        double lo = total / cus, hi = std::max(time(0, 1), 2 * lo);
+        std::vector<int> kk(np);
+        for (int it = 0; it < 20; ++it) {
+            const double T = it == 0 ? hi : 0.5 * (lo + hi);
+            long used = 0;
+            double rest = 0;
+            for (int q = 0; q < np; ++q) {
+                const int cap = most(q);
+                int k = 1;
+                while (k < cap && time(q, k) > T) ++k;
+                kk[q] = k;
+                if (k > 1 || np < cus) used += k;
+                else rest += time(q, 1);
+            }
+            if (used + rest / (0.9 * T) <= cus) {
+                hi = T;
+                Kq = kk;
+            } else {
+                lo = T;
             }
         }
+        for (int q = 0; q < np; ++q)
+            if (Kq[q] > 1) nst = q + 1;
     }
-    B.pbp.wg_per_pair = K;
+    B.pf_split = B.pf_nsplit = 0;
+    for (int q = 0; q < np; ++q)
+        if (Kq[q] > 1) {
+            B.pf_split = B.pf_split ? std::min(B.pf_split, Kq[q]) : Kq[q];
+            ++B.pf_nsplit;
+        }
     B.pbp.nstatic = nst;
     // schedule: per row, the groups dealt to the K members (longest first to
     // the least loaded), then per member in rounds of at most pf_waves;
@@ -2561,7 +2580,12 @@ int pf_setup(lcg_batch &B) {
     // -1).  Word: round | wave<<12 | member<<16.
     std::vector<int32_t> sched;
     std::vector<int> Kp(np, 1);  // workgroups of each pair
-    for (int q = 0; q < nst; ++q) Kp[B.order[q]] = K;
+    std::vector<int32_t> deal;   // place in the work order, member, members
+    for (int q = 0; q < nst; ++q) {
+        Kp[B.order[q]] = Kq[q];
+        for (int mm = 0; mm < Kq[q]; ++mm) deal.insert(deal.end(), {q, mm, Kq[q]});
+    }
+    B.pbp.dealt = (int32_t)(deal.size() / 3);
     for (int k = 0; k < np; ++k) {
         const PairDesc &d = B.descs[k];
         PfDesc &f = B.pdescs[k];
@@ -2655,9 +2679,11 @@ int pf_setup(lcg_batch &B) {
     B.pbp.scratch_stride = (int32_t)((stride + 31) & ~(size_t)31);
     hipError_t e;
     // all workgroups resident at once (one per CU): static members + the rest
-    B.pf_grid = nst == np ? np * K : (nst > 0 ? cus : std::min(np, cus));
+    B.pf_grid = std::min(std::max(cus, B.pbp.dealt), B.pbp.dealt + np - nst);
     B.eff.pf_waves = B.pf_waves;
-    B.eff.pf_wg_per_pair = forced ? K : 0;  // 0: chosen per pair by the makespan rule above
+    B.eff.pf_wg_per_pair = forced ? Kq[0] : 0;  // 0: chosen per pair by the makespan rule above
+    B.pbp.deal = (int32_t)sched.size();
+    sched.insert(sched.end(), deal.begin(), deal.end());
     HIPCHECK(hipMalloc(&B.d_pfa, std::max<size_t>(1, off) * 8));
     HIPCHECK(hipMalloc(&B.d_pdescs, sizeof(PfDesc) * np));
     HIPCHECK(hipMalloc(&B.d_pfscratch, (size_t)B.pf_grid * B.pf_waves * B.pbp.scratch_stride * 8));
@@ -2805,8 +2831,8 @@ extern "C" int lcg_batch_pf_config(lcg_batch *B, int32_t *wg_per_pair, int32_t *
     if (!B) return LCG_E_ARG;
     if (B->device_built) return LCG_E_STATE;
     if (int rc = pf_setup(*B)) return rc;
-    if (wg_per_pair) *wg_per_pair = B->pbp.wg_per_pair;
-    if (nstatic) *nstatic = B->pbp.nstatic;
+    if (wg_per_pair) *wg_per_pair = std::max(1, B->pf_split);
+    if (nstatic) *nstatic = B->pf_nsplit;
     if (workgroups) *workgroups = B->pf_grid;
     return LCG_OK;
 }

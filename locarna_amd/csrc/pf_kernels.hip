@@ -921,19 +921,20 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
     double *egA = dl, *egB = dl + (L + 1), *es = dl + 2 * (L + 1);
     double *pool = es + LCG_NCODES * LCG_NCODES;
     double *wscr = scratch + (size_t)(blockIdx.x * nwaves + wave) * bp.scratch_stride;
-    // The first nstatic pairs of the queue order have wg_per_pair workgroups
-    // (members) each, blocks K k .. K k + K - 1, all resident; the groups of a
-    // row are dealt to the members, which meet at a barrier after every row
-    // (arrival counter per pair, bounded wait).  The other workgroups take
-    // the remaining pairs from the queue, one workgroup per pair.
-    const bool stat = (int)blockIdx.x < bp.wg_per_pair * bp.nstatic;
-    const int K = stat ? bp.wg_per_pair : 1;
-    const int member = stat ? (int)blockIdx.x % K : 0;
+    // The first nstatic pairs of the work order have workgroups (members) of
+    // their own, all resident; the groups of a row are dealt to the members,
+    // which meet at a barrier after every row (arrival counter per pair,
+    // bounded wait).  The other workgroups take the remaining pairs from the
+    // queue, one workgroup per pair.
+    const bool stat = (int)blockIdx.x < bp.dealt;
+    const int *deal = sched + bp.deal + 3 * (stat ? (int)blockIdx.x : 0);
+    const int K = stat ? deal[2] : 1;
+    const int member = stat ? deal[1] : 0;
     const int spin_lim = bp.spin_limit ? bp.spin_limit : LCG_PF_SPIN_LIMIT;
     for (int iter = 0;; ++iter) {
         if (stat) {
             if (iter > 0) break;
-            if (threadIdx.x == 0) s_pair = (int)blockIdx.x / K;
+            if (threadIdx.x == 0) s_pair = deal[0];
         } else if (threadIdx.x == 0) {
             s_pair = bp.nstatic + atomicAdd(queue, 1);
         }
@@ -1290,7 +1291,7 @@ extern "C" int lcg_launch_pf(const PairDesc *descs, const PfDesc *pdescs, const 
         attr_set = true;
     }
     hipLaunchKernelGGL(lcg_pf_reset_queue, dim3(1), dim3(64), 0, stream, queue);
-    if (bp.wg_per_pair > 1)
+    if (bp.dealt > 0)
         hipLaunchKernelGGL(lcg_pf_reset_barriers, dim3(1), dim3(256), 0, stream, barriers, bp.npairs);
     hipLaunchKernelGGL(lcg_pf_pairs, dim3(grid), dim3(waves * 64), lds_bytes, stream, descs, pdescs, order, queue,
                        arena, pfa, scratch, sched, barriers, fstore, bp);

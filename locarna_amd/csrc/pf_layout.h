@@ -53,10 +53,11 @@ typedef struct {
     int32_t scratch_stride;  // doubles of global scratch per (workgroup, wave)
     int32_t pool;            // doubles of LDS pool for group regions
     int32_t nfblk_max;       // fill blocks of the largest pair (LDS header)
-    int32_t wg_per_pair;     // workgroups sharing one of the first nstatic pairs
-    int32_t nstatic;         // pairs (in queue order) with wg_per_pair
-                             // workgroups each, assigned by block index; the
-                             // other workgroups take the rest from the queue
+    int32_t dealt;           // workgroups with a pair of their own (a list at
+    int32_t deal;            // sched + deal: place in the work order, member,
+                             // members), and
+    int32_t nstatic;         // the pairs they have, first in the work order;
+                             // the other workgroups take the rest from the queue
     int32_t spin_limit;      // polls of a bounded cross-workgroup wait (0: default,
                              // -1: every wait gives up at once, for error-path tests)
 } PfBatchParams;
