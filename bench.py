@@ -220,22 +220,23 @@ def main():
         plain = npairs / (plain_ms / 1e3)
         plain_one_cu = npairs / (batch.run(mode=1, trace=True) / 1e3)
 
-    # integer-op roofline of the dominant kernel, lcg_fill_pairs (fill of D
-    # over all arc-match groups): W_int = 11 C + 2 K + A over its own cells
+    # integer-op roofline of the dominant kernel, lcg_fill_band (fill of D
+    # over all arc-match groups; lcg_fill_pairs counts its work and takes the
+    # pairs with band rows of more than 128 columns): W_int = 11 C + 2 K + A over its own cells
     # C and candidates K, divided by its device time (HIP events around it
     # on its stream)
     w_fill = 11 * fill_cells + 2 * fill_cands + arcm
     fill_avg = sum(fill_ms) / len(fill_ms) if fill_ms else None
     achieved = w_fill / (fill_avg / 1e3) / 1e12 if fill_avg else None
     traffic = None
-    tpath = os.path.join(ROOT, "profiles", "lcg_fill_pairs_%s_traffic.json" % args.workload)
+    tpath = os.path.join(ROOT, "profiles", "lcg_fill_band_%s_traffic.json" % args.workload)
     if os.path.exists(tpath):
         with open(tpath) as f:
             traffic = json.load(f).get("hbm_bytes_per_launch")
     roofline = {"bound": "valu", "achieved": round(achieved, 4) if achieved else None,
                 "peak": round(P_INT32_TOPS, 2), "unit": "TOPS",
                 "frac": round(achieved / P_INT32_TOPS, 5) if achieved else None, "traffic": traffic,
-                "kernel": "lcg_fill_pairs", "kernel_ms": round(fill_avg, 3) if fill_avg else None,
+                "kernel": "lcg_fill_band", "kernel_ms": round(fill_avg, 3) if fill_avg else None,
                 "int_ops_per_launch": w_fill,
                 "other_kernel": {"name": "lcg_top_pairs",
                                  "ms": round(sum(top_ms) / len(top_ms), 3) if top_ms else None,
