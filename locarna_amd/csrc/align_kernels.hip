@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "device_layout.h"
+#include "member_barrier.h"
 
 namespace {
 
@@ -1592,17 +1593,9 @@ __device__ __forceinline__ Pair load_pair(const PairDesc &d, int *arena, int *ld
 // Group schedule word G[5] = round | wave << 12 | member << 16.
 #define LCG_SPIN_LIMIT (1 << 22)
 
-// Arrival at a pair's barrier and bounded wait for `target` arrivals (one
-// thread of each member); an expired wait marks the pair's status.
+// An expired wait marks the pair's status (one thread).
 __device__ __forceinline__ void meet(int *counter, int target, int spin_lim, int *status) {
-    atomicAdd(counter, 1);
-    for (int spin = 0; spin_lim < 0 || atomicAdd(counter, 0) < target; ++spin) {
-        if (spin > spin_lim) {
-            atomicExch(status, 2);
-            break;
-        }
-        __builtin_amdgcn_s_sleep(2);
-    }
+    if (!arrive_and_wait(counter, target, spin_lim)) atomicExch(status, 2);
 }
 
 template <bool TAB, bool SL>
@@ -1825,18 +1818,9 @@ __device__ __forceinline__ void fill_band(const PairDesc *__restrict__ descs, co
                 band_row<TAB>(P, V, bp, now, gtask + g0, gams, al, ng, member, K, pool);
                 if (K > 1) {
                     // every member's D of the row is written before any member
-                    // reads it in a later row: the waves' stores are in the L2
-                    // before one wave writes it back, and after the barrier
-                    // drops what the CU's L1 holds
-                    __threadfence_block();
-                    __syncthreads();
+                    // reads it in a later row
                     ++passed;
-                    if (threadIdx.x == 0) {
-                        __threadfence();
-                        meet(&barriers[k], K * passed, spin_lim, &arena[d.out + 3]);
-                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                    }
-                    __syncthreads();
+                    member_barrier(&barriers[k], K * passed, spin_lim, [&]() { atomicExch(&arena[d.out + 3], 2); });
                 } else {
                     __threadfence_block();
                     __syncthreads();

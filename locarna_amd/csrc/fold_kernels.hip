@@ -35,11 +35,13 @@
 #include <type_traits>
 
 #include "fold_layout.h"
+#include "member_barrier.h"
 
 namespace {
 
 constexpr int FT = LCG_FOLD_THREADS, NWV = FT / 64;
 constexpr int MAXLOOP = LCG_FOLD_MAXLOOP;
+constexpr int LCG_FOLD_SPIN_LIMIT = 1 << 22;
 
 __device__ __forceinline__ int weak(int t) { return (0x72 >> t) & 1; }
 __device__ __forceinline__ double readlane_d(double v, int l) {
@@ -85,18 +87,6 @@ __device__ __forceinline__ Terms wave_terms(int w, int lane, const double *tabs,
         t.f = tabs[LCG_FOLD_TAB_LOOP + t.l1 * (MAXLOOP + 1) + l2] * exp(-(double)(t.s + 2) * log_sigma);
     }
     return t;
-}
-
-// Arrival at a sequence's barrier and bounded wait for `target` arrivals.
-__device__ __forceinline__ void meet(int *counter, int target, int *status) {
-    atomicAdd(counter, 1);
-    for (int spin = 0; atomicAdd(counter, 0) < target; ++spin) {
-        if (spin > (1 << 22)) {
-            atomicExch(status, 2);
-            break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-    }
 }
 
 }  // namespace
@@ -183,17 +173,8 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
     // workgroup reads them
     auto diagonal_done = [&]() {
         if (K > 1) {
-            // the waves' stores are in the L2 before one wave writes it back
-            // and, after the barrier, drops what the CU's L1 holds
-            __threadfence_block();
-            __syncthreads();
             ++passed;
-            if (tid == 0) {
-                __threadfence();
-                meet(counter, K * passed, status);
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            }
-            __syncthreads();
+            member_barrier(counter, K * passed, LCG_FOLD_SPIN_LIMIT, [&]() { atomicExch(status, 2); });
         } else {
             __threadfence_block();
             __syncthreads();

@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include "device_layout.h"
+#include "member_barrier.h"
 #include "pf_layout.h"
 
 namespace {
@@ -979,26 +980,10 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
         }
         if (threadIdx.x == 0) s_open = 0.0;
         int passed = 0;  // barrier generations passed
-        // all members' global writes before any member goes on; one wave's
-        // device-scope fences after the workgroup's own barrier (each writes the
-        // L2 back or drops the L1)
+        // all members' global writes before any member goes on
         auto pair_barrier = [&]() {
-            __threadfence_block();
-            __syncthreads();
             ++passed;
-            if (threadIdx.x == 0) {
-                __threadfence();
-                atomicAdd(&barriers[k], 1);
-                for (int spin = 0; spin_lim < 0 || atomicAdd(&barriers[k], 0) < K * passed; ++spin) {
-                    if (spin > spin_lim) {
-                        pfa[f.out + 2] = 1.0;
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(2);
-                }
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            }
-            __syncthreads();
+            member_barrier(&barriers[k], K * passed, spin_lim, [&]() { pfa[f.out + 2] = 1.0; });
         };
         PfPair P;
         P.mn = mn;
