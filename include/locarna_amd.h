@@ -533,6 +533,12 @@ typedef struct {
 } lcg_fold_params;
 int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fold_params *params, int32_t device,
                  lcg_fold **out, char *err, int errlen);
+/* lcg_fold_run with a bound of the waits between the workgroups that share a
+ * sequence of more than 256 nt (no counterpart in the reference; for tests):
+ * polls as in lcg_batch_set_spin_limit.  Where a wait expires, the sequences
+ * are folded again on one workgroup each. */
+int lcg_fold_run_limited(const char *const *seqs, int32_t count, const lcg_fold_params *params, int32_t device,
+                         int32_t polls, lcg_fold **out, char *err, int errlen);
 /* pp text of sequence k under `name` (RnaData::write_pp): pairs with
  * p > min_prob in order i, j ascending; returns the length, writes the text
  * with its terminating 0 when cap exceeds it.  The handle keeps the last
@@ -547,6 +553,9 @@ int lcg_fold_probs(const lcg_fold *f, int32_t k, double *P, double *P2, int64_t 
 int lcg_fold_log_z(const lcg_fold *f, int32_t k, double *log_z);
 /* device time of the folding kernel, wall time of lcg_fold_run */
 int lcg_fold_stats(const lcg_fold *f, float *device_ms, float *wall_ms);
+/* launches of the folding kernel (more than one where a scale or an expired
+ * wait made it run again) */
+int lcg_fold_launches(const lcg_fold *f);
 void lcg_fold_free(lcg_fold *f);
 
 /* mlocarna's default pipeline from sequences to the multiple alignment

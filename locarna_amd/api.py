@@ -154,6 +154,8 @@ def _sig(L):
     L.lcg_progressive_free.restype = None
     L.lcg_fold_run.argtypes = [c.POINTER(c.c_char_p), c.c_int32, c.POINTER(FoldParams), c.c_int32,
                                c.POINTER(c.c_void_p), c.c_char_p, c.c_int]
+    L.lcg_fold_run_limited.argtypes = L.lcg_fold_run.argtypes[:4] + [c.c_int32] + L.lcg_fold_run.argtypes[4:]
+    L.lcg_fold_launches.argtypes = [c.c_void_p]
     L.lcg_fold_write_pp.argtypes = [c.c_void_p, c.c_int32, c.c_char_p, c.c_char_p, c.c_int64]
     L.lcg_fold_write_pp.restype = c.c_int64
     L.lcg_fold_probs.argtypes = [c.c_void_p, c.c_int32, c.c_void_p, c.c_void_p, c.c_int64]
@@ -745,9 +747,11 @@ class Fold:
     """Base-pair probabilities of single sequences on one GPU
     (lcg_fold_run; the step locarna_rnafold_pp performs for mlocarna,
     src/locarna_rnafold_pp.cc:209-271): pp(k, name), probs(k), log_z(k),
-    stats()."""
+    stats().  polls: bound of the waits between workgroups
+    (lcg_fold_run_limited, for tests)."""
 
-    def __init__(self, seqs, max_bp_span=-1, min_prob=0.001, stacking=False, device=0, scale_kcal_per_nt=0.0):
+    def __init__(self, seqs, max_bp_span=-1, min_prob=0.001, stacking=False, device=0, scale_kcal_per_nt=0.0,
+                 polls=0):
         n = len(seqs)
         arr = (ctypes.c_char_p * n)(*[s.encode() for s in seqs])
         fp = FoldParams(max_bp_span, 1 if stacking else 0, min_prob, scale_kcal_per_nt)
@@ -755,7 +759,7 @@ class Fold:
         err = ctypes.create_string_buffer(1024)
         self.h = None
         self.lens = [len(s) for s in seqs]
-        rc = lib().lcg_fold_run(arr, n, ctypes.byref(fp), device, ctypes.byref(h), err, 1024)
+        rc = lib().lcg_fold_run_limited(arr, n, ctypes.byref(fp), device, polls, ctypes.byref(h), err, 1024)
         if rc != 0:
             raise LcgError("lcg_fold_run (%d): %s" % (rc, err.value.decode()))
         self.h = h
@@ -790,6 +794,9 @@ class Fold:
         d, w = ctypes.c_float(), ctypes.c_float()
         lib().lcg_fold_stats(self.h, ctypes.byref(d), ctypes.byref(w))
         return dict(device_ms=d.value, wall_ms=w.value)
+
+    def launches(self):
+        return lib().lcg_fold_launches(self.h)
 
     def destroy(self):
         if self.h:

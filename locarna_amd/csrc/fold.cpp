@@ -26,7 +26,7 @@
 extern "C" size_t lcg_fold_lds_bytes(int nmax, int nch);
 extern "C" int lcg_launch_fold(const FoldDesc *descs, const signed char *codes, const double *tabs, double *mats,
                                double *outs, double *zout, int *counters, int *status, const int *seq_of, int grid,
-                               int nmax, int nch, hipStream_t stream);
+                               int polls, int nmax, int nch, hipStream_t stream);
 
 struct lcg_fold {
     lcg_fold_params p{};
@@ -107,12 +107,13 @@ signed char code_of(char c) {
 // 256 nt a sequence has one workgroup: 64 of 60-200 nt take 2.45 ms so and
 // 2.79 ms on several, one of 75 nt 1.10 and 1.17 ms (a barrier per diagonal
 // takes longer than the cells it divides).  Longer ones get one per 64 cells
-// as far as the CUs go: two of 700-800 nt 26.8 ms against 121 ms.
-std::vector<int> deal_workgroups(std::vector<FoldDesc> &descs, int cus, int nmax, int &nch) {
+// as far as the CUs go: two of 700-800 nt 26.8 ms against 121 ms.  `single`:
+// one for every sequence.
+std::vector<int> deal_workgroups(std::vector<FoldDesc> &descs, int cus, int nmax, bool single, int &nch) {
     const int count = (int)descs.size();
     auto chunks = [&](const FoldDesc &d) { return std::max(1, (d.n + 63) / 64); };
     int cap = 1;
-    if (nmax > 256)
+    if (nmax > 256 && !single)
         for (int c = 2; c <= 64; ++c) {
             long sum = 0;
             for (const FoldDesc &d : descs) sum += std::min(c, chunks(d));
@@ -145,7 +146,12 @@ struct DevBuf {
 
 extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fold_params *params, int32_t device,
                             lcg_fold **out, char *err, int errlen) {
-    if (!seqs || count < 1 || !params || !out) return LCG_E_ARG;
+    return lcg_fold_run_limited(seqs, count, params, device, 0, out, err, errlen);
+}
+
+extern "C" int lcg_fold_run_limited(const char *const *seqs, int32_t count, const lcg_fold_params *params,
+                                    int32_t device, int32_t polls, lcg_fold **out, char *err, int errlen) {
+    if (!seqs || count < 1 || !params || polls < -1 || !out) return LCG_E_ARG;
     *out = nullptr;
     if (!(params->min_prob >= 0 && params->min_prob < 1) ||
         (params->max_bp_span != -1 && params->max_bp_span < 1) || (params->stacking & ~1)) {
@@ -209,8 +215,7 @@ extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fo
     if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device)) != hipSuccess)
         return hip_fail(e);
     int nch = 4;
-    const std::vector<int> seq_of = deal_workgroups(descs, cus, nmax, nch);
-    const int grid = (int)seq_of.size() / 2;
+    std::vector<int> seq_of = deal_workgroups(descs, cus, nmax, false, nch);
     DevBuf dd, dc, dt, dm, dout, dz, db, ds;
     if ((e = hipMalloc(&dd.p, sizeof(FoldDesc) * count)) || (e = hipMalloc(&dc.p, codes.size())) ||
         (e = hipMalloc(&dt.p, tabs.size() * sizeof(double))) || (e = hipMalloc(&dm.p, mat * sizeof(double))) ||
@@ -256,7 +261,7 @@ extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fo
         (void)hipEventRecord(ev0, 0);
         int lr = lcg_launch_fold((const FoldDesc *)dd.p, (const signed char *)dc.p, (const double *)dt.p,
                                  (double *)dm.p, (double *)dout.p, (double *)dz.p, (int *)db.p, (int *)db.p + count,
-                                 (const int *)ds.p, grid, nmax, nch, 0);
+                                 (const int *)ds.p, (int)seq_of.size() / 2, polls ? polls : 1 << 22, nmax, nch, 0);
         (void)hipEventRecord(ev1, 0);
         if (lr) {
             rc = hip_fail((hipError_t)lr);
@@ -274,16 +279,20 @@ extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fo
             rc = hip_fail(e);
             break;
         }
-        if (grid > count) {  // some sequences on several workgroups
+        if ((int)seq_of.size() > 2 * count) {  // some sequences on several workgroups
             int expired = 0;
             if ((e = hipMemcpy(&expired, (int *)db.p + count, sizeof(int), hipMemcpyDeviceToHost))) {
                 rc = hip_fail(e);
                 break;
             }
             if (expired) {
-                set_err(err, errlen, "a wait between the workgroups of a sequence expired");
-                rc = LCG_E_STATE;
-                break;
+                // the workgroups of a sequence were not resident together (a
+                // busy device): again on one each, where nothing waits
+                seq_of = deal_workgroups(descs, cus, nmax, true, nch);
+                if ((e = hipMemcpy(ds.p, seq_of.data(), seq_of.size() * sizeof(int), hipMemcpyHostToDevice)))
+                    rc = hip_fail(e);
+                --attempt;
+                continue;
             }
         }
         bool all = true;
@@ -403,5 +412,7 @@ extern "C" int lcg_fold_stats(const lcg_fold *f, float *device_ms, float *wall_m
     if (wall_ms) *wall_ms = f->wall_ms;
     return LCG_OK;
 }
+
+extern "C" int lcg_fold_launches(const lcg_fold *f) { return f ? f->launches : LCG_E_ARG; }
 
 extern "C" void lcg_fold_free(lcg_fold *f) { delete f; }

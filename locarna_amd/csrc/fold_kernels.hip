@@ -41,7 +41,6 @@ namespace {
 
 constexpr int FT = LCG_FOLD_THREADS, NWV = FT / 64;
 constexpr int MAXLOOP = LCG_FOLD_MAXLOOP;
-constexpr int LCG_FOLD_SPIN_LIMIT = 1 << 22;
 
 __device__ __forceinline__ int weak(int t) { return (0x72 >> t) & 1; }
 __device__ __forceinline__ double readlane_d(double v, int l) {
@@ -108,7 +107,7 @@ __device__ __forceinline__ Terms wave_terms(int w, int lane, const double *tabs,
 template <int NCH>
 __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const signed char *codes, const double *tabs,
                                          double *mats, double *outs, double *zout, int *counter, int *status,
-                                         double *lds) {
+                                         int polls, double *lds) {
     constexpr int NB = 64 * NCH;  // cells per batch
     const int n = D.n, W = D.W, S = D.S, K = D.K;
     double *part = lds;                    // [sum][wave][cell]: M2 or Qmb, interior loops, Qm1b
@@ -174,7 +173,7 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
     auto diagonal_done = [&]() {
         if (K > 1) {
             ++passed;
-            member_barrier(counter, K * passed, LCG_FOLD_SPIN_LIMIT, [&]() { atomicExch(status, 2); });
+            member_barrier(counter, K * passed, polls, [&]() { atomicExch(status, 2); });
         } else {
             __threadfence_block();
             __syncthreads();
@@ -453,16 +452,16 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
 extern "C" __global__ __launch_bounds__(FT) void lcg_fold_seqs(const FoldDesc *descs, const signed char *codes,
                                                                const double *tabs, double *mats, double *outs,
                                                                double *zout, int *counters, int *status,
-                                                               const int *seq_of, int nch) {
+                                                               const int *seq_of, int polls, int nch) {
     extern __shared__ double lds[];
     const int sq = seq_of[2 * blockIdx.x], member = seq_of[2 * blockIdx.x + 1];
     const FoldDesc D = descs[sq];
     if (D.K > 1 || D.n <= 64 || nch == 1)
-        fold_seq<1>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, lds);
+        fold_seq<1>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
     else if (D.n <= 128)
-        fold_seq<2>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, lds);
+        fold_seq<2>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
     else
-        fold_seq<4>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, lds);
+        fold_seq<4>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
 }
 
 extern "C" size_t lcg_fold_lds_bytes(int nmax, int nch) {
@@ -472,16 +471,17 @@ extern "C" size_t lcg_fold_lds_bytes(int nmax, int nch) {
            (size_t)(nmax + 2);
 }
 
-// grid workgroups: sequence and member of each in seq_of; nch 1, 2 or 4.
+// grid workgroups: sequence and member of each in seq_of; polls: bound of the
+// waits between the members of a sequence; nch 1, 2 or 4.
 extern "C" int lcg_launch_fold(const FoldDesc *descs, const signed char *codes, const double *tabs, double *mats,
                                double *outs, double *zout, int *counters, int *status, const int *seq_of, int grid,
-                               int nmax, int nch, hipStream_t stream) {
+                               int polls, int nmax, int nch, hipStream_t stream) {
     const size_t lds = lcg_fold_lds_bytes(nmax, nch);
     if (hipError_t e = hipFuncSetAttribute((const void *)lcg_fold_seqs, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)lds))
         return (int)e;
     if (grid <= 0) return 0;
     hipLaunchKernelGGL(lcg_fold_seqs, dim3(grid), dim3(FT), lds, stream, descs, codes, tabs, mats, outs, zout, counters,
-                       status, seq_of, nch);
+                       status, seq_of, polls, nch);
     return (int)hipGetLastError();
 }

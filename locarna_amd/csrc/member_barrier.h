@@ -3,15 +3,24 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-// Arrival and wait for `target` arrivals in at most `polls` polls (one thread
-// of each member); false: the wait expired.
+#define LCG_WAIT_EXPIRED (1 << 30)  // in the counter; arrivals stay far below
+
+// Arrival and wait for `target` arrivals in at most `polls` polls, -1: none
+// (one thread of each member); false: this wait or an earlier one of any
+// member expired.  An expired wait stays in the counter, so that no later one
+// waits for members that are behind, and so that these learn of it when they
+// come (what they then write, others may have read before).
 __device__ __forceinline__ bool arrive_and_wait(int *counter, int target, int polls) {
-    atomicAdd(counter, 1);
-    for (int spin = 0; polls < 0 || atomicAdd(counter, 0) < target; ++spin) {
-        if (spin > polls) return false;
+    int seen = atomicAdd(counter, 1) + 1;
+    for (int spin = 0; polls < 0 || seen < target; ++spin) {
+        if (spin > polls) {
+            atomicOr(counter, LCG_WAIT_EXPIRED);
+            return false;
+        }
         __builtin_amdgcn_s_sleep(2);
+        seen = atomicAdd(counter, 0);
     }
-    return true;
+    return seen < LCG_WAIT_EXPIRED;
 }
 
 // What every member wrote to global memory before it, every member reads after
@@ -19,9 +28,9 @@ __device__ __forceinline__ bool arrive_and_wait(int *counter, int target, int po
 // the L2 (vmcnt(0); neither s_barrier nor a fence of workgroup scope waits for
 // them), and only then does one wave write the L2 back, arrive and, once all
 // have arrived, drop what the CU's L1 and the L2 hold of other XCDs' memory: a
-// write-back and an invalidation per member, not per wave.  With a write-back
-// per wave a diagonal of lcg_fold_seqs takes 30 us, so 7.
-// `expired` is called by one thread if the wait expired.
+// write-back and an invalidation per member, not per wave (a barrier of 16
+// waves 30 us with one per wave, 7 us so).
+// `expired` is called by one thread where arrive_and_wait returns false.
 template <class Expired>
 __device__ __forceinline__ void member_barrier(int *counter, int target, int polls, Expired expired) {
     __threadfence_block();

@@ -4,7 +4,9 @@ request of that run fails with LCG_E_STATE, the first one and all later
 ones, on the integer and the LocARNA-P path; the next run that completes
 its waits is valid again.  The condition is forced from the host (a spin
 limit of -1 makes every wait give up at once, so every kernel still exits
-normally); one-pair batches run on several workgroups per pair."""
+normally); one-pair batches run on several workgroups per pair.  Folding
+runs the sequences again on one workgroup each instead."""
+import numpy as np
 import pytest
 
 from locarna_amd import api, synth
@@ -64,6 +66,27 @@ def test_expired_wait_pf_path():
     assert z2[0] == pytest.approx(z[0], rel=1e-12)
     assert grad2 == pytest.approx(grad, rel=1e-9, abs=1e-12)
     batch.destroy()
+
+
+def test_expired_wait_folding():
+    """Waits that give up at every diagonal of two long sequences: folded again
+    without any, with the same values."""
+    seqs = [synth.sequences(60 + n, 1, n, n, 0.5, 0.5)[0] for n in (300, 290, 70)]
+    print("folding with waits", flush=True)
+    ref = api.Fold(seqs, max_bp_span=90)
+    print("folding with every wait given up", flush=True)
+    F = api.Fold(seqs, max_bp_span=90, polls=-1)
+    assert ref.launches() == 1 and F.launches() == 2
+    for k in range(3):
+        assert F.log_z(k) == ref.log_z(k)
+        for a, b in zip(F.probs(k), ref.probs(k)):
+            assert np.array_equal(a, b)
+    F.destroy()
+    print("folding with waits again", flush=True)
+    F = api.Fold(seqs, max_bp_span=90)
+    assert F.launches() == 1 and F.log_z(0) == ref.log_z(0)
+    F.destroy()
+    ref.destroy()
 
 
 def test_penalty_out_of_range_refused():
