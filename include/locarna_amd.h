@@ -539,6 +539,12 @@ int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fold_params *
  * are folded again on one workgroup each. */
 int lcg_fold_run_limited(const char *const *seqs, int32_t count, const lcg_fold_params *params, int32_t device,
                          int32_t polls, lcg_fold **out, char *err, int errlen);
+/* How lcg_fold_run would run sequences of these lengths on a device of `cus`
+ * CUs (host logic, no counterpart in the reference): workgroups of each,
+ * chunks of 64 cells per batch of each and the LDS bytes these lay out.
+ * Returns the LDS bytes of a workgroup. */
+int64_t lcg_fold_plan(const int32_t *lens, int32_t count, int32_t cus, int32_t *members, int32_t *chunks,
+                      int64_t *lds);
 /* pp text of sequence k under `name` (RnaData::write_pp): pairs with
  * p > min_prob in order i, j ascending; returns the length, writes the text
  * with its terminating 0 when cap exceeds it.  The handle keeps the last

@@ -155,6 +155,8 @@ def _sig(L):
     L.lcg_fold_run.argtypes = [c.POINTER(c.c_char_p), c.c_int32, c.POINTER(FoldParams), c.c_int32,
                                c.POINTER(c.c_void_p), c.c_char_p, c.c_int]
     L.lcg_fold_run_limited.argtypes = L.lcg_fold_run.argtypes[:4] + [c.c_int32] + L.lcg_fold_run.argtypes[4:]
+    L.lcg_fold_plan.argtypes = [c.c_void_p, c.c_int32, c.c_int32] + [c.c_void_p] * 3
+    L.lcg_fold_plan.restype = c.c_int64
     L.lcg_fold_launches.argtypes = [c.c_void_p]
     L.lcg_fold_write_pp.argtypes = [c.c_void_p, c.c_int32, c.c_char_p, c.c_char_p, c.c_int64]
     L.lcg_fold_write_pp.restype = c.c_int64
@@ -741,6 +743,18 @@ class Progressive:
             self.destroy()
         except Exception:
             pass
+
+
+def fold_plan(lens, cus=256):
+    """(workgroups, chunks per batch, LDS bytes) of each sequence and the LDS
+    bytes of a workgroup of the launch (lcg_fold_plan)."""
+    n = len(lens)
+    a = (ctypes.c_int32 * n)(*lens)
+    mem, chunks, lds = (ctypes.c_int32 * n)(), (ctypes.c_int32 * n)(), (ctypes.c_int64 * n)()
+    rc = lib().lcg_fold_plan(a, n, cus, mem, chunks, lds)
+    if rc < 0:
+        raise LcgError("lcg_fold_plan (%d)" % rc)
+    return list(zip(mem, chunks, lds)), rc
 
 
 class Fold:

@@ -144,6 +144,25 @@ struct DevBuf {
 
 }  // namespace
 
+extern "C" int64_t lcg_fold_plan(const int32_t *lens, int32_t count, int32_t cus, int32_t *members, int32_t *chunks,
+                                 int64_t *lds) {
+    if (!lens || count < 1 || cus < 1 || !members || !chunks || !lds) return LCG_E_ARG;
+    std::vector<FoldDesc> descs(count);
+    int nmax = 0, nch = 4;
+    for (int k = 0; k < count; ++k) {
+        if (lens[k] < 0 || lens[k] > LCG_FOLD_MAX_LEN) return LCG_E_ARG;
+        descs[k].n = lens[k];
+        nmax = std::max(nmax, lens[k]);
+    }
+    deal_workgroups(descs, cus, nmax, false, nch);
+    for (int k = 0; k < count; ++k) {
+        members[k] = descs[k].K;
+        chunks[k] = lcg_fold_chunks(lens[k], descs[k].K, nch);
+        lds[k] = (int64_t)lcg_fold_lds_bytes(lens[k], chunks[k]);
+    }
+    return (int64_t)lcg_fold_lds_bytes(nmax, nch);
+}
+
 extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fold_params *params, int32_t device,
                             lcg_fold **out, char *err, int errlen) {
     return lcg_fold_run_limited(seqs, count, params, device, 0, out, err, errlen);

@@ -447,8 +447,6 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
     }
 }
 
-// Chunks per batch: one with several workgroups on the sequence, else as many
-// as its diagonals have, up to nch (what the LDS allows).
 extern "C" __global__ __launch_bounds__(FT) void lcg_fold_seqs(const FoldDesc *descs, const signed char *codes,
                                                                const double *tabs, double *mats, double *outs,
                                                                double *zout, int *counters, int *status,
@@ -456,9 +454,10 @@ extern "C" __global__ __launch_bounds__(FT) void lcg_fold_seqs(const FoldDesc *d
     extern __shared__ double lds[];
     const int sq = seq_of[2 * blockIdx.x], member = seq_of[2 * blockIdx.x + 1];
     const FoldDesc D = descs[sq];
-    if (D.K > 1 || D.n <= 64 || nch == 1)
+    const int chunks = lcg_fold_chunks(D.n, D.K, nch);
+    if (chunks == 1)
         fold_seq<1>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
-    else if (D.n <= 128)
+    else if (chunks == 2)
         fold_seq<2>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
     else
         fold_seq<4>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);

@@ -36,6 +36,20 @@
 #define LCG_FOLD_RINGS 16
 #define LCG_FOLD_PAD 1024         // doubles past a sequence's matrices (chunks of 64 cells run past a diagonal)
 
+#ifdef __HIPCC__
+#define LCG_FOLD_HD __host__ __device__
+#else
+#define LCG_FOLD_HD
+#endif
+
+// Chunks of 64 cells per batch of a sequence of n bases on K workgroups: one
+// with several workgroups, else as many as its diagonals have, up to nch (1, 2
+// or 4: what the LDS of the launch was allocated for).
+LCG_FOLD_HD inline int lcg_fold_chunks(int n, int K, int nch) {
+    const int c = K > 1 || n <= 64 ? 1 : n <= 128 ? 2 : 4;
+    return c < nch ? c : nch;
+}
+
 struct FoldDesc {
     int n;           // sequence length
     int W;           // band width

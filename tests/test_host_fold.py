@@ -1,6 +1,7 @@
 """Argument checks of the folding entry points that return before any
 device work (CPU): parameter ranges, the length limit, the pipeline's
-minimum of two sequences, and the locarna_rnafold_pp program's refusals."""
+minimum of two sequences, the locarna_rnafold_pp program's refusals, and the
+workgroups and LDS that a launch is planned with (lcg_fold_plan)."""
 import os
 import subprocess
 
@@ -34,3 +35,17 @@ def test_rnafold_pp_refusals(args, stdin, msg):
     exe = os.path.join(os.path.dirname(api.__file__), "_build", "locarna_rnafold_pp")
     r = subprocess.run([exe] + args, input=stdin, text=True, capture_output=True, timeout=60)
     assert r.returncode != 0 and msg in r.stderr
+
+
+@pytest.mark.parametrize("lens", [[75], [64, 128, 256], [300, 700], [65] * 130 + [3700], [65] * 130 + [129, 3602, 1200],
+                                  [100] * 300 + [4096, 650], [200] * 255 + [257], [4096] * 5, [64] * 200 + [4096],
+                                  [1, 4096] * 128])
+def test_plan_fits(lens):
+    """Every sequence's part of the LDS is inside what the launch allocates, and
+    workgroups that wait for each other are resident together."""
+    plan, allocated = api.fold_plan(lens, 256)
+    assert allocated <= 160 * 1024
+    assert max(lds for _, _, lds in plan) <= allocated
+    members = [k for k, _, _ in plan]
+    assert min(members) >= 1 and (max(members) == 1 or sum(members) <= 256)
+    assert all(c in (1, 2, 4) and (k == 1 or c == 1) for k, c, _ in plan)
