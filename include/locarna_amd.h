@@ -377,6 +377,15 @@ int lcg_batch_D(const lcg_batch *batch, int32_t k, int64_t *D, int32_t cap);
  * share the pair.  Returns the number of groups. */
 int lcg_pair_schedule(const lcg_pair *pair, int32_t waves, int32_t pool_ints, int32_t members,
                       int32_t *group_words, int32_t *rounds, int32_t cap);
+/* Workgroups of the pairs of a batch as the band fill and LocARNA-P deal them
+ * by estimated work (no counterpart in the reference; exported for
+ * inspection): work[npairs] descending, most[npairs] the largest number for
+ * each pair, `slots` resident workgroups; k workgroups take
+ * (1 + meet (k - 1)) / k of the time of one.  Returns the number of pairs,
+ * first in the order, that have workgroups of their own; the others are
+ * queued. */
+int lcg_deal_workgroups(const double *work, const int32_t *most, int32_t npairs, int32_t slots, double meet,
+                        int32_t *members);
 
 /* Work counted by the last run with trace bit 1 set: DP cells and arc-match
  * candidates evaluated by the fill of D and the top level of pair k. */

@@ -100,6 +100,7 @@ def _sig(L):
     L.lcg_pair_arcmatches.argtypes = [c.c_void_p] + [c.c_void_p] * 5 + [c.c_int32]
     L.lcg_pair_score_tables.argtypes = [c.c_void_p] + [c.c_void_p] * 5
     L.lcg_pair_schedule.argtypes = [c.c_void_p, c.c_int32, c.c_int32, c.c_int32, c.c_void_p, c.c_void_p, c.c_int32]
+    L.lcg_deal_workgroups.argtypes = [c.c_void_p, c.c_void_p, c.c_int32, c.c_int32, c.c_double, c.c_void_p]
     L.lcg_batch_create.argtypes = [c.POINTER(c.c_void_p), c.c_int32, c.c_int32, c.POINTER(c.c_void_p),
                                    c.c_char_p, c.c_int]
     L.lcg_batch_destroy.argtypes = [c.c_void_p]
@@ -352,6 +353,17 @@ def prepare_pairs(pp_pairs, params=None, device_compaction=False, device_band=Fa
     pairs = [Pair(None, None, params, device_compaction, _handle=ctypes.c_void_p(out[k])) for k in range(n)]
     return pairs, {"band_ms": st.band_ms, "device_banded": st.device_banded, "host_banded": st.host_banded,
                    "parse_ms": st.parse_ms, "band_wall_ms": st.band_wall_ms, "finish_ms": st.finish_ms}
+
+
+def deal_workgroups(work, most, slots, meet):
+    """(workgroups of each pair, pairs with workgroups of their own)
+    (lcg_deal_workgroups)."""
+    n = len(work)
+    K = (ctypes.c_int32 * n)()
+    rc = lib().lcg_deal_workgroups((ctypes.c_double * n)(*work), (ctypes.c_int32 * n)(*most), n, slots, meet, K)
+    if rc < 0:
+        raise LcgError("lcg_deal_workgroups (%d)" % rc)
+    return list(K), rc
 
 
 class Batch:

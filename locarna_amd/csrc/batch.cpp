@@ -1428,57 +1428,69 @@ bool schedule_all(lcg_batch &B, const FillShape &s) {
     return true;
 }
 
-// Deals the first pairs of the work order to workgroups of the band fill:
-// K each where that is asked for, else as many to each as keep the estimated
-// makespan smallest (a pair of work w on k workgroups takes w (1 + 0.14 (k -
-// 1)) / k: 80, 43, 27 and 20 ms for k = 1, 2, 4 and 8 on four 500-nt pairs),
-// with a group of an average row of left ends for every one.
-// All of them are resident at once (at most one per CU); the pairs that are
-// not dealt are queued.  Three ints per workgroup: place in the order, member,
-// members.
-void deal_pairs(lcg_batch &B, const FillShape &s) {
-    const int np = B.npairs, slots = B.cus;
-    auto time = [&](int q, int k) { return (double)B.work[B.order[q]] * (1 + 0.14 * (k - 1)) / k; };
-    auto most = [&](int q) {
-        const PairDesc &d = B.descs[B.order[q]];
-        if (!d.band_need || d.band_need > s.band_pool) return 1;
-        return std::max(2, std::min(16, d.ngroups / std::max(1, d.n)));
-    };
-    std::vector<int> K(np, 1);
+// Workgroups (members) of the pairs of a batch, by place in the work order
+// (largest first), at most most[q] for pair q: the numbers that keep the
+// estimated makespan smallest, a pair of work w taking w (1 + meet (k - 1)) / k
+// on k workgroups.  The first pairs (the returned number) have workgroups of
+// their own, all resident at once (at most `slots`, one per CU); the others
+// are queued for the remaining workgroups, which they fill to about 0.9.
+int deal_workgroups(const std::vector<double> &work, const std::vector<int> &most, int slots, double meet,
+                    std::vector<int> &K) {
+    const int np = (int)work.size();
+    auto time = [&](int q, int k) { return work[q] * (1 + meet * (k - 1)) / k; };
+    K.assign(np, 1);
+    double total = 0;
+    for (int q = 0; q < np; ++q) total += work[q];
+    // smallest makespan that the slots allow, by bisection
+    double lo = total / slots, hi = std::max(work[0], 2 * lo);
+    std::vector<int> kk(np);
+    for (int it = 0; it < 20; ++it) {
+        const double T = it == 0 ? hi : 0.5 * (lo + hi);
+        long used = 0;
+        double rest = 0;
+        for (int q = 0; q < np; ++q) {
+            int k = 1;
+            while (k < most[q] && time(q, k) > T) ++k;
+            kk[q] = k;
+            if (k > 1 || np < slots) used += k;
+            else rest += work[q];
+        }
+        if (used + rest / (0.9 * T) <= slots) {
+            hi = T;
+            K = kk;
+        } else {
+            lo = T;
+        }
+    }
     int dealt = np < slots ? np : 0;
+    for (int q = 0; q < np; ++q)
+        if (K[q] > 1) dealt = std::max(dealt, q + 1);
+    return dealt;
+}
+
+// Deals pairs to workgroups of the band fill: K each where that is asked for,
+// else by estimated work (80, 43, 27 and 20 ms for 1, 2, 4 and 8 workgroups on
+// four 500-nt pairs), with a group of an average row of left ends for every
+// one.  Three ints per workgroup: place in the order, member, members.
+void deal_pairs(lcg_batch &B, const FillShape &s) {
+    const int np = B.npairs;
+    std::vector<int> K(np, 1);
+    int dealt = np < B.cus ? np : 0;
     if (s.band_K > 0) {
         if (s.band_K > 1) {
             dealt = np;  // band_K * np workgroups at most one per CU
             std::fill(K.begin(), K.end(), s.band_K);
         }
     } else {
-        double total = 0;
-        for (int q = 0; q < np; ++q) total += time(q, 1);
-        // smallest makespan that the slots allow, by bisection
-        double lo = total / slots, hi = std::max(time(0, 1), 2 * lo);
-        std::vector<int> kk(np);
-        for (int it = 0; it < 20; ++it) {
-            const double T = it == 0 ? hi : 0.5 * (lo + hi);
-            long used = 0;
-            double rest = 0;
-            for (int q = 0; q < np; ++q) {
-                const int cap = most(q);
-                int k = 1;
-                while (k < cap && time(q, k) > T) ++k;
-                kk[q] = k;
-                if (k > 1 || np < slots) used += k;
-                else rest += time(q, 1);
-            }
-            // queued pairs fill their workgroups to about 0.9
-            if (used + rest / (0.9 * T) <= slots) {
-                hi = T;
-                K = kk;
-            } else {
-                lo = T;
-            }
+        std::vector<double> work(np);
+        std::vector<int> most(np, 1);
+        for (int q = 0; q < np; ++q) {
+            const PairDesc &d = B.descs[B.order[q]];
+            work[q] = (double)B.work[B.order[q]];
+            if (d.band_need && d.band_need <= s.band_pool)
+                most[q] = std::max(2, std::min(16, d.ngroups / std::max(1, d.n)));
         }
-        for (int q = 0; q < np; ++q)
-            if (K[q] > 1) dealt = std::max(dealt, q + 1);
+        dealt = deal_workgroups(work, most, B.cus, 0.14, K);
     }
     B.deal.clear();
     for (int q = 0; q < dealt; ++q)
@@ -1489,6 +1501,19 @@ void deal_pairs(lcg_batch &B, const FillShape &s) {
     B.parts.band.grid = std::max(wgs, dealt == np ? 0 : std::min(np, B.cus * s.band_wgs_per_cu));
 }
 
+}  // namespace
+
+extern "C" int lcg_deal_workgroups(const double *work, const int32_t *most, int32_t npairs, int32_t slots, double meet,
+                                   int32_t *members) {
+    if (!work || !most || !members || npairs < 1 || slots < 1) return LCG_E_ARG;
+    std::vector<int> K;
+    const int dealt = deal_workgroups(std::vector<double>(work, work + npairs), std::vector<int>(most, most + npairs),
+                                      slots, meet, K);
+    std::copy(K.begin(), K.end(), members);
+    return dealt;
+}
+
+namespace {
 // Launch parameters of both kernels for the chosen shapes.
 void apply_shape(lcg_batch &B, const FillShape &s, const TopShape &t) {
     const int np = B.npairs;
@@ -2514,14 +2539,11 @@ int pf_setup(lcg_batch &B) {
     if (pool < 64) return LCG_E_CAPACITY;
     B.pbp.pool = pool;
     B.pf_lds = (size_t)4 * hdr_ints + (size_t)8 * (hdr_doubles + pool);
-    // Workgroups per pair (members; all workgroups resident, one per CU): the
-    // numbers that make the slowest pair's estimated time smallest, the pairs
-    // that are not dealt being queued for the remaining workgroups.  A pair on
-    // k workgroups takes about (1 + 0.08 (k - 1)) / k of its time on one (120
-    // pairs of 150 nt 109 -> 62 ms on two each; 48 ragged pairs 202, 116 and 99
-    // ms on two, four and five each).  No more than a pair has groups per row:
-    // one pair of 88 nt (14 groups a row) takes 7.12 ms on 4, 6.90 on 16 and
-    // 7.03 on 64.
+    // Workgroups per pair (members): a pair on k workgroups takes about
+    // (1 + 0.08 (k - 1)) / k of its time on one (120 pairs of 150 nt 109 -> 62
+    // ms on two each; 48 ragged pairs 202, 116 and 99 ms on two, four and five
+    // each).  No more than a pair has groups per row: one pair of 88 nt (14
+    // groups a row) takes 7.12 ms on 4, 6.90 on 16 and 7.03 on 64.
     int cus = 0;
     HIPCHECK(hipSetDevice(B.device));
     HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, B.device));
@@ -2533,38 +2555,14 @@ int pf_setup(lcg_batch &B) {
         std::fill(Kq.begin(), Kq.end(), K);
         nst = K > 1 ? np : 0;
     } else {
-        auto time = [&](int q, int k) { return (double)B.work[B.order[q]] * (1 + 0.08 * (k - 1)) / k; };
-        auto most = [&](int q) {
+        std::vector<double> work(np);
+        std::vector<int> most(np);
+        for (int q = 0; q < np; ++q) {
             const PairDesc &d = B.descs[B.order[q]];
-            return std::max(2, std::min(64, d.ngroups / std::max(1, d.n)));
-        };
-        double total = 0;
-        for (int q = 0; q < np; ++q) total += time(q, 1);
-        // smallest makespan that the workgroups allow, by bisection; queued
-        // pairs fill theirs to about 0.9
-        double lo = total / cus, hi = std::max(time(0, 1), 2 * lo);
-        std::vector<int> kk(np);
-        for (int it = 0; it < 20; ++it) {
-            const double T = it == 0 ? hi : 0.5 * (lo + hi);
-            long used = 0;
-            double rest = 0;
-            for (int q = 0; q < np; ++q) {
-                const int cap = most(q);
-                int k = 1;
-                while (k < cap && time(q, k) > T) ++k;
-                kk[q] = k;
-                if (k > 1 || np < cus) used += k;
-                else rest += time(q, 1);
-            }
-            if (used + rest / (0.9 * T) <= cus) {
-                hi = T;
-                Kq = kk;
-            } else {
-                lo = T;
-            }
+            work[q] = (double)B.work[B.order[q]];
+            most[q] = std::max(2, std::min(64, d.ngroups / std::max(1, d.n)));
         }
-        for (int q = 0; q < np; ++q)
-            if (Kq[q] > 1) nst = q + 1;
+        nst = deal_workgroups(work, most, cus, 0.08, Kq);
     }
     B.pf_split = B.pf_nsplit = 0;
     for (int q = 0; q < np; ++q)

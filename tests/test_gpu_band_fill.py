@@ -83,6 +83,21 @@ def test_profiles(monkeypatch):
     assert _results(texts, pa, monkeypatch, None) == ref
 
 
+def _shared(texts, params):
+    """Whether several workgroups share a pair: a run whose waits all expire is
+    invalid then."""
+    B = api.Batch([api.Pair(a, b, params) for a, b in texts])
+    B.set_spin_limit(-1)
+    B.run(mode=0, trace=False)
+    try:
+        B.score(0)
+        return False
+    except api.LcgError:
+        return True
+    finally:
+        B.destroy()
+
+
 def test_many_pairs_dealt(monkeypatch):
     """More pairs than CUs, one of them far larger: dealt to several
     workgroups, the others queued."""
@@ -90,5 +105,16 @@ def test_many_pairs_dealt(monkeypatch):
     t = _texts([30 + k for k in range(24)], 970)
     texts = [(big[0], big[1])] + [(t[a], t[b]) for a in range(24) for b in range(a)]
     pa = api.locarna_params(max_bp_span=150)
-    assert len(texts) > 256
+    assert len(texts) > 256 and _shared(texts, pa)
+    assert _results(texts, pa, monkeypatch, None) == _results(texts, pa, monkeypatch, "0")
+
+
+def test_many_pairs_dealt_after_wide_ones(monkeypatch):
+    """The same with pairs before it in the work order that are too wide for the
+    band fill (no trace band: 134 columns and more)."""
+    big = _texts([140, 133, 127, 125], 980, span=150)
+    t = _texts([20 + k for k in range(24)], 990)
+    texts = [(big[0], big[1]), (big[1], big[0]), (big[2], big[3])] + [(t[a], t[b]) for a in range(24) for b in range(a)]
+    pa = api.locarna_params(max_bp_span=150, min_trace_prob=0.0)
+    assert len(texts) > 256 and _shared(texts, pa)
     assert _results(texts, pa, monkeypatch, None) == _results(texts, pa, monkeypatch, "0")

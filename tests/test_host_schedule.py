@@ -2,8 +2,11 @@
 lcg_batch_create uses): every group of a row is placed once, a round of a
 workgroup member holds at most `waves` groups on distinct waves, their LDS
 regions are disjoint and inside the pool, and the row's round count covers
-them.  Runs on the CPU."""
+them.  And the dealing of pairs to workgroups (lcg_deal_workgroups, the function
+of the band fill and of LocARNA-P): the workgroups that wait for each other are
+resident together, and queued pairs have some left.  Runs on the CPU."""
 import collections
+import random
 
 import pytest
 
@@ -45,3 +48,39 @@ def test_schedule_rejects_small_pool():
     P = _pairs()[0]
     with pytest.raises(api.LcgError):
         P.schedule(16, 64, 1)
+
+
+def _works(rng, n, kind):
+    if kind == "equal":
+        return [1e6] * n
+    if kind == "one":
+        return sorted([1e3 * rng.uniform(1, 2) for _ in range(n - 1)] + [1e7], reverse=True)
+    return sorted((rng.lognormvariate(10, 1.5) for _ in range(n)), reverse=True)
+
+
+@pytest.mark.parametrize("kind", ["ragged", "equal", "one"])
+@pytest.mark.parametrize("npairs", [1, 2, 30, 255, 256, 257, 300, 2016])
+@pytest.mark.parametrize("first", [0, 1, 40, 400])
+def test_dealt_workgroups_are_resident(kind, npairs, first):
+    """`first` pairs that cannot be split (too wide for the band fill) come
+    before those that can."""
+    rng = random.Random(7 * npairs + first)
+    for slots in (256, 64):
+        for meet in (0.14, 0.08):
+            work = _works(rng, npairs, kind)
+            most = [1 if q < first else rng.randint(2, 16) for q in range(npairs)]
+            K, dealt = api.deal_workgroups(work, most, slots, meet)
+            assert all(1 <= k <= m for k, m in zip(K, most))
+            assert all(k == 1 for k in K[dealt:])
+            used = sum(K[:dealt])
+            assert used <= slots and (dealt == npairs or used < slots)
+            if npairs < slots:
+                assert dealt == npairs
+
+            def span(K, dealt):  # the dealt pairs' slowest, the others spread over the rest
+                t = [w * (1 + meet * (k - 1)) / k for w, k in zip(work, K)]
+                load = [0.0] * max(1, slots - sum(K[:dealt]))
+                for x in t[dealt:]:
+                    load[load.index(min(load))] += x
+                return max(t[:dealt] + load)
+            assert span(K, dealt) <= 1.2 * span([1] * npairs, 0)
