@@ -1759,11 +1759,11 @@ __device__ __forceinline__ void fill_band(const PairDesc *__restrict__ descs, co
         const bool mine = iter == 0 && (int)blockIdx.x < bp.dealt;
         int K = 1, member = 0;
         if (mine) {
-            member = deal[3 * blockIdx.x + 1];
-            K = deal[3 * blockIdx.x + 2];
+            member = deal ? deal[3 * blockIdx.x + 1] : blockIdx.x;
+            K = deal ? deal[3 * blockIdx.x + 2] : gridDim.x;
         }
         if (threadIdx.x == 0)
-            s_pair = mine ? deal[3 * blockIdx.x] : bp.dealt_pairs + atomicAdd(queue, 1);
+            s_pair = !mine ? bp.dealt_pairs + atomicAdd(queue, 1) : deal ? deal[3 * blockIdx.x] : 0;
         __syncthreads();
         const int k = uniform(s_pair);
         if (k >= bp.npairs) break;

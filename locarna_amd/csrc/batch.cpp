@@ -1468,10 +1468,17 @@ int deal_workgroups(const std::vector<double> &work, const std::vector<int> &mos
     return dealt;
 }
 
+// Workgroups that the band fill can use for a pair: a group of an average row
+// of left ends for every one; 1: not a pair of the band fill.
+int band_members(const PairDesc &d, int pool) {
+    if (!d.band_need || d.band_need > pool) return 1;
+    return std::max(2, std::min(16, d.ngroups / std::max(1, d.n)));
+}
+
 // Deals pairs to workgroups of the band fill: K each where that is asked for,
 // else by estimated work (80, 43, 27 and 20 ms for 1, 2, 4 and 8 workgroups on
-// four 500-nt pairs), with a group of an average row of left ends for every
-// one.  Three ints per workgroup: place in the order, member, members.
+// four 500-nt pairs).  Three ints per workgroup: place in the order, member,
+// members.
 void deal_pairs(lcg_batch &B, const FillShape &s) {
     const int np = B.npairs;
     std::vector<int> K(np, 1);
@@ -1485,10 +1492,8 @@ void deal_pairs(lcg_batch &B, const FillShape &s) {
         std::vector<double> work(np);
         std::vector<int> most(np, 1);
         for (int q = 0; q < np; ++q) {
-            const PairDesc &d = B.descs[B.order[q]];
             work[q] = (double)B.work[B.order[q]];
-            if (d.band_need && d.band_need <= s.band_pool)
-                most[q] = std::max(2, std::min(16, d.ngroups / std::max(1, d.n)));
+            most[q] = band_members(B.descs[B.order[q]], s.band_pool);
         }
         dealt = deal_workgroups(work, most, B.cus, 0.14, K);
     }
@@ -1935,7 +1940,9 @@ extern "C" int lcg_batch_run(lcg_batch *B, int32_t mode, int32_t trace, float *d
     if (mode == 0) {
         if (int rc = launch(B->d_order, B->ev_mid, B->stream)) return hip_fail((hipError_t)rc);
     } else if (mode == 1) {
-        // one pair per launch, by the fill that takes it
+        // one pair per launch, by the fill that takes it, on as many workgroups
+        // as it can use where the batch has fewer pairs than CUs (the band
+        // fill of a 500-nt pair: 80 ms on one, 20 on eight)
         const LaunchParts all = parts;
         for (int k = 0; k < B->npairs; ++k) {
             const PairDesc &d = B->descs[B->order[k]];
@@ -1946,7 +1953,12 @@ extern "C" int lcg_batch_run(lcg_batch *B, int32_t mode, int32_t trace, float *d
                 x->bp.npairs = 1;
                 x->grid = x == &parts.fill ? x->bp.wg_per_pair : 1;
             }
-            parts.band.bp.dealt = parts.band.bp.dealt_pairs = 0;  // one workgroup from the queue
+            int K = all.band.bp.wg_per_pair;
+            if (K == 0) K = B->npairs < B->cus ? band_members(d, all.band.bp.pool_ints) : 1;
+            parts.deal = nullptr;  // all workgroups share the pair
+            parts.band.grid = std::min(K, B->cus);
+            parts.band.bp.dealt = parts.band.grid;
+            parts.band.bp.dealt_pairs = 1;
             if (int rc = launch(B->d_order + k, nullptr, B->stream)) return hip_fail((hipError_t)rc);
         }
     } else {

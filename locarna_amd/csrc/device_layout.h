@@ -149,7 +149,7 @@ typedef struct {
 } LaunchPart;
 // The launches of a run: general fill, band fill, top level / traceback.
 // deal (device): 3 per workgroup of the band fill below bp.dealt: place in
-// the work order, member, members.
+// the work order, member, members; null: all workgroups share the first pair.
 typedef struct {
     LaunchPart fill, band, top;
     const int32_t *deal;

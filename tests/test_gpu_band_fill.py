@@ -83,12 +83,12 @@ def test_profiles(monkeypatch):
     assert _results(texts, pa, monkeypatch, None) == ref
 
 
-def _shared(texts, params):
+def _shared(texts, params, mode=0, shape=None):
     """Whether several workgroups share a pair: a run whose waits all expire is
     invalid then."""
-    B = api.Batch([api.Pair(a, b, params) for a, b in texts])
+    B = api.Batch([api.Pair(a, b, params) for a, b in texts], shape=shape)
     B.set_spin_limit(-1)
-    B.run(mode=0, trace=False)
+    B.run(mode=mode, trace=False)
     try:
         B.score(0)
         return False
@@ -118,3 +118,20 @@ def test_many_pairs_dealt_after_wide_ones(monkeypatch):
     pa = api.locarna_params(max_bp_span=150, min_trace_prob=0.0)
     assert len(texts) > 256 and _shared(texts, pa)
     assert _results(texts, pa, monkeypatch, None) == _results(texts, pa, monkeypatch, "0")
+
+
+def test_one_pair_per_launch():
+    """Mode 1: with fewer pairs than CUs several workgroups share the launch's
+    pair, with the wanted number where one is asked for."""
+    t = _texts([150, 143, 60, 64], 940)
+    texts = [(t[2], t[3]), (t[0], t[1]), (t[1], t[2])]
+    pa = api.locarna_params()
+    assert _shared(texts, pa, mode=1) and _shared(texts, pa, mode=1, shape=dict(wg_per_pair=3))
+    assert not _shared(texts, pa, mode=1, shape=dict(wg_per_pair=1))
+    B = api.Batch([api.Pair(a, b, pa) for a, b in texts])
+    res = []
+    for mode in (0, 1, 2, 1):
+        B.run(mode=mode)
+        res.append([(B.score(k), B.alignment(k), B.D(k)) for k in range(3)])
+    B.destroy()
+    assert res[1:] == [res[0]] * 3
