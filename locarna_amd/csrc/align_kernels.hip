@@ -853,37 +853,39 @@ __device__ __forceinline__ void store_D(const Pair &P, const int4 &ga, int v) {
     P.D[ga.z] = v;
 }
 
-// A group of a row's task list, of the list that the lanes hold (places below
-// 64) or of the list in memory.
+// A group of a row of left ends: left end and largest right end (bl | ar <<
+// 16), range in gams.
 struct BandGroup {
-    int bl, ar, b, e;  // left end, largest right end, range in gams
-};
-__device__ __forceinline__ BandGroup band_group(const int4 &held, const int4 *__restrict__ tasks, int u) {
     int x, b, e;
-    if (u < 64) {
-        x = readlane(held.x, u), b = readlane(held.y, u), e = readlane(held.z, u);
-    } else {
-        const int4 t = tasks[u];
-        x = uniform(t.x), b = uniform(t.y), e = uniform(t.z);
-    }
-    return BandGroup{x & 0xffff, (int)((unsigned)x >> 16), b, e};
+    __device__ __forceinline__ int bl() const { return x & 0xffff; }
+    __device__ __forceinline__ int ar() const { return (int)((unsigned)x >> 16); }
+};
+__device__ __forceinline__ BandGroup load_group(const int *__restrict__ groups, int u) {
+    const int4 *G = reinterpret_cast<const int4 *>(groups + LCG_GROUP_INTS * u);
+    const int4 v = G[0];
+    return BandGroup{(int)((unsigned)v.x >> 16) | (v.y << 16), v.w, G[1].x};
+}
+// Group u of the row: of those that the lanes hold (places below 64) or in memory.
+__device__ __forceinline__ BandGroup band_group(const BandGroup &held, const int *__restrict__ groups, int u) {
+    if (u < 64) return BandGroup{readlane(held.x, u), readlane(held.b, u), readlane(held.e, u)};
+    const BandGroup t = load_group(groups, u);
+    return BandGroup{uniform(t.x), uniform(t.b), uniform(t.e)};
 }
 
-// The groups of a row of left ends at places u and, with LPG 32, u + 1 of
-// their list filled, and the D of their arc matches written.  The first 64
+// The groups of a row of left ends at places u and, with LPG 32, u + 1 filled, and the D of their arc matches written.  The first 64
 // arc matches and their scores are loaded before they are needed.
 template <bool TAB, int LPG, int NC>
-__device__ __forceinline__ void band_task(const Pair &P, const BandView &V, const int4 &held,
-                                          const int4 *__restrict__ tasks, const int4 *__restrict__ gams, int al, int u,
+__device__ __forceinline__ void band_task(const Pair &P, const BandView &V, const BandGroup &held,
+                                          const int *__restrict__ groups, const int4 *__restrict__ gams, int al, int u,
                                           bool two, int *base) {
     constexpr int G = 64 / LPG;
     const int lane = lane_id();
-    const BandGroup a = band_group(held, tasks, u), b = two ? band_group(held, tasks, u + 1) : a;
+    const BandGroup a = band_group(held, groups, u), b = two ? band_group(held, groups, u + 1) : a;
     const int na = a.e - a.b, nt = na + (two ? b.e - b.b : 0);
     auto place = [&](int t) LCG_INLINE { return t >= na ? b.b + t - na : a.b + t; };
     int4 ga = gams[place(min(lane, nt - 1))];
     int sc = 0;
-    band_fill<TAB, LPG, NC>(P, V, al, a.bl, b.bl, a.ar, base, [&]() LCG_INLINE { sc = P.amscore[ga.z]; });
+    band_fill<TAB, LPG, NC>(P, V, al, a.bl(), b.bl(), a.ar(), base, [&]() LCG_INLINE { sc = P.amscore[ga.z]; });
     const int *Mo = base + 4 * LPG * NC * G - G * P.coff[al];
     for (int t = lane; t < nt; t += 64) {
         if (t >= 64) {
@@ -895,8 +897,7 @@ __device__ __forceinline__ void band_task(const Pair &P, const BandView &V, cons
     }
 }
 
-// The groups g0 .. g1-1 of row al (tasks: their list, longest first; held:
-// its first 64 by lane): dealt in this order to the K members and the waves of
+// The ng groups of row al (longest first; held: the first 64 by lane): dealt in this order to the K members and the waves of
 // each, which take them in turns up and down; a wave's region is as large as
 // its first task's, the number of waves is what the pool holds, and a wave
 // passes from one task to the next without a barrier.  Two groups per wave
@@ -904,9 +905,9 @@ __device__ __forceinline__ void band_task(const Pair &P, const BandView &V, cons
 // every group gets a wave of its own (the row's time is then that of its
 // longest task).
 template <bool TAB>
-__device__ __forceinline__ void band_row(const Pair &P, const BandView &V, const BatchParams &bp, const int4 &held,
-                                         const int4 *__restrict__ tasks, const int4 *__restrict__ gams, int al, int ng,
-                                         int member, int K, int *pool) {
+__device__ __forceinline__ void band_row(const Pair &P, const BandView &V, const BatchParams &bp,
+                                         const BandGroup &held, const int *__restrict__ groups,
+                                         const int4 *__restrict__ gams, int al, int ng, int member, int K, int *pool) {
     const int lane = lane_id(), wave = uniform(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const int c0 = P.coff[al];
     const int ar = (int)((unsigned)readlane(held.x, 0) >> 16);
@@ -933,7 +934,7 @@ __device__ __forceinline__ void band_row(const Pair &P, const BandView &V, const
         int *base = pool + (readlane(end, wave) - readlane(size, wave));
         for (int r = 0; per * (member + K * r * ns) < ng; ++r) {
             const int u = per * (member + K * (r * ns + ((r & 1) ? ns - 1 - wave : wave)));
-            if (u < ng) band_task<TAB, LPG, NC>(P, V, held, tasks, gams, al, u, per == 2 && u + 1 < ng, base);
+            if (u < ng) band_task<TAB, LPG, NC>(P, V, held, groups, gams, al, u, per == 2 && u + 1 < ng, base);
         }
     };
     using std::integral_constant;
@@ -1799,23 +1800,23 @@ __device__ __forceinline__ void fill_band(const PairDesc *__restrict__ descs, co
             for (int i = threadIdx.x; i <= d.n; i += blockDim.x) cursor[i] = P.fbp[i];
             int al = next_row(d.n), buf = 0, passed = 0;
             advance(ends, al);
-            const int4 *gtask = reinterpret_cast<const int4 *>(arena + d.gtask);
+            const int *groups = arena + d.groups;
             const int4 *gams = reinterpret_cast<const int4 *>(arena + d.gams);
             // the next row's first 64 groups, by lane
             auto hold = [&](int al) {
                 const int g0 = uniform(lrows[al + 1]), ng = uniform(lrows[al]) - g0;
-                return gtask[g0 + min(lane, ng - 1)];
+                return load_group(groups, g0 + min(lane, ng - 1));
             };
-            int4 held = al >= 1 ? hold(al) : make_int4(0, 0, 0, 0);
+            BandGroup held = al >= 1 ? hold(al) : BandGroup{0, 0, 0};
             __syncthreads();
             while (al >= 1) {
                 const int nal = next_row(al - 1);
-                const int4 now = held;
+                const BandGroup now = held;
                 if (nal >= 1) held = hold(nal);
                 advance(ends + (buf ^ 1) * step, nal);
                 const BandView V{pc, ends + buf * step};
                 const int g0 = uniform(lrows[al + 1]), ng = uniform(lrows[al]) - g0;
-                band_row<TAB>(P, V, bp, now, gtask + g0, gams, al, ng, member, K, pool);
+                band_row<TAB>(P, V, bp, now, groups + LCG_GROUP_INTS * g0, gams, al, ng, member, K, pool);
                 if (K > 1) {
                     // every member's D of the row is written before any member
                     // reads it in a later row

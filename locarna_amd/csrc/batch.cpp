@@ -100,8 +100,6 @@ size_t layout_pair(PairDesc &d, int n, int m, int ncells, int ngroups, int nam, 
     d.rounds = take((size_t)n + 2);
     align(4);
     d.groups = take((size_t)LCG_GROUP_INTS * ngroups);
-    d.gtask = take(4 * (size_t)ngroups);
-    align(4);
     d.gams = take(4 * (size_t)nam);
     d.amscore = take(nam);
     d.cptr = take((size_t)ncells + 1);
@@ -112,7 +110,6 @@ size_t layout_pair(PairDesc &d, int n, int m, int ncells, int ngroups, int nam, 
     d.fcand = take(2 * (size_t)nam);
     d.fband = take(2 * (size_t)nam);
     d.fblk = take(2 * (size_t)nfblk);
-    d.f2c = take(nam);
     d.D = take(nam);
     d.edges = take((size_t)n + m + 1);
     d.structs = take((size_t)n + m);
@@ -131,7 +128,7 @@ size_t layout_pair(PairDesc &d, int n, int m, int ncells, int ngroups, int nam, 
 void rebase(PairDesc &d, int32_t base) {
     int32_t *offs[] = {&d.band, &d.codes, &d.gaps, &d.sigma, &d.rows, &d.groups, &d.gams, &d.amscore,
                        &d.cptr, &d.cand, &d.D, &d.edges, &d.structs, &d.tstack, &d.out, &d.rounds,
-                       &d.fptr, &d.fblk, &d.fcand, &d.f2c, &d.inner, &d.c2a, &d.amst, &d.fband, &d.gtask};
+                       &d.fptr, &d.fblk, &d.fcand, &d.inner, &d.c2a, &d.amst, &d.fband};
     for (int32_t *o : offs) *o += base;
 }
 
@@ -141,8 +138,8 @@ void rebase(PairDesc &d, int32_t base) {
 bool image_in_place(const PairDesc &d, int32_t base, int32_t size, const std::vector<int32_t> &arena,
                     bool stacking = false) {
     const int32_t offs[] = {d.band, d.codes, d.gaps, d.sigma, d.rows, d.groups, d.gams, d.amscore, d.cptr, d.cand,
-                            d.D, d.edges, d.structs, d.tstack, d.out, d.rounds, d.fptr, d.fblk, d.fcand, d.f2c,
-                            d.inner, d.c2a, d.amst, d.fband, d.gtask};
+                            d.D, d.edges, d.structs, d.tstack, d.out, d.rounds, d.fptr, d.fblk, d.fcand,
+                            d.inner, d.c2a, d.amst, d.fband};
     for (int32_t o : offs)
         if (o < base || o > base + size) return false;
     if (stacking && d.amst + d.nam > base + size) return false;  // --stacking scores present
@@ -335,6 +332,8 @@ void pack(lcg_pair &P) {
         rows[al] = (int)groups.size();
     }
     rows[0] = (int)groups.size();
+    std::stable_sort(groups.begin(), groups.end(),
+                     [](const G &x, const G &y) { return x.al != y.al ? x.al > y.al : x.ar > y.ar; });
     d.ngroups = (int)groups.size();
     d.rows = reserve(blob, rows.size());
     std::copy(rows.begin(), rows.end(), blob.begin() + d.rows);
@@ -350,23 +349,6 @@ void pack(lcg_pair &P) {
         G8[4] = groups[g].e;
         G8[7] = groups[g].lds;
     }
-    d.gtask = reserve(blob, 4 * groups.size());
-    {
-        std::vector<int> idx(groups.size());
-        std::iota(idx.begin(), idx.end(), 0);
-        std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) {
-            return groups[x].al != groups[y].al ? groups[x].al > groups[y].al : groups[x].ar > groups[y].ar;
-        });
-        for (size_t t = 0; t < idx.size(); ++t) {
-            const G &g = groups[idx[t]];
-            int32_t *T = &blob[d.gtask + 4 * t];
-            T[0] = g.bl | (g.ar << 16);
-            T[1] = g.b;
-            T[2] = g.e;
-            T[3] = idx[t];
-        }
-    }
-    while (blob.size() & 3) blob.push_back(0);
     d.gams = reserve(blob, 4 * (size_t)nam);  // (--noLP: only the arc matches with an inner one have an entry)
     d.amscore = reserve(blob, nam);
     for (int k = 0; k < nam; ++k) blob[d.amscore + k] = (int32_t)sc.arcmatch(k);
@@ -452,8 +434,6 @@ void pack(lcg_pair &P) {
         gams[q + 1] = entry_of[gams[q + 2]];
         gams[q + 3] = fentry_of[gams[q + 2]];
     }
-    d.f2c = reserve(blob, nam);
-    for (int k = 0; k < nam; ++k) blob[d.f2c + fentry_of[k]] = entry_of[k];
     P.entry_of = entry_of;
     std::copy(gams.begin(), gams.end(), blob.begin() + d.gams);
     // every D is written by the fill, except with --noLP those of the arc

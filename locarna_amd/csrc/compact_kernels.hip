@@ -212,7 +212,10 @@ __device__ GroupCell group_cell(const CPair &P, int al, int bl) {
 
 // stored row width W, LDS ints of the region [E | S | M] and the DP cells of
 // the group (al, bl) with maximal right ends (ar, br)
-__device__ void group_geom(const CPair &P, int al, int bl, int ar, int br, int &W, int &lds, long long &cells) {
+__device__ __forceinline__ int region_ints(int al, int bl, int ar, int br, int W) {
+    return ((br - bl) + W + (ar - al) * W + 3) & ~3;
+}
+__device__ void group_geom(const CPair &P, int al, int bl, int ar, int br, int &W, long long &cells) {
     W = 0;
     cells = 0;
     for (int i = al; i < ar; ++i) {
@@ -221,7 +224,6 @@ __device__ void group_geom(const CPair &P, int al, int bl, int ar, int br, int &
         W = max(W, max(0, hi - lo + 1));
         if (i > al) cells += max(0, min(br - 1, P.mx[i]) - max(bl + 1, P.mn[i]) + 1);
     }
-    lds = ((br - bl) + W + (ar - al) * W + 3) & ~3;
 }
 
 }  // namespace
@@ -281,11 +283,11 @@ __global__ __launch_bounds__(CT) void lcg_compact_count(const CompactDesc *__res
         cell_rc(P, c, al, bl);
         const GroupCell g = group_cell(P, al, bl);
         if (g.cnt > 0) {
-            int W, L;
+            int W;
             long long cells;
-            group_geom(P, al, bl, g.ar, g.br, W, L, cells);
+            group_geom(P, al, bl, g.ar, g.br, W, cells);
             atomicAdd(&s_groups, 1);
-            atomicMax(&s_gmax, L);
+            atomicMax(&s_gmax, region_ints(al, bl, g.ar, g.br, W));
             atomicMax(&s_ecap, g.br - bl);
             atomicAdd(&s_cells, (unsigned long long)cells);
         }
@@ -395,19 +397,16 @@ __global__ __launch_bounds__(CT) void lcg_compact_build(const CompactDesc *__res
             if (flag) {
                 const int gi = ngroups - 1 - (cf + ef);
                 const int amb = nam - (cc + ec) - g.cnt;
-                int W, L;
+                int W;
                 long long cells;
-                group_geom(P, al, bl, g.ar, g.br, W, L, cells);
+                group_geom(P, al, bl, g.ar, g.br, W, cells);
                 if (gi >= 0 && gi < ngroups && amb >= 0) {
-                    int *G = arena + d.groups + (size_t)gi * LCG_GROUP_INTS;
-                    G[0] = al | (bl << 16);
-                    G[1] = g.ar | (g.br << 16);
-                    G[2] = W;
-                    G[3] = amb;
-                    G[4] = amb + g.cnt;
-                    G[5] = 0;
-                    G[6] = 0;
-                    G[7] = L;
+                    // kept in the place of the group arc-match lists until
+                    // the rows are sorted; G[0] for the search of the rows
+                    arena[d.groups + (size_t)gi * LCG_GROUP_INTS] = al;
+                    P.sched[gi] = al;
+                    reinterpret_cast<int4 *>(arena + d.gams)[gi] =
+                        make_int4(bl | (W << 16), g.ar | (g.br << 16), amb, amb + g.cnt);
                 } else {
                     s_status = 2;
                 }
@@ -544,15 +543,28 @@ __global__ __launch_bounds__(CT) void lcg_compact_build(const CompactDesc *__res
         arena[d.rows + al] = lo;
     }
     __syncthreads();
-    // 6. fill entry -> candidate entry; per group its arc matches in the
-    // reference order (ar | br<<16, candidate entry, arc match, fill entry)
-    for (int x = threadIdx.x; x < nam; x += CT) {
-        const int t = P.fof[x];
-        if (t >= 0 && t < nam)
-            arena[d.f2c + t] = P.eof[x];
-        else
-            s_status = 2;
+    // groups of a row by ar descending (bl descending within equal ar): the
+    // place of each from a count over its row
+    const bool counted = s_status == 0;
+    __syncthreads();
+    for (int gi = threadIdx.x; gi < ngroups && counted; gi += CT) {
+        const int4 *T = reinterpret_cast<const int4 *>(arena + d.gams);
+        const int4 g = T[gi];
+        const int al = P.sched[gi], bl = g.x & 0xffff, W = (int)((unsigned)g.x >> 16);
+        const int ar = g.y & 0xffff, br = g.y >> 16;
+        const int g0 = arena[d.rows + al + 1], g1 = arena[d.rows + al];
+        int place = g0;
+        for (int t = g0; t < g1; ++t) {
+            const int o = T[t].y & 0xffff;
+            place += o > ar || (o == ar && t < gi);
+        }
+        int4 *G = reinterpret_cast<int4 *>(arena + d.groups + (size_t)place * LCG_GROUP_INTS);
+        G[0] = make_int4(al | (bl << 16), g.y, W, g.z);
+        G[1] = make_int4(g.w, 0, 0, region_ints(al, bl, ar, br, W));
     }
+    __syncthreads();
+    // 6. per group its arc matches in the reference order
+    // (ar | br<<16, candidate entry, arc match, fill entry)
     for (int gi = threadIdx.x; gi < ngroups; gi += CT) {
         const int *G = arena + d.groups + (size_t)gi * LCG_GROUP_INTS;
         const int al = G[0] & 0xffff, bl = G[0] >> 16;
@@ -593,21 +605,7 @@ __global__ __launch_bounds__(CT) void lcg_compact_build(const CompactDesc *__res
         };
         auto mem_of = [&](int g) { return Gt[(size_t)g * LCG_GROUP_INTS + 5] >> 16; };
         auto lds_of = [&](int g) { return Gt[(size_t)g * LCG_GROUP_INTS + 7]; };
-        for (int t = 0; t < cnt; ++t) idx[t] = g0 + t;
-        for (int t = 1; t < cnt; ++t) {  // stable: rows descending
-            const int x = idx[t], kx = rows_of(x);
-            int s = t;
-            while (s > 0 && rows_of(idx[s - 1]) < kx) {
-                idx[s] = idx[s - 1];
-                --s;
-            }
-            idx[s] = x;
-        }
-        for (int t = 0; t < cnt; ++t) {  // the band fill's order: ar descending
-            const int *G = Gt + (size_t)idx[t] * LCG_GROUP_INTS;
-            reinterpret_cast<int4 *>(arena + d.gtask)[g0 + t] =
-                make_int4((G[0] >> 16) | ((G[1] & 0xffff) << 16), G[3], G[4], idx[t]);
-        }
+        for (int t = 0; t < cnt; ++t) idx[t] = g0 + t;  // rows descending
         for (int mm = 0; mm < K; ++mm) load[mm] = 0;
         for (int t = 0; t < cnt; ++t) {
             const int g = idx[t];

@@ -20,9 +20,13 @@
 //                                        round | wave<<12 | member<<16,
 //                                        lds offset, lds ints) where ar, br are
 //                                       the maximal right ends and W the
-//                                       stored row width of the group region
-//   gams:     4 per arc match, group order: (ar | br<<16, candidate entry,
-//             arc match, fill entry)
+//                                       stored row width of the group region;
+//                                       the groups of a left end al by ar
+//                                       descending (bl descending within
+//                                       equal ar): the band fill takes them
+//                                       in this order
+//   gams:     4 per arc match, by group (al, then bl descending): (ar |
+//             br<<16, candidate entry, arc match, fill entry)
 //   amscore:  s(am) per arc match (reference index order)
 //   cptr:     ncells + 1                CSR over band cells of the arc matches
 //   cand:     4 per entry               with those right ends, sorted by cell
@@ -43,11 +47,6 @@
 //                                       (LCG_FBAND of the cell (p-1, q-1)
 //                                       and of the column of j in row i,
 //                                       D(am))
-//   gtask:    4 per group               the groups of each left end by ar
-//                                       descending (their order within
-//                                       equal ar): (bl | ar<<16, am_begin,
-//                                       am_end, group)
-//   f2c:      per fill entry            its index in cand (cell order)
 //   D:        per arc match (output of the fill, reference index order)
 //   edges:    n + m + 1 slots (output): slot i+j holds the edge that reaches
 //             cell (i, j): (a << 16) | b with 0 for a gap side, -1 if empty
@@ -94,16 +93,14 @@ typedef struct {
     int32_t top_ints;  // LDS ints of the top-level region
     int32_t fptr, fblk, fcand;
     int32_t nfblk;     // fill blocks including the sentinel
-    int32_t f2c;       // fill entry -> candidate entry (cell order)
     int32_t inner;     // --noLP / --stacking only: per arc match the arc match directly inside it, -1 if none
     int32_t c2a;       // --noLP / --stacking only: candidate entry -> arc match
     int32_t amst;      // --stacking only: per arc match its stacked score, LCG_NEG if not stackable
     int32_t slmax;     // --struct-local: ints of the largest group region (eight states)
-    int32_t fband, gtask;
+    int32_t fband;
     int32_t band_need; // pool ints the band kernels need for this pair, 0: they do not
                        // apply (a band row wider than LCG_BAND_COLS, or bounds that decrease)
-    int32_t pad;
-} PairDesc;  // 37 ints
+} PairDesc;  // 34 ints
 
 typedef struct {
     int32_t alpha;           // indel opening

@@ -115,8 +115,7 @@ struct PfPair {
     double eo, ps;
     int n, m;
     const int *fbp, *fbk;  // LDS: fill blocks of row i (left end p, first entry)
-    const int *fcand;      // int arena: fill entries (p | q<<16, j | min_col(p-1)<<16, -)
-    const int *f2c;        // fill entry -> candidate entry
+    const int *fcand;      // int arena: fill entries (p | q<<16, j | min_col(p-1)<<16)
     double *fD;            // inside D per fill entry
     double *fDb;           // outside dZ/dD per fill entry: the fixed-column kernels' part
     double *fq;            // fragment match queries (8 doubles each)
@@ -1008,7 +1007,6 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
         P.fbp = fbp;
         P.fbk = fbk;
         P.fcand = arena + d.fcand;
-        P.f2c = arena + d.f2c;
         P.fD = pfa + f.fD;
         P.fDb = pfa + f.fDb;
         P.fq = pfa + f.frag;
@@ -1233,8 +1231,10 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
             }
             if (K > 1) pair_barrier();
         }
-        for (int t = member * blockDim.x + threadIdx.x; t < d.nam; t += K * blockDim.x)
-            P.Dbar[P.f2c[t]] += P.fDb[t];
+        for (int t = member * blockDim.x + threadIdx.x; t < d.nam; t += K * blockDim.x) {
+            const int4 ga = gams[t];
+            P.Dbar[ga.y] += P.fDb[ga.w];
+        }
         // fragment queries: the inside of each block (the virtual arc match
         // (i-1, j+1; k-1, l+1), AlignerP::compute_fragment_match_prob,
         // aligner_p.icc:1440-1479), one wave per query in its global scratch

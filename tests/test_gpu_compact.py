@@ -6,6 +6,8 @@ host packing of the same pairs int for int, and both batches align to the
 same scores, alignments and D tables.  The host packing itself is checked
 against the oracle in test_gpu_align.py; the tiny pairs are also checked
 against the oracle here.  Calls the kernels through the C ABI."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -97,3 +99,20 @@ def test_compact_long500(local):
     # 4 pairs: several workgroups per pair, the schedule deals groups to members
     pps, pairs, span = synth.workload("long500")
     _run([(pps[a], pps[b]) for a, b in pairs], dict(max_bp_span=span, sequ_local=local), "long500-%d" % local)
+
+
+def test_image_size():
+    """What an arc match and a group take of the arena (2^31 ints hold a batch):
+    14 and 8 ints, beside what the lengths, the band and the arcs need."""
+    pps, pairs, span = synth.workload("allpairs64", limit_pairs=6)
+    pa = api.locarna_params(max_bp_span=span)
+    for device in (False, True):
+        B = api.Batch([api.Pair(pps[a], pps[b], pa, device_compaction=device) for a, b in pairs])
+        for k, P in enumerate(B.pairs):
+            nam, ng, ints = B.pair_info(k)
+            n, m = P.lenA, P.lenB
+            na, nb = ctypes.c_int32(), ctypes.c_int32()
+            api.lib().lcg_pair_num_arcs(P.h, ctypes.byref(na), ctypes.byref(nb))
+            rest = 12 * n + 4 * m + P.band_cells + 2 * na.value + 112
+            assert nam > 1000 and ints <= 14 * nam + 8 * ng + rest, (device, k, nam, ng, ints, rest)
+        B.destroy()
