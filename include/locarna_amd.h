@@ -433,6 +433,11 @@ int64_t lcg_batch_write_bm_probs(const lcg_batch *batch, int32_t k, int32_t incl
  * T d log Z / d theta (lcg_batch_pf_grad). */
 int lcg_batch_pf_sample(const lcg_batch *batch, int32_t k, uint64_t seed, int32_t nsamples, double *mean,
                         double *var, int32_t cap);
+/* Doubles of LDS of a region of LocARNA-P's fixed-column kernels (no
+ * counterpart in the reference; exported for inspection): `rows` stored rows
+ * of `width` columns, `cols` columns of the region; outside 0: inside pass,
+ * 1: outside pass and top level. */
+int64_t lcg_pf_region_doubles(int32_t rows, int32_t width, int32_t cols, int32_t outside);
 /* LocARNA-P launch configuration of the batch (no counterpart in the
  * reference): `nstatic` pairs, the first of the work order (largest first), run
  * on `wg_per_pair` workgroups each or more, the others on one workgroup each;

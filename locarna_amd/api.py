@@ -125,6 +125,8 @@ def _sig(L):
     L.lcg_batch_pf_grad.argtypes = [c.c_void_p, c.c_int32, c.c_void_p, c.c_int32]
     L.lcg_batch_pf_sample.argtypes = [c.c_void_p, c.c_int32, c.c_uint64, c.c_int32, c.c_void_p, c.c_void_p,
                                       c.c_int32]
+    L.lcg_pf_region_doubles.argtypes = [c.c_int32] * 4
+    L.lcg_pf_region_doubles.restype = c.c_int64
     L.lcg_batch_pf_config.argtypes = [c.c_void_p] + [c.POINTER(c.c_int32)] * 3
     L.lcg_batch_suboptimal.argtypes = [c.c_void_p, c.c_int32, c.c_int32, c.c_int64, c.c_void_p, c.c_int32]
     L.lcg_batch_suboptimal_alignment.argtypes = [c.c_void_p, c.c_int32, c.c_void_p, c.c_void_p, c.c_int32,

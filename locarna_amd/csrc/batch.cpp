@@ -2596,7 +2596,7 @@ int pf_setup(lcg_batch &B) {
                     const int gal = G[0] & 0xffff, gbl = G[0] >> 16, gar = G[1] & 0xffff, gbr = G[1] >> 16;
                     if (gbr - gbl - 1 > 128 || gar - gal - 1 > 128) return -1;
                     const long cells = (long)(gar - gal) * G[2];
-                    const long sz = 4 * (gbr - gbl) + (pass == 0 ? 1 : 2) * cells;
+                    const long sz = lcg_pf_region(cells, gbr - gbl, pass);
                     return sz <= pool ? ((sz + 1) & ~1L) : -1;
                 };
                 auto rows_of = [&](int g) {
@@ -2632,9 +2632,7 @@ int pf_setup(lcg_batch &B) {
                         int32_t *S = &sched[f.sched + 4 * (size_t)g + 2 * pass];
                         S[0] = (int32_t)r | (cnt[r] << 12) | (mm << 16);
                         S[1] = sz > 0 ? (int32_t)used[r] : -1;
-                        if (sz > 0) {
-                            used[r] += sz;
-                        }
+                        if (sz > 0) used[r] += sz;
                         cnt[r] += 1;
                     }
                     nr = std::max(nr, used.size());
@@ -2815,6 +2813,11 @@ extern "C" int lcg_batch_pf_fragment_probs(const lcg_batch *B, int32_t k, double
     if (cap < (int32_t)p.size() || (!prob && !p.empty())) return LCG_E_ARG;
     std::copy(p.begin(), p.end(), prob);
     return (int)p.size();
+}
+
+extern "C" int64_t lcg_pf_region_doubles(int32_t rows, int32_t width, int32_t cols, int32_t outside) {
+    if (rows < 1 || width < 1 || cols < 1) return LCG_E_ARG;
+    return lcg_pf_region((long)rows * width, cols, outside);
 }
 
 extern "C" int lcg_batch_pf_config(lcg_batch *B, int32_t *wg_per_pair, int32_t *nstatic, int32_t *workgroups) {

@@ -383,8 +383,9 @@ __device__ void pf_reverse(const PfPair &P, const Region &R, bool want_dbar, dou
 
 // ---- fixed-column group kernels (columns bl+1 .. br-1 in NC chunks of 64
 // lanes, the same column on the same lane in every row; rows al+1 .. ar-1).
-// Region in LDS (doubles): [S: 4 (br-bl)] [M: (ar-al) W] [Mbar: (ar-al) W],
-// rows stored from max(bl, min_col(i)) as in the general layout.
+// Region in LDS (doubles, lcg_pf_region): [M: (ar-al) W], rows stored from
+// max(bl, min_col(i)) as in the general layout; after it S, the arc sums of four
+// rows (4 (br-bl)), in the forward fill and Mbar ((ar-al) W) in the adjoint.
 //
 // Four rows are one block, rows al+r0 .. al+r0+3 (r0 a multiple of 4).  An
 // arc (p, i) spans at least three positions, so an arc term of row i reads
@@ -524,7 +525,7 @@ __device__ __forceinline__ void pf_fwd_fixed(const PfPair &P, int al, int bl, in
     const int lane = lane_id();
     const double eo = P.eo, ps = P.ps;
     const int SR = br - bl, nrows = ar - al - 1;
-    double *S = base, *Mst = base + 4 * SR;
+    double *Mst = base, *S = base + (ar - al) * W;
     for (int c = lane; c < 4 * SR; c += 64) S[c] = 0.0;
     PfRows T;
     T.load(P, al, bl, ar, br, 0);
@@ -674,8 +675,8 @@ __device__ __forceinline__ double pf_rev_fixed(const PfPair &P, int al, int bl, 
                                double *edge, double *edge2 = nullptr) {
     const int lane = lane_id();
     const double eo = P.eo, ec = 1.0 - P.eo, ps = P.ps;
-    const double *Mst = base + 4 * (br - bl);
-    double *Mb = base + 4 * (br - bl) + (ar - al) * W;
+    const double *Mst = base;
+    double *Mb = base + (ar - al) * W;
     const int nrows = ar - al - 1;
     double cf[NC][6], ac[NC], uf[NC][6], au[NC], gBo[NC], gBn[NC];
     double cv[NC], cd[NC], Eb[NC], Ue[NC], left[NC];
@@ -1064,7 +1065,7 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                             pf_fwd_fixed<1>(P, gal, gbl, gar, gbr, W, base);
                         else
                             pf_fwd_fixed<2>(P, gal, gbl, gar, gbr, W, base);
-                        const double *Mst = base + 4 * (gbr - gbl);
+                        const double *Mst = base;
                         if (so >= 0) {  // M, which the outside pass reads
                             double *Ms = fstore + 4 * (size_t)so;
                             for (int c = lane; c < cells; c += 64) Ms[c] = Mst[c];
@@ -1101,12 +1102,12 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
         if (wave == 0 && member == 0) {
             const int W = d.wtop;
             const size_t cells = (size_t)(n + 1) * W;
-            if (n <= 192 && m <= 192 && 4 * (size_t)(m + 1) + 2 * cells <= (size_t)bp.pool) {
+            if (n <= 192 && m <= 192 && lcg_pf_region(cells, m + 1, 1) <= bp.pool) {
                 // the whole LDS pool is free while the other waves wait
                 double *base = pool;
                 pf_fwd_fixed<3>(P, 0, 0, n + 1, m + 1, W, base);
                 const int xz = fixed_at(0, 0, m + 1, W, n, m);
-                double *Mst = base + 4 * (m + 1);
+                double *Mst = base;
                 const double Z = xz >= 0 ? Mst[xz] : 0.0;
                 if (lane == 0) pfa[f.out + 0] = Z;
                 double *Mb = Mst + cells;
@@ -1158,7 +1159,7 @@ extern "C" __global__ void __launch_bounds__(512) lcg_pf_pairs(const PairDesc *_
                     if (off >= 0) {
                         double *base = pool + off;
                         const int cells = (gar - gal) * W;
-                        double *Mst = base + 4 * (gbr - gbl), *Mb = Mst + cells;
+                        double *Mst = base, *Mb = Mst + cells;
                         const bool nc1 = gbr - gbl - 1 <= 64;
                         const int so = sched[f.fso + g];
                         if (so >= 0) {

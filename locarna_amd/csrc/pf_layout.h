@@ -36,6 +36,17 @@
 #pragma once
 #include <stdint.h>
 
+// Doubles of a region of the fixed-column kernels, `cells` cells in rows, `cols`
+// columns from bl to below br: inside [M: cells][S: 4 cols], outside and top
+// level [M: cells][Mbar: cells], where S of a forward fill, which is over before
+// Mbar is cleared, takes Mbar's place.
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline long lcg_pf_region(long cells, long cols, int outside) {
+    return cells + (outside && cells > 4 * cols ? cells : 4 * cols);
+}
+
 typedef struct {
     int32_t egA, egB, es, eam;
     int32_t Dc, Dbar, edge_full, edge_ref;

@@ -4,7 +4,8 @@ workgroup member holds at most `waves` groups on distinct waves, their LDS
 regions are disjoint and inside the pool, and the row's round count covers
 them.  And the dealing of pairs to workgroups (lcg_deal_workgroups, the function
 of the band fill and of LocARNA-P): the workgroups that wait for each other are
-resident together, and queued pairs have some left.  Runs on the CPU."""
+resident together, and queued pairs have some left.  And the LDS of LocARNA-P's
+regions.  Runs on the CPU."""
 import collections
 import random
 
@@ -84,3 +85,18 @@ def test_dealt_workgroups_are_resident(kind, npairs, first):
                     load[load.index(min(load))] += x
                 return max(t[:dealt] + load)
             assert span(K, dealt) <= 1.2 * span([1] * npairs, 0)
+
+
+def test_pf_regions_at_the_edge_of_the_pool():
+    """In the outside pass and at the top level a region of the sizes that an LDS
+    pool ends at (6,000 doubles for the longest pairs, up to 20,000) takes no
+    more than its two matrices and one row."""
+    size = api.lib().lcg_pf_region_doubles
+    for rows in (20, 60, 129, 193):
+        for width in (20, 64, 129, 193):
+            for cols in (width, 2 * width):
+                cells = rows * width
+                assert size(rows, width, cols, 0) == cells + 4 * cols
+                assert size(rows, width, cols, 1) >= cells + 4 * cols  # a forward fill fits too
+                if 2 * cells + cols > 6000:
+                    assert size(rows, width, cols, 1) <= 2 * cells + cols
