@@ -109,7 +109,9 @@ struct Pair {
     int4 *cand;                     // global: (al|bl<<16, j, D, min_col(al-1))
     const int *fbp, *fbk;           // LDS: fill blocks of row i, (p, first entry)
     const int2 *__restrict__ fcand; // global: fill entries (p | q<<16, j | min_col(p-1)<<16)
-    int2 *fband;                    // global: fill entries by band cells (LCG_FBAND, D)
+    int2 *fband;                    // global: fill entries by band cells (LCG_FBAND, D), fds 2 only
+    int *fD;                        // global: D of the fill entries, fds words apart
+    int fds;
     const int *__restrict__ amscore;
     int *D;
     int *edges;
@@ -141,7 +143,7 @@ __device__ __forceinline__ int sig_col(const Pair &P, int j) {
 __device__ __forceinline__ int row_lo(const Pair &P, int i, int bl) { return max(bl, P.mn[i]); }
 __device__ __forceinline__ int row_hi(const Pair &P, int i, int br) { return min(br - 1, P.mx[i]); }
 
-// fill-list entry (fcand and the D of fband)
+// fill-list entry (fcand and its D)
 struct FillEntry {
     int pq, jm, D;
 };
@@ -356,7 +358,7 @@ __device__ void group_fill_fixed(const Pair &P, int al, int bl, int ar, int br, 
     auto fetch = [&](int t, int t1) {
         const int tt = t < t1 ? t : max(t1 - 1, 0);
         const int2 e = P.fcand[tt];
-        return FillEntry{e.x, e.y, P.fband[tt].y};
+        return FillEntry{e.x, e.y, P.fD[P.fds * tt]};
     };
     for (int c = lane; c < br - bl; c += 64) Srow[c] = LCG_NEG;
     // row al (init row): M(al, bl) = 0, M(al, j) = alpha + sum gapB
@@ -846,10 +848,11 @@ __device__ __forceinline__ int arcmatch_D(const Pair &P, const int4 &ga, int mv,
     return v;
 }
 
-// D of an arc match, not normalized (the reference's InftyInt sum)
-__device__ __forceinline__ void store_D(const Pair &P, const int4 &ga, int v) {
+// D of an arc match, not normalized (the reference's InftyInt sum); entry: the
+// D of its fill entry
+__device__ __forceinline__ void store_D(const Pair &P, const int4 &ga, int *entry, int v) {
     P.cand[ga.y].z = v;
-    P.fband[ga.w].y = v;
+    *entry = v;
     P.D[ga.z] = v;
 }
 
@@ -893,7 +896,7 @@ __device__ __forceinline__ void band_task(const Pair &P, const BandView &V, cons
             sc = P.amscore[ga.z];
         }
         const int i = (ga.x & 0xffff) - 1, j = (ga.x >> 16) - 1;
-        store_D(P, ga, arcmatch_D(P, ga, Mo[(P.coff[i] + j - P.mn[i]) * G + (t >= na)], sc));
+        store_D(P, ga, &P.fband[ga.w].y, arcmatch_D(P, ga, Mo[(P.coff[i] + j - P.mn[i]) * G + (t >= na)], sc));
     }
 }
 
@@ -1566,6 +1569,8 @@ __device__ __forceinline__ Pair load_pair(const PairDesc &d, int *arena, int *ld
     P.fbk = fbk;
     P.fcand = reinterpret_cast<const int2 *>(arena + d.fcand);
     P.fband = reinterpret_cast<int2 *>(arena + d.fband);
+    P.fD = arena + d.fband + d.fds - 1;
+    P.fds = d.fds;
     P.amscore = arena + d.amscore;
     P.D = arena + d.D;
     P.edges = arena + d.edges;
@@ -1672,7 +1677,7 @@ __device__ __forceinline__ void fill_pairs(const PairDesc *__restrict__ descs, c
                         const int4 ga = gams[t];
                         const int ar = ga.x & 0xffff, br = ga.x >> 16;
                         const int v = sl_best(P, base, gal, gbl, gar, gbr, W, ar - 1, br - 1, nullptr) + P.amscore[ga.z];
-                        store_D(P, ga, v);
+                        store_D(P, ga, P.fD + P.fds * ga.w, v);
                     }
                     region_sync<true>();
                 } else if (!SL && mg >= 0) {
@@ -1690,7 +1695,7 @@ __device__ __forceinline__ void fill_pairs(const PairDesc *__restrict__ descs, c
                         const int4 ga = gams[t];
                         const int ar = ga.x & 0xffff, br = ga.x >> 16;
                         const int mv = Mst[(ar - 1 - gal) * W + (br - 1 - row_lo(P, ar - 1, gbl))];
-                        store_D(P, ga, arcmatch_D(P, ga, mv, P.amscore[ga.z]));
+                        store_D(P, ga, P.fD + P.fds * ga.w, arcmatch_D(P, ga, mv, P.amscore[ga.z]));
                     }
                 }
                 __threadfence_block();

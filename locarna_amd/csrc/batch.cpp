@@ -83,7 +83,7 @@ int32_t reserve(std::vector<int32_t> &blob, size_t count, int32_t fill = 0) {
 // Offsets of a pair's arena image (device_layout.h) from its sizes, in the
 // order the host packing reserves them; the device compaction lays out its
 // pairs with it, so both produce the same image.  Returns the image size.
-size_t layout_pair(PairDesc &d, int n, int m, int ncells, int ngroups, int nam, int nfblk, bool nolp = false,
+size_t layout_pair(PairDesc &d, int n, int m, int ncells, int ngroups, int nam, int nfblk, bool band, bool nolp = false,
                    bool stacking = false, bool table = false) {
     size_t off = 0;
     auto take = [&](size_t count) {
@@ -108,7 +108,8 @@ size_t layout_pair(PairDesc &d, int n, int m, int ncells, int ngroups, int nam, 
     d.fptr = take((size_t)n + 2);
     align(2);
     d.fcand = take(2 * (size_t)nam);
-    d.fband = take(2 * (size_t)nam);
+    d.fds = band ? 2 : 1;
+    d.fband = take(d.fds * (size_t)nam);
     d.fblk = take(2 * (size_t)nfblk);
     d.D = take(nam);
     d.edges = take((size_t)n + m + 1);
@@ -167,15 +168,34 @@ void top_region(const std::vector<int> &mn, const std::vector<int> &mx, int n, i
     top_ints = ((m + 1) + wtop + (n + 1) * wtop + 3) & ~3;
 }
 
+// Whether the band fill can take a pair: band bounds that do not decrease, rows
+// of at most LCG_BAND_COLS columns.
+bool band_rows(const lcg_pair &P) {
+    const std::vector<int> &mn = P.tc->min_cols(), &mx = P.tc->max_cols();
+    if (P.params.struct_local || !std::is_sorted(mn.begin(), mn.end()) || !std::is_sorted(mx.begin(), mx.end()))
+        return false;
+    for (size_t i = 0; i < mn.size(); ++i)
+        if (mx[i] - mn[i] + 1 > LCG_BAND_COLS) return false;
+    return true;
+}
+
 // Order of the arcs of B within a fill block (the arc matches of one arc of
-// A): first the first arc of every right end (ascending), then the second
-// ones, and so on (right ends by right adjacency order), so that neighbouring
-// fill entries end in different columns: the fill combines the entries of a
-// row by LDS atomics, which are serialized where lanes meet in a column.
-// Returns the place of every arc in that order.
-std::vector<int> fill_order(const BasePairs &bB, int m) {
+// A).  For the band fill first the first arc of every right end (ascending),
+// then the second ones, and so on (right ends by right adjacency order), so
+// that neighbouring fill entries end in different columns: the fill combines
+// the entries of a row by LDS atomics, which are serialized where lanes meet in
+// a column.  Else by right adjacency order, in which the general fill, whose
+// rows are longer, gathers from neighbouring cells (128 pairs of 150 nt without
+// a band 472 ms in the first order, 452 in this one).  Returns the place of
+// every arc in that order.
+std::vector<int> fill_order(const BasePairs &bB, int m, bool band) {
     std::vector<int> place(bB.num_bps(), 0);
     int t = 0;
+    if (!band) {
+        for (int j = 0; j <= m; ++j)
+            for (int a : bB.right_adj(j)) place[a] = t++;
+        return place;
+    }
     for (size_t r = 0, left = 1; left; ++r) {
         left = 0;
         for (int j = 0; j <= m; ++j) {
@@ -388,13 +408,15 @@ void pack(lcg_pair &P) {
     if (t != nam) throw failure("internal: arc match right-end lists incomplete");
     // fill-D candidate list: the arc matches of row i (right end in A),
     // blocks of one arc of A by left end p descending, in fill order in a block
-    const std::vector<int> place = fill_order(bB, m);
+    const bool band = band_rows(P);
+    const std::vector<int> place = fill_order(bB, m, band);
     std::vector<std::vector<int>> by_rightA(n + 1);
     for (int k = 0; k < nam; ++k) by_rightA[bA.arc(ams.arcmatch(k).arcA).right].push_back(k);
     d.fptr = reserve(blob, (size_t)n + 2);
     while (blob.size() & 1) blob.push_back(0);
     d.fcand = reserve(blob, 2 * (size_t)nam);
-    d.fband = reserve(blob, 2 * (size_t)nam);
+    d.fds = band ? 2 : 1;
+    d.fband = reserve(blob, d.fds * (size_t)nam, LCG_NEG);
     std::vector<int32_t> blk;
     std::vector<int> fentry_of(nam, -1);
     int tf = 0;
@@ -419,8 +441,7 @@ void pack(lcg_pair &P) {
             blob[d.fcand + 2 * tf] = p | (q << 16);
             blob[d.fcand + 2 * tf + 1] = j | (tc.min_col(p - 1) << 16);
             const int src = blob[d.band + 2 * (n + 1) + p - 1] + (q - 1 - tc.min_col(p - 1));
-            blob[d.fband + 2 * tf] = (int32_t)LCG_FBAND(src, j - tc.min_col(i));
-            blob[d.fband + 2 * tf + 1] = LCG_NEG;
+            if (band) blob[d.fband + 2 * tf] = (int32_t)LCG_FBAND(src, j - tc.min_col(i));
             fentry_of[k] = tf++;
         }
     }
@@ -468,7 +489,7 @@ void pack(lcg_pair &P) {
     d.slmax = slmax;
     {
         PairDesc L = d;
-        const size_t size = layout_pair(L, n, m, ncells, d.ngroups, nam, d.nfblk, nolp, stacking, table);
+        const size_t size = layout_pair(L, n, m, ncells, d.ngroups, nam, d.nfblk, band, nolp, stacking, table);
         if (size != blob.size() || std::memcmp(&L, &d, sizeof d) != 0) throw failure("internal: arena layout");
     }
     P.desc = d;
@@ -554,7 +575,7 @@ void prepare_compaction_inputs(lcg_pair &P) {
     side(bB, *P.B, m, false);
     c.fordB = reserve(img, NB);
     {
-        const std::vector<int> place = fill_order(bB, m);
+        const std::vector<int> place = fill_order(bB, m, band_rows(P));
         for (int b = 0; b < NB; ++b) img[c.fordB + place[b]] = b;
     }
     c.band = reserve(img, 2 * (size_t)(n + 1));
@@ -565,7 +586,7 @@ void prepare_compaction_inputs(lcg_pair &P) {
     {
         PairDesc L;
         std::memset(&L, 0, sizeof L);
-        layout_pair(L, n, m, 0, 0, 0, 1);
+        layout_pair(L, n, m, 0, 0, 0, 1, false);
         c.hdr_len = L.rows;  // band, codes, gaps, sigma are the head of the image
         c.hdr = reserve(img, c.hdr_len);
         L.n = n;
@@ -1247,7 +1268,7 @@ int device_count_and_layout(lcg_batch &B, lcg_pair *const *pairs, int npairs, st
         int ncells = 0;
         for (int i = 0; i <= d.n; ++i) ncells += std::max(0, P.tc->max_col(i) - P.tc->min_col(i) + 1);
         d.ncells = ncells;
-        size[k] = layout_pair(d, d.n, d.m, ncells, d.ngroups, d.nam, d.nfblk);
+        size[k] = layout_pair(d, d.n, d.m, ncells, d.ngroups, d.nam, d.nfblk, band_rows(P));
         d.gmax = S[LCG_CS_GMAX];
         int64_t cells = (int64_t)(((uint64_t)(uint32_t)S[LCG_CS_CELLS + 1] << 32) | (uint32_t)S[LCG_CS_CELLS]);
         top_region(P.tc->min_cols(), P.tc->max_cols(), d.n, d.m, d.wtop, d.top_ints, cells);
@@ -1643,17 +1664,16 @@ extern "C" int lcg_batch_create_shaped(lcg_pair *const *pairs, int32_t npairs, i
             work[k] = P->cells;
         }
     }
-    // pairs the band fill takes: band bounds that do not decrease, rows of at
-    // most LCG_BAND_COLS columns; the pool must hold a region of one group
-    // (rows al .. below the largest right end of A's arcs with left end al)
+    // pairs the band fill takes (fds 2); the pool must hold a region of one
+    // group (rows al .. below the largest right end of A's arcs with left end al)
     const char *fc = std::getenv("LCG_FIXED_COLS");
     const bool fixed_cols = !fc || std::atoi(fc) != 0;
     bool band = false;
-    for (int k = 0; k < npairs && fixed_cols && !p0.struct_local; ++k) {
+    for (int k = 0; k < npairs && fixed_cols; ++k) {
+        if (B->descs[k].fds != 2) continue;
         const lcg_pair &X = *pairs[k];
         const std::vector<int> &mn = X.tc->min_cols(), &mx = X.tc->max_cols();
         const int n = X.A->length();
-        if (!std::is_sorted(mn.begin(), mn.end()) || !std::is_sorted(mx.begin(), mx.end())) continue;
         std::vector<int> coff(n + 2, 0);
         int w = 0;
         for (int i = 0; i <= n; ++i) {
@@ -1661,7 +1681,6 @@ extern "C" int lcg_batch_create_shaped(lcg_pair *const *pairs, int32_t npairs, i
             w = std::max(w, x);
             coff[i + 1] = coff[i] + x;
         }
-        if (w > LCG_BAND_COLS) continue;
         int cells = 0;
         for (int a = 0; a < X.bA->num_bps(); ++a) {
             const Arc &x = X.bA->arc(a);

@@ -520,8 +520,11 @@ __global__ __launch_bounds__(CT) void lcg_compact_build(const CompactDesc *__res
                     const int q = left_of(arcB), j = right_of(arcB);
                     *reinterpret_cast<int2 *>(arena + d.fcand + 2 * (size_t)t) =
                         make_int2(p | (q << 16), j | (mnp << 16));
-                    *reinterpret_cast<int2 *>(arena + d.fband + 2 * (size_t)t) =
-                        make_int2((int)LCG_FBAND(P.coff[p - 1] + (q - 1 - mnp), j - mni), LCG_NEG);
+                    if (d.fds == 2)
+                        *reinterpret_cast<int2 *>(arena + d.fband + 2 * (size_t)t) =
+                            make_int2((int)LCG_FBAND(P.coff[p - 1] + (q - 1 - mnp), j - mni), LCG_NEG);
+                    else
+                        arena[d.fband + (size_t)t] = LCG_NEG;
                     P.fof[x] = t;
                 } else {
                     s_status = 2;

@@ -38,15 +38,16 @@
 //                                       right end i), rows i ascending, p
 //                                       descending within a row: (p, first
 //                                       fill entry); sentinel (0, nam)
-//   fcand:    2 per entry               the arc matches again, by block, a
-//                                       block's in fill order: (p | q<<16,
-//                                       j | min_col(p-1)<<16); a group
-//                                       with left end al reads the prefix
-//                                       p > al of each row
-//   fband:    2 per entry               the same entries by band cells:
-//                                       (LCG_FBAND of the cell (p-1, q-1)
-//                                       and of the column of j in row i,
-//                                       D(am))
+//   fcand:    2 per entry               the arc matches again, by block:
+//                                       (p | q<<16, j | min_col(p-1)<<16); a
+//                                       group with left end al reads the
+//                                       prefix p > al of each row.  A block's
+//                                       entries by j, of pairs for the band
+//                                       fill (fds 2) spread over the columns
+//   fband:    fds per entry             fds 1: D(am); fds 2: the same entries
+//                                       by band cells: (LCG_FBAND of the cell
+//                                       (p-1, q-1) and of the column of j in
+//                                       row i, D(am))
 //   D:        per arc match (output of the fill, reference index order)
 //   edges:    n + m + 1 slots (output): slot i+j holds the edge that reaches
 //             cell (i, j): (a << 16) | b with 0 for a gap side, -1 if empty
@@ -98,9 +99,10 @@ typedef struct {
     int32_t amst;      // --stacking only: per arc match its stacked score, LCG_NEG if not stackable
     int32_t slmax;     // --struct-local: ints of the largest group region (eight states)
     int32_t fband;
-    int32_t band_need; // pool ints the band kernels need for this pair, 0: they do not
-                       // apply (a band row wider than LCG_BAND_COLS, or bounds that decrease)
-} PairDesc;  // 34 ints
+    int32_t fds;       // words per entry of fband: 2 where the band kernels can apply (band rows of at
+                       // most LCG_BAND_COLS columns, bounds that do not decrease), else 1
+    int32_t band_need; // pool ints the band kernels need for this pair, 0: they do not apply
+} PairDesc;  // 35 ints
 
 typedef struct {
     int32_t alpha;           // indel opening

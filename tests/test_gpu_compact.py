@@ -101,18 +101,22 @@ def test_compact_long500(local):
     _run([(pps[a], pps[b]) for a, b in pairs], dict(max_bp_span=span, sequ_local=local), "long500-%d" % local)
 
 
-def test_image_size():
+@pytest.mark.parametrize("words,kw", [(14, {}), (13, dict(min_trace_prob=0.0))], ids=["banded", "wide"])
+def test_image_size(words, kw):
     """What an arc match and a group take of the arena (2^31 ints hold a batch):
-    14 and 8 ints, beside what the lengths, the band and the arcs need."""
-    pps, pairs, span = synth.workload("allpairs64", limit_pairs=6)
-    pa = api.locarna_params(max_bp_span=span)
+    14 (13 of pairs too wide for the band fill) and 8 ints, beside what the
+    lengths, the band and the arcs need."""
+    pps, pairs, span = synth.workload("allpairs64")
+    pa = api.locarna_params(max_bp_span=span, **kw)
     for device in (False, True):
-        B = api.Batch([api.Pair(pps[a], pps[b], pa, device_compaction=device) for a, b in pairs])
-        for k, P in enumerate(B.pairs):
+        P = [api.Pair(pps[a], pps[b], pa, device_compaction=device) for a, b in pairs[:12]]
+        P = [p for p in P if not kw or p.lenB >= 128]
+        assert P
+        B = api.Batch(P)
+        for k, p in enumerate(P):
             nam, ng, ints = B.pair_info(k)
-            n, m = P.lenA, P.lenB
             na, nb = ctypes.c_int32(), ctypes.c_int32()
-            api.lib().lcg_pair_num_arcs(P.h, ctypes.byref(na), ctypes.byref(nb))
-            rest = 12 * n + 4 * m + P.band_cells + 2 * na.value + 112
-            assert nam > 1000 and ints <= 14 * nam + 8 * ng + rest, (device, k, nam, ng, ints, rest)
+            api.lib().lcg_pair_num_arcs(p.h, ctypes.byref(na), ctypes.byref(nb))
+            rest = 12 * p.lenA + 4 * p.lenB + p.band_cells + 2 * na.value + 112
+            assert nam > 1000 and ints <= words * nam + 8 * ng + rest, (device, k, nam, ng, ints, rest)
         B.destroy()
