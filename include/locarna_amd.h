@@ -380,7 +380,7 @@ int lcg_pair_schedule(const lcg_pair *pair, int32_t waves, int32_t pool_ints, in
 /* Workgroups of the pairs of a batch as the band fill and LocARNA-P deal them
  * by estimated work (no counterpart in the reference; exported for
  * inspection): work[npairs] descending, most[npairs] the largest number for
- * each pair, `slots` resident workgroups; k workgroups take
+ * each pair (0: none, a pair of the other fill), `slots` resident workgroups; k workgroups take
  * (1 + meet (k - 1)) / k of the time of one.  Returns the number of pairs,
  * first in the order, that have workgroups of their own; the others are
  * queued. */

@@ -1626,10 +1626,6 @@ __device__ __forceinline__ void fill_pairs(const PairDesc *__restrict__ descs, c
         const int k = s_pair;
         if (k >= bp.npairs) break;
         const PairDesc d = descs[order[k]];
-        if (d.band_need && d.band_need <= bp.band) {  // the band fill's
-            __syncthreads();
-            continue;
-        }
         if (member == 0) {
             if (bp.count && threadIdx.x < 4) arena[d.out + 4 + threadIdx.x] = 0;
             if (threadIdx.x == 0) arena[d.out + 3] = 0;  // status
@@ -2144,17 +2140,30 @@ extern "C" int lcg_launch_align(const PairDesc *descs, const int *order, int *qu
     // the multi-workgroup fills (a pair is in one of them)
     hipLaunchKernelGGL(lcg_reset_queue, dim3(1), dim3(64), 0, stream, queue);
     if (!top_only) {  // the fill of D (skipped when only the top level is redone)
+        const int np = T.bp.npairs;
         if ((F.waves && F.bp.wg_per_pair > 1) || (B.waves && B.bp.dealt))
-            hipLaunchKernelGGL(lcg_reset_barriers, dim3(1), dim3(256), 0, stream, barriers, T.bp.npairs);
-        if (B.waves)
-            hipLaunchKernelGGL(B.bp.sigma_table ? lcg_fill_band_tab : lcg_fill_band, dim3(B.grid), dim3(B.waves * 64),
-                               B.lds_bytes, stream, descs, order, queue + 32, arena, barriers, parts->deal, B.bp);
+            hipLaunchKernelGGL(lcg_reset_barriers, dim3(1), dim3(256), 0, stream, barriers, parts->rest ? 2 * np : np);
+        // with pairs for both fills the general one first, beside the other
+        const bool both = F.waves && B.waves && parts->side;
+        hipStream_t fs = both ? (hipStream_t)parts->side : stream;
+        if (both) {
+            if (hipError_t e = hipEventRecord((hipEvent_t)parts->fork, stream)) return (int)e;
+            if (hipError_t e = hipStreamWaitEvent(fs, (hipEvent_t)parts->fork, 0)) return (int)e;
+        }
         if (F.waves)
             hipLaunchKernelGGL(F.bp.struct_local  ? lcg_fill_pairs_sl
                                : F.bp.sigma_table ? lcg_fill_pairs_tab
                                                   : lcg_fill_pairs,
-                               dim3(F.grid), dim3(F.waves * 64), F.lds_bytes, stream, descs, order, queue, arena,
-                               barriers, scratch, F.bp);
+                               dim3(F.grid), dim3(F.waves * 64), F.lds_bytes, fs, descs,
+                               parts->rest ? parts->rest : order, queue, arena, parts->rest ? barriers + np : barriers,
+                               scratch, F.bp);
+        if (B.waves)
+            hipLaunchKernelGGL(B.bp.sigma_table ? lcg_fill_band_tab : lcg_fill_band, dim3(B.grid), dim3(B.waves * 64),
+                               B.lds_bytes, stream, descs, order, queue + 32, arena, barriers, parts->deal, B.bp);
+        if (both) {
+            if (hipError_t e = hipEventRecord((hipEvent_t)parts->join, fs)) return (int)e;
+            if (hipError_t e = hipStreamWaitEvent(stream, (hipEvent_t)parts->join, 0)) return (int)e;
+        }
     }
     if (mid) (void)hipEventRecord(mid, stream);
     hipLaunchKernelGGL(T.bp.struct_local  ? lcg_top_pairs_sl

@@ -960,6 +960,11 @@ struct lcg_batch {
     LaunchParts parts{};  // grids, waves and LDS of the three launches (their bp is filled in per run)
     std::vector<int32_t> deal;    // workgroups of the band fill with a pair of their own (deal_pairs)
     int32_t *d_deal = nullptr;    // 3 per CU
+    std::vector<int32_t> rest;    // pairs of the general fill where the band fill has others, in work order
+                                  // (device: after d_order)
+    int rest_grid = 0, count_grid = 0;  // general fill: workgroups without the band fill beside it; of a counting run
+    hipStream_t side = nullptr;         // the general fill beside the band fill, and its fork and join
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     int fill_waves = 1;   // waves of the general fill, also where no pair of the batch takes it
     bool have_results = false;
     bool fetched = false;
@@ -1430,7 +1435,8 @@ bool schedule_all(lcg_batch &B, const FillShape &s) {
 }
 
 // Workgroups (members) of the pairs of a batch, by place in the work order
-// (largest first), at most most[q] for pair q: the numbers that keep the
+// (largest first), at most most[q] for pair q (0: none, not a pair of this
+// launch): the numbers that keep the
 // estimated makespan smallest, a pair of work w taking w (1 + meet (k - 1)) / k
 // on k workgroups.  The first pairs (the returned number) have workgroups of
 // their own, all resident at once (at most `slots`, one per CU); the others
@@ -1440,21 +1446,31 @@ int deal_workgroups(const std::vector<double> &work, const std::vector<int> &mos
     const int np = (int)work.size();
     auto time = [&](int q, int k) { return work[q] * (1 + meet * (k - 1)) / k; };
     K.assign(np, 1);
-    double total = 0;
-    for (int q = 0; q < np; ++q) total += work[q];
+    double total = 0, longest = 0;
+    int takes = 0;
+    for (int q = 0; q < np; ++q) {
+        if (most[q] < 1) {
+            K[q] = 0;
+            continue;
+        }
+        total += work[q];
+        longest = std::max(longest, work[q]);
+        ++takes;
+    }
+    const bool few = takes < slots;
     // smallest makespan that the slots allow, by bisection
-    double lo = total / slots, hi = std::max(work[0], 2 * lo);
+    double lo = total / slots, hi = std::max(longest, 2 * lo);
     std::vector<int> kk(np);
     for (int it = 0; it < 20; ++it) {
         const double T = it == 0 ? hi : 0.5 * (lo + hi);
         long used = 0;
         double rest = 0;
         for (int q = 0; q < np; ++q) {
-            int k = 1;
+            int k = std::min(1, most[q]);
             while (k < most[q] && time(q, k) > T) ++k;
             kk[q] = k;
-            if (k > 1 || np < slots) used += k;
-            else rest += work[q];
+            if (k > 1 || few) used += k;
+            else if (k == 1) rest += work[q];
         }
         if (used + rest / (0.9 * T) <= slots) {
             hi = T;
@@ -1463,40 +1479,53 @@ int deal_workgroups(const std::vector<double> &work, const std::vector<int> &mos
             lo = T;
         }
     }
-    int dealt = np < slots ? np : 0;
+    int dealt = few ? np : 0;
     for (int q = 0; q < np; ++q)
         if (K[q] > 1) dealt = std::max(dealt, q + 1);
     return dealt;
 }
 
 // Workgroups that the band fill can use for a pair: a group of an average row
-// of left ends for every one; 1: not a pair of the band fill.
+// of left ends for every one; 0: not a pair of the band fill.
 int band_members(const PairDesc &d, int pool) {
-    if (!d.band_need || d.band_need > pool) return 1;
+    if (!d.band_need || d.band_need > pool) return 0;
     return std::max(2, std::min(16, d.ngroups / std::max(1, d.n)));
 }
 
 // Deals pairs to workgroups of the band fill: K each where that is asked for,
 // else by estimated work (80, 43, 27 and 20 ms for 1, 2, 4 and 8 workgroups on
 // four 500-nt pairs).  Three ints per workgroup: place in the order, member,
-// members.
+// members.  The pairs of the general fill go to `rest`.
+//
+// The two fills run side by side, so the workgroups that wait for others, of
+// either, are together at most one per CU: with fewer pairs than CUs a pair of
+// the general fill keeps its s.K; else it has one, which waits for nobody, and
+// the general fill's grid leaves room for the dealt ones.  That grid: one
+// workgroup per pair or three times the share of the CUs that its pairs' work
+// asks for (a wide pair's work takes two to three times as long); what is too
+// much the band fill's queue gets later.
 void deal_pairs(lcg_batch &B, const FillShape &s) {
     const int np = B.npairs;
     std::vector<int> K(np, 1);
+    std::vector<double> work(np);
+    std::vector<int> most(np);
+    B.rest.clear();
+    double rest_work = 0, total = 0;
+    for (int q = 0; q < np; ++q) {
+        work[q] = (double)B.work[B.order[q]];
+        most[q] = band_members(B.descs[B.order[q]], s.band_pool);
+        total += work[q];
+        if (most[q]) continue;
+        B.rest.push_back(B.order[q]);
+        rest_work += work[q];
+    }
+    const int nrest = (int)B.rest.size();
     int dealt = np < B.cus ? np : 0;
     if (s.band_K > 0) {
-        if (s.band_K > 1) {
-            dealt = np;  // band_K * np workgroups at most one per CU
-            std::fill(K.begin(), K.end(), s.band_K);
-        }
-    } else {
-        std::vector<double> work(np);
-        std::vector<int> most(np, 1);
-        for (int q = 0; q < np; ++q) {
-            work[q] = (double)B.work[B.order[q]];
-            most[q] = band_members(B.descs[B.order[q]], s.band_pool);
-        }
-        dealt = deal_workgroups(work, most, B.cus, 0.14, K);
+        if (s.band_K > 1) dealt = np;  // band_K * np workgroups at most one per CU
+        for (int q = 0; q < np; ++q) K[q] = most[q] ? s.band_K : 0;
+    } else if (nrest < np) {
+        dealt = deal_workgroups(work, most, B.cus - (s.K > 1 ? nrest * s.K : nrest ? 1 : 0), 0.14, K);
     }
     B.deal.clear();
     for (int q = 0; q < dealt; ++q)
@@ -1505,6 +1534,12 @@ void deal_pairs(lcg_batch &B, const FillShape &s) {
     B.bp_band.dealt = wgs;
     B.bp_band.dealt_pairs = dealt;
     B.parts.band.grid = std::max(wgs, dealt == np ? 0 : std::min(np, B.cus * s.band_wgs_per_cu));
+    const int alone = std::min(nrest, B.cus * s.wgs_per_cu);
+    B.rest_grid = s.K > 1 ? nrest * s.K : alone;
+    B.parts.fill.grid = B.rest_grid;
+    if (s.K == 1 && nrest > 0 && nrest < np)
+        B.parts.fill.grid = std::max(1, std::min({alone, B.cus - wgs, (int)(3 * B.cus * rest_work / total) + 1}));
+    if (nrest == np) B.rest.clear();
 }
 
 }  // namespace
@@ -1524,13 +1559,12 @@ namespace {
 void apply_shape(lcg_batch &B, const FillShape &s, const TopShape &t) {
     const int np = B.npairs;
     B.bp.hdr_ints = B.hdr;
-    B.bp.band = s.band_pool;
     B.bp.pool_ints = s.pool;
     B.bp.wg_per_pair = s.K;
     int nband = 0;
     for (const PairDesc &d : B.descs) nband += d.band_need && d.band_need <= s.band_pool;
     B.parts.fill.waves = nband < np ? s.waves : 0;
-    B.parts.fill.grid = s.K > 1 ? np * s.K : std::min(np, B.cus * s.wgs_per_cu);
+    B.count_grid = s.K > 1 ? np * s.K : std::min(np, B.cus * s.wgs_per_cu);
     B.parts.fill.lds_bytes = (size_t)(B.hdr + s.pool) * 4;
     B.fill_waves = s.waves;
     B.parts.band.waves = nband > 0 ? s.band_waves : 0;
@@ -1559,13 +1593,22 @@ void apply_shape(lcg_batch &B, const FillShape &s, const TopShape &t) {
 // --struct-local, the fill's and traceback's eight-state regions
 size_t scratch_ints(const lcg_batch &B) {
     const size_t top = (size_t)B.parts.top.grid * B.parts.top.waves * std::max(B.top_max, B.sl_max);
-    const size_t fill = (size_t)B.parts.fill.grid * B.fill_waves * B.sl_max;
+    const size_t fill = (size_t)B.count_grid * B.fill_waves * B.sl_max;
     return std::max(top, fill);
 }
 
-hipError_t upload_deal(lcg_batch &B) {
-    if (B.deal.empty()) return hipSuccess;
-    return hipMemcpy(B.d_deal, B.deal.data(), B.deal.size() * 4, hipMemcpyHostToDevice);
+hipError_t prepare_fills(lcg_batch &B) {
+    hipError_t e = hipSuccess;
+    if (!B.deal.empty()) e = hipMemcpy(B.d_deal, B.deal.data(), B.deal.size() * 4, hipMemcpyHostToDevice);
+    if (!e && !B.rest.empty())
+        e = hipMemcpy(B.d_order + B.npairs, B.rest.data(), B.rest.size() * 4, hipMemcpyHostToDevice);
+    // the second stream and its events where both fills have pairs
+    if (!e && !B.rest.empty() && !B.side) {
+        e = hipStreamCreate(&B.side);
+        if (!e) e = hipEventCreateWithFlags(&B.ev_fork, hipEventDisableTiming);
+        if (!e) e = hipEventCreateWithFlags(&B.ev_join, hipEventDisableTiming);
+    }
+    return e;
 }
 
 // The launches of a run.  A counting run takes the general fill for every
@@ -1582,8 +1625,14 @@ LaunchParts run_parts(const lcg_batch &B, int trace, int count) {
     }
     if (count) {
         L.fill.waves = B.fill_waves;
-        L.fill.bp.band = 0;
+        L.fill.grid = B.count_grid;
         L.band.waves = 0;
+    } else if (!B.rest.empty()) {
+        L.fill.bp.npairs = (int32_t)B.rest.size();
+        L.rest = B.d_order + B.npairs;
+        L.side = B.side;
+        L.fork = B.ev_fork;
+        L.join = B.ev_join;
     }
     return L;
 }
@@ -1762,12 +1811,12 @@ extern "C" int lcg_batch_create_shaped(lcg_pair *const *pairs, int32_t npairs, i
     apply_shape(*B, fs, ts);
     if ((e = hipMalloc(&B->d_arena, (B->arena_ints + LCG_ARENA_PAD) * 4)) != hipSuccess) return hip_fail(e, err, errlen);
     if ((e = hipMalloc(&B->d_descs, sizeof(PairDesc) * npairs)) != hipSuccess) return hip_fail(e, err, errlen);
-    if ((e = hipMalloc(&B->d_order, 4 * (size_t)npairs)) != hipSuccess) return hip_fail(e, err, errlen);
+    if ((e = hipMalloc(&B->d_order, 8 * (size_t)npairs)) != hipSuccess) return hip_fail(e, err, errlen);
     if ((e = hipMalloc(&B->d_queue, 256)) != hipSuccess) return hip_fail(e, err, errlen);
-    if ((e = hipMalloc(&B->d_barriers, 4 * (size_t)npairs)) != hipSuccess) return hip_fail(e, err, errlen);
+    if ((e = hipMalloc(&B->d_barriers, 8 * (size_t)npairs)) != hipSuccess) return hip_fail(e, err, errlen);
     if ((e = hipMalloc(&B->d_scratch, scratch_ints(*B) * 4)) != hipSuccess) return hip_fail(e, err, errlen);
     if ((e = hipMalloc(&B->d_deal, 12 * (size_t)cus)) != hipSuccess) return hip_fail(e, err, errlen);
-    if ((e = upload_deal(*B)) != hipSuccess) return hip_fail(e, err, errlen);
+    if ((e = prepare_fills(*B)) != hipSuccess) return hip_fail(e, err, errlen);
     if (deferred)  // the compaction writes the image over a cleared arena
         e = hipMemsetAsync(B->d_arena, 0, B->arena_ints * 4, B->stream);
     else
@@ -1826,6 +1875,9 @@ lcg_batch::~lcg_batch() {
     if (B->d_queue) hipFree(B->d_queue);
     if (B->d_barriers) hipFree(B->d_barriers);
     if (B->d_deal) hipFree(B->d_deal);
+    if (B->ev_fork) hipEventDestroy(B->ev_fork);
+    if (B->ev_join) hipEventDestroy(B->ev_join);
+    if (B->side) hipStreamDestroy(B->side);
     if (B->d_scratch) hipFree(B->d_scratch);
     if (B->d_restr) hipFree(B->d_restr);
     if (B->d_kscratch) hipFree(B->d_kscratch);
@@ -1945,15 +1997,16 @@ extern "C" int lcg_batch_run(lcg_batch *B, int32_t mode, int32_t trace, float *d
         const LaunchParts all = parts;
         for (int k = 0; k < B->npairs; ++k) {
             const PairDesc &d = B->descs[B->order[k]];
-            const bool band = d.band_need && d.band_need <= all.fill.bp.band;
-            parts.fill.waves = band ? 0 : all.fill.waves;
-            parts.band.waves = band ? all.band.waves : 0;
+            const int members = count ? 0 : band_members(d, all.band.bp.pool_ints);
+            parts.fill.waves = members ? 0 : all.fill.waves;
+            parts.band.waves = members ? all.band.waves : 0;
+            parts.rest = nullptr;
             for (LaunchPart *x : {&parts.fill, &parts.band, &parts.top}) {
                 x->bp.npairs = 1;
                 x->grid = x == &parts.fill ? x->bp.wg_per_pair : 1;
             }
             int K = all.band.bp.wg_per_pair;
-            if (K == 0) K = B->npairs < B->cus ? band_members(d, all.band.bp.pool_ints) : 1;
+            if (K == 0) K = B->npairs < B->cus ? std::max(1, members) : 1;
             parts.deal = nullptr;  // all workgroups share the pair
             parts.band.grid = std::min(K, B->cus);
             parts.band.bp.dealt = parts.band.grid;
@@ -2014,11 +2067,13 @@ extern "C" int lcg_batch_run_noalloc(lcg_batch *B, int32_t trace) {
     int *S = nullptr;
     long long cap = 0;
     if (int rc = lcg_noalloc_scratch(B->device, &S, &cap)) return hip_fail((hipError_t)rc);
-    const long long bar_off = 64;                                 // queues at 0 and 16
-    const long long top_off = (bar_off + B->npairs + 63) & ~63LL;  // 256-byte aligned
+    const long long bar_off = 64;                                     // queues at 0, 16 and 32
+    const long long top_off = (bar_off + 2 * B->npairs + 63) & ~63LL;  // 256-byte aligned
     const long long per_wg = (long long)B->parts.top.waves * B->top_max;
     if (top_off + per_wg > cap) return LCG_E_CAPACITY;
     LaunchParts parts = run_parts(*B, trace & 1, 0);
+    parts.side = nullptr;  // no events: the fills one after the other
+    parts.fill.grid = B->rest_grid;
     parts.top.grid = (int)std::min<long long>(parts.top.grid, (cap - top_off) / per_wg);
     if (int rc = lcg_launch_align(B->d_descs, B->d_order, S, B->d_arena, S + top_off, S + bar_off, &parts, nullptr, 0,
                                   nullptr, B->stream))
@@ -3391,7 +3446,7 @@ extern "C" int lcg_batch_reshape(lcg_batch *B, const lcg_shape *shape, char *err
     }
     const size_t old_scratch = scratch_ints(*B);
     apply_shape(*B, fs, ts);
-    HIPCHECK(upload_deal(*B));
+    HIPCHECK(prepare_fills(*B));
     const size_t new_scratch = scratch_ints(*B);
     if (new_scratch > old_scratch) {
         HIPCHECK(hipFree(B->d_scratch));

@@ -131,8 +131,6 @@ typedef struct {
     int32_t exclusion;       // --exclusion: score of one excluded block
     int32_t sl_stride;       // ints of global scratch per (workgroup, wave) of the
                              // fill with --struct-local
-    int32_t band;            // general fill: pool ints of the band fill, which takes the
-                             // pairs that need no more (0: no band fill)
     int32_t band_lds;        // band fill: LDS offset (ints, even) of its part of the header
     int32_t dealt;           // band fill: workgroups with a pair of their own to start
     int32_t dealt_pairs;     // with, and the pairs they have; the others are queued
@@ -149,9 +147,14 @@ typedef struct {
 // The launches of a run: general fill, band fill, top level / traceback.
 // deal (device): 3 per workgroup of the band fill below bp.dealt: place in
 // the work order, member, members; null: all workgroups share the first pair.
+// rest (device): the pairs of the general fill where the band fill has others
+// (fill.bp.npairs of them, longest first; null: the work order); its arrival
+// counters follow those of the batch's pairs.  side, fork, join (a stream and two
+// events of the batch, or null): the general fill runs beside the band fill.
 typedef struct {
     LaunchPart fill, band, top;
-    const int32_t *deal;
+    const int32_t *deal, *rest;
+    void *side, *fork, *join;
 } LaunchParts;
 
 // LDS ints of a region of the band fill: rows of CW columns per group, G

@@ -109,15 +109,31 @@ def test_many_pairs_dealt(monkeypatch):
     assert _results(texts, pa, monkeypatch, None) == _results(texts, pa, monkeypatch, "0")
 
 
-def test_many_pairs_dealt_after_wide_ones(monkeypatch):
-    """The same with pairs before it in the work order that are too wide for the
-    band fill (no trace band: 134 columns and more)."""
+@pytest.mark.parametrize("short", [2, 8, 24], ids=["3", "31", "279"])
+def test_mixed_batches(short, monkeypatch):
+    """Pairs for both fills, which run side by side (no trace band: 134 columns
+    and more are too wide for the band fill), with fewer pairs than CUs, where
+    several workgroups share a pair of either, and with more, where the wide ones
+    come first in the work order: eagerly, as a graph replayed between other
+    runs, one pair per launch and without allocations."""
     big = _texts([140, 133, 127, 125], 980, span=150)
-    t = _texts([20 + k for k in range(24)], 990)
-    texts = [(big[0], big[1]), (big[1], big[0]), (big[2], big[3])] + [(t[a], t[b]) for a in range(24) for b in range(a)]
+    t = _texts([20 + k for k in range(short)], 990)
+    texts = [(big[0], big[1]), (big[1], big[0])][:1 if short == 2 else 2] + [(big[2], big[3])]
+    texts += [(t[a], t[b]) for a in range(short) for b in range(a)]
     pa = api.locarna_params(max_bp_span=150, min_trace_prob=0.0)
-    assert len(texts) > 256 and _shared(texts, pa)
-    assert _results(texts, pa, monkeypatch, None) == _results(texts, pa, monkeypatch, "0")
+    assert _shared(texts, pa)
+    ref = _results(texts, pa, monkeypatch, "0")
+    monkeypatch.delenv("LCG_FIXED_COLS")
+    B = api.Batch([api.Pair(a, b, pa) for a, b in texts])
+    for mode in (0, 2, 2, 0, 2, 1):
+        print("mode", mode, flush=True)
+        B.run(mode=mode)
+        assert [(B.score(k), B.alignment(k), B.D(k)) for k in range(len(texts))] == ref, mode
+    B.run_noalloc()
+    assert [(B.score(k), B.alignment(k), B.D(k)) for k in range(len(texts))] == ref
+    B.run(mode=0, count=True)
+    assert [B.score(k) for k in range(len(texts))] == [x[0] for x in ref]
+    B.destroy()
 
 
 def test_one_pair_per_launch():

@@ -63,20 +63,24 @@ def _works(rng, n, kind):
 @pytest.mark.parametrize("npairs", [1, 2, 30, 255, 256, 257, 300, 2016])
 @pytest.mark.parametrize("first", [0, 1, 40, 400])
 def test_dealt_workgroups_are_resident(kind, npairs, first):
-    """`first` pairs that cannot be split (too wide for the band fill) come
-    before those that can."""
+    """`first` pairs of the other fill (too wide for the band fill) and as many
+    that cannot be split come before those that can."""
     rng = random.Random(7 * npairs + first)
     for slots in (256, 64):
         for meet in (0.14, 0.08):
             work = _works(rng, npairs, kind)
-            most = [1 if q < first else rng.randint(2, 16) for q in range(npairs)]
+            most = [q // first if q < 2 * first else rng.randint(2, 16) for q in range(npairs)]
             K, dealt = api.deal_workgroups(work, most, slots, meet)
-            assert all(1 <= k <= m for k, m in zip(K, most))
-            assert all(k == 1 for k in K[dealt:])
+            assert all(min(1, m) <= k <= m for k, m in zip(K, most))
+            assert all(k <= 1 for k in K[dealt:])
             used = sum(K[:dealt])
-            assert used <= slots and (dealt == npairs or used < slots)
-            if npairs < slots:
+            assert used <= slots and (sum(K[dealt:]) == 0 or used < slots)
+            if sum(m > 0 for m in most) < slots:
                 assert dealt == npairs
+            own = [q for q in range(npairs) if most[q]]
+            if not own:
+                continue
+            work, K, dealt = [work[q] for q in own], [K[q] for q in own], sum(q < dealt for q in own)
 
             def span(K, dealt):  # the dealt pairs' slowest, the others spread over the rest
                 t = [w * (1 + meet * (k - 1)) / k for w, k in zip(work, K)]
@@ -84,7 +88,7 @@ def test_dealt_workgroups_are_resident(kind, npairs, first):
                 for x in t[dealt:]:
                     load[load.index(min(load))] += x
                 return max(t[:dealt] + load)
-            assert span(K, dealt) <= 1.2 * span([1] * npairs, 0)
+            assert span(K, dealt) <= 1.2 * span([1] * len(own), 0)
 
 
 def test_pf_regions_at_the_edge_of_the_pool():
