@@ -1498,12 +1498,12 @@ int band_members(const PairDesc &d, int pool) {
 // members.  The pairs of the general fill go to `rest`.
 //
 // The two fills run side by side, so the workgroups that wait for others, of
-// either, are together at most one per CU: with fewer pairs than CUs a pair of
-// the general fill keeps its s.K; else it has one, which waits for nobody, and
-// the general fill's grid leaves room for the dealt ones.  That grid: one
-// workgroup per pair or three times the share of the CUs that its pairs' work
-// asks for (a wide pair's work takes two to three times as long); what is too
-// much the band fill's queue gets later.
+// either, are together at most one per CU.  Pairs of the general fill that have
+// s.K > 1 keep them.  With one each, which waits for nobody, the band fill
+// deals the CUs that are left by the general fill's share of the work (three
+// times its estimate: a wide pair's work takes two to three times as long) or
+// by one workgroup per pair; the general fill then takes all that were not
+// dealt where the band fill queues no pairs, else its share.
 void deal_pairs(lcg_batch &B, const FillShape &s) {
     const int np = B.npairs;
     std::vector<int> K(np, 1);
@@ -1520,12 +1520,16 @@ void deal_pairs(lcg_batch &B, const FillShape &s) {
         rest_work += work[q];
     }
     const int nrest = (int)B.rest.size();
+    const int share =
+        nrest ? std::max(1, std::min(std::min(nrest, B.cus - 1),
+                                     (int)(B.cus * 3 * rest_work / std::max(1.0, total + 2 * rest_work))))
+              : 0;
     int dealt = np < B.cus ? np : 0;
     if (s.band_K > 0) {
         if (s.band_K > 1) dealt = np;  // band_K * np workgroups at most one per CU
         for (int q = 0; q < np; ++q) K[q] = most[q] ? s.band_K : 0;
     } else if (nrest < np) {
-        dealt = deal_workgroups(work, most, B.cus - (s.K > 1 ? nrest * s.K : nrest ? 1 : 0), 0.14, K);
+        dealt = deal_workgroups(work, most, B.cus - (s.K > 1 ? nrest * s.K : share), 0.14, K);
     }
     B.deal.clear();
     for (int q = 0; q < dealt; ++q)
@@ -1538,7 +1542,7 @@ void deal_pairs(lcg_batch &B, const FillShape &s) {
     B.rest_grid = s.K > 1 ? nrest * s.K : alone;
     B.parts.fill.grid = B.rest_grid;
     if (s.K == 1 && nrest > 0 && nrest < np)
-        B.parts.fill.grid = std::max(1, std::min({alone, B.cus - wgs, (int)(3 * B.cus * rest_work / total) + 1}));
+        B.parts.fill.grid = std::max(1, std::min({alone, B.cus - wgs, dealt == np ? alone : share}));
     if (nrest == np) B.rest.clear();
 }
 
