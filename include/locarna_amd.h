@@ -555,7 +555,8 @@ int lcg_fold_run_limited(const char *const *seqs, int32_t count, const lcg_fold_
                          int32_t polls, lcg_fold **out, char *err, int errlen);
 /* How lcg_fold_run would run sequences of these lengths on a device of `cus`
  * CUs (host logic, no counterpart in the reference): workgroups of each,
- * chunks of 64 cells per batch of each and the LDS bytes these lay out.
+ * chunks of 64 cells per batch of each (0: the kernel for short sequences) and
+ * the LDS bytes these lay out.
  * Returns the LDS bytes of a workgroup. */
 int64_t lcg_fold_plan(const int32_t *lens, int32_t count, int32_t cus, int32_t *members, int32_t *chunks,
                       int64_t *lds);

@@ -23,10 +23,10 @@
 #include "host.hpp"
 #include "locarna_amd.h"
 
-extern "C" size_t lcg_fold_lds_bytes(int nmax, int nch);
+extern "C" size_t lcg_fold_lds_bytes(int nmax, int nch, int W);
 extern "C" int lcg_launch_fold(const FoldDesc *descs, const signed char *codes, const double *tabs, double *mats,
                                double *outs, double *zout, int *counters, int *status, const int *seq_of, int grid,
-                               int polls, int nmax, int nch, hipStream_t stream);
+                               int polls, int nch, size_t lds, hipStream_t stream);
 
 struct lcg_fold {
     lcg_fold_params p{};
@@ -108,8 +108,13 @@ signed char code_of(char c) {
 // 2.79 ms on several, one of 75 nt 1.10 and 1.17 ms (a barrier per diagonal
 // takes longer than the cells it divides).  Longer ones get one per 64 cells
 // as far as the CUs go: two of 700-800 nt 26.8 ms against 121 ms.  `single`:
-// one for every sequence.
-std::vector<int> deal_workgroups(std::vector<FoldDesc> &descs, int cus, int nmax, bool single, int &nch) {
+// one for every sequence.  lds: bytes of a workgroup.  nch 0: lcg_fold_short,
+// where the matrices of all sequences fit the LDS (up to 52 nt, to 64 with a
+// span limit) and every sequence has a CU to itself (else two share one).
+std::vector<int> deal_workgroups(std::vector<FoldDesc> &descs, int cus, bool single, int &nch, size_t &lds) {
+    const size_t limit = 160 * 1024 - 1024;
+    int nmax = 0;
+    for (const FoldDesc &d : descs) nmax = std::max(nmax, d.n);
     const int count = (int)descs.size();
     auto chunks = [&](const FoldDesc &d) { return std::max(1, (d.n + 63) / 64); };
     int cap = 1;
@@ -121,7 +126,7 @@ std::vector<int> deal_workgroups(std::vector<FoldDesc> &descs, int cus, int nmax
             cap = c;
         }
     nch = cap > 1 || nmax <= 64 ? 1 : nmax <= 128 ? 2 : 4;
-    while (nch > 1 && lcg_fold_lds_bytes(nmax, nch) > 160 * 1024 - 1024) nch /= 2;
+    while (nch > 1 && lcg_fold_lds_bytes(nmax, nch, 0) > limit) nch /= 2;
     std::vector<int> by_len(count), out;
     for (int k = 0; k < count; ++k) by_len[k] = k;
     std::stable_sort(by_len.begin(), by_len.end(), [&](int a, int b) { return descs[a].n > descs[b].n; });
@@ -132,6 +137,12 @@ std::vector<int> deal_workgroups(std::vector<FoldDesc> &descs, int cus, int nmax
             out.push_back(m);
         }
     }
+    lds = 0;
+    for (const FoldDesc &d : descs) lds = std::max(lds, lcg_fold_lds_bytes(d.n, 0, d.W));
+    if (nmax <= 64 && lds <= limit && count <= cus)
+        nch = 0;
+    else
+        lds = lcg_fold_lds_bytes(nmax, nch, 0);
     return out;
 }
 
@@ -148,19 +159,21 @@ extern "C" int64_t lcg_fold_plan(const int32_t *lens, int32_t count, int32_t cus
                                  int64_t *lds) {
     if (!lens || count < 1 || cus < 1 || !members || !chunks || !lds) return LCG_E_ARG;
     std::vector<FoldDesc> descs(count);
-    int nmax = 0, nch = 4;
+    int nch = 4;
+    size_t all = 0;
     for (int k = 0; k < count; ++k) {
         if (lens[k] < 0 || lens[k] > LCG_FOLD_MAX_LEN) return LCG_E_ARG;
         descs[k].n = lens[k];
-        nmax = std::max(nmax, lens[k]);
+        descs[k].W = std::max(1, lens[k]);
     }
-    deal_workgroups(descs, cus, nmax, false, nch);
+    deal_workgroups(descs, cus, false, nch, all);
     for (int k = 0; k < count; ++k) {
-        members[k] = descs[k].K;
-        chunks[k] = lcg_fold_chunks(lens[k], descs[k].K, nch);
-        lds[k] = (int64_t)lcg_fold_lds_bytes(lens[k], chunks[k]);
+        const FoldDesc &d = descs[k];
+        members[k] = d.K;
+        chunks[k] = nch ? lcg_fold_chunks(d.n, d.K, nch) : 0;
+        lds[k] = (int64_t)lcg_fold_lds_bytes(d.n, chunks[k], d.W);
     }
-    return (int64_t)lcg_fold_lds_bytes(nmax, nch);
+    return (int64_t)all;
 }
 
 extern "C" int lcg_fold_run(const char *const *seqs, int32_t count, const lcg_fold_params *params, int32_t device,
@@ -234,10 +247,12 @@ extern "C" int lcg_fold_run_limited(const char *const *seqs, int32_t count, cons
     if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device)) != hipSuccess)
         return hip_fail(e);
     int nch = 4;
-    std::vector<int> seq_of = deal_workgroups(descs, cus, nmax, false, nch);
+    size_t lds = 0;
+    std::vector<int> seq_of = deal_workgroups(descs, cus, false, nch, lds);
     DevBuf dd, dc, dt, dm, dout, dz, db, ds;
     if ((e = hipMalloc(&dd.p, sizeof(FoldDesc) * count)) || (e = hipMalloc(&dc.p, codes.size())) ||
-        (e = hipMalloc(&dt.p, tabs.size() * sizeof(double))) || (e = hipMalloc(&dm.p, mat * sizeof(double))) ||
+        (e = hipMalloc(&dt.p, tabs.size() * sizeof(double))) ||
+        (nch && (e = hipMalloc(&dm.p, mat * sizeof(double)))) ||
         (e = hipMalloc(&dout.p, outd * sizeof(double))) || (e = hipMalloc(&dz.p, count * sizeof(double))) ||
         (e = hipMalloc(&db.p, (count + 1) * sizeof(int))) || (e = hipMalloc(&ds.p, seq_of.size() * sizeof(int))))
         return hip_fail(e);
@@ -245,7 +260,7 @@ extern "C" int lcg_fold_run_limited(const char *const *seqs, int32_t count, cons
         (e = hipMemcpy(dt.p, tabs.data(), tabs.size() * sizeof(double), hipMemcpyHostToDevice)) ||
         (e = hipMemcpy(ds.p, seq_of.data(), seq_of.size() * sizeof(int), hipMemcpyHostToDevice)))
         return hip_fail(e);
-    if ((e = hipMemsetAsync(dm.p, 0, mat * sizeof(double), 0))) return hip_fail(e);
+    if (nch && (e = hipMemsetAsync(dm.p, 0, mat * sizeof(double), 0))) return hip_fail(e);
     hipEvent_t ev0, ev1;
     if ((e = hipEventCreate(&ev0))) return hip_fail(e);
     if ((e = hipEventCreate(&ev1))) {
@@ -273,14 +288,14 @@ extern "C" int lcg_fold_run_limited(const char *const *seqs, int32_t count, cons
             break;
         }
         // arrival counters of the sequences on several workgroups, and the status
-        if ((e = hipMemsetAsync(db.p, 0, (count + 1) * sizeof(int), 0))) {
+        if ((int)seq_of.size() > 2 * count && (e = hipMemsetAsync(db.p, 0, (count + 1) * sizeof(int), 0))) {
             rc = hip_fail(e);
             break;
         }
         (void)hipEventRecord(ev0, 0);
         int lr = lcg_launch_fold((const FoldDesc *)dd.p, (const signed char *)dc.p, (const double *)dt.p,
                                  (double *)dm.p, (double *)dout.p, (double *)dz.p, (int *)db.p, (int *)db.p + count,
-                                 (const int *)ds.p, (int)seq_of.size() / 2, polls ? polls : 1 << 22, nmax, nch, 0);
+                                 (const int *)ds.p, (int)seq_of.size() / 2, polls ? polls : 1 << 22, nch, lds, 0);
         (void)hipEventRecord(ev1, 0);
         if (lr) {
             rc = hip_fail((hipError_t)lr);
@@ -307,7 +322,7 @@ extern "C" int lcg_fold_run_limited(const char *const *seqs, int32_t count, cons
             if (expired) {
                 // the workgroups of a sequence were not resident together (a
                 // busy device): again on one each, where nothing waits
-                seq_of = deal_workgroups(descs, cus, nmax, true, nch);
+                seq_of = deal_workgroups(descs, cus, true, nch, lds);
                 if ((e = hipMemcpy(ds.p, seq_of.data(), seq_of.size() * sizeof(int), hipMemcpyHostToDevice)))
                     rc = hip_fail(e);
                 --attempt;

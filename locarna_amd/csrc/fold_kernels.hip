@@ -39,7 +39,6 @@
 
 namespace {
 
-constexpr int FT = LCG_FOLD_THREADS, NWV = FT / 64;
 constexpr int MAXLOOP = LCG_FOLD_MAXLOOP;
 
 __device__ __forceinline__ int weak(int t) { return (0x72 >> t) & 1; }
@@ -56,25 +55,27 @@ struct Seq {
     __device__ __forceinline__ int pt(int i, int j) const { return ptab[cs[i] * 5 + cs[j]]; }
 };
 
-// The loop terms of a wave, one per lane: lanes 0..3 bulges of two bases and
-// more, lanes 4..31 interior loops, by loop size within each kind.  Wave w
-// has every 16th of the 58 bulges and 435 interior loops.
+// The loop terms of a wave of NWV, one per lane: the first 64 / NWV lanes
+// bulges of two bases and more, then interior loops, by loop size within each
+// kind.  Wave w has every NWV-th of the 58 bulges and 435 interior loops.
 struct Terms {
     int s, l1;     // unpaired bases (99: none), those of the 5' side
     double f;      // factor with two strong pairs, times sigma^-(s + 2)
 };
 
+template <int NWV>
 __device__ __forceinline__ Terms wave_terms(int w, int lane, const double *tabs, double log_sigma) {
     Terms t{99, 0, 0.0};
     int l2 = 0;
-    if (lane < 4) {
+    constexpr int NBU = 64 / NWV;
+    if (lane < NBU) {
         const int e = w + NWV * lane;
         if (e < 2 * (MAXLOOP - 1)) {
             t.s = 2 + e / 2;
             t.l1 = (e & 1) ? t.s : 0;
         }
-    } else if (lane < 32) {
-        int x = w + NWV * (lane - 4), s = 2;
+    } else {
+        int x = w + NWV * (lane - NBU), s = 2;
         while (s <= MAXLOOP && x >= s - 1) x -= s - 1, ++s;
         if (s <= MAXLOOP) {
             t.s = s;
@@ -92,7 +93,7 @@ __device__ __forceinline__ Terms wave_terms(int w, int lane, const double *tabs,
 
 // K workgroups fold a sequence, each the batches of 64 NCH cells of a
 // diagonal that are its own.  The lanes of a wave are the cells of a chunk of
-// 64; the waves of the workgroup split the terms of their sums (every 16th
+// 64; the waves of the workgroup split the terms of their sums (every NWV-th
 // each), so that a load is 64 neighbours, many are in flight, and no lane
 // waits for another; the partial sums meet in LDS, one wave per chunk adds
 // them up and finishes its cells.  The interior loops are summed for the
@@ -104,14 +105,21 @@ __device__ __forceinline__ Terms wave_terms(int w, int lane, const double *tabs,
 // quarter wave per cell with gathered terms and five more sums over the
 // splits: 64 sequences of 60-200 nt, span 100, 5.53 -> 2.45 ms; two of
 // 700-800 nt without a limit 300 -> 26.8 ms; one of 75 nt 1.21 -> 1.10 ms.
-template <int NCH>
+// IN_LDS (short sequences, 8 waves): the matrices are in LDS, and both split sums
+// of the outside pass have a part of their own (two barriers fewer).  One
+// sequence of 20, 30, 40 and 50 nt 0.082, 0.160, 0.252 and 0.357 ms; in global
+// memory with 16 waves 0.162, 0.306, 0.466 and 0.625 (the quarter wave per cell
+// 0.082, 0.200, 0.375 and 0.597), in LDS with 16 waves 0.114, 0.213 and 0.319.
+template <int NCH, int NWV, bool IN_LDS>
 __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const signed char *codes, const double *tabs,
                                          double *mats, double *outs, double *zout, int *counter, int *status,
                                          int polls, double *lds) {
     constexpr int NB = 64 * NCH;  // cells per batch
-    const int n = D.n, W = D.W, S = D.S, K = D.K;
-    double *part = lds;                    // [sum][wave][cell]: M2 or Qmb, interior loops, Qm1b
-    double *T = part + 3 * NWV * NB;       // factor table from the stacks on
+    constexpr int NP = IN_LDS ? 4 : 3, FT = 64 * NWV, NBU = 64 / NWV;
+    const int n = D.n, W = D.W, S = IN_LDS ? n + 2 : D.S, K = NCH == 1 && !IN_LDS ? D.K : 1;
+    double *part = lds + (IN_LDS ? lcg_fold_matrix_doubles(n, W) : 0);  // [sum][wave][cell]: M2 or Qmb, bulges,
+                                                                        // interior loops, (NP 4) Qm1b
+    double *T = part + NP * NWV * NB;      // factor table from the stacks on
     double *Z5 = T + (LCG_FOLD_TAB_HP - LCG_FOLD_TAB_STACK), *Z5b = Z5 + (n + 1);  // n + 1 each
     int *ptab = (int *)(Z5b + (n + 1));    // 25
     unsigned short *list = (unsigned short *)(ptab + 28);  // two buffers of NB: cells that can pair
@@ -136,12 +144,12 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
         ptab[tid] = t;
     }
     const Seq Q{cs, ptab};
-    const Terms tm = wave_terms(wave, lane, tabs, D.log_sigma);
+    const Terms tm = wave_terms<NWV>(wave, lane, tabs, D.log_sigma);
     // place of a term's cell from the cell (i, d) inside and outside
     const int off_in = tm.s < 99 ? -(2 + tm.s) * S + 1 + tm.l1 : 0, off_out = -off_in;
     const double s1 = exp(-D.log_sigma), s2 = s1 * s1, s3 = s2 * s1;
     const size_t sz = (size_t)W * S;
-    double *Qb = mats + D.mat, *QI = Qb + sz, *QU = QI + sz, *Qm = QU + sz, *Qm1 = Qm + sz, *X = Qm1 + sz;
+    double *Qb = IN_LDS ? lds : mats + D.mat, *QI = Qb + sz, *QU = QI + sz, *Qm = QU + sz, *Qm1 = Qm + sz, *X = Qm1 + sz;
     double *ring = X + sz;
     double *M2 = ring, *Y = ring + 3 * (size_t)S;  // inside: 3 and 2 diagonals
     double *U = ring + 5 * (size_t)S, *R = ring + 7 * (size_t)S, *Qbb = ring + 9 * (size_t)S;  // outside: 2, 2, 4
@@ -149,6 +157,8 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
     double *P = outs + D.out, *P2 = P + osz;
     const double *hp = tabs + LCG_FOLD_TAB_HP;
     int passed = 0, buf = 0;
+    if (IN_LDS)
+        for (int x = tid; x < (int)lcg_fold_matrix_doubles(n, W); x += FT) lds[x] = 0.0;
     __syncthreads();
 
     // the cells of batch b of diagonal d that can pair, into a list buffer
@@ -184,7 +194,7 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
     auto loops = [&](int b, int lim, const double *band_u, const double *band_i, int off) {
         const int c = count[buf];
         const unsigned long long in = __ballot(tm.s <= lim);
-        const int nu = __popcll(in & 15), ni = __popcll(in >> 4);
+        const int nu = __popcll(in & ((1 << NBU) - 1)), ni = __popcll(in >> NBU);
         for (int h = 0; 64 * h < c; ++h) {
             const int x = 64 * h + lane;
             const unsigned i = b * NB + list[buf * NB + (x < c ? x : 0)] + 1;
@@ -202,8 +212,9 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
                 return acc;
             };
             double au = 0, ai = 0;
-            if (nu > 0) au = terms(std::integral_constant<int, 4>(), band_u, 0, nu, au);
-            for (int q = 4; q < 4 + ni; q += 14) ai = terms(std::integral_constant<int, 14>(), band_i, q, 4 + ni, ai);
+            for (int q = 0; q < nu; q += 4) au = terms(std::integral_constant<int, 4>(), band_u, q, nu, au);
+            for (int q = NBU; q < NBU + ni; q += 14)
+                ai = terms(std::integral_constant<int, 14>(), band_i, q, NBU + ni, ai);
             part[(NWV + wave) * NB + x] = au;
             part[(2 * NWV + wave) * NB + x] = ai;
         }
@@ -220,7 +231,8 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
     if (wave == 0) make_list(4, member, 0);
     __syncthreads();
     for (int d = 4; d < W; ++d) {
-        const double hs = exp(-(double)(d + 1) * D.log_sigma);
+        const double hs = D.log_sigma == 0 ? 1.0 : exp(-(double)(d + 1) * D.log_sigma);
+        const double hs0 = hp[(d - 1) * 2] * hs, hs1 = hp[(d - 1) * 2 + 1] * hs;  // loaded ahead of the cells
         for (int b = member; b < nbatch && b * NB < n - d; b += K) {
             // partial sums
             double m2[NCH];
@@ -256,7 +268,7 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
                         l += s3 * (tab(LCG_FOLD_TAB_BULGE1 + t * 8 + Q.pt(i + 1, j - 2)) * Qb[x - 3 * S + 1] +
                                    tab(LCG_FOLD_TAB_BULGE1 + t * 8 + Q.pt(i + 2, j - 1)) * Qb[x - 3 * S + 2]);
                     const double mq = d > 5 ? M2[(size_t)((d - 2) % 3) * S + i + 1] : 0.0;
-                    qb = hp[(d - 1) * 2 + wk] * hs + l + mq * tab(LCG_FOLD_TAB_MLC) * tab(LCG_FOLD_TAB_TP + wk) * s2;
+                    qb = (wk ? hs1 : hs0) + l + mq * tab(LCG_FOLD_TAB_MLC) * tab(LCG_FOLD_TAB_TP + wk) * s2;
                     Qb[x] = qb;
                     QI[x] = qb * tab(LCG_FOLD_TAB_GI + wk);
                     QU[x] = qb * tab(LCG_FOLD_TAB_GU + wk);
@@ -269,7 +281,8 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
                 Qm[x] = y + m;
                 M2[(size_t)(d % 3) * S + i] = m;
                 Y[(size_t)(d & 1) * S + i] = y;
-                P[(size_t)i * W + d] = t ? qb * tab(LCG_FOLD_TAB_EXT + weak(t)) : 0.0;
+                // for the exterior loop, which reads rows (from LDS any order)
+                (IN_LDS ? X[x] : P[(size_t)i * W + d]) = t ? qb * tab(LCG_FOLD_TAB_EXT + weak(t)) : 0.0;
             }
             buf ^= 1;
             if (nb != member) __syncthreads();
@@ -288,6 +301,7 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
     // are taken at once.
     for (int x = tid; x <= n; x += FT) Z5[x] = Z5b[x] = 0.0;
     __syncthreads();
+    auto ext = [&](int i, int d) { return IN_LDS ? X[(size_t)d * S + i] : P[(size_t)i * W + d]; };
     if (wave == 0) {
         double z = 1.0;  // Z5(k0 - 1)
         if (lane == 0) Z5[0] = 1.0;
@@ -308,7 +322,7 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const int e = j - k0 - k;
-                    if (j <= n && e >= 4 && e < W && k0 + k <= n) f += zk[k] * P[(size_t)(k0 + k) * W + e];
+                    if (j <= n && e >= 4 && e < W && k0 + k <= n) f += zk[k] * ext(k0 + k, e);
                 }
                 if (j <= n) Z5[j] += f;
             }
@@ -324,7 +338,7 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const int m = m0 - k, e = j - m - 1;  // row m + 1
-                    if (m >= 0 && j <= n && e >= 4 && e < W) f[k] += zb * P[(size_t)(m + 1) * W + e];
+                    if (m >= 0 && j <= n && e >= 4 && e < W) f[k] += zb * ext(m + 1, e);
                 }
             }
 #pragma unroll
@@ -372,9 +386,12 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
                 for (int h = 0; h < NCH; ++h) q2[h] += x[64 * h] * y[64 * h];
             }
             loops(b, min(MAXLOOP, W - 3 - d), QU + (size_t)d * S, QI + (size_t)d * S, off_out);
-            // the sums of the splits share the first third in turn
+            // with three parts the sums of the splits share the first in turn
 #pragma unroll
             for (int h = 0; h < NCH; ++h) part[wave * NB + 64 * h + lane] = q1[h];
+            if (NP == 4)
+#pragma unroll
+                for (int h = 0; h < NCH; ++h) part[(3 * NWV + wave) * NB + 64 * h + lane] = q2[h];
             __syncthreads();
             double qmb = 0, lu = 0, li = 0;
             const int c = 64 * wave + lane, a = b * NB + c + 1, e = a + d;
@@ -388,15 +405,17 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
             }
             const int nb = b + K < nbatch && (b + K) * NB < n - d ? b + K : member;
             if (wave == NWV - 1) make_list(nb == member ? d - 1 : d, nb, buf ^ 1);
-            __syncthreads();
+            if (NP == 3) {
+                __syncthreads();
 #pragma unroll
-            for (int h = 0; h < NCH; ++h) part[wave * NB + 64 * h + lane] = q2[h];
-            __syncthreads();
+                for (int h = 0; h < NCH; ++h) part[wave * NB + 64 * h + lane] = q2[h];
+                __syncthreads();
+            }
             if (mine) {
                 const size_t x = (size_t)d * S + a;
                 const bool up = a >= 2, right = e < n;
                 const double u = qmb + (up && d + 1 < W ? s1 * U[(size_t)((d + 1) & 1) * S + a - 1] : 0.0);
-                const double qm1b = total(0, c) + u;
+                const double qm1b = total(NP == 4 ? 3 : 0, c) + u;
                 const double sb = right && d + 1 < W ? s1 * R[(size_t)((d + 1) & 1) * S + a] : 0.0;
                 double xv = qmb;
                 if (up && right && d + 2 < W) {
@@ -447,40 +466,57 @@ __device__ __forceinline__ void fold_seq(const FoldDesc &D, int member, const si
     }
 }
 
-extern "C" __global__ __launch_bounds__(FT) void lcg_fold_seqs(const FoldDesc *descs, const signed char *codes,
-                                                               const double *tabs, double *mats, double *outs,
-                                                               double *zout, int *counters, int *status,
-                                                               const int *seq_of, int polls, int nch) {
+extern "C" __global__ __launch_bounds__(LCG_FOLD_THREADS) void lcg_fold_seqs(
+    const FoldDesc *descs, const signed char *codes, const double *tabs, double *mats, double *outs, double *zout,
+    int *counters, int *status, const int *seq_of, int polls, int nch) {
+    constexpr int NWV = LCG_FOLD_THREADS / 64;
     extern __shared__ double lds[];
     const int sq = seq_of[2 * blockIdx.x], member = seq_of[2 * blockIdx.x + 1];
     const FoldDesc D = descs[sq];
     const int chunks = lcg_fold_chunks(D.n, D.K, nch);
     if (chunks == 1)
-        fold_seq<1>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
+        fold_seq<1, NWV, false>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
     else if (chunks == 2)
-        fold_seq<2>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
+        fold_seq<2, NWV, false>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
     else
-        fold_seq<4>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
+        fold_seq<4, NWV, false>(D, member, codes, tabs, mats, outs, zout + sq, counters + sq, status, polls, lds);
 }
 
-extern "C" size_t lcg_fold_lds_bytes(int nmax, int nch) {
-    const int nb = 64 * nch;
-    const size_t doubles = 3 * NWV * nb + (LCG_FOLD_TAB_HP - LCG_FOLD_TAB_STACK) + 2 * (nmax + 1);
+// Short sequences, one workgroup each, the matrices in LDS: a diagonal has few
+// terms, so half the waves (fewer partial sums to add up, shorter barriers).
+extern "C" __global__ __launch_bounds__(LCG_FOLD_SHORT_THREADS) void lcg_fold_short(
+    const FoldDesc *descs, const signed char *codes, const double *tabs, double *outs, double *zout,
+    const int *seq_of) {
+    extern __shared__ double lds[];
+    const int sq = seq_of[2 * blockIdx.x];
+    const FoldDesc D = descs[sq];
+    fold_seq<1, LCG_FOLD_SHORT_THREADS / 64, true>(D, 0, codes, tabs, nullptr, outs, zout + sq, nullptr, nullptr, 0, lds);
+}
+
+// LDS bytes of a workgroup; nch 0: of lcg_fold_short for a band of W.
+extern "C" size_t lcg_fold_lds_bytes(int nmax, int nch, int W) {
+    const size_t nb = nch ? 64 * nch : 64;
+    const size_t sums = nch ? 3 * (LCG_FOLD_THREADS / 64) * nb
+                            : 4 * (LCG_FOLD_SHORT_THREADS / 64) * nb + lcg_fold_matrix_doubles(nmax, W);
+    const size_t doubles = sums + (LCG_FOLD_TAB_HP - LCG_FOLD_TAB_STACK) + 2 * (nmax + 1);
     return doubles * sizeof(double) + 28 * sizeof(int) + 4 * nb * sizeof(unsigned short) + 2 * sizeof(int) +
            (size_t)(nmax + 2);
 }
 
 // grid workgroups: sequence and member of each in seq_of; polls: bound of the
-// waits between the members of a sequence; nch 1, 2 or 4.
+// waits between the members of a sequence; nch 1, 2 or 4, 0: lcg_fold_short;
+// lds: bytes.
 extern "C" int lcg_launch_fold(const FoldDesc *descs, const signed char *codes, const double *tabs, double *mats,
                                double *outs, double *zout, int *counters, int *status, const int *seq_of, int grid,
-                               int polls, int nmax, int nch, hipStream_t stream) {
-    const size_t lds = lcg_fold_lds_bytes(nmax, nch);
-    if (hipError_t e = hipFuncSetAttribute((const void *)lcg_fold_seqs, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)lds))
-        return (int)e;
+                               int polls, int nch, size_t lds, hipStream_t stream) {
+    const void *kernel = nch ? (const void *)lcg_fold_seqs : (const void *)lcg_fold_short;
+    if (hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)) return (int)e;
     if (grid <= 0) return 0;
-    hipLaunchKernelGGL(lcg_fold_seqs, dim3(grid), dim3(FT), lds, stream, descs, codes, tabs, mats, outs, zout, counters,
-                       status, seq_of, polls, nch);
+    if (nch)
+        hipLaunchKernelGGL(lcg_fold_seqs, dim3(grid), dim3(LCG_FOLD_THREADS), lds, stream, descs, codes, tabs, mats, outs,
+                           zout, counters, status, seq_of, polls, nch);
+    else
+        hipLaunchKernelGGL(lcg_fold_short, dim3(grid), dim3(LCG_FOLD_SHORT_THREADS), lds, stream, descs, codes, tabs, outs,
+                           zout, seq_of);
     return (int)hipGetLastError();
 }

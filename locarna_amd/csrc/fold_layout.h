@@ -19,6 +19,8 @@
 #ifndef LOCARNA_AMD_FOLD_LAYOUT_H
 #define LOCARNA_AMD_FOLD_LAYOUT_H
 
+#include <stddef.h>
+
 #define LCG_FOLD_MAXLOOP 30
 // factor table (doubles): Boltzmann factors of the loop terms
 #define LCG_FOLD_TAB_LOOP 0       // [l1 * 31 + l2], l1 + l2 >= 2, two strong pairs
@@ -33,6 +35,7 @@
 #define LCG_FOLD_TAB_HP 1100      // [L * 2 + weak]: hairpin of L unpaired bases
 #define LCG_FOLD_MAX_LEN 4096     // longest sequence (Z5 and Z5b live in LDS)
 #define LCG_FOLD_THREADS 1024
+#define LCG_FOLD_SHORT_THREADS 512  // lcg_fold_short
 #define LCG_FOLD_RINGS 16
 #define LCG_FOLD_PAD 1024         // doubles past a sequence's matrices (chunks of 64 cells run past a diagonal)
 
@@ -48,6 +51,12 @@
 LCG_FOLD_HD inline int lcg_fold_chunks(int n, int K, int nch) {
     const int c = K > 1 || n <= 64 ? 1 : n <= 128 ? 2 : 4;
     return c < nch ? c : nch;
+}
+
+// Doubles of a sequence's matrices in LDS (lcg_fold_short): rows of n + 2, and what the lanes past
+// the end of the last row read.
+LCG_FOLD_HD inline size_t lcg_fold_matrix_doubles(int n, int W) {
+    return ((size_t)6 * W + LCG_FOLD_RINGS) * (n + 2) + 64;
 }
 
 struct FoldDesc {

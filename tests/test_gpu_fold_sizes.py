@@ -1,6 +1,6 @@
 """The folding kernel at the edges of its batches and workgroups: lengths
-around 64, 128 and 256 nt (1, 2, 4 chunks of cells a batch) and above (several
-workgroups per sequence), spans below and above the interior-loop limit, alone
+up to 52 nt (matrices in LDS), around 64, 128 and 256 nt (1, 2, 4 chunks of
+cells a batch) and above (several workgroups per sequence), spans below and above the interior-loop limit, alone
 and together (with half as many sequences as CUs and more, the long ones too on
 one workgroup each, with two chunks a batch where Z5 of the longest takes the
 LDS), against the folding oracle (1e-10 absolute on probabilities, as sums of up
@@ -37,13 +37,13 @@ def _check(seqs, span, first=None):
     F.destroy()
 
 
-@pytest.mark.parametrize("n", [5, 9, 10, 11, 40, 63, 64, 65, 127, 128, 129, 192, 255, 256, 257, 321])
+@pytest.mark.parametrize("n", [5, 9, 10, 11, 30, 40, 52, 53, 63, 64, 65, 127, 128, 129, 192, 255, 256, 257, 321])
 @pytest.mark.parametrize("span", [-1, 7, 36, 70])
 def test_one_sequence(n, span):
     _check(_seqs([n], 40 + n), span)
 
 
-@pytest.mark.parametrize("lens", [[1, 4, 64, 65, 128, 129, 250], [300, 12, 90, 64, 257]])
+@pytest.mark.parametrize("lens", [[1, 4, 64, 65, 128, 129, 250], [300, 12, 90, 64, 257], [52, 1, 4, 30, 17, 40]])
 def test_together(lens):
     _check(_seqs(lens, 90), 100)
 

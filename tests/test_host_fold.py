@@ -39,7 +39,7 @@ def test_rnafold_pp_refusals(args, stdin, msg):
 
 @pytest.mark.parametrize("lens", [[75], [64, 128, 256], [300, 700], [65] * 130 + [3700], [65] * 130 + [129, 3602, 1200],
                                   [100] * 300 + [4096, 650], [200] * 255 + [257], [4096] * 5, [64] * 200 + [4096],
-                                  [1, 4096] * 128])
+                                  [1, 4096] * 128, [52, 1, 30], [53, 20], [20] * 256, [20] * 257, [0]])
 def test_plan_fits(lens):
     """Every sequence's part of the LDS is inside what the launch allocates, and
     workgroups that wait for each other are resident together."""
@@ -48,4 +48,5 @@ def test_plan_fits(lens):
     assert max(lds for _, _, lds in plan) <= allocated
     members = [k for k, _, _ in plan]
     assert min(members) >= 1 and (max(members) == 1 or sum(members) <= 256)
-    assert all(c in (1, 2, 4) and (k == 1 or c == 1) for k, c, _ in plan)
+    assert all(c in (1, 2, 4) and (k == 1 or c == 1) for k, c, _ in plan) or {c for _, c, _ in plan} == {0}
+    assert (max(lens) <= 52 and len(lens) <= 256) == (plan[0][1] == 0)
