@@ -55,6 +55,7 @@ struct lcg_pair {
     std::vector<int32_t> blob;
     PairDesc desc;
     int64_t cells = 0;  // DP cells (groups + top level) as a work estimate
+    int band_need = 0;  // PairDesc.band_need
     int ecap = 0;       // max columns of a group region (E vector)
     std::vector<int> entry_of;  // arc match -> candidate entry
     // prepared for the device compaction (lcg_pair_prepare_device): no arc
@@ -168,15 +169,26 @@ void top_region(const std::vector<int> &mn, const std::vector<int> &mx, int n, i
     top_ints = ((m + 1) + wtop + (n + 1) * wtop + 3) & ~3;
 }
 
-// Whether the band fill can take a pair: band bounds that do not decrease, rows
-// of at most LCG_BAND_COLS columns.
-bool band_rows(const lcg_pair &P) {
+// Pool ints that the band fill needs for a pair: a region of one group (rows al
+// .. below the largest right end of A's arcs with left end al); 0 if it cannot
+// take the pair: a band bound decreases or a row has more than LCG_BAND_COLS
+// columns.
+int band_pool_need(const lcg_pair &P) {
     const std::vector<int> &mn = P.tc->min_cols(), &mx = P.tc->max_cols();
-    if (P.params.struct_local || !std::is_sorted(mn.begin(), mn.end()) || !std::is_sorted(mx.begin(), mx.end()))
-        return false;
-    for (size_t i = 0; i < mn.size(); ++i)
-        if (mx[i] - mn[i] + 1 > LCG_BAND_COLS) return false;
-    return true;
+    if (P.params.struct_local || !std::is_sorted(mn.begin(), mn.end()) || !std::is_sorted(mx.begin(), mx.end())) return 0;
+    std::vector<int> coff(mn.size() + 1, 0);
+    int w = 0, cells = 0;
+    for (size_t i = 0; i < mn.size(); ++i) {
+        const int x = std::max(0, mx[i] - mn[i] + 1);
+        w = std::max(w, x);
+        coff[i + 1] = coff[i] + x;
+    }
+    if (w > LCG_BAND_COLS) return 0;
+    for (int a = 0; a < P.bA->num_bps(); ++a) {
+        const Arc &x = P.bA->arc(a);
+        cells = std::max(cells, coff[x.right] - coff[x.left]);
+    }
+    return LCG_BAND_REGION(1, w <= 64 ? 64 : 128, cells);
 }
 
 // Order of the arcs of B within a fill block (the arc matches of one arc of
@@ -408,7 +420,8 @@ void pack(lcg_pair &P) {
     if (t != nam) throw failure("internal: arc match right-end lists incomplete");
     // fill-D candidate list: the arc matches of row i (right end in A),
     // blocks of one arc of A by left end p descending, in fill order in a block
-    const bool band = band_rows(P);
+    P.band_need = band_pool_need(P);
+    const bool band = P.band_need != 0;
     const std::vector<int> place = fill_order(bB, m, band);
     std::vector<std::vector<int>> by_rightA(n + 1);
     for (int k = 0; k < nam; ++k) by_rightA[bA.arc(ams.arcmatch(k).arcA).right].push_back(k);
@@ -575,7 +588,8 @@ void prepare_compaction_inputs(lcg_pair &P) {
     side(bB, *P.B, m, false);
     c.fordB = reserve(img, NB);
     {
-        const std::vector<int> place = fill_order(bB, m, band_rows(P));
+        P.band_need = band_pool_need(P);
+        const std::vector<int> place = fill_order(bB, m, P.band_need != 0);
         for (int b = 0; b < NB; ++b) img[c.fordB + place[b]] = b;
     }
     c.band = reserve(img, 2 * (size_t)(n + 1));
@@ -1273,7 +1287,7 @@ int device_count_and_layout(lcg_batch &B, lcg_pair *const *pairs, int npairs, st
         int ncells = 0;
         for (int i = 0; i <= d.n; ++i) ncells += std::max(0, P.tc->max_col(i) - P.tc->min_col(i) + 1);
         d.ncells = ncells;
-        size[k] = layout_pair(d, d.n, d.m, ncells, d.ngroups, d.nam, d.nfblk, band_rows(P));
+        size[k] = layout_pair(d, d.n, d.m, ncells, d.ngroups, d.nam, d.nfblk, P.band_need != 0);
         d.gmax = S[LCG_CS_GMAX];
         int64_t cells = (int64_t)(((uint64_t)(uint32_t)S[LCG_CS_CELLS + 1] << 32) | (uint32_t)S[LCG_CS_CELLS]);
         top_region(P.tc->min_cols(), P.tc->max_cols(), d.n, d.m, d.wtop, d.top_ints, cells);
@@ -1717,30 +1731,13 @@ extern "C" int lcg_batch_create_shaped(lcg_pair *const *pairs, int32_t npairs, i
             work[k] = P->cells;
         }
     }
-    // pairs the band fill takes (fds 2); the pool must hold a region of one
-    // group (rows al .. below the largest right end of A's arcs with left end al)
+    // pairs the band fill takes
     const char *fc = std::getenv("LCG_FIXED_COLS");
     const bool fixed_cols = !fc || std::atoi(fc) != 0;
     bool band = false;
     for (int k = 0; k < npairs && fixed_cols; ++k) {
-        if (B->descs[k].fds != 2) continue;
-        const lcg_pair &X = *pairs[k];
-        const std::vector<int> &mn = X.tc->min_cols(), &mx = X.tc->max_cols();
-        const int n = X.A->length();
-        std::vector<int> coff(n + 2, 0);
-        int w = 0;
-        for (int i = 0; i <= n; ++i) {
-            const int x = std::max(0, mx[i] - mn[i] + 1);
-            w = std::max(w, x);
-            coff[i + 1] = coff[i] + x;
-        }
-        int cells = 0;
-        for (int a = 0; a < X.bA->num_bps(); ++a) {
-            const Arc &x = X.bA->arc(a);
-            cells = std::max(cells, coff[x.right] - coff[x.left]);
-        }
-        B->descs[k].band_need = LCG_BAND_REGION(1, w <= 64 ? 64 : 128, cells);
-        band = true;
+        B->descs[k].band_need = pairs[k]->band_need;
+        band |= pairs[k]->band_need != 0;
     }
     int max_len = 1, gmax = 4, top_max = 4, nfblk_max = 1;
     for (const PairDesc &d : B->descs) B->sl_max = std::max(B->sl_max, d.slmax);
