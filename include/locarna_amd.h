@@ -213,8 +213,7 @@ typedef struct {
     int32_t top_waves;      /* top level + traceback: waves per workgroup, 1..16 (4) */
     int32_t top_wgs_per_cu; /* top level + traceback: workgroups per CU, 1..4 (4) */
     int32_t pf_waves;       /* LocARNA-P: waves per workgroup, 1..8 (8) */
-    int32_t pf_wg_per_pair; /* LocARNA-P: workgroups per pair, 1..64; 0: two for the largest pairs where
-                               that shortens the estimated makespan, else CUs / pairs */
+    int32_t pf_wg_per_pair; /* LocARNA-P: workgroups per pair, 1..64; 0: chosen per pair by its estimated work */
     int32_t reserved;
 } lcg_shape;
 /* lcg_batch_create with a requested launch shape (NULL: defaults). */

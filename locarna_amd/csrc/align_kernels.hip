@@ -555,14 +555,15 @@ __device__ void fill_group(const Pair &P, int al, int bl, int ar, int br, int W,
 // operands, read together beforehand).  Rows al+1 .. al+3 have no arc terms;
 // they run while the entries of the next four rows are loaded, and every
 // block's entries are loaded while the block before runs.
-// Bound: a wave's instruction stream (about 450 instructions per block of
-// four rows at 4-5 cycles each, most of a row of left ends' waves idle while
-// its longest group runs) and, with many arc terms, the LDS (an atomic of 64
-// lanes on 25 columns takes 8-19 cycles by how the lanes meet, a random
-// gather 10).  The LDS holds the regions of only 7-12 waves per CU.  Against
-// the fixed-column kernel: 2016 pairs of 60-200 nt 53.5 -> 36.6 ms, 120
-// local pairs of 35-149 nt 65.9 -> 18.8 ms (with the pairs dealt by work),
-// four 500-nt pairs 61.9 -> 17.4 ms, one pair of 75 nt 2.10 -> 0.78 ms.
+// Bound: latency with few waves.  A block of four rows is about 450
+// instructions, with many arc terms LDS trips (an atomic of 64 lanes on 25
+// columns takes 8-19 cycles by how the lanes meet, a random gather 10); the LDS
+// holds the regions of 9.5 waves per CU on average (60-200 nt), 8.7 of which
+// have a task, as the tasks of a row of left ends differ in length; vector
+// instructions take 31 % of the issue cycles.  Against the fixed-column kernel:
+// 2016 pairs of 60-200 nt 53.5 -> 36.8 ms, 120 local pairs of 35-149 nt 65.9 ->
+// 17.6 ms (with the pairs dealt by work), four 500-nt pairs 61.9 -> 17.1 ms, one
+// pair of 75 nt 2.10 -> 0.78 ms.
 // Tried and slower or equal: the rows' scalars through the scalar cache
 // (34.9 / 17.8 / 18.2 / 0.84 ms), regions of one size per row (37.3 ms for
 // the first), 128 instead of 256 entries of a row loaded ahead (37.7 ms).

@@ -99,9 +99,11 @@ __device__ __forceinline__ Terms wave_terms(int w, int lane, const double *tabs,
 // them up and finishes its cells.  The interior loops are summed for the
 // cells that can pair only (3 of 8 on random sequences), listed by a wave
 // that has no chunk to finish.
-// Bound: per diagonal the instructions of 16 waves (about 200 each for the
-// interior loops), three trips to the L2 and two barriers: 6-10 us, and with
-// several workgroups 7 us more for the barrier between them.  Against a
+// Bound: the chain of a diagonal, 6-10 us: of about 20,000 cycles with a clock
+// in it (75 nt) the split sums take 3,500 (inside) to 6,600, the loops 5,000,
+// the barrier behind them 3,500, the wave that adds up the parts and finishes
+// the cells 5,000 to 6,300; with several workgroups 7 us more for the barrier
+// between them.  Against a
 // quarter wave per cell with gathered terms and five more sums over the
 // splits: 64 sequences of 60-200 nt, span 100, 5.53 -> 2.45 ms; two of
 // 700-800 nt without a limit 300 -> 26.8 ms; one of 75 nt 1.21 -> 1.10 ms.
